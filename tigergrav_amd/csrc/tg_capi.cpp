@@ -152,6 +152,7 @@ int leaf_call(const tg_params* p, tg_force* f, const int32_t* x, int64_t ns, con
 	a.list = nullptr;
 	a.out = static_cast<double*>(T->out.p);
 	a.nitems = int(ngroups);
+	a.nlist = ngroups * nj;
 	a.wrap = p->ewald ? 1 : 0;
 	a.uniform = 1;
 	a.m = m;

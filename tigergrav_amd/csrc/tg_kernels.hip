@@ -73,6 +73,49 @@ __device__ __forceinline__ int ceil_log2_64(int n) { return n <= 1 ? 0 : 32 - __
 
 __device__ __forceinline__ double wave_xor(double v, int off) { return __shfl_xor(v, off, 64); }
 
+// orders a wave's accesses to its own LDS tile, which no other wave of the work group touches.  The
+// LDS serves a wave's accesses in order, so with several waves only the compiler has to keep them
+// apart.  The wait on the LDS and scalar counter costs little here and lets the loops behind it wait
+// for each LDS read as it comes (a scalar load that may be pending makes every such wait one for
+// all reads: 4% of the far-pair loop); a one-wave group's barrier is that wait.
+template <int NW>
+__device__ __forceinline__ void wave_lds_sync() {
+	if (NW == 1) {
+		__syncthreads();
+	} else {
+		__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+		__builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+		__builtin_amdgcn_wave_barrier();
+		__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+	}
+}
+
+// Leaf kinds: NW waves share an item, each taking a contiguous run of its 64-source tiles; their
+// sums are added in wave order.  [begin, end) of wave w's sources in the list [b, e).
+template <int NW>
+__device__ __forceinline__ int2 wave_share(int b, int e, int w) {
+	if (NW == 1) return make_int2(b, e);
+	const int tiles = (e - b + 63) >> 6;
+	const int per = (tiles + NW - 1) / NW;
+	const int lo = min(int64_t(e), int64_t(b) + int64_t(64) * per * w);
+	const int hi = min(int64_t(e), int64_t(lo) + int64_t(64) * per);
+	return make_int2(lo, hi);
+}
+
+// Waves per leaf item.  One wave's chain of tiles is serial, so few items with long lists leave the
+// chip idle, and on clustered sets the longest lists set the kernel's time.  The waves are raised
+// up to TARGET in all (four rounds of the chip: 256 CUs, 4 SIMDs each, eight waves a SIMD, for the
+// uneven lists to even out), as long as each keeps two tiles or more on average.  Sets of more than
+// TARGET / 2 items (2M particles: 65,000 and more) keep one wave each, whose sums need no second
+// pass.
+static int leaf_waves(int nitems, int64_t sources, int most) {
+	constexpr int64_t TARGET = 32768;
+	const int64_t tiles = (sources / (nitems > 0 ? nitems : 1) + 63) / 64;
+	int w = 1;
+	while (w < most && int64_t(nitems) * (2 * w) <= TARGET && tiles >= 4 * w) w *= 2;
+	return w;
+}
+
 // ---- PP direct -------------------------------------------------------------------------------
 // Spline-softened (GADGET-2 cubic spline, support h) potential and acceleration
 // (src/gravity.cpp:231-287).  Beyond h it is Newton's 1/r.  A leaf item's source list starts with
@@ -155,7 +198,8 @@ __device__ __forceinline__ bool off_big(float ox, float oy, float oz) {
 	return fabsf(ox) >= 1073741824.0f || fabsf(oy) >= 1073741824.0f || fabsf(oz) >= 1073741824.0f;
 }
 
-// one PP item (<= 64 sinks of a leaf against its source list), by one 64-lane work group.
+// one PP item (<= 64 sinks of a leaf against its source list), by one work group of NW waves, each
+// on its own share of the list.
 // Lane = (sink si, phase ph) with P = 64 / ns phases (lanes from P ns on idle), so a leaf of ns
 // sinks keeps P ns of the 64 lanes busy.  A 64-source tile is staged phase-major in LDS: phase ph
 // takes sources ph, ph + P, ... from K = ceil(64 / P) consecutive slots (slots no source fills hold
@@ -171,15 +215,18 @@ __device__ __forceinline__ bool off_big(float ox, float oy, float oz) {
 // carries at most the rounding of the larger offset (2^-24 of it) beside its own.  Periodic tiles
 // with an offset of a quarter box or more (possible only when leaves span that much) keep the
 // exact form, so the wrap-around always picks the nearest image.
-struct PPShared {
+struct PPShared {  // one wave's
 	int4 tile[128];
 	float4 ftile[128];
 	double red[4][64];
 };
 
-template <bool WRAP, bool PHI, bool UNIFORM>
-__device__ __forceinline__ void pp_item(const LeafArgs& A, const int4 it, PPShared& S) {
-	const int lane = threadIdx.x;
+template <int NW, bool WRAP, bool PHI, bool UNIFORM>
+__device__ __forceinline__ void pp_item(const LeafArgs& A, const int4 it, PPShared* SS) {
+	const int lane = threadIdx.x & 63;
+	const int wave = NW == 1 ? 0 : int(threadIdx.x >> 6);
+	PPShared& S = SS[wave];
+	const int2 share = wave_share<NW>(it.z, it.w, wave);
 	const int ns = max(it.y & PP_COUNT_MASK, 1);
 	const int near_len = int(unsigned(it.y) >> PP_NEAR_SHIFT);
 	const int near_end = near_len == PP_NEAR_ALL ? INT_MAX : it.z + near_len;
@@ -208,7 +255,7 @@ __device__ __forceinline__ void pp_item(const LeafArgs& A, const int4 it, PPShar
 	double dax = 0.0, day = 0.0, daz = 0.0, dpp = 0.0;
 	// software pipeline: the next tile's source record (and the list index after it) are loaded
 	// while the current tile is evaluated
-	auto index_at = [&](int b) { return b + lane < it.w ? (A.list ? A.list[b + lane] : b + lane) : -1; };
+	auto index_at = [&](int b) { return b + lane < share.y ? (A.list ? A.list[b + lane] : b + lane) : -1; };
 	auto source_at = [&](int j) {
 		int4 v = pad;  // zero weight
 		if (j >= 0) {
@@ -217,12 +264,12 @@ __device__ __forceinline__ void pp_item(const LeafArgs& A, const int4 it, PPShar
 		}
 		return v;
 	};
-	int next_idx0 = index_at(it.z);
+	int next_idx0 = index_at(share.x);
 	int4 next = source_at(next_idx0);
 	bool next_pad = next_idx0 < 0;
-	int next_idx = index_at(it.z + 64);
-	for (int base = it.z; base < it.w; base += 64) {
-		const int n = min(64, it.w - base);
+	int next_idx = index_at(share.x + 64);
+	for (int base = share.x; base < share.y; base += 64) {
+		const int n = min(64, share.y - base);
 		const bool near = base < near_end;
 		// the staged source as an offset from the centre; a pad sits out of reach (r2 overflows to
 		// infinity, its reciprocal root and weight are zero)
@@ -231,10 +278,10 @@ __device__ __forceinline__ void pp_item(const LeafArgs& A, const int4 it, PPShar
 				__int_as_float(next.w));
 		const unsigned long long bigs = WRAP ? __ballot(!next_pad && off_big(f.x, f.y, f.z)) : 0ull;
 		const bool use_off = item_off && !near && bigs == 0ull;
-		__syncthreads();
+		wave_lds_sync<NW>();
 		S.tile[dst] = next;
 		S.ftile[dst] = f;
-		__syncthreads();
+		wave_lds_sync<NW>();
 		next_pad = next_idx < 0;
 		next = source_at(next_idx);
 		next_idx = index_at(base + 128);
@@ -261,18 +308,20 @@ __device__ __forceinline__ void pp_item(const LeafArgs& A, const int4 it, PPShar
 		dpp += pp;
 		ax = ay = az = pp = 0.f;
 	}
-	// the phases of each sink, added in phase order
+	// the phases of each sink, added in phase order, wave after wave
 	S.red[0][lane] = dax;
 	S.red[1][lane] = day;
 	S.red[2][lane] = daz;
 	S.red[3][lane] = dpp;
 	__syncthreads();
-	if (lane < ns) {
-		for (int q = 1; q < P; q++) {
-			dax += S.red[0][q * ns + lane];
-			day += S.red[1][q * ns + lane];
-			daz += S.red[2][q * ns + lane];
-			dpp += S.red[3][q * ns + lane];
+	if (wave == 0 && lane < ns) {
+		for (int q = 1; q < NW * P; q++) {
+			const PPShared& R = SS[NW == 1 ? 0 : q / P];
+			const int l = (NW == 1 ? q : q % P) * ns + lane;
+			dax += R.red[0][l];
+			day += R.red[1][l];
+			daz += R.red[2][l];
+			dpp += R.red[3][l];
 		}
 		// position units: g = -sum w dx r^-3 = -2^64 sum (w du ru^-3), phi = -2^32 sum (w / ru)
 		const double ms = UNIFORM ? double(A.m) : 1.0;
@@ -285,17 +334,17 @@ __device__ __forceinline__ void pp_item(const LeafArgs& A, const int4 it, PPShar
 }
 
 // one work group per item; the dispatcher hands items out in array order (heaviest first)
-template <bool WRAP, bool PHI, bool UNIFORM>
-__global__ __launch_bounds__(64) void k_pp_direct(LeafArgs A) {
-	__shared__ PPShared S;
-	pp_item<WRAP, PHI, UNIFORM>(A, A.items[blockIdx.x], S);
+template <int NW, bool WRAP, bool PHI, bool UNIFORM>
+__global__ __launch_bounds__(64 * NW) void k_pp_direct(LeafArgs A) {
+	__shared__ PPShared S[NW];
+	pp_item<NW, WRAP, PHI, UNIFORM>(A, A.items[blockIdx.x], S);
 }
 
 // persistent form: as many work groups as the machine keeps resident, each taking the next
 // item from a queue counter (A.queue, zero at launch) until the items run out
-template <bool WRAP, bool PHI, bool UNIFORM>
-__global__ __launch_bounds__(64) void k_pp_direct_queue(LeafArgs A) {
-	__shared__ PPShared S;
+template <int NW, bool WRAP, bool PHI, bool UNIFORM>
+__global__ __launch_bounds__(64 * NW) void k_pp_direct_queue(LeafArgs A) {
+	__shared__ PPShared S[NW];
 	__shared__ int next;
 	for (;;) {
 		__syncthreads();
@@ -303,7 +352,7 @@ __global__ __launch_bounds__(64) void k_pp_direct_queue(LeafArgs A) {
 		__syncthreads();
 		const int k = next;
 		if (k >= A.nitems) break;
-		pp_item<WRAP, PHI, UNIFORM>(A, A.items[k], S);
+		pp_item<NW, WRAP, PHI, UNIFORM>(A, A.items[k], S);
 	}
 }
 
@@ -311,42 +360,71 @@ __global__ void k_zero_counter(int* c) {
 	if (threadIdx.x == 0) c[0] = 0;
 }
 
-hipError_t launch_pp_direct(const LeafArgs& a, bool do_phi, hipStream_t s) {
-	if (a.nitems <= 0) return hipSuccess;
+template <int NW, bool WRAP, bool PHI, bool UNIFORM>
+static void pp_launch(const LeafArgs& a, hipStream_t s) {
 	if (a.queue) {
 		// the counter is cleared by a kernel (not a memset) so the launch sequence stays graph-safe
 		hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, s, a.queue);
 		const int groups = a.nitems < a.resident ? a.nitems : a.resident;
-#define TG_PPQ(W, PH, U) hipLaunchKernelGGL((k_pp_direct_queue<W, PH, U>), dim3(groups), dim3(64), 0, s, a)
-		const bool u = a.uniform != 0;
-		if (a.wrap) {
-			if (do_phi) { if (u) TG_PPQ(true, true, true); else TG_PPQ(true, true, false); }
-			else { if (u) TG_PPQ(true, false, true); else TG_PPQ(true, false, false); }
-		} else {
-			if (do_phi) { if (u) TG_PPQ(false, true, true); else TG_PPQ(false, true, false); }
-			else { if (u) TG_PPQ(false, false, true); else TG_PPQ(false, false, false); }
-		}
-#undef TG_PPQ
-		return hipGetLastError();
+		hipLaunchKernelGGL((k_pp_direct_queue<NW, WRAP, PHI, UNIFORM>), dim3(groups), dim3(64 * NW), 0, s, a);
+	} else {
+		hipLaunchKernelGGL((k_pp_direct<NW, WRAP, PHI, UNIFORM>), dim3(a.nitems), dim3(64 * NW), 0, s, a);
 	}
-#define TG_PP(W, PH, U) hipLaunchKernelGGL((k_pp_direct<W, PH, U>), dim3(a.nitems), dim3(64), 0, s, a)
+}
+
+template <bool WRAP, bool PHI, bool UNIFORM>
+static void pp_waves(const LeafArgs& a, hipStream_t s) {
+	switch (leaf_waves(a.nitems, a.nlist, 8)) {
+		case 1: pp_launch<1, WRAP, PHI, UNIFORM>(a, s); break;
+		case 2: pp_launch<2, WRAP, PHI, UNIFORM>(a, s); break;
+		case 4: pp_launch<4, WRAP, PHI, UNIFORM>(a, s); break;
+		default: pp_launch<8, WRAP, PHI, UNIFORM>(a, s); break;
+	}
+}
+
+hipError_t launch_pp_direct(const LeafArgs& a, bool do_phi, hipStream_t s) {
+	if (a.nitems <= 0) return hipSuccess;
 	const bool u = a.uniform != 0;
 	if (a.wrap) {
-		if (do_phi) { if (u) TG_PP(true, true, true); else TG_PP(true, true, false); }
-		else { if (u) TG_PP(true, false, true); else TG_PP(true, false, false); }
+		if (do_phi) { if (u) pp_waves<true, true, true>(a, s); else pp_waves<true, true, false>(a, s); }
+		else { if (u) pp_waves<true, false, true>(a, s); else pp_waves<true, false, false>(a, s); }
 	} else {
-		if (do_phi) { if (u) TG_PP(false, true, true); else TG_PP(false, true, false); }
-		else { if (u) TG_PP(false, false, true); else TG_PP(false, false, false); }
+		if (do_phi) { if (u) pp_waves<false, true, true>(a, s); else pp_waves<false, true, false>(a, s); }
+		else { if (u) pp_waves<false, false, true>(a, s); else pp_waves<false, false, false>(a, s); }
 	}
-#undef TG_PP
 	return hipGetLastError();
 }
 
 // ---- PC (multipole -> particle) ----------------------------------------------------------------
-template <bool EWALD, bool WRAP>
-__global__ __launch_bounds__(64) void k_pc(LeafArgs A) {
+// The waves of a sink add up: the phases of each wave by cross-lane adds, then the waves in order
+// (wave 0's first NSP lanes hold the sums).  Every lane of the group calls this.
+template <int NW>
+__device__ __forceinline__ void leaf_sums(double& dphi, double* dg, int nsp, int lane, int wave, double (*red)[4][64]) {
+	for (int off = nsp; off < 64; off <<= 1) {
+		dphi += wave_xor(dphi, off);
+		dg[0] += wave_xor(dg[0], off);
+		dg[1] += wave_xor(dg[1], off);
+		dg[2] += wave_xor(dg[2], off);
+	}
+	if (NW == 1) return;
+	if (wave > 0 && lane < nsp) {
+		red[wave - 1][0][lane] = dphi;
+		for (int d = 0; d < 3; d++) red[wave - 1][1 + d][lane] = dg[d];
+	}
+	__syncthreads();
+	if (wave == 0 && lane < nsp)
+		for (int w = 0; w < NW - 1; w++) {
+			dphi += red[w][0][lane];
+			for (int d = 0; d < 3; d++) dg[d] += red[w][1 + d][lane];
+		}
+}
+
+template <int NW, bool EWALD, bool WRAP>
+__global__ __launch_bounds__(64 * NW) void k_pc(LeafArgs A) {
 	const int4 it = A.items[blockIdx.x];
-	const int lane = threadIdx.x;
+	const int lane = threadIdx.x & 63;
+	const int wave = NW == 1 ? 0 : int(threadIdx.x >> 6);
+	const int2 share = wave_share<NW>(it.z, it.w, wave);
 	const int ns = it.y & PP_COUNT_MASK;
 	const int lg = ceil_log2_64(ns);
 	const int nsp = 1 << lg;
@@ -354,12 +432,14 @@ __global__ __launch_bounds__(64) void k_pc(LeafArgs A) {
 	const int si = lane & (nsp - 1);
 	const int ph = lane >> lg;
 	const int4 me = A.sinks[it.x + min(si, ns - 1)];
-	__shared__ float tile[64][20];
+	__shared__ float tiles[NW][64][20];
+	__shared__ double red[NW > 1 ? NW - 1 : 1][4][64];
+	float (*tile)[20] = tiles[wave];
 	float phi = 0.f, g[3] = {0.f, 0.f, 0.f};
 	double dphi = 0.0, dg[3] = {0.0, 0.0, 0.0};
-	for (int base = it.z; base < it.w; base += 64) {
-		const int n = min(64, it.w - base);
-		__syncthreads();
+	for (int base = share.x; base < share.y; base += 64) {
+		const int n = min(64, share.y - base);
+		wave_lds_sync<NW>();
 		if (lane < n) {
 			const float4* src = reinterpret_cast<const float4*>(A.multis + (A.list ? A.list[base + lane] : base + lane));
 #pragma unroll
@@ -371,7 +451,7 @@ __global__ __launch_bounds__(64) void k_pc(LeafArgs A) {
 				tile[lane][4 * q + 3] = v.w;
 			}
 		}
-		__syncthreads();
+		wave_lds_sync<NW>();
 		for (int k = ph; k < n; k += P) {
 			float M[17];
 #pragma unroll
@@ -392,13 +472,8 @@ __global__ __launch_bounds__(64) void k_pc(LeafArgs A) {
 		dg[2] += g[2];
 		phi = g[0] = g[1] = g[2] = 0.f;
 	}
-	for (int off = nsp; off < 64; off <<= 1) {
-		dphi += wave_xor(dphi, off);
-		dg[0] += wave_xor(dg[0], off);
-		dg[1] += wave_xor(dg[1], off);
-		dg[2] += wave_xor(dg[2], off);
-	}
-	if (ph == 0 && si < ns) {
+	leaf_sums<NW>(dphi, dg, nsp, lane, wave, red);
+	if (wave == 0 && ph == 0 && si < ns) {
 		double* o = A.out + 4 * (size_t) (it.x + si);
 		o[0] += dphi;
 		o[1] += dg[0];
@@ -407,14 +482,24 @@ __global__ __launch_bounds__(64) void k_pc(LeafArgs A) {
 	}
 }
 
+template <int NW>
+static void pc_launch(const LeafArgs& a, bool ewald, hipStream_t s) {
+	if (ewald)
+		hipLaunchKernelGGL((k_pc<NW, true, true>), dim3(a.nitems), dim3(64 * NW), 0, s, a);
+	else if (a.wrap)
+		hipLaunchKernelGGL((k_pc<NW, false, true>), dim3(a.nitems), dim3(64 * NW), 0, s, a);
+	else
+		hipLaunchKernelGGL((k_pc<NW, false, false>), dim3(a.nitems), dim3(64 * NW), 0, s, a);
+}
+
 hipError_t launch_pc(const LeafArgs& a, bool ewald, hipStream_t s) {
 	if (a.nitems <= 0) return hipSuccess;
-	if (ewald)
-		hipLaunchKernelGGL((k_pc<true, true>), dim3(a.nitems), dim3(64), 0, s, a);
-	else if (a.wrap)
-		hipLaunchKernelGGL((k_pc<false, true>), dim3(a.nitems), dim3(64), 0, s, a);
-	else
-		hipLaunchKernelGGL((k_pc<false, false>), dim3(a.nitems), dim3(64), 0, s, a);
+	switch (leaf_waves(a.nitems, a.nlist, 8)) {
+		case 1: pc_launch<1>(a, ewald, s); break;
+		case 2: pc_launch<2>(a, ewald, s); break;
+		case 4: pc_launch<4>(a, ewald, s); break;
+		default: pc_launch<8>(a, ewald, s); break;
+	}
 	return hipGetLastError();
 }
 
@@ -424,9 +509,12 @@ hipError_t launch_pc(const LeafArgs& a, bool ewald, hipStream_t s) {
 // Fourier terms, n = 0 term and pi/4 in one table), weighted by the source mass; pairs closer than
 // 1e-6 take the reference's constant 2.8372975 and zero force (its zmask).  Sinks and sources are
 // laid out as in k_pc: 2^lg lanes per sink, the other lane bits split the tile's sources.
-__global__ __launch_bounds__(64) void k_pp_ewald(LeafArgs A) {
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void k_pp_ewald(LeafArgs A) {
 	const int4 it = A.items[blockIdx.x];
-	const int lane = threadIdx.x;
+	const int lane = threadIdx.x & 63;
+	const int wave = NW == 1 ? 0 : int(threadIdx.x >> 6);
+	const int2 share = wave_share<NW>(it.z, it.w, wave);
 	const int ns = it.y & PP_COUNT_MASK;
 	const int lg = ceil_log2_64(ns);
 	const int nsp = 1 << lg;
@@ -434,13 +522,15 @@ __global__ __launch_bounds__(64) void k_pp_ewald(LeafArgs A) {
 	const int si = lane & (nsp - 1);
 	const int ph = lane >> lg;
 	const int4 me = A.sinks[it.x + min(si, ns - 1)];
-	__shared__ int4 tile[64];
+	__shared__ int4 tiles[NW][64];
+	__shared__ double red[NW > 1 ? NW - 1 : 1][4][64];
+	int4* tile = tiles[wave];
 	double dphi = 0.0, dg[3] = {0.0, 0.0, 0.0};
-	for (int base = it.z; base < it.w; base += 64) {
-		const int n = min(64, it.w - base);
-		__syncthreads();
+	for (int base = share.x; base < share.y; base += 64) {
+		const int n = min(64, share.y - base);
+		wave_lds_sync<NW>();
 		if (lane < n) tile[lane] = A.srcs[A.list ? A.list[base + lane] : base + lane];
-		__syncthreads();
+		wave_lds_sync<NW>();
 		float phi = 0.f, g[3] = {0.f, 0.f, 0.f};
 		for (int k = ph; k < n; k += P) {
 			const int4 s = tile[k];
@@ -459,13 +549,8 @@ __global__ __launch_bounds__(64) void k_pp_ewald(LeafArgs A) {
 		dg[1] += g[1];
 		dg[2] += g[2];
 	}
-	for (int off = nsp; off < 64; off <<= 1) {
-		dphi += wave_xor(dphi, off);
-		dg[0] += wave_xor(dg[0], off);
-		dg[1] += wave_xor(dg[1], off);
-		dg[2] += wave_xor(dg[2], off);
-	}
-	if (ph == 0 && si < ns) {
+	leaf_sums<NW>(dphi, dg, nsp, lane, wave, red);
+	if (wave == 0 && ph == 0 && si < ns) {
 		double* o = A.out + 4 * (size_t) (it.x + si);
 		o[0] += dphi;
 		o[1] += dg[0];
@@ -476,7 +561,13 @@ __global__ __launch_bounds__(64) void k_pp_ewald(LeafArgs A) {
 
 hipError_t launch_pp_ewald(const LeafArgs& a, hipStream_t s) {
 	if (a.nitems <= 0) return hipSuccess;
-	hipLaunchKernelGGL(k_pp_ewald, dim3(a.nitems), dim3(64), 0, s, a);
+	switch (leaf_waves(a.nitems, a.nlist, 16)) {
+		case 1: hipLaunchKernelGGL(k_pp_ewald<1>, dim3(a.nitems), dim3(64), 0, s, a); break;
+		case 2: hipLaunchKernelGGL(k_pp_ewald<2>, dim3(a.nitems), dim3(128), 0, s, a); break;
+		case 4: hipLaunchKernelGGL(k_pp_ewald<4>, dim3(a.nitems), dim3(256), 0, s, a); break;
+		case 8: hipLaunchKernelGGL(k_pp_ewald<8>, dim3(a.nitems), dim3(512), 0, s, a); break;
+		default: hipLaunchKernelGGL(k_pp_ewald<16>, dim3(a.nitems), dim3(1024), 0, s, a); break;
+	}
 	return hipGetLastError();
 }
 

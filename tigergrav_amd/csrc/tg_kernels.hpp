@@ -59,6 +59,7 @@ struct LeafArgs {
 	const int* list;
 	double* out;             // 4 doubles per sink
 	int nitems;
+	int64_t nlist;           // sources of all items (their lists' lengths added up)
 	int wrap;                // periodic minimum-image separations (direct kinds)
 	int uniform;             // all source masses equal to m (PP direct sums once, scales at the end)
 	float m;                 // the common mass when uniform

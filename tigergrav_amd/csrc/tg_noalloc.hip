@@ -158,6 +158,7 @@ extern "C" int tg_gravity_PP_direct_noalloc(const tg_params* p, tg_force* f, con
 		a.list = nullptr;
 		a.out = sums;
 		a.nitems = int((ns + 63) / 64);
+		a.nlist = int64_t(a.nitems) * nj;
 		a.wrap = p->ewald ? 1 : 0;
 		a.uniform = 1;
 		a.m = m;

@@ -806,6 +806,7 @@ int Solver::enqueue_solve(bool timed) {
 		la.items = work[k].items.as<int4>();
 		la.list = work[k].list.as<int>();
 		la.nitems = work[k].nitems;
+		la.nlist = work[k].nlist;
 		SCHK(mark(2 * k));
 		if (k == PC_DIRECT || k == PC_EWALD)
 			SCHK(launch_pc(la, k == PC_EWALD, s));
