@@ -7,13 +7,20 @@
 //   periodic:  spline-softened Newton on the nearest image plus the converged Ewald correction
 //              of the periodic Green's function minus 1/r (the function tigergrav's Ewald kernels
 //              truncate, tigergrav/green.hpp:189-286), with its +pi/alpha^2 constant.
-// The Ewald sum is split at alpha = 6: the real-space part runs over the 27 images with
-// |n_i| <= 1 (every omitted image is >= 1.5 away, erfc(9) ~ 1e-37) with a cutoff at r = 1
-// (erfc(6) ~ 2e-17); the Fourier part over 0 < |h|^2 <= 144 (exp(-pi^2 145 / 36) ~ 5e-18),
-// evaluated through structure factors C(h) = sum_j m_j cos(2 pi h.x_j), S(h) = sum_j m_j sin(...),
-// one half-space of h with a factor 2.  Every sum has a fixed order: results are deterministic.
+// The forces' Ewald sum is split at alpha = 12: the real-space part then lives on the nearest image
+// alone within r = 1/2 (every omitted term is below erfc(6) / 0.5 ~ 4e-17), and the Fourier part over
+// 0 < |h|^2 <= 576 (exp(-pi^2 577 / 144) ~ 7e-18) is separable: cos(2 pi h.(x_i - x_j)) summed over the
+// signs of h's components is a product of cosines, so the structure factors are the eight sums
+// T = sum_j m_j {cos, sin}(a x_j) {cos, sin}(b y_j) {cos, sin}(c z_j) per octant vector (a, b, c), eight FMAs each
+// from per-particle tables of {cos, sin}(2 pi k x), k <= 24.  (alpha = 6 with its 27 images and a sincos
+// per vector and particle took 285 ms for 256 sinks of 2M particles.)  The gradient's sum is
+// split at alpha = 6: 27 images with |n_i| <= 1 (every omitted image is >= 1.5 away, erfc(9) ~ 1e-37),
+// cut off at r = 1 (erfc(6) ~ 2e-17); the Fourier part over 0 < |h|^2 <= 144 (exp(-pi^2 145 / 36) ~
+// 5e-18) through structure factors of one half-space of h with a factor 2.
+// Every sum has a fixed order: results are deterministic.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <string>
 #include <vector>
@@ -23,10 +30,15 @@
 
 namespace {
 
-constexpr double kAlpha = 6.0;
+constexpr double kAlphaF = 12.0;  // the forces' split
+constexpr int kHF = 24;           // their highest Fourier index per axis
+constexpr int kHF2 = kHF * kHF;
+constexpr int kZG = 9;            // z indices of one structure-factor task: three tasks cover 0..26
+constexpr int kTab = 3 * kZG;     // table entries per axis, zero past kHF
+constexpr double kAlpha = 6.0;    // the gradient's split
 constexpr int kHMax2 = 144;
-constexpr int kSFChunks = 128;   // particle chunks of the structure-factor pass
-constexpr int kSrcChunks = 64;   // source chunks of the pair pass
+constexpr int kSFChunks = 128;   // the gradient's particle chunks of the structure-factor pass
+constexpr int kSrcChunks = 64;   // and source chunks of the pair pass
 constexpr double kPosInv = 1.0 / 4294967296.0;
 
 thread_local std::string g_direct_err;
@@ -52,45 +64,38 @@ __device__ __forceinline__ void spline64(double r, double h, double& f, double& 
 	}
 }
 
-// the real-space part of the correction for one pair at nearest-image offset x:
-//   U(r0) - sum_{n != 0, r_n < 1} erfc(a r_n)/r_n,  U(r) = erf(a r)/r  (= erfc(a r)/r's n = 0 term minus -1/r)
-// returned as the potential term u and d = (1/r) du/dr per image folded into the gradient.
-__device__ void real_space(const double* x, double& u, double* du) {
-	const double a = kAlpha, two_over_sqrtpi = 1.1283791670955126;
-	u = 0.0;
-	du[0] = du[1] = du[2] = 0.0;
-	for (int i = -1; i <= 1; i++)
-		for (int j = -1; j <= 1; j++)
-			for (int k = -1; k <= 1; k++) {
-				const double y[3] = {x[0] + i, x[1] + j, x[2] + k};
-				const double r2 = y[0] * y[0] + y[1] * y[1] + y[2] * y[2];
-				double val, dr;  // potential term and (1/r) d/dr of it
-				if (i == 0 && j == 0 && k == 0) {
-					const double z = a * sqrt(r2), z2 = z * z;
-					if (z < 0.1) {
-						// erf(z)/r and its (1/r) d/dr as series in z^2
-						const double c = two_over_sqrtpi * a;
-						val = c * (1.0 + z2 * (-1.0 / 3.0 + z2 * (1.0 / 10.0 + z2 * (-1.0 / 42.0 + z2 * (1.0 / 216.0 + z2 * (-1.0 / 1320.0 + z2 / 9360.0))))));
-						dr = c * a * a *
-						     (-2.0 / 3.0 + z2 * (4.0 / 10.0 + z2 * (-6.0 / 42.0 + z2 * (8.0 / 216.0 + z2 * (-10.0 / 1320.0 + z2 * (12.0 / 9360.0 - z2 * 14.0 / 75600.0))))));
-					} else {
-						const double r = sqrt(r2);
-						const double e = erf(z);
-						val = e / r;
-						dr = (-e / r + two_over_sqrtpi * a * exp(-z2)) / r2;
-					}
-				} else {
-					if (r2 >= 1.0) continue;
-					const double r = sqrt(r2), z = a * r;
-					const double ec = erfc(z);
-					val = -ec / r;
-					dr = (ec / r + two_over_sqrtpi * a * exp(-z * z)) / r2;
-				}
-				u += val;
-				du[0] += y[0] * dr;
-				du[1] += y[1] * dr;
-				du[2] += y[2] * dr;
-			}
+// the same inside the softening length, out of line: a handful of pairs in a million, and its erf
+// would hold half the registers of the loop
+__device__ __attribute__((noinline)) void softened_pair64(double r, double h, double& f, double& p) {
+	const double a = kAlphaF, c = 1.1283791670955126 * kAlphaF;
+	const double r2 = r * r, z2 = a * a * r2;
+	spline64(r, h, f, p);
+	double u, d;  // erf(alpha r) / r and -(1/r) d/dr of it
+	if (z2 < 0.01) {  // as series in z^2
+		u = c * (1.0 + z2 * (-1.0 / 3.0 + z2 * (1.0 / 10.0 + z2 * (-1.0 / 42.0 + z2 * (1.0 / 216.0 + z2 * (-1.0 / 1320.0 + z2 / 9360.0))))));
+		d = -c * a * a *
+		    (-2.0 / 3.0 + z2 * (4.0 / 10.0 + z2 * (-6.0 / 42.0 + z2 * (8.0 / 216.0 + z2 * (-10.0 / 1320.0 + z2 * (12.0 / 9360.0 - z2 * 14.0 / 75600.0))))));
+	} else {
+		u = erf(a * r) / r;
+		d = (u - c * exp(-z2)) / r2;
+	}
+	p -= u;
+	f -= d;
+}
+
+// the periodic pair within the cut-off (nearest image at distance r): g = -m dx f, phi = -m p, the
+// spline-softened Newton pair less the Gaussian-smoothed one that the Fourier part sums.  Past h
+// the difference is erfc(alpha r) / r.
+__device__ __forceinline__ void ewald_pair64(double r2, double h, double& f, double& p) {
+	const double a = kAlphaF, c = 1.1283791670955126 * kAlphaF;  // 2 alpha / sqrt(pi)
+	const double r = sqrt(r2), z2 = a * a * r2;
+	if (r >= h) {
+		const double ri = 1.0 / r;
+		p = erfc(a * r) * ri;
+		f = (p + c * exp(-z2)) * (ri * ri);
+		return;
+	}
+	softened_pair64(r, h, f, p);
 }
 
 // the real-space correction's gradient and Hessian for one pair at nearest-image offset x:
@@ -168,65 +173,91 @@ __device__ __forceinline__ void spline64_grad(double r, double h, double& f, dou
 	}
 }
 
-// structure factors of one particle chunk: thread = half-space vector h, block = 64 vectors
-__global__ __launch_bounds__(64) void k_structure(const int4* __restrict__ hv, int nh, const int* __restrict__ x,
+// The forces' structure factors: thread = task (a, b, g), the eight sums of the octant vectors
+// (a, b, 9 g .. 9 g + 8); block = 256 tasks x one particle chunk.  The block makes each particle's
+// tables of (cos, sin)(2 pi k x) together, 75 sincospi a particle (2 k x is exact in FP64: x carries 32
+// fraction bits, so sincospi reduces exactly), and every task takes 76 FP64 operations a particle from
+// them: bound by FP64 arithmetic.  64 FMAs and 9 broadcast LDS reads a particle and task: nine z
+// indices a task balance the two (one index a task would read as often as it multiplies), and their
+// 72 sums fit the registers.
+constexpr int kSFTile = 16;  // particles staged at a time
+__global__ __launch_bounds__(256) void k_structure(const int4* __restrict__ tasks, int nt, const int* __restrict__ x,
 		const float* __restrict__ mass, double m, int64_t n, double* __restrict__ part) {
-	const int t = blockIdx.x * 64 + threadIdx.x;
-	const int64_t per = (n + kSFChunks - 1) / kSFChunks;
+	__shared__ double2 tab[kSFTile][3][kTab];
+	const int t = blockIdx.x * 256 + threadIdx.x;
+	const int4 task = tasks[min(t, nt - 1)];
+	const int64_t per = (n + gridDim.y - 1) / gridDim.y;
 	const int64_t b = int64_t(blockIdx.y) * per, e = min(n, b + per);
-	__shared__ double sx[256][4];
-	const int4 h = t < nh ? hv[t] : make_int4(0, 0, 0, 0);
-	double C = 0.0, S = 0.0;
-	for (int64_t base = b; base < e; base += 256) {
+	double acc[kZG][8];
+#pragma unroll
+	for (int z = 0; z < kZG; z++)
+#pragma unroll
+		for (int q = 0; q < 8; q++) acc[z][q] = 0.0;
+	for (int64_t base = b; base < e; base += kSFTile) {
 		__syncthreads();
-		for (int q = threadIdx.x; q < 256; q += 64) {
-			const int64_t j = base + q;
-			if (j < e) {
-				sx[q][0] = double(x[3 * j]) * kPosInv + 0.5;
-				sx[q][1] = double(x[3 * j + 1]) * kPosInv + 0.5;
-				sx[q][2] = double(x[3 * j + 2]) * kPosInv + 0.5;
-				sx[q][3] = mass ? double(mass[j]) : m;
-			} else {
-				sx[q][0] = sx[q][1] = sx[q][2] = sx[q][3] = 0.0;
+		for (int q = threadIdx.x; q < kSFTile * 3 * kTab; q += 256) {
+			const int p = q / (3 * kTab), axis = q / kTab % 3, k = q % kTab;
+			const int64_t j = base + p;
+			double2 v = make_double2(0.0, 0.0);
+			if (j < e && k <= kHF) {
+				sincospi(2.0 * k * (double(x[3 * j + axis]) * kPosInv + 0.5), &v.y, &v.x);
+				if (axis == 0) {
+					const double mj = mass ? double(mass[j]) : m;
+					v.x *= mj;
+					v.y *= mj;
+				}
+			}
+			tab[p][axis][k] = v;
+		}
+		__syncthreads();
+		const int cnt = int(min<int64_t>(kSFTile, e - base));
+		for (int p = 0; p < cnt; p++) {
+			const double2 X = tab[p][0][task.x], Y = tab[p][1][task.y];
+			const double w[4] = {X.x * Y.x, X.x * Y.y, X.y * Y.x, X.y * Y.y};
+			const double2* zt = &tab[p][2][kZG * task.z];
+#pragma unroll
+			for (int z = 0; z < kZG; z++) {
+				const double2 Z = zt[z];
+#pragma unroll
+				for (int q = 0; q < 4; q++) {
+					acc[z][2 * q] = fma(w[q], Z.x, acc[z][2 * q]);
+					acc[z][2 * q + 1] = fma(w[q], Z.y, acc[z][2 * q + 1]);
+				}
 			}
 		}
-		__syncthreads();
-		const int cnt = int(min<int64_t>(256, e - base));
-		for (int q = 0; q < cnt; q++) {
-			// 2 h.x is exact in FP64 (x carries 32 fraction bits), so sincospi reduces exactly
-			const double arg = 2.0 * (h.x * sx[q][0] + h.y * sx[q][1] + h.z * sx[q][2]);
-			double s, c;
-			sincospi(arg, &s, &c);
-			C = fma(sx[q][3], c, C);
-			S = fma(sx[q][3], s, S);
-		}
 	}
-	if (t < nh) {
-		part[2 * (int64_t(blockIdx.y) * nh + t)] = C;
-		part[2 * (int64_t(blockIdx.y) * nh + t) + 1] = S;
+	if (t < nt) {
+		// element-major within the chunk, so that neighbouring tasks write neighbouring words
+		double* o = part + int64_t(blockIdx.y) * nt * (8 * kZG) + t;
+#pragma unroll
+		for (int z = 0; z < kZG; z++)
+#pragma unroll
+			for (int q = 0; q < 8; q++) o[int64_t(8 * z + q) * nt] = acc[z][q];
 	}
 }
 
-__global__ __launch_bounds__(256) void k_structure_sum(const double* __restrict__ part, int nh, double* __restrict__ cs) {
-	const int t = blockIdx.x * 256 + threadIdx.x;
-	if (t >= nh) return;
-	double C = 0.0, S = 0.0;
-	for (int c = 0; c < kSFChunks; c++) {
-		C += part[2 * (int64_t(c) * nh + t)];
-		S += part[2 * (int64_t(c) * nh + t) + 1];
-	}
-	cs[2 * t] = C;
-	cs[2 * t + 1] = S;
+// the chunks added in order: cs[task][z][8]
+__global__ __launch_bounds__(256) void k_structure_sum(const double* __restrict__ part, int nt, int chunks, double* __restrict__ cs) {
+	const int i = blockIdx.x * 256 + threadIdx.x;
+	if (i >= nt * 8 * kZG) return;
+	double s = 0.0;
+	for (int c = 0; c < chunks; c++) s += part[int64_t(c) * nt * (8 * kZG) + i];
+	cs[int64_t(i % nt) * (8 * kZG) + i / nt] = s;
 }
 
-// pair pass: thread = sink, block = 64 sinks x one source chunk
+// Pair pass: block = one wave, 64 / P sinks x P phases of one source chunk, P a power of two that
+// fills the wave where there are fewer than 64 sinks.  Periodic pairs past the cut-off (r >= 1/2,
+// half of them) are done after the distance.
+template <bool EWALD>
 __global__ __launch_bounds__(64) void k_pairs(const int* __restrict__ x, const float* __restrict__ mass, double m, int64_t n,
-		const int64_t* __restrict__ sinks, int64_t ns, int ewald, double h, double* __restrict__ part) {
-	const int64_t si = int64_t(blockIdx.x) * 64 + threadIdx.x;
+		const int64_t* __restrict__ sinks, int64_t ns, int lanes, double h, double* __restrict__ part) {
+	const int P = 64 / lanes, ph = threadIdx.x / lanes;
+	const int64_t si = int64_t(blockIdx.x) * lanes + threadIdx.x % lanes;
 	const int64_t i = sinks[min(si, ns - 1)];
 	const int xi[3] = {x[3 * i], x[3 * i + 1], x[3 * i + 2]};
-	const int64_t per = (n + kSrcChunks - 1) / kSrcChunks;
+	const int64_t per = (n + gridDim.y - 1) / gridDim.y;
 	const int64_t b = int64_t(blockIdx.y) * per, e = min(n, b + per);
+	const double cut2 = fmax(0.25, h * h);
 	__shared__ int sx[256][3];
 	__shared__ double sm[256];
 	double phi = 0.0, g[3] = {0.0, 0.0, 0.0};
@@ -242,28 +273,29 @@ __global__ __launch_bounds__(64) void k_pairs(const int* __restrict__ x, const f
 		}
 		__syncthreads();
 		const int cnt = int(min<int64_t>(256, e - base));
-		for (int q = 0; q < cnt; q++) {
-			const double dx[3] = {sep(ewald, xi[0], sx[q][0]), sep(ewald, xi[1], sx[q][1]), sep(ewald, xi[2], sx[q][2])};
-			const double mj = sm[q];
-			const double r = sqrt(dx[0] * dx[0] + dx[1] * dx[1] + dx[2] * dx[2]);
+		for (int q = ph; q < cnt; q += P) {
+			const double dx[3] = {sep(EWALD, xi[0], sx[q][0]), sep(EWALD, xi[1], sx[q][1]), sep(EWALD, xi[2], sx[q][2])};
+			const double r2 = dx[0] * dx[0] + dx[1] * dx[1] + dx[2] * dx[2];
+			if (EWALD && r2 >= cut2) continue;
 			double f, p;
-			spline64(r, h, f, p);
-			phi -= mj * p;
-			g[0] -= mj * dx[0] * f;
-			g[1] -= mj * dx[1] * f;
-			g[2] -= mj * dx[2] * f;
-			if (ewald) {
-				double u, du[3];
-				real_space(dx, u, du);
-				phi += mj * u;
-				g[0] -= mj * du[0];
-				g[1] -= mj * du[1];
-				g[2] -= mj * du[2];
-			}
+			if (EWALD)
+				ewald_pair64(r2, h, f, p);
+			else
+				spline64(sqrt(r2), h, f, p);
+			const double mj = sm[q];
+			f *= mj;
+			phi = fma(-mj, p, phi);
+			g[0] = fma(-dx[0], f, g[0]);
+			g[1] = fma(-dx[1], f, g[1]);
+			g[2] = fma(-dx[2], f, g[2]);
 		}
 	}
-	if (si < ns) {
-		double* o = part + 4 * (si * kSrcChunks + blockIdx.y);
+	for (int o = lanes; o < 64; o <<= 1) {
+		phi += __shfl_xor(phi, o, 64);
+		for (int d = 0; d < 3; d++) g[d] += __shfl_xor(g[d], o, 64);
+	}
+	if (ph == 0 && si < ns) {
+		double* o = part + 4 * (si * gridDim.y + blockIdx.y);
 		o[0] = phi;
 		o[1] = g[0];
 		o[2] = g[1];
@@ -271,49 +303,62 @@ __global__ __launch_bounds__(64) void k_pairs(const int* __restrict__ x, const f
 	}
 }
 
-// per sink: pair partials in chunk order, then the Fourier part and the constant
-__global__ __launch_bounds__(64) void k_finish(const int* __restrict__ x, const int64_t* __restrict__ sinks, int64_t ns,
-		const double* __restrict__ part, int ewald, const int4* __restrict__ hv, const double* __restrict__ cs, int nh,
+// Per sink (one block): pair partials, then the Fourier part over the octant vectors, thread by
+// thread, and the constant.  With K = exp(-pi^2 h^2 / alpha^2) / h^2 and every sign of (a, b, c) distinct
+// (half for each zero component), phi = -(8 / pi) sum K C_x C_y C_z, where C = cos_i cos_j + sin_i sin_j per axis;
+// the gradient along an axis takes k (cos_i sin_j - sin_i cos_j) there.
+__global__ __launch_bounds__(256) void k_finish(const int* __restrict__ x, const int64_t* __restrict__ sinks, int chunks,
+		const double* __restrict__ part, int ewald, const int4* __restrict__ tasks, const double* __restrict__ cs, int nt,
 		double mtot, double* __restrict__ out) {
-	const int64_t si = int64_t(blockIdx.x) * 64 + threadIdx.x;
-	if (si >= ns) return;
-	double phi = 0.0, g[3] = {0.0, 0.0, 0.0};
-	for (int c = 0; c < kSrcChunks; c++) {
-		const double* o = part + 4 * (si * kSrcChunks + c);
-		phi += o[0];
-		g[0] += o[1];
-		g[1] += o[2];
-		g[2] += o[3];
-	}
+	__shared__ double2 tab[3][kTab];
+	__shared__ double red[4][256];
+	const int64_t si = blockIdx.x;
+	const int t = threadIdx.x;
+	double v[4] = {0.0, 0.0, 0.0, 0.0};
+	for (int c = t; c < chunks; c += 256)
+		for (int q = 0; q < 4; q++) v[q] += part[4 * (si * chunks + c) + q];
 	if (ewald) {
-		const int64_t i = sinks[si];
-		const double xi[3] = {double(x[3 * i]) * kPosInv + 0.5, double(x[3 * i + 1]) * kPosInv + 0.5,
-				double(x[3 * i + 2]) * kPosInv + 0.5};
-		const double pi = 3.141592653589793, a2 = kAlpha * kAlpha;
-		double fp = 0.0, fg[3] = {0.0, 0.0, 0.0};
-		for (int t = 0; t < nh; t++) {
-			const int4 h = hv[t];
-			const double h2 = double(h.x * h.x + h.y * h.y + h.z * h.z);
-			const double c0 = 2.0 * exp(-pi * pi * h2 / a2) / h2;  // both h and -h
-			double s, c;
-			sincospi(2.0 * (h.x * xi[0] + h.y * xi[1] + h.z * xi[2]), &s, &c);
-			const double C = cs[2 * t], S = cs[2 * t + 1];
-			fp += c0 * (c * C + s * S);
-			const double gg = 2.0 * c0 * (s * C - c * S);
-			fg[0] += h.x * gg;
-			fg[1] += h.y * gg;
-			fg[2] += h.z * gg;
+		if (t < 3 * kTab) {
+			const int axis = t / kTab, k = t % kTab;
+			double2 w = make_double2(0.0, 0.0);
+			if (k <= kHF) sincospi(2.0 * k * (double(x[3 * sinks[si] + axis]) * kPosInv + 0.5), &w.y, &w.x);
+			tab[axis][k] = w;
 		}
-		phi += -fp / pi + mtot * pi / a2;
-		g[0] -= fg[0];
-		g[1] -= fg[1];
-		g[2] -= fg[2];
+		__syncthreads();
+		const double pi = 3.141592653589793;
+		for (int j = t; j < nt * kZG; j += 256) {
+			const int4 task = tasks[j / kZG];
+			const int a = task.x, b = task.y, c = kZG * task.z + j % kZG;
+			const int h2 = a * a + b * b + c * c;
+			if (h2 == 0 || h2 > kHF2) continue;
+			const double K = exp(-pi * pi / (kAlphaF * kAlphaF) * h2) / h2 * (a ? 2.0 : 1.0) * (b ? 2.0 : 1.0) * (c ? 2.0 : 1.0);
+			const double2 X = tab[0][a], Y = tab[1][b], Z = tab[2][c];
+			const double* T = cs + int64_t(j) * 8;  // (cos, sin) of x, y, z from the highest bit down
+			// contract z, then y, then x: P with C, Q with the derivative's sine
+			double Pz[4], Qz[4], PP[2], QP[2], PQ[2];
+			for (int q = 0; q < 4; q++) {
+				Pz[q] = Z.x * T[2 * q] + Z.y * T[2 * q + 1];
+				Qz[q] = Z.x * T[2 * q + 1] - Z.y * T[2 * q];
+			}
+			for (int q = 0; q < 2; q++) {
+				PP[q] = Y.x * Pz[2 * q] + Y.y * Pz[2 * q + 1];
+				QP[q] = Y.x * Pz[2 * q + 1] - Y.y * Pz[2 * q];
+				PQ[q] = Y.x * Qz[2 * q] + Y.y * Qz[2 * q + 1];
+			}
+			v[0] -= K / pi * (X.x * PP[0] + X.y * PP[1]);
+			v[1] += 2.0 * K * a * (X.x * PP[1] - X.y * PP[0]);
+			v[2] += 2.0 * K * b * (X.x * QP[0] + X.y * QP[1]);
+			v[3] += 2.0 * K * c * (X.x * PQ[0] + X.y * PQ[1]);
+		}
 	}
-	double* o = out + 4 * si;
-	o[0] = phi;
-	o[1] = g[0];
-	o[2] = g[1];
-	o[3] = g[2];
+	for (int q = 0; q < 4; q++) red[q][t] = v[q];
+	for (int o = 128; o > 0; o >>= 1) {
+		__syncthreads();
+		if (t < o)
+			for (int q = 0; q < 4; q++) red[q][t] += red[q][t + o];
+	}
+	__syncthreads();
+	if (t < 4) out[4 * si + t] = red[t][0] + (t == 0 && ewald ? mtot * 3.141592653589793 / (kAlphaF * kAlphaF) : 0.0);
 }
 
 // gradient: structure factors C, S (mass weighted) and Cw, Sw (weight weighted), 8 per h
@@ -484,17 +529,23 @@ extern "C" int tg_direct_forces(const tg_params* prm, const int32_t* x, const fl
 		for (int64_t j = 0; j < n; j++) mtot += mass[j];
 	else
 		mtot = prm->m * double(n);
-	// half-space of 0 < |h|^2 <= kHMax2
+	// the structure-factor tasks: octant columns (a, b) in runs of kZG z indices that reach into the sphere
 	std::vector<int4> hv;
-	for (int i = -12; i <= 12; i++)
-		for (int j = -12; j <= 12; j++)
-			for (int k = -12; k <= 12; k++) {
-				const int h2 = i * i + j * j + k * k;
-				if (h2 == 0 || h2 > kHMax2) continue;
-				if (i < 0 || (i == 0 && (j < 0 || (j == 0 && k < 0)))) continue;
-				hv.push_back(make_int4(i, j, k, 0));
-			}
-	const int nh = int(hv.size());
+	if (ewald)
+		for (int g = 0; kZG * g <= kHF; g++)
+			for (int i = 0; i <= kHF; i++)
+				for (int j = 0; j <= kHF; j++)
+					if (i * i + j * j + kZG * g * kZG * g <= kHF2) hv.push_back(make_int4(i, j, g, 0));
+	const int nt = int(hv.size());
+	// Particle chunks of the structure factors: one round of the chip (two blocks of four waves per CU by
+	// its registers), a chunk of 64 particles or more.  Source chunks of the pair pass: 16,384 waves (four rounds of the chip at four
+	// waves a SIMD), a chunk of 512 sources or more.
+	const int sf_chunks = int(std::max<int64_t>(1, std::min<int64_t>(512 / std::max(1, (nt + 255) / 256), n / 64)));
+	int lanes = 1;
+	while (lanes < 64 && lanes < ns) lanes *= 2;
+	const int64_t sblocks = (ns + lanes - 1) / lanes;
+	const int src_chunks = int(std::max<int64_t>(1, std::min<int64_t>((16384 + sblocks - 1) / sblocks, n / 512)));
+	if (sblocks > INT32_MAX || ns > INT32_MAX) return TG_EINVAL;
 	Buf dx, dm, ds, dh, dsf, dcs, dpart, dout;
 	hipStream_t st = nullptr;
 	int rc = TG_OK;
@@ -518,28 +569,32 @@ extern "C" int tg_direct_forces(const tg_params* prm, const int32_t* x, const fl
 		}
 		DCHK(hipMalloc(&ds.p, size_t(ns) * 8));
 		DCHK(hipMemcpyAsync(ds.p, sinks, size_t(ns) * 8, hipMemcpyHostToDevice, st));
-		DCHK(hipMalloc(&dh.p, hv.size() * sizeof(int4)));
-		DCHK(hipMemcpyAsync(dh.p, hv.data(), hv.size() * sizeof(int4), hipMemcpyHostToDevice, st));
-		DCHK(hipMalloc(&dcs.p, size_t(nh) * 16));
 		if (ewald) {
-			DCHK(hipMalloc(&dsf.p, size_t(kSFChunks) * nh * 16));
-			hipLaunchKernelGGL(k_structure, dim3((nh + 63) / 64, kSFChunks), dim3(64), 0, st, static_cast<const int4*>(dh.p), nh,
+			DCHK(hipMalloc(&dh.p, hv.size() * sizeof(int4)));
+			DCHK(hipMemcpyAsync(dh.p, hv.data(), hv.size() * sizeof(int4), hipMemcpyHostToDevice, st));
+			DCHK(hipMalloc(&dcs.p, size_t(nt) * 8 * kZG * 8));
+			DCHK(hipMalloc(&dsf.p, size_t(sf_chunks) * nt * 8 * kZG * 8));
+			hipLaunchKernelGGL(k_structure, dim3((nt + 255) / 256, sf_chunks), dim3(256), 0, st, static_cast<const int4*>(dh.p), nt,
 					static_cast<const int*>(dx.p), static_cast<const float*>(dm.p), prm->m, n, static_cast<double*>(dsf.p));
 			DCHK(hipGetLastError());
-			hipLaunchKernelGGL(k_structure_sum, dim3((nh + 255) / 256), dim3(256), 0, st, static_cast<const double*>(dsf.p), nh,
-					static_cast<double*>(dcs.p));
+			hipLaunchKernelGGL(k_structure_sum, dim3((nt * 8 * kZG + 255) / 256), dim3(256), 0, st, static_cast<const double*>(dsf.p), nt,
+					sf_chunks, static_cast<double*>(dcs.p));
 			DCHK(hipGetLastError());
 		}
-		DCHK(hipMalloc(&dpart.p, size_t(ns) * kSrcChunks * 32));
-		const unsigned sblocks = unsigned((ns + 63) / 64);
-		hipLaunchKernelGGL(k_pairs, dim3(sblocks, kSrcChunks), dim3(64), 0, st, static_cast<const int*>(dx.p),
-				static_cast<const float*>(dm.p), prm->m, n, static_cast<const int64_t*>(ds.p), ns, ewald, prm->soft_len,
-				static_cast<double*>(dpart.p));
+		DCHK(hipMalloc(&dpart.p, size_t(ns) * src_chunks * 32));
+		if (ewald)
+			hipLaunchKernelGGL(k_pairs<true>, dim3(unsigned(sblocks), src_chunks), dim3(64), 0, st, static_cast<const int*>(dx.p),
+					static_cast<const float*>(dm.p), prm->m, n, static_cast<const int64_t*>(ds.p), ns, lanes, prm->soft_len,
+					static_cast<double*>(dpart.p));
+		else
+			hipLaunchKernelGGL(k_pairs<false>, dim3(unsigned(sblocks), src_chunks), dim3(64), 0, st, static_cast<const int*>(dx.p),
+					static_cast<const float*>(dm.p), prm->m, n, static_cast<const int64_t*>(ds.p), ns, lanes, prm->soft_len,
+					static_cast<double*>(dpart.p));
 		DCHK(hipGetLastError());
 		DCHK(hipMalloc(&dout.p, size_t(ns) * 32));
-		hipLaunchKernelGGL(k_finish, dim3(sblocks), dim3(64), 0, st, static_cast<const int*>(dx.p),
-				static_cast<const int64_t*>(ds.p), ns, static_cast<const double*>(dpart.p), ewald, static_cast<const int4*>(dh.p),
-				static_cast<const double*>(dcs.p), nh, mtot, static_cast<double*>(dout.p));
+		hipLaunchKernelGGL(k_finish, dim3(unsigned(ns)), dim3(256), 0, st, static_cast<const int*>(dx.p),
+				static_cast<const int64_t*>(ds.p), src_chunks, static_cast<const double*>(dpart.p), ewald, static_cast<const int4*>(dh.p),
+				static_cast<const double*>(dcs.p), nt, mtot, static_cast<double*>(dout.p));
 		DCHK(hipGetLastError());
 		DCHK(hipMemcpyAsync(out, dout.p, size_t(ns) * 32, hipMemcpyDeviceToHost, st));
 		DCHK(hipStreamSynchronize(st));
