@@ -538,7 +538,7 @@ __global__ __launch_bounds__(64) void k_tw_pleaf(const int4* __restrict__ leaf_i
 
 }  // namespace
 
-hipError_t walk_nodes_device(const DeviceTree& D, WalkNode** out, hipStream_t s, std::string& err) {
+hipError_t walk_nodes_device(const DeviceTree& D, WalkNode** out, hipStream_t s, std::string& err, std::vector<void*>& later) {
 	*out = nullptr;
 	const int64_t nn = D.nn;
 	WalkNode* wn = nullptr;
@@ -551,10 +551,9 @@ hipError_t walk_nodes_device(const DeviceTree& D, WalkNode** out, hipStream_t s,
 		hipLaunchKernelGGL(k_tw_walk_nodes, dim3(blocks(nl, 256)), dim3(256), 0, s, D.nodes, D.multi, b, nl, sbox, wn);
 		e = hipGetLastError();
 	}
-	if (e == hipSuccess) e = hipStreamSynchronize(s);
-	if (sbox) dev_free(sbox);
+	if (sbox) later.push_back(sbox);
 	if (e != hipSuccess) {
-		if (wn) dev_free(wn);
+		if (wn) later.push_back(wn);
 		err = std::string("walk node table: ") + hipGetErrorString(e);
 		return e;
 	}

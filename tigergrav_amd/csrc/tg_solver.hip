@@ -391,14 +391,24 @@ int Solver::set_particles(const int32_t* x, const float* mass, int64_t count, bo
 	for (auto& w : work)
 		if (!w.list.owned) w.list.release();
 	lists_on_device = false;
+	// the build's working buffers, freed when its stream has drained
+	struct Later {
+		hipStream_t s;
+		std::vector<void*> blocks;
+		~Later() {
+			if (blocks.empty()) return;
+			(void) hipStreamSynchronize(s);
+			for (void* p : blocks) dev_free(p);
+		}
+	} later{stream, {}};
 	if (gpu_walk) {
 		// the lists stay on the device; the work is built from them there (upload_lists_device)
 		WalkNode* wn = nullptr;
 		if (tree_on_device) {
-			const hipError_t e = walk_nodes_device(dtree, &wn, stream, err);
+			const hipError_t e = walk_nodes_device(dtree, &wn, stream, err, later.blocks);
 			if (e != hipSuccess) return e == hipErrorOutOfMemory ? TG_ENOMEM : TG_EHIP;
 		}
-		const hipError_t e = device_walk(tree, device, stream, err, t_detail, &dlists, wn, n_nodes, &walk_hint);
+		const hipError_t e = device_walk(tree, device, stream, err, t_detail, &dlists, wn, n_nodes, &walk_hint, later.blocks);
 		if (e != hipSuccess) return e == hipErrorOutOfMemory ? TG_ENOMEM : TG_EHIP;
 		lists_on_device = true;
 	} else {

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <string>
+#include <vector>
 
 #include "tg_tree.hpp"
 
@@ -32,29 +33,35 @@ struct DeviceLists {
 	void release();
 };
 
-// Tree::walk on the device: fills T.lists and T.census with exactly the lists the host walk
-// builds (same entries, same order).  Returns hipSuccess or the first HIP error; err names it.
-// t, if given, receives the seconds spent in set-up, the walk steps, list assembly with the copy
-// to the host, and the census.  With keep, nothing is copied to the host: the lists stay on the
-// device in *keep (released first), T.lists is left empty and T.census zero.
-// With nodes (a device table of nn nodes, which device_walk then owns and frees or hands to keep),
-// T supplies only its parameters: the tree itself may be on the device only.
-// With hint, the walk's working buffers start at the sizes *hint holds (those the caller's last
-// walk reached, which this walk writes back), so a rebuild of similar particles grows none of them:
-// a grown output pool copies what it holds, and a grown per-step buffer waits for the stream.
+// The sizes a walk reached, for the next one's working buffers and grids.
 struct WalkHint {
 	int64_t out[8] = {};    // entries of each output kind
 	int64_t lists = 0;      // the longest checklist set of a step
-	int64_t counts = 0;     // per-step count buffer
-	int64_t codes = 0;      // per-step category bytes
+	int64_t units = 0;      // the most units of a step
+	int64_t drains = 0;     // drain rounds
+	int steps = 0;          // steps (0: no walk yet)
+	std::vector<int32_t> step_units;  // units of the first steps
 };
-hipError_t device_walk(Tree& T, int device, hipStream_t s, std::string& err, double* t = nullptr, DeviceLists* keep = nullptr,
-		WalkNode* nodes = nullptr, int64_t nn = 0, WalkHint* hint = nullptr);
+
+// Tree::walk on the device: exactly the lists the host walk builds (same entries, same order), left
+// on the device in *keep (released first); T supplies the parameters, its lists are left empty and
+// its census zero.  Returns hipSuccess or the first HIP error; err names it.  t, if given,
+// receives the seconds spent in set-up, the walk steps and list assembly (enqueued), and zero.
+// With nodes (a device table of nn nodes, which device_walk then owns and frees or hands to keep),
+// the tree itself may be on the device only.
+// With hint, the walk's working buffers start at the sizes *hint holds (those the caller's last
+// walk reached, which this walk writes back) and its steps are enqueued without a host wait; a walk
+// that passes one of those sizes runs again, waiting for each step's.
+// The work may still be running on s when this returns: the caller frees the blocks added to `later`
+// (dev_free) once s has drained.
+hipError_t device_walk(Tree& T, int device, hipStream_t s, std::string& err, double* t, DeviceLists* keep, WalkNode* nodes, int64_t nn,
+		WalkHint* hint, std::vector<void*>& later);
 
 struct DeviceTree;
 // the walk's node table of a device-built tree, made on the device (*out: nn nodes, device memory
 // the caller frees): the centres, radii and children, and each node's sink span from a bottom-up
-// union of its non-empty leaves' particle boxes, as Tree::sink_spans forms it
-hipError_t walk_nodes_device(const DeviceTree& D, WalkNode** out, hipStream_t s, std::string& err);
+// union of its non-empty leaves' particle boxes, as Tree::sink_spans forms it.  Enqueued on s; `later`
+// as for device_walk.
+hipError_t walk_nodes_device(const DeviceTree& D, WalkNode** out, hipStream_t s, std::string& err, std::vector<void*>& later);
 
 }  // namespace tg
