@@ -15,16 +15,17 @@
 // length of the sink leaf's box, the test made in FP64 with the host's operations.  Scans over
 // the leaves give the offsets; the PP ranges are expanded (PP direct: near ranges first, both
 // groups in list order), the items of <= 64 sinks written, and every kind's items put in the
-// order of a stable sort by descending cost class (a radix sort of (class, index) pairs).  The PC lists
-// are the walk's own.
-#include <hipcub/hipcub.hpp>
-
+// order of a stable sort by descending cost class (a counting sort).  The PC lists are the walk's own.
+// Every kernel covers its four kinds at once and all arrays of a stage are scanned together
+// (tg_scan.hpp): a small set's preparation is a matter of launches, 25 of them, and two host waits
+// for the sizes.
 #include <algorithm>
 #include <cstring>
 
 #include "tg_gravity.h"
 #include "tg_solver.hpp"
 #include "tg_devmem.hpp"
+#include "tg_scan.hpp"
 
 namespace tg {
 namespace {
@@ -119,70 +120,131 @@ __global__ __launch_bounds__(256) void k_node_chunks(NodeIn A, const int64_t* __
 	}
 }
 
-// the partial slot of every entry: one wave per chunk
-__global__ __launch_bounds__(256) void k_node_owner(const int2* __restrict__ chunks, const int* __restrict__ chunk_slot, int64_t nch,
-		int* __restrict__ owner) {
+struct ChunkSet {
+	const int2* chunks[4];
+	const int* slot[4];
+	int* owner[4];
+	int64_t nch[4];
+};
+
+// The partial slot of the entries: one wave per chunk, kinds in grid.y.  The solve reads the slot of
+// a wave's first 64 entries only (a longer chunk is a wave of its own), so no more are written
+// unless `all` asks (0.35 ms of 1.3 GB at 2M theta 0.3 leaf 8).
+__global__ __launch_bounds__(256) void k_node_owner(ChunkSet S, int all) {
+	const int q = blockIdx.y;
 	const int64_t c = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
-	if (c >= nch) return;
-	const int2 ch = chunks[c];
-	const int sl = chunk_slot[c];
-	for (int j = ch.x + int(threadIdx.x & 63); j < ch.y; j += 64) owner[j] = sl;
+	if (c >= S.nch[q]) return;
+	const int2 ch = S.chunks[q][c];
+	const int sl = S.slot[q][c];
+	const int end = all ? ch.y : min(ch.y, ch.x + 64);
+	for (int j = ch.x + int(threadIdx.x & 63); j < end; j += 64) S.owner[q][j] = sl;
 }
 
-// greedy packing of chunks [c0, c1) into waves of <= 64 entries: calls emit(begin, end) per wave
+// Greedy packing of a segment's chunks into waves of <= 64 entries (a longer chunk is a wave alone):
+// a wave that starts at chunk c ends before next(c), the first chunk whose end lies more than 64
+// entries past c's begin.  The waves' first chunks are the orbit of the segment's first under
+// next, marked by doubling: eight tables of 2^k-fold jumps, eight rounds of marks.  (One thread walking a
+// segment's 256 chunks took 37 us whatever the set's size.)
+struct PackShared {
+	int begin[WAVE_SEGMENT], end[WAVE_SEGMENT];
+	short jump[8][WAVE_SEGMENT + 1];
+	uint8_t mark[WAVE_SEGMENT + 1];
+	int wsum[WAVE_SEGMENT / 64];
+};
+static_assert(WAVE_SEGMENT == 256, "eight doublings cover a segment");
+
+// calls emit(rank, begin, end) in the thread of every wave's first chunk; returns the wave count
 template <class F>
-__device__ __forceinline__ void pack_waves(const int2* __restrict__ chunks, int64_t c0, int64_t c1, F emit) {
-	int2 cur = make_int2(0, 0);
-	bool open = false;
-	for (int64_t c = c0; c < c1; c++) {
-		const int2 ch = chunks[c];
-		if (open && ch.y - cur.x > 64) {
-			emit(cur);
-			open = false;
-		}
-		if (!open) {
-			cur = ch;
-			open = true;
-		} else {
-			cur.y = ch.y;
-		}
+__device__ __forceinline__ int pack_segment(const int2* __restrict__ chunks, int64_t c0, int cnt, PackShared& S, F emit) {
+	const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+	if (t < cnt) {
+		const int2 c = chunks[c0 + t];
+		S.begin[t] = c.x;
+		S.end[t] = c.y;
 	}
-	if (open) emit(cur);
+	S.mark[t] = t == 0;
+	__syncthreads();
+	if (t < cnt) {
+		int lo = t + 1, hi = cnt;
+		while (lo < hi) {
+			const int mid = (lo + hi) >> 1;
+			if (S.end[mid] - S.begin[t] > 64)
+				hi = mid;
+			else
+				lo = mid + 1;
+		}
+		S.jump[0][t] = short(lo);
+	} else {
+		S.jump[0][t] = short(cnt);
+	}
+	if (t == 0) {
+		for (int k = 0; k < 8; k++) S.jump[k][cnt] = short(cnt);
+		S.mark[cnt] = 0;
+	}
+	__syncthreads();
+	for (int k = 1; k < 8; k++) {
+		if (t < cnt) S.jump[k][t] = S.jump[k - 1][S.jump[k - 1][t]];
+		__syncthreads();
+	}
+	for (int k = 7; k >= 0; k--) {
+		const int to = t < cnt && S.mark[t] ? int(S.jump[k][t]) : cnt;
+		if (to < cnt) S.mark[to] = 1;
+		__syncthreads();
+	}
+	const bool first = t < cnt && S.mark[t];
+	const unsigned long long m = __ballot(first);
+	if (lane == 0) S.wsum[wave] = __popcll(m);
+	__syncthreads();
+	int before = 0, all = 0;
+	for (int w = 0; w < WAVE_SEGMENT / 64; w++) {
+		if (w < wave) before += S.wsum[w];
+		all += S.wsum[w];
+	}
+	if (first) emit(before + __popcll(m & (lane ? ~0ull >> (64 - lane) : 0ull)), S.begin[t], S.end[S.jump[0][t] - 1]);
+	return all;
 }
 
-// waves per segment of WAVE_SEGMENT chunks (array of nseg + 1, the last zero)
-__global__ __launch_bounds__(256) void k_wave_count(const int2* __restrict__ chunks, int64_t nch, int64_t nseg, int64_t* __restrict__ nw) {
-	const int64_t sg = int64_t(blockIdx.x) * 256 + threadIdx.x;
-	if (sg > nseg) return;
-	if (sg == nseg) {
-		nw[sg] = 0;
-		return;
-	}
-	const int64_t c0 = sg * WAVE_SEGMENT, c1 = c0 + WAVE_SEGMENT < nch ? c0 + WAVE_SEGMENT : nch;
-	int64_t k = 0;
-	pack_waves(chunks, c0, c1, [&](int2) { k++; });
-	nw[sg] = k;
+// waves per segment of WAVE_SEGMENT chunks, kinds in grid.y
+struct PackOut {
+	int64_t nseg[4];
+	int64_t* nw[4];
+	const int64_t* ow[4];
+	int2* waves[4];
+};
+__global__ __launch_bounds__(WAVE_SEGMENT) void k_wave_count(ChunkSet S, PackOut O) {
+	__shared__ PackShared P;
+	const int q = blockIdx.y;
+	const int64_t sg = blockIdx.x;
+	if (sg >= O.nseg[q]) return;
+	const int64_t c0 = sg * WAVE_SEGMENT;
+	const int n = pack_segment(S.chunks[q], c0, int(S.nch[q] - c0 < WAVE_SEGMENT ? S.nch[q] - c0 : WAVE_SEGMENT), P, [](int, int, int) {});
+	if (threadIdx.x == 0) O.nw[q][sg] = n;
 }
 
-__global__ __launch_bounds__(256) void k_wave_write(const int2* __restrict__ chunks, int64_t nch, int64_t nseg, const int64_t* __restrict__ ow,
-		int2* __restrict__ waves) {
-	const int64_t sg = int64_t(blockIdx.x) * 256 + threadIdx.x;
-	if (sg >= nseg) return;
-	const int64_t c0 = sg * WAVE_SEGMENT, c1 = c0 + WAVE_SEGMENT < nch ? c0 + WAVE_SEGMENT : nch;
-	int64_t k = ow[sg];
-	pack_waves(chunks, c0, c1, [&](int2 w) { waves[k++] = w; });
+__global__ __launch_bounds__(WAVE_SEGMENT) void k_wave_write(ChunkSet S, PackOut O) {
+	__shared__ PackShared P;
+	const int q = blockIdx.y;
+	const int64_t sg = blockIdx.x;
+	if (sg >= O.nseg[q]) return;
+	const int64_t c0 = sg * WAVE_SEGMENT;
+	int2* out = O.waves[q] + O.ow[q][sg];
+	pack_segment(S.chunks[q], c0, int(S.nch[q] - c0 < WAVE_SEGMENT ? S.nch[q] - c0 : WAVE_SEGMENT), P,
+			[&](int r, int b, int e) { out[r] = make_int2(b, e); });
 }
 
 // ---- range expansion (CP, PP) --------------------------------------------------------------------
 
 // One wave writes the entries of the non-empty ranges of v[kb, ke) (2 ints each) that keep()
-// accepts, consecutively from out: 64 ranges per round, an inclusive scan of their lengths, then
-// every lane writes entries base + lane + 64 t, finding its range by binary search of the scan.
-// Returns the entries written.  The block is this one wave (the barriers are the wave's).
+// accepts, consecutively from out: 64 ranges per round, an exclusive scan of their lengths, the
+// non-empty ones moved to the first lanes; then 64 entries at a time, each finding its range from a
+// mask of the entries at which ranges start (a binary search of the scan per entry took 1.6 times
+// as long).  Returns the entries written.  The block is this one wave (the barriers are the wave's).
 template <class Keep>
 __device__ int64_t expand_ranges(const int32_t* __restrict__ v, int64_t kb, int64_t ke, Keep keep, int32_t* __restrict__ out) {
-	__shared__ int incl[64], first[64];
+	__shared__ int s_start[64], s_off[64];
+	__shared__ uint8_t s_flag[64];
 	const int lane = threadIdx.x;
+	const unsigned long long below = lane ? ~0ull >> (64 - lane) : 0ull;
 	int64_t pos = 0;
 	for (int64_t j0 = kb; j0 < ke; j0 += 128) {
 		const int64_t j = j0 + 2 * lane;
@@ -199,22 +261,30 @@ __device__ int64_t expand_ranges(const int32_t* __restrict__ v, int64_t kb, int6
 			if (lane >= o) s += t;
 		}
 		const int tot = __shfl(s, 63, 64);
-		incl[lane] = s;
-		first[lane] = b;
-		__syncthreads();
-		for (int p = lane; p < tot; p += 64) {
-			int lo = 0, hi = 63;  // the first range whose inclusive end passes p
-			while (lo < hi) {
-				const int mid = (lo + hi) >> 1;
-				if (incl[mid] > p)
-					hi = mid;
-				else
-					lo = mid + 1;
-			}
-			const int before = lo ? incl[lo - 1] : 0;
-			out[pos + p] = first[lo] + (p - before);
+		const unsigned long long some = __ballot(len > 0);
+		const int nr = __popcll(some);
+		if (len > 0) {
+			const int r = __popcll(some & below);
+			s_start[r] = s - len;
+			s_off[r] = b - (s - len);
 		}
 		__syncthreads();
+		const int start = lane < nr ? s_start[lane] : INT32_MAX;
+		const int off = lane < nr ? s_off[lane] : 0;
+		int r0 = 0;  // ranges that started before the 64 entries
+		for (int p0 = 0; p0 < tot; p0 += 64) {
+			s_flag[lane] = 0;
+			__syncthreads();
+			const int at = start - p0;
+			if (at >= 0 && at < 64) s_flag[at] = 1;
+			__syncthreads();
+			const unsigned long long m = __ballot(s_flag[lane] != 0);
+			const int r = r0 + __popcll(m & (below | (1ull << lane))) - 1;
+			const int o = __shfl(off, r & 63, 64);
+			if (p0 + lane < tot) out[pos + p0 + lane] = o + p0 + lane;
+			r0 += __popcll(m);
+			__syncthreads();
+		}
 		pos += tot;
 	}
 	return pos;
@@ -240,8 +310,7 @@ struct LeafIn {
 	const int4* leaf_items;  // (node, first particle, end, -)
 	const int4* parts;
 	const int* pleaf;        // particle -> leaf
-	const WalkNode* nodes;
-	const int4* box;         // per node, 2 records: lowest and highest particle coordinates (leaves)
+	const int4* box;         // per node, 2 records: lowest and highest particle coordinates, first particle, end (leaves)
 	uint8_t* near;           // PP direct: per range (entry pair j / 2), the near test's outcome
 	int64_t nl;
 	int ewald;
@@ -266,8 +335,8 @@ __global__ __launch_bounds__(64) void k_leaf_boxes(const int4* __restrict__ leaf
 		hi[d] = wave_max(hi[d]);
 	}
 	if (threadIdx.x == 0) {
-		box[2 * li.x] = make_int4(lo[0], lo[1], lo[2], 0);
-		box[2 * li.x + 1] = make_int4(hi[0], hi[1], hi[2], 0);
+		box[2 * li.x] = make_int4(lo[0], lo[1], lo[2], li.y);
+		box[2 * li.x + 1] = make_int4(hi[0], hi[1], hi[2], li.z);
 	}
 }
 
@@ -290,16 +359,28 @@ __device__ bool may_be_near(int4 slo, int4 shi, int4 lo, int4 hi, int ewald, dou
 	return d2 <= hnear * hnear;
 }
 
+// the same decided by one axis alone where that is clear: a gap beyond the softening length by more
+// than FP32's error (3e-7 of the box) on any axis, and no periodic axis near the quarter-box rule
+__device__ __forceinline__ bool surely_far(int4 slo, int4 shi, int4 lo, int4 hi, int ewald, float hnear) {
+	const int a0[3] = {slo.x, slo.y, slo.z}, a1[3] = {shi.x, shi.y, shi.z};
+	const int b0[3] = {lo.x, lo.y, lo.z}, b1[3] = {hi.x, hi.y, hi.z};
+	float gap = -1.0f, wide = 0.0f;
+	for (int d = 0; d < 3; d++) {
+		const float hh = (float(unsigned(a1[d]) - unsigned(a0[d])) + float(unsigned(b1[d]) - unsigned(b0[d]))) * 1.1641532182693481e-10f;  // 2^-33
+		float dc = float((int64_t(a0[d]) + a1[d]) - (int64_t(b0[d]) + b1[d])) * 1.1641532182693481e-10f;
+		if (ewald) dc -= rintf(dc);
+		gap = fmaxf(gap, fabsf(dc) - hh);
+		wide = fmaxf(wide, hh);
+	}
+	return gap > hnear + 1e-6f && !(ewald && wide > 0.2499f);
+}
+
 // the near test of the source range [b, e) (non-empty) for a sink leaf of box [slo, shi]: a whole
-// leaf takes that leaf's box, any other range its particles' box
+// leaf (which the walk's ranges are) takes that leaf's box, any other range its particles' box
 __device__ bool range_near(const LeafIn& A, int4 slo, int4 shi, int b, int e) {
 	const int lf = A.pleaf[b];
-	const WalkNode& nd = A.nodes[lf];
-	int4 lo, hi;
-	if (nd.pbegin == b && nd.pend == e) {
-		lo = A.box[2 * lf];
-		hi = A.box[2 * lf + 1];
-	} else {
+	int4 lo = A.box[2 * lf], hi = A.box[2 * lf + 1];
+	if (lo.w != b || hi.w != e) {
 		lo = make_int4(INT32_MAX, INT32_MAX, INT32_MAX, 0);
 		hi = make_int4(INT32_MIN, INT32_MIN, INT32_MIN, 0);
 		for (int p = b; p < e; p++) {
@@ -308,6 +389,7 @@ __device__ bool range_near(const LeafIn& A, int4 slo, int4 shi, int b, int e) {
 			hi = make_int4(max(hi.x, x.x), max(hi.y, x.y), max(hi.z, x.z), 0);
 		}
 	}
+	if (surely_far(slo, shi, lo, hi, A.ewald, float(A.hnear))) return false;
 	return may_be_near(slo, shi, lo, hi, A.ewald, A.hnear);
 }
 
@@ -362,10 +444,9 @@ __global__ __launch_bounds__(64) void k_leaf_count(LeafIn A, int64_t* __restrict
 struct LeafOut {
 	int32_t* list[4];  // PP kinds: expanded lists (PC: unused)
 	int4* items[4];    // unsorted items
-	unsigned long long* key[4];
-	int* idx[4];
+	uint8_t* cls[4];   // their cost classes (item_class, below CLASSES)
 };
-
+constexpr int CLASSES = 64;
 
 // the expanded PP lists and every kind's items, in leaf order: one wave per leaf
 __global__ __launch_bounds__(64) void k_leaf_write(LeafIn A, const int64_t* __restrict__ lent, const int64_t* __restrict__ olent,
@@ -405,25 +486,62 @@ __global__ __launch_bounds__(64) void k_leaf_write(LeafIn A, const int64_t* __re
 			const int y = (q & 1) ? pp_item_y(cnt, nearl) : cnt;
 			const int64_t it = it0 + k;
 			O.items[q][it] = make_int4(b, y, int(lb), int(le));
-			O.key[q][it] = (unsigned long long) item_class(le - lb, cnt);
-			O.idx[q][it] = int(it);
+			O.cls[q][it] = uint8_t(item_class(le - lb, cnt));
 		}
 	}
 }
 
-__global__ __launch_bounds__(256) void k_gather_items(const int4* __restrict__ in, const int* __restrict__ idx, int64_t m, int4* __restrict__ out) {
-	const int64_t r = int64_t(blockIdx.x) * 256 + threadIdx.x;
-	if (r < m) out[r] = in[idx[r]];
+// Counting sort of the items by descending class, stable: tiles of SORT_TILE items, per tile the items
+// of each class (hist[(CLASSES - 1 - class) tiles + tile], kinds in grid.y); a scan of those gives the
+// place of each tile's first item of each class, and an item's rank among the tile's earlier ones of
+// its class the rest.
+constexpr int SORT_TILE = 1024;
+struct SortSet {
+	const int4* in[4];
+	const uint8_t* cls[4];
+	int4* out[4];
+	int64_t* hist[4];
+	const int64_t* place[4];
+	int64_t n[4];
+};
+
+__global__ __launch_bounds__(SORT_TILE) void k_item_hist(SortSet S) {
+	__shared__ int h[CLASSES];
+	const int q = blockIdx.y;
+	const int64_t tiles = (S.n[q] + SORT_TILE - 1) / SORT_TILE;
+	if (int64_t(blockIdx.x) >= tiles) return;
+	if (threadIdx.x < CLASSES) h[threadIdx.x] = 0;
+	__syncthreads();
+	const int64_t i = int64_t(blockIdx.x) * SORT_TILE + threadIdx.x;
+	if (i < S.n[q]) atomicAdd(&h[S.cls[q][i]], 1);
+	__syncthreads();
+	if (threadIdx.x < CLASSES) S.hist[q][(CLASSES - 1 - int(threadIdx.x)) * tiles + blockIdx.x] = h[threadIdx.x];
 }
 
-__global__ void k_zero_u64(unsigned long long* p, int m) {
-	if (int(threadIdx.x) < m) p[threadIdx.x] = 0;
-}
-
-// the last element of each array, gathered for one copy to the host
-__global__ void k_last(const int64_t* const* __restrict__ arrs, const int64_t* __restrict__ at, int m, int64_t* __restrict__ out) {
-	const int k = threadIdx.x;
-	if (k < m) out[k] = arrs[k][at[k]];
+__global__ __launch_bounds__(SORT_TILE) void k_item_scatter(SortSet S) {
+	__shared__ int h[SORT_TILE / 64][CLASSES];
+	const int q = blockIdx.y;
+	const int64_t tiles = (S.n[q] + SORT_TILE - 1) / SORT_TILE;
+	if (int64_t(blockIdx.x) >= tiles) return;
+	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	for (int k = threadIdx.x; k < SORT_TILE / 64 * CLASSES; k += SORT_TILE) h[k / CLASSES][k % CLASSES] = 0;
+	__syncthreads();
+	const int64_t i = int64_t(blockIdx.x) * SORT_TILE + threadIdx.x;
+	const bool in = i < S.n[q];
+	const int c = in ? int(S.cls[q][i]) : 0;
+	// the lanes of the wave with this lane's class
+	unsigned long long same = __ballot(in);
+	for (int bit = 0; bit < 6; bit++) {
+		const unsigned long long set = __ballot((c >> bit) & 1);
+		same &= (c >> bit) & 1 ? set : ~set;
+	}
+	const int rank = __popcll(same & (lane ? ~0ull >> (64 - lane) : 0ull));
+	if (in && rank == 0) h[wave][c] = __popcll(same);
+	__syncthreads();
+	if (!in) return;
+	int64_t pos = S.place[q][(CLASSES - 1 - c) * tiles + blockIdx.x] + rank;
+	for (int w = 0; w < wave; w++) pos += h[w][c];
+	S.out[q][pos] = S.in[q][i];
 }
 
 unsigned blocks(int64_t n, int per) { return unsigned((n + per - 1) / per); }
@@ -483,27 +601,22 @@ __global__ __launch_bounds__(256) void k_tw_walk_nodes(const DNode* __restrict__
 	wn[k] = w;
 }
 
-// particle records (x, y, z, mass bits)
-__global__ __launch_bounds__(256) void k_tw_parts(const int32_t* __restrict__ pos, const float* __restrict__ mass, int64_t n, int4* __restrict__ parts) {
+// particle records (x, y, z, mass bits) and the input order
+__global__ __launch_bounds__(256) void k_tw_parts(const int32_t* __restrict__ pos, const float* __restrict__ mass, const int64_t* __restrict__ order,
+		int64_t n, int4* __restrict__ parts, int64_t* __restrict__ order_out) {
 	const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
-	if (i < n) parts[i] = make_int4(pos[3 * i], pos[3 * i + 1], pos[3 * i + 2], __float_as_int(mass[i]));
+	if (i >= n) return;
+	parts[i] = make_int4(pos[3 * i], pos[3 * i + 1], pos[3 * i + 2], __float_as_int(mass[i]));
+	order_out[i] = order[i];
 }
 
 // per node: source multipole, centre, level, parent; flags of the non-empty leaves and their
-// root-path lengths (arrays of nn + 1, the last zero); the leaf count (empty leaves included)
+// root-path lengths, and of every leaf, empty ones included
 __global__ __launch_bounds__(256) void k_tw_nodes(const DNode* __restrict__ nodes, const DMulti* __restrict__ multi, int64_t nn,
 		MultiSrc* __restrict__ multis, int4* __restrict__ npos, int* __restrict__ level, int* __restrict__ parent, int64_t* __restrict__ lflag,
-		int64_t* __restrict__ plen, unsigned long long* __restrict__ n_leaves) {
+		int64_t* __restrict__ plen, int64_t* __restrict__ leaves) {
 	const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
-	// the leaf count: one atomic per wave
-	const bool is_leaf = i < nn && nodes[i].c0 < 0;
-	const unsigned long long lv = __ballot(is_leaf);
-	if ((threadIdx.x & 63) == 0 && lv) atomicAdd(n_leaves, (unsigned long long) __popcll(lv));
-	if (i > nn) return;
-	if (i == nn) {
-		lflag[i] = plen[i] = 0;
-		return;
-	}
+	if (i >= nn) return;
 	const DNode nd = nodes[i];
 	const DMulti& m = multi[i];
 	MultiSrc ms;
@@ -517,6 +630,7 @@ __global__ __launch_bounds__(256) void k_tw_nodes(const DNode* __restrict__ node
 	const bool use = leaf && nd.pend > nd.pbegin;
 	lflag[i] = use ? 1 : 0;
 	plen[i] = use ? nd.level + 1 : 0;
+	leaves[i] = leaf ? 1 : 0;
 }
 
 // the non-empty leaves in node order: (node, first particle, end, root-path offset) and the paths
@@ -590,45 +704,34 @@ int Solver::upload_tree_device() {
 	PCHK(d_pleaf.alloc(std::max<size_t>(size_t(n) * 4, 16)));
 	PCHK(d_order.alloc(std::max<size_t>(size_t(n) * 8, 16)));
 	PCHK(d_Lnode.alloc(std::max<size_t>(size_t(nn) * 35 * sizeof(double), 16)));
-	DeviceArray flag, loff, plen, poff, cnt, scan_tmp;
-	struct Free {
-		hipStream_t s;
-		DeviceArray* a[6];
-		~Free() {
-			(void) hipStreamSynchronize(s);
-			for (auto* x : a) x->release();
-		}
-	} free_on_return{s, {&flag, &loff, &plen, &poff, &cnt, &scan_tmp}};
-	const int64_t np = nn + 1;
-	PCHK(flag.alloc(np * 8));
-	PCHK(loff.alloc(np * 8));
-	PCHK(plen.alloc(np * 8));
-	PCHK(poff.alloc(np * 8));
-	PCHK(cnt.alloc(64));
+	// scratch, freed with the build's working buffers: six columns of nn words, the scan's workspace
+	void* cols = nullptr;
+	void* work = nullptr;
+	PCHK(dev_malloc(&cols, size_t(6 * nn + 1) * 8));
+	build_later.push_back(cols);
+	int64_t* flag = static_cast<int64_t*>(cols);
+	int64_t *loff = flag + nn, *plen = flag + 2 * nn, *poff = flag + 3 * nn, *lall = flag + 4 * nn, *aoff = flag + 5 * nn;
 	if (n > 0) {
-		hipLaunchKernelGGL(k_tw_parts, dim3(blocks(n, 256)), dim3(256), 0, s, D.pos, D.mass, n, d_parts.as<int4>());
+		hipLaunchKernelGGL(k_tw_parts, dim3(blocks(n, 256)), dim3(256), 0, s, D.pos, D.mass, D.order, n, d_parts.as<int4>(), d_order.as<int64_t>());
 		PCHK(hipGetLastError());
-		PCHK(hipMemcpyAsync(d_order.p, D.order, size_t(n) * 8, hipMemcpyDeviceToDevice, s));
 	}
 	order_on_device = true;
-	hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, s, cnt.as<unsigned long long>(), 1);
-	PCHK(hipGetLastError());
-	hipLaunchKernelGGL(k_tw_nodes, dim3(blocks(np, 256)), dim3(256), 0, s, D.nodes, D.multi, nn, d_multis.as<MultiSrc>(), d_nodepos.as<int4>(),
-			d_level.as<int>(), d_parent.as<int>(), flag.as<int64_t>(), plen.as<int64_t>(), cnt.as<unsigned long long>());
-	PCHK(hipGetLastError());
-	for (int k = 0; k < 2; k++) {
-		const int64_t* in = (k ? plen : flag).as<const int64_t>();
-		int64_t* out = (k ? poff : loff).as<int64_t>();
-		size_t need = 0;
-		PCHK(hipcub::DeviceScan::ExclusiveSum(nullptr, need, in, out, np, s));
-		PCHK(scan_tmp.alloc(std::max<size_t>(need, 16)));
-		PCHK(hipcub::DeviceScan::ExclusiveSum(scan_tmp.p, need, in, out, np, s));
+	int64_t tot[3] = {0, 0, 0};
+	if (nn > 0) {
+		hipLaunchKernelGGL(k_tw_nodes, dim3(blocks(nn, 256)), dim3(256), 0, s, D.nodes, D.multi, nn, d_multis.as<MultiSrc>(), d_nodepos.as<int4>(),
+				d_level.as<int>(), d_parent.as<int>(), flag, plen, lall);
+		PCHK(hipGetLastError());
+		ScanSet sc;
+		sc.add(flag, loff, nn);
+		sc.add(plen, poff, nn);
+		sc.add(lall, aoff, nn);
+		PCHK(dev_malloc(&work, size_t(scan_workspace(sc) + sc.cols) * 8));
+		build_later.push_back(work);
+		int64_t* wt = static_cast<int64_t*>(work);
+		PCHK(scan_columns(sc, wt + sc.cols, wt, s));
+		PCHK(hipMemcpyAsync(tot, wt, sizeof(tot), hipMemcpyDeviceToHost, s));
+		PCHK(hipStreamSynchronize(s));
 	}
-	int64_t tot[3];
-	PCHK(hipMemcpyAsync(tot, loff.as<int64_t>() + nn, 8, hipMemcpyDeviceToHost, s));
-	PCHK(hipMemcpyAsync(tot + 1, poff.as<int64_t>() + nn, 8, hipMemcpyDeviceToHost, s));
-	PCHK(hipMemcpyAsync(tot + 2, cnt.p, 8, hipMemcpyDeviceToHost, s));
-	PCHK(hipStreamSynchronize(s));
 	if (tot[1] > int64_t(INT32_MAX)) {
 		err = "root-to-leaf paths exceed 2^31 entries";
 		return TG_EINVAL;
@@ -639,8 +742,8 @@ int Solver::upload_tree_device() {
 	PCHK(d_leaf_items.alloc(std::max<size_t>(size_t(tot[0]) * sizeof(int4), 16)));
 	PCHK(d_path.alloc(std::max<size_t>(size_t(tot[1]) * 4, 16)));
 	if (nn > 0) {
-		hipLaunchKernelGGL(k_tw_leaves, dim3(blocks(nn, 256)), dim3(256), 0, s, D.nodes, nn, flag.as<const int64_t>(), loff.as<const int64_t>(),
-				poff.as<const int64_t>(), d_leaf_items.as<int4>(), d_path.as<int>());
+		hipLaunchKernelGGL(k_tw_leaves, dim3(blocks(nn, 256)), dim3(256), 0, s, D.nodes, nn, flag, loff, poff, d_leaf_items.as<int4>(),
+				d_path.as<int>());
 		PCHK(hipGetLastError());
 	}
 	if (tot[0] > 0) {
@@ -648,7 +751,6 @@ int Solver::upload_tree_device() {
 		PCHK(hipGetLastError());
 	}
 	level_begin.assign(D.level_begin.begin(), D.level_begin.end());
-	PCHK(hipStreamSynchronize(s));
 	return TG_OK;
 }
 
@@ -667,54 +769,16 @@ int Solver::upload_lists_device() {
 			err = "an interaction list exceeds 2^31 entries (32-bit list offsets)";
 			return TG_EINVAL;
 		}
-	std::vector<DeviceArray> tmp;  // scratch, freed on return (after the stream drains)
-	struct Drain {
-		hipStream_t s;
-		std::vector<DeviceArray>& t;
-		~Drain() {
-			(void) hipStreamSynchronize(s);
-			for (auto& a : t) a.release();
-		}
-	} drain{s, tmp};
-	tmp.reserve(64);
-	auto scratch = [&](size_t bytes) -> void* {
-		tmp.emplace_back();
-		if (tmp.back().alloc(std::max<size_t>(bytes, 16)) != hipSuccess) return nullptr;
-		return tmp.back().p;
+	auto scratch = [&](size_t bytes) -> void* {  // freed with the build's working buffers
+		void* p = nullptr;
+		if (dev_malloc(&p, std::max<size_t>(bytes, 16)) != hipSuccess) return nullptr;
+		build_later.push_back(p);
+		return p;
 	};
-	void* scan_tmp = nullptr;
-	size_t scan_bytes = 0;
-	auto exclusive_scan = [&](const int64_t* in, int64_t* out, int64_t m) -> hipError_t {
-		size_t need = 0;
-		hipError_t e = hipcub::DeviceScan::ExclusiveSum(nullptr, need, in, out, m, s);
-		if (e != hipSuccess) return e;
-		if (need > scan_bytes) {
-			scan_bytes = std::max(need, 2 * scan_bytes);
-			scan_tmp = scratch(scan_bytes);
-			if (!scan_tmp) return hipErrorOutOfMemory;
-		}
-		size_t b = scan_bytes;
-		return hipcub::DeviceScan::ExclusiveSum(scan_tmp, b, in, out, m, s);
-	};
-	// the last elements of up to 16 arrays to the host (one copy, one wait)
-	int64_t** d_arrs = static_cast<int64_t**>(scratch(16 * sizeof(int64_t*)));
-	int64_t* d_at = static_cast<int64_t*>(scratch(16 * sizeof(int64_t)));
-	int64_t* d_last = static_cast<int64_t*>(scratch(16 * sizeof(int64_t)));
-	if (!d_arrs || !d_at || !d_last) PCHK(hipErrorOutOfMemory);
-	auto lasts = [&](const std::vector<const int64_t*>& arrs, const std::vector<int64_t>& at, int64_t* out) -> hipError_t {
-		const int m = int(arrs.size());
-		hipError_t e = hipMemcpyAsync(d_arrs, arrs.data(), m * sizeof(int64_t*), hipMemcpyHostToDevice, s);
-		if (e == hipSuccess) e = hipMemcpyAsync(d_at, at.data(), m * sizeof(int64_t), hipMemcpyHostToDevice, s);
-		if (e != hipSuccess) return e;
-		hipLaunchKernelGGL(k_last, dim3(1), dim3(64), 0, s, d_arrs, d_at, m, d_last);
-		if ((e = hipGetLastError()) != hipSuccess) return e;
-		if ((e = hipMemcpyAsync(out, d_last, m * sizeof(int64_t), hipMemcpyDeviceToHost, s)) != hipSuccess) return e;
-		return hipStreamSynchronize(s);
-	};
+	auto words = [&](int64_t count) { return static_cast<int64_t*>(scratch(size_t(count) * 8)); };
 	list_bytes = 0;
-	const int64_t np = nn + 1;
 
-	// ---- node kinds ----
+	// ---- sizes: node kinds per node (entries, chunks, slots), leaf kinds per leaf (entries, items, census) ----
 	NodeIn ni{};
 	for (int q = 0; q < 4; q++) {
 		ni.ptr[q] = L.ptr(q);
@@ -722,66 +786,106 @@ int Solver::upload_lists_device() {
 	}
 	ni.nn = nn;
 	ni.chunk = chunk;
-	int64_t* nent = static_cast<int64_t*>(scratch(4 * np * 8));
-	int64_t* oent = static_cast<int64_t*>(scratch(4 * np * 8));
-	int64_t* nchk = static_cast<int64_t*>(scratch(4 * np * 8));
-	int64_t* ochk = static_cast<int64_t*>(scratch(4 * np * 8));
-	int64_t* nslot = static_cast<int64_t*>(scratch(np * 8));
-	if (!nent || !oent || !nchk || !ochk || !nslot) PCHK(hipErrorOutOfMemory);
+	const int64_t np = nn + 1, lp = nl + 1;
+	int64_t* nent = words(4 * np);
+	int64_t* oent = words(4 * np);
+	int64_t* nchk = words(4 * np);
+	int64_t* ochk = words(4 * np);
+	int64_t* nslot = words(np);
+	int64_t* lent = words(4 * lp);
+	int64_t* olent = words(4 * lp);
+	int64_t* litem = words(4 * lp);
+	int64_t* olitem = words(4 * lp);
+	int64_t* lnear = words(lp);
+	int64_t* sums = words(8 * lp);   // per leaf, 8 columns
+	int64_t* osums = words(8 * lp);  // (their totals only)
+	int4* box = static_cast<int4*>(scratch(size_t(std::max<int64_t>(nn, 1)) * 2 * sizeof(int4)));
+	if (!nent || !oent || !nchk || !ochk || !nslot || !lent || !olent || !litem || !olitem || !lnear || !sums || !osums || !box)
+		PCHK(hipErrorOutOfMemory);
 	PCHK(d_node_slot_ptr.alloc(np * 8));
 	int64_t* slot_ptr = d_node_slot_ptr.as<int64_t>();
+	LeafIn li{};
+	for (int q = 0; q < 4; q++) {
+		li.ptr[q] = L.ptr(4 + q);
+		li.val[q] = L.val[4 + q];
+	}
+	li.leaf_items = d_leaf_items.as<int4>();
+	li.parts = d_parts.as<int4>();
+	li.pleaf = d_pleaf.as<int>();
+	li.nl = nl;
+	li.ewald = ewald;
+	li.hnear = soft_len * 1.001 + 1e-9;  // the host's margin over the kernel's single-precision test
+	li.box = box;
+	li.near = static_cast<uint8_t*>(scratch(size_t(std::max<int64_t>(L.len[5], 2)) / 2 + 1));
+	if (!li.near) PCHK(hipErrorOutOfMemory);
 	hipLaunchKernelGGL(k_node_count, dim3(blocks(np, 256)), dim3(256), 0, s, ni, nent, nchk, nslot);
 	PCHK(hipGetLastError());
-	for (int q = 0; q < 4; q++) {
-		PCHK(exclusive_scan(nent + q * np, oent + q * np, np));
-		PCHK(exclusive_scan(nchk + q * np, ochk + q * np, np));
+	if (nl > 0) {
+		hipLaunchKernelGGL(k_leaf_boxes, dim3(unsigned(nl)), dim3(64), 0, s, li.leaf_items, li.parts, box);
+		PCHK(hipGetLastError());
 	}
-	PCHK(exclusive_scan(nslot, slot_ptr, np));
-	int64_t nlen[4], nch[4], nslots;
+	hipLaunchKernelGGL(k_leaf_count, dim3(unsigned(lp)), dim3(64), 0, s, li, lent, lnear, litem, sums);
+	PCHK(hipGetLastError());
+	int64_t nlen[4], nch[4], nslots, llen[4], nitems[4];
+	uint64_t census[8];
 	{
-		int64_t v[9];
-		std::vector<const int64_t*> arrs;
-		std::vector<int64_t> at;
+		// two sets of columns, one wait
+		ScanSet a, b;
+		for (int q = 0; q < 4; q++) a.add(nent + q * np, oent + q * np, np);
+		for (int q = 0; q < 4; q++) a.add(nchk + q * np, ochk + q * np, np);
+		a.add(nslot, slot_ptr, np);
+		for (int q = 0; q < 4; q++) b.add(lent + q * lp, olent + q * lp, lp);
+		for (int q = 0; q < 4; q++) b.add(litem + q * lp, olitem + q * lp, lp);
+		for (int k = 0; k < 8; k++) b.add(sums + k * lp, osums + k * lp, lp);
+		int64_t* wa = words(scan_workspace(a));
+		int64_t* wb = words(scan_workspace(b));
+		int64_t* tot = words(32);
+		if (!wa || !wb || !tot) PCHK(hipErrorOutOfMemory);
+		PCHK(scan_columns(a, wa, tot, s));
+		PCHK(scan_columns(b, wb, tot + a.cols, s));
+		int64_t v[25];
+		PCHK(hipMemcpyAsync(v, tot, sizeof(v), hipMemcpyDeviceToHost, s));
+		PCHK(hipStreamSynchronize(s));
 		for (int q = 0; q < 4; q++) {
-			arrs.push_back(oent + q * np);
-			at.push_back(nn);
-			arrs.push_back(ochk + q * np);
-			at.push_back(nn);
-		}
-		arrs.push_back(slot_ptr);
-		at.push_back(nn);
-		PCHK(lasts(arrs, at, v));
-		for (int q = 0; q < 4; q++) {
-			nlen[q] = v[2 * q];
-			nch[q] = v[2 * q + 1];
+			nlen[q] = v[q];
+			nch[q] = v[4 + q];
+			llen[q] = v[9 + q];
+			nitems[q] = v[13 + q];
 		}
 		nslots = v[8];
+		for (int k = 0; k < 8; k++) census[k] = uint64_t(v[17 + k]);
 	}
-	for (int q = 0; q < 4; q++)
-		if (nlen[q] > int64_t(INT32_MAX)) {
+	for (int q = 0; q < 4; q++) {
+		if (int64_t(census[4 + q]) != L.len[4 + q]) {
+			err = "device list work: leaf-kind entries outside the non-empty leaves";
+			return TG_EINVAL;
+		}
+		if (nlen[q] > int64_t(INT32_MAX) || llen[q] > int64_t(INT32_MAX) || nitems[q] > int64_t(INT32_MAX)) {
 			err = "an interaction list exceeds 2^31 entries (32-bit list offsets)";
 			return TG_EINVAL;
 		}
+	}
 	if (nslots > int64_t(INT32_MAX)) {
 		err = "partial slots exceed 2^31";
 		return TG_EINVAL;
 	}
+
+	// ---- node kinds ----
 	n_slots = nslots;
 	PCHK(d_slot_node.alloc(std::max<size_t>(size_t(nslots) * 4, 16)));
 	NodeOut no{};
 	no.slot_node = d_slot_node.as<int>();
-	for (int q = 0; q < 4; q++) {
-		no.chunks[q] = static_cast<int2*>(scratch(size_t(nch[q]) * sizeof(int2)));
-		no.chunk_slot[q] = static_cast<int*>(scratch(size_t(nch[q]) * 4));
-		if (!no.chunks[q] || !no.chunk_slot[q]) PCHK(hipErrorOutOfMemory);
-	}
-	if (nn > 0) {
-		hipLaunchKernelGGL(k_node_chunks, dim3(blocks(nn, 256)), dim3(256), 0, s, ni, nent, oent, ochk, slot_ptr, no);
-		PCHK(hipGetLastError());
-	}
-	// lists: CC the walk's own, CP expanded; owners; waves
+	ChunkSet cs{};
+	int64_t nch_max = 0;
 	for (int q = 0; q < 4; q++) {
 		KindWork& w = work[NODE_KIND[q]];
+		// kept with the work: the slots of all entries are written from them on demand (complete_owners)
+		PCHK(w.chunks.alloc(std::max<size_t>(size_t(nch[q]) * sizeof(int2), 16)));
+		PCHK(w.chunk_slot.alloc(std::max<size_t>(size_t(nch[q]) * 4, 16)));
+		w.nchunks = nch[q];
+		no.chunks[q] = w.chunks.as<int2>();
+		no.chunk_slot[q] = w.chunk_slot.as<int>();
+		// lists: CC the walk's own, CP expanded
 		w.list.release();
 		if (q & 1) {
 			PCHK(w.list.alloc(std::max<size_t>(size_t(nlen[q]) * 4, 16)));
@@ -792,125 +896,61 @@ int Solver::upload_lists_device() {
 		}
 		w.nlist = nlen[q];
 		PCHK(w.owner.alloc(std::max<size_t>(size_t(nlen[q]) * 4, 16)));
-		if (nch[q] > 0) {
-			hipLaunchKernelGGL(k_node_owner, dim3(blocks(nch[q], 4)), dim3(256), 0, s, no.chunks[q], no.chunk_slot[q], nch[q], w.owner.as<int>());
+		PCHK(w.items.alloc(std::max<size_t>(size_t(nch[q]) * sizeof(int2), 16)));  // a wave holds a chunk or more
+		cs.chunks[q] = no.chunks[q];
+		cs.slot[q] = no.chunk_slot[q];
+		cs.owner[q] = w.owner.as<int>();
+		cs.nch[q] = nch[q];
+		nch_max = std::max(nch_max, nch[q]);
+	}
+	owners_complete = false;
+	if (nn > 0) {
+		hipLaunchKernelGGL(k_node_chunks, dim3(blocks(nn, 256)), dim3(256), 0, s, ni, nent, oent, ochk, slot_ptr, no);
+		PCHK(hipGetLastError());
+		if (L.len[1] > 0 || L.len[3] > 0) {
+			hipLaunchKernelGGL(k_node_expand, dim3(unsigned(nn)), dim3(64), 0, s, ni, oent, work[CP_DIRECT].list.as<int32_t>(),
+					work[CP_EWALD].list.as<int32_t>());
 			PCHK(hipGetLastError());
 		}
 	}
-	if (nn > 0 && (L.len[1] > 0 || L.len[3] > 0)) {
-		hipLaunchKernelGGL(k_node_expand, dim3(unsigned(nn)), dim3(64), 0, s, ni, oent, work[CP_DIRECT].list.as<int32_t>(),
-				work[CP_EWALD].list.as<int32_t>());
+	int64_t* d_nwaves = words(4);
+	if (!d_nwaves) PCHK(hipErrorOutOfMemory);
+	if (nch_max > 0) {
+		hipLaunchKernelGGL(k_node_owner, dim3(blocks(nch_max, 4), 4), dim3(256), 0, s, cs, 0);
 		PCHK(hipGetLastError());
 	}
 	{
-		int64_t* nw[4];
-		int64_t* ow[4];
-		int64_t nseg[4];
-		std::vector<const int64_t*> arrs;
-		std::vector<int64_t> at;
+		PackOut po{};
+		ScanSet sc;
+		int64_t nseg_max = 0;
 		for (int q = 0; q < 4; q++) {
-			nseg[q] = (nch[q] + WAVE_SEGMENT - 1) / WAVE_SEGMENT;
-			nw[q] = static_cast<int64_t*>(scratch(size_t(nseg[q] + 1) * 8));
-			ow[q] = static_cast<int64_t*>(scratch(size_t(nseg[q] + 1) * 8));
-			if (!nw[q] || !ow[q]) PCHK(hipErrorOutOfMemory);
-			hipLaunchKernelGGL(k_wave_count, dim3(blocks(nseg[q] + 1, 256)), dim3(256), 0, s, no.chunks[q], nch[q], nseg[q], nw[q]);
-			PCHK(hipGetLastError());
-			PCHK(exclusive_scan(nw[q], ow[q], nseg[q] + 1));
-			arrs.push_back(ow[q]);
-			at.push_back(nseg[q]);
+			po.nseg[q] = (nch[q] + WAVE_SEGMENT - 1) / WAVE_SEGMENT;
+			po.nw[q] = words(po.nseg[q] + 1);
+			int64_t* ow = words(po.nseg[q] + 1);
+			if (!po.nw[q] || !ow) PCHK(hipErrorOutOfMemory);
+			po.ow[q] = ow;
+			po.waves[q] = work[NODE_KIND[q]].items.as<int2>();
+			sc.add(po.nw[q], ow, po.nseg[q]);
+			nseg_max = std::max(nseg_max, po.nseg[q]);
 		}
-		int64_t nwaves[4];
-		PCHK(lasts(arrs, at, nwaves));
-		for (int q = 0; q < 4; q++) {
-			KindWork& w = work[NODE_KIND[q]];
-			PCHK(w.items.alloc(std::max<size_t>(size_t(nwaves[q]) * sizeof(int2), 16)));
-			w.nitems = int(nwaves[q]);
-			if (nseg[q] > 0) {
-				hipLaunchKernelGGL(k_wave_write, dim3(blocks(nseg[q], 256)), dim3(256), 0, s, no.chunks[q], nch[q], nseg[q], ow[q],
-						w.items.as<int2>());
-				PCHK(hipGetLastError());
-			}
-			list_bytes += int64_t(nwaves[q]) * int64_t(sizeof(int2)) + nlen[q] * 4;
+		int64_t* ws = words(scan_workspace(sc));
+		if (!ws) PCHK(hipErrorOutOfMemory);
+		if (nseg_max > 0) {
+			hipLaunchKernelGGL(k_wave_count, dim3(unsigned(nseg_max), 4), dim3(WAVE_SEGMENT), 0, s, cs, po);
+			PCHK(hipGetLastError());
+		}
+		PCHK(scan_columns(sc, ws, d_nwaves, s));
+		if (nseg_max > 0) {
+			hipLaunchKernelGGL(k_wave_write, dim3(unsigned(nseg_max), 4), dim3(WAVE_SEGMENT), 0, s, cs, po);
+			PCHK(hipGetLastError());
 		}
 	}
 
 	// ---- leaf kinds ----
-	LeafIn li{};
-	for (int q = 0; q < 4; q++) {
-		li.ptr[q] = L.ptr(4 + q);
-		li.val[q] = L.val[4 + q];
-	}
-	li.leaf_items = d_leaf_items.as<int4>();
-	li.parts = d_parts.as<int4>();
-	li.pleaf = d_pleaf.as<int>();
-	li.nodes = L.nodes;
-	li.nl = nl;
-	li.ewald = ewald;
-	li.hnear = soft_len * 1.001 + 1e-9;  // the host's margin over the kernel's single-precision test
-	int4* box = static_cast<int4*>(scratch(size_t(std::max<int64_t>(nn, 1)) * 2 * sizeof(int4)));
-	const int64_t lp = nl + 1;
-	int64_t* lent = static_cast<int64_t*>(scratch(4 * lp * 8));
-	int64_t* olent = static_cast<int64_t*>(scratch(4 * lp * 8));
-	int64_t* litem = static_cast<int64_t*>(scratch(4 * lp * 8));
-	int64_t* olitem = static_cast<int64_t*>(scratch(4 * lp * 8));
-	int64_t* lnear = static_cast<int64_t*>(scratch(lp * 8));
-	int64_t* sums = static_cast<int64_t*>(scratch(8 * lp * 8));   // per leaf, 8 columns
-	int64_t* sum_tot = static_cast<int64_t*>(scratch(8 * 8));     // their totals
-	if (!box || !lent || !olent || !litem || !olitem || !lnear || !sums || !sum_tot) PCHK(hipErrorOutOfMemory);
-	li.box = box;
-	li.near = static_cast<uint8_t*>(scratch(size_t(std::max<int64_t>(L.len[5], 2)) / 2 + 1));
-	if (!li.near) PCHK(hipErrorOutOfMemory);
-	if (nl > 0) {
-		hipLaunchKernelGGL(k_leaf_boxes, dim3(unsigned(nl)), dim3(64), 0, s, li.leaf_items, li.parts, box);
-		PCHK(hipGetLastError());
-	}
-	hipLaunchKernelGGL(k_leaf_count, dim3(unsigned(lp)), dim3(64), 0, s, li, lent, lnear, litem, sums);
-	PCHK(hipGetLastError());
-	for (int q = 0; q < 4; q++) {
-		PCHK(exclusive_scan(lent + q * lp, olent + q * lp, lp));
-		PCHK(exclusive_scan(litem + q * lp, olitem + q * lp, lp));
-	}
-	for (int k = 0; k < 8; k++) {
-		size_t need = 0;
-		PCHK(hipcub::DeviceReduce::Sum(nullptr, need, sums + k * lp, sum_tot + k, lp, s));
-		void* tmp_r = scratch(need);
-		if (!tmp_r) PCHK(hipErrorOutOfMemory);
-		PCHK(hipcub::DeviceReduce::Sum(tmp_r, need, sums + k * lp, sum_tot + k, lp, s));
-	}
-	int64_t llen[4], nitems[4];
-	uint64_t census[8];
-	{
-		std::vector<const int64_t*> arrs;
-		std::vector<int64_t> at;
-		for (int q = 0; q < 4; q++) {
-			arrs.push_back(olent + q * lp);
-			at.push_back(nl);
-			arrs.push_back(olitem + q * lp);
-			at.push_back(nl);
-		}
-		for (int k = 0; k < 8; k++) {
-			arrs.push_back(sum_tot);
-			at.push_back(k);
-		}
-		int64_t v[16];
-		PCHK(lasts(arrs, at, v));
-		for (int q = 0; q < 4; q++) {
-			llen[q] = v[2 * q];
-			nitems[q] = v[2 * q + 1];
-		}
-		for (int k = 0; k < 8; k++) census[k] = uint64_t(v[8 + k]);
-	}
-	for (int q = 0; q < 4; q++) {
-		if (int64_t(census[4 + q]) != L.len[4 + q]) {
-			err = "device list work: leaf-kind entries outside the non-empty leaves";
-			return TG_EINVAL;
-		}
-		if (llen[q] > int64_t(INT32_MAX) || nitems[q] > int64_t(INT32_MAX)) {
-			err = "an interaction list exceeds 2^31 entries (32-bit list offsets)";
-			return TG_EINVAL;
-		}
-	}
 	LeafOut lo{};
+	SortSet so{};
+	int64_t tiles_max = 0;
+	ScanSet sc;
 	for (int q = 0; q < 4; q++) {
 		KindWork& w = work[LEAF_KIND[q]];
 		w.list.release();
@@ -924,34 +964,43 @@ int Solver::upload_lists_device() {
 		}
 		w.owner.release();
 		w.nlist = llen[q];
+		w.nitems = int(nitems[q]);
+		PCHK(w.items.alloc(std::max<size_t>(size_t(nitems[q]) * sizeof(int4), 16)));
+		list_bytes += nitems[q] * int64_t(sizeof(int4));
 		lo.items[q] = static_cast<int4*>(scratch(size_t(nitems[q]) * sizeof(int4)));
-		lo.key[q] = static_cast<unsigned long long*>(scratch(size_t(nitems[q]) * 8));
-		lo.idx[q] = static_cast<int*>(scratch(size_t(nitems[q]) * 4));
-		if (!lo.items[q] || !lo.key[q] || !lo.idx[q]) PCHK(hipErrorOutOfMemory);
+		lo.cls[q] = static_cast<uint8_t*>(scratch(size_t(nitems[q])));
+		const int64_t tiles = (nitems[q] + SORT_TILE - 1) / SORT_TILE;
+		tiles_max = std::max(tiles_max, tiles);
+		so.hist[q] = words(CLASSES * tiles);
+		int64_t* place = words(CLASSES * tiles);
+		if (!lo.items[q] || !lo.cls[q] || !so.hist[q] || !place) PCHK(hipErrorOutOfMemory);
+		so.place[q] = place;
+		so.in[q] = lo.items[q];
+		so.cls[q] = lo.cls[q];
+		so.out[q] = w.items.as<int4>();
+		so.n[q] = nitems[q];
+		sc.add(so.hist[q], place, CLASSES * tiles);
 	}
 	if (nl > 0) {
 		hipLaunchKernelGGL(k_leaf_write, dim3(unsigned(nl)), dim3(64), 0, s, li, lent, olent, lnear, olitem, lo);
 		PCHK(hipGetLastError());
 	}
-	// heaviest cost class first, leaf order within a class: a stable radix sort of (class, index),
-	// descending
-	for (int q = 0; q < 4; q++) {
-		KindWork& w = work[LEAF_KIND[q]];
-		const int m = int(nitems[q]);
-		PCHK(w.items.alloc(std::max<size_t>(size_t(m) * sizeof(int4), 16)));
-		w.nitems = m;
-		list_bytes += int64_t(m) * int64_t(sizeof(int4));
-		if (m == 0) continue;
-		unsigned long long* key_out = static_cast<unsigned long long*>(scratch(size_t(m) * 8));
-		int* idx_out = static_cast<int*>(scratch(size_t(m) * 4));
-		if (!key_out || !idx_out) PCHK(hipErrorOutOfMemory);
-		size_t need = 0;
-		PCHK(hipcub::DeviceRadixSort::SortPairsDescending(nullptr, need, lo.key[q], key_out, lo.idx[q], idx_out, m, 0, 8, s));
-		void* sort_tmp = scratch(need);
-		if (!sort_tmp) PCHK(hipErrorOutOfMemory);
-		PCHK(hipcub::DeviceRadixSort::SortPairsDescending(sort_tmp, need, lo.key[q], key_out, lo.idx[q], idx_out, m, 0, 8, s));
-		hipLaunchKernelGGL(k_gather_items, dim3(blocks(m, 256)), dim3(256), 0, s, lo.items[q], idx_out, int64_t(m), w.items.as<int4>());
+	if (tiles_max > 0) {
+		// heaviest cost class first, leaf order within a class
+		hipLaunchKernelGGL(k_item_hist, dim3(unsigned(tiles_max), 4), dim3(SORT_TILE), 0, s, so);
 		PCHK(hipGetLastError());
+		int64_t* ws = words(scan_workspace(sc) + 4);
+		if (!ws) PCHK(hipErrorOutOfMemory);
+		PCHK(scan_columns(sc, ws + 4, ws, s));
+		hipLaunchKernelGGL(k_item_scatter, dim3(unsigned(tiles_max), 4), dim3(SORT_TILE), 0, s, so);
+		PCHK(hipGetLastError());
+	}
+	int64_t nwaves[4];
+	PCHK(hipMemcpyAsync(nwaves, d_nwaves, sizeof(nwaves), hipMemcpyDeviceToHost, s));
+	PCHK(hipStreamSynchronize(s));
+	for (int q = 0; q < 4; q++) {
+		work[NODE_KIND[q]].nitems = int(nwaves[q]);
+		list_bytes += nwaves[q] * int64_t(sizeof(int2)) + nlen[q] * 4;
 	}
 	// the census as the reference counts it (node kinds: sources; leaf kinds: sinks x sources)
 	Census& C = tree.census;
@@ -963,7 +1012,28 @@ int Solver::upload_lists_device() {
 	C.PP_direct = census[1];
 	C.PC_ewald = census[2];
 	C.PP_ewald = census[3];
-	PCHK(hipStreamSynchronize(s));
+	return TG_OK;
+}
+
+int Solver::complete_owners() {
+	if (owners_complete) return TG_OK;
+	PCHK(hipSetDevice(device));
+	ChunkSet cs{};
+	int64_t nch_max = 0;
+	for (int q = 0; q < 4; q++) {
+		KindWork& w = work[NODE_KIND[q]];
+		cs.chunks[q] = w.chunks.as<int2>();
+		cs.slot[q] = w.chunk_slot.as<int>();
+		cs.owner[q] = w.owner.as<int>();
+		cs.nch[q] = w.nchunks;
+		nch_max = std::max(nch_max, w.nchunks);
+	}
+	if (nch_max > 0) {
+		hipLaunchKernelGGL(k_node_owner, dim3(blocks(nch_max, 4), 4), dim3(256), 0, stream, cs, 1);
+		PCHK(hipGetLastError());
+		PCHK(hipStreamSynchronize(stream));
+	}
+	owners_complete = true;
 	return TG_OK;
 }
 

@@ -322,6 +322,8 @@ Solver::~Solver() {
 			w.items.release();
 			w.list.release();
 			w.owner.release();
+			w.chunks.release();
+			w.chunk_slot.release();
 		}
 		dlists.release();
 		dtree.release();
@@ -391,24 +393,25 @@ int Solver::set_particles(const int32_t* x, const float* mass, int64_t count, bo
 	for (auto& w : work)
 		if (!w.list.owned) w.list.release();
 	lists_on_device = false;
-	// the build's working buffers, freed when its stream has drained
+	// the build's working buffers are freed when its stream has drained, on every way out
 	struct Later {
-		hipStream_t s;
-		std::vector<void*> blocks;
+		Solver& S;
 		~Later() {
-			if (blocks.empty()) return;
-			(void) hipStreamSynchronize(s);
-			for (void* p : blocks) dev_free(p);
+			if (S.build_later.empty()) return;
+			(void) hipStreamSynchronize(S.stream);
+			for (void* p : S.build_later) dev_free(p);
+			S.build_later.clear();
 		}
-	} later{stream, {}};
+	} later{*this};
+	owners_complete = true;
 	if (gpu_walk) {
 		// the lists stay on the device; the work is built from them there (upload_lists_device)
 		WalkNode* wn = nullptr;
 		if (tree_on_device) {
-			const hipError_t e = walk_nodes_device(dtree, &wn, stream, err, later.blocks);
+			const hipError_t e = walk_nodes_device(dtree, &wn, stream, err, build_later);
 			if (e != hipSuccess) return e == hipErrorOutOfMemory ? TG_ENOMEM : TG_EHIP;
 		}
-		const hipError_t e = device_walk(tree, device, stream, err, t_detail, &dlists, wn, n_nodes, &walk_hint, later.blocks);
+		const hipError_t e = device_walk(tree, device, stream, err, t_detail, &dlists, wn, n_nodes, &walk_hint, build_later);
 		if (e != hipSuccess) return e == hipErrorOutOfMemory ? TG_ENOMEM : TG_EHIP;
 		lists_on_device = true;
 	} else {
@@ -1249,6 +1252,8 @@ int64_t tg_solver_export(tg_solver* h, const char* name, void* dst, int64_t capa
 				a = &w.list;
 				bytes = size_t(w.nlist) * 4;
 			} else if (what == "work_owner" && node_kind) {
+				const int rc = S.complete_owners();
+				if (rc != TG_OK) return fail(h, rc);
 				a = &w.owner;
 				bytes = size_t(w.nlist) * 4;
 			} else {

@@ -30,7 +30,10 @@ struct DeviceArray {
 struct KindWork {
 	DeviceArray items;  // int4 leaf items (PP/PC) or int2 waves (CC/CP)
 	DeviceArray list;   // int32 source indices
-	DeviceArray owner;  // int32 partial slot per list entry (CC/CP)
+	DeviceArray owner;  // int32 partial slot per list entry (CC/CP); of a chunk's first 64 entries until complete_owners
+	// device-prepared node kinds: [begin, end) entries and partial slot of each chunk
+	DeviceArray chunks, chunk_slot;
+	int64_t nchunks = 0;
 	int nitems = 0;
 	int64_t nlist = 0;
 };
@@ -120,6 +123,9 @@ struct Solver {
 	int upload();
 	int upload_lists_device();  // every kind's work from dlists, on the device (tg_prep.hip)
 	int upload_tree_device();   // the tree's arrays from dtree, on the device (tg_prep.hip)
+	int complete_owners();      // the partial slots of all entries of device-prepared node kinds (the solve reads the first 64 of a chunk)
+	bool owners_complete = true;
+	std::vector<void*> build_later;  // a build's working buffers, freed when its stream has drained
 	int host_tree();            // copies the device build's tree into tree
 	int host_lists();  // copies the device walk's lists into tree.lists
 	int upload_sources();
