@@ -31,5 +31,5 @@ def test_stages(n, leaf, theta, chunk, ewald):
         s.close()
     for name in NAMES:
         assert np.array_equal(got[0][name], got[1][name]), name
-    for key in ("count", "items", "list_len", "list_bytes"):
+    for key in ("count", "items", "list_len"):
         assert got[0]["info"][key] == got[1]["info"][key], key

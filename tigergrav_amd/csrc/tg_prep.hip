@@ -548,59 +548,6 @@ unsigned blocks(int64_t n, int per) { return unsigned((n + per - 1) / per); }
 
 // ---- the tree's arrays from a device-built tree ---------------------------------------------------
 
-// the walk's node table: one level of nodes, deepest levels first.  sbox: per node the box of its
-// particles (leaves) or the union of its non-empty children's (Tree::sink_spans); span its
-// diagonal, in FP64 with the host's operations
-__global__ __launch_bounds__(256) void k_tw_walk_nodes(const DNode* __restrict__ nodes, const DMulti* __restrict__ multi, int lb, int nl,
-		double* __restrict__ sbox, WalkNode* __restrict__ wn) {
-#pragma clang fp contract(off)
-	const int j = blockIdx.x * 256 + threadIdx.x;
-	if (j >= nl) return;
-	const int k = lb + j;
-	const DNode nd = nodes[k];
-	const DMulti& m = multi[k];
-	double mn[3] = {1.0, 1.0, 1.0}, mx[3] = {0.0, 0.0, 0.0};
-	const bool empty = nd.pend == nd.pbegin;
-	if (!empty) {
-		if (nd.c0 < 0) {
-			for (int d = 0; d < 3; d++) {
-				mn[d] = m.rmin[d];
-				mx[d] = m.rmax[d];
-			}
-		} else {
-			const int ch[2] = {nd.c0, nd.c1};
-			for (int c = 0; c < 2; c++) {
-				if (nodes[ch[c]].pend == nodes[ch[c]].pbegin) continue;
-				const double* b = sbox + 6 * int64_t(ch[c]);
-				for (int d = 0; d < 3; d++) {
-					mx[d] = mx[d] < b[3 + d] ? b[3 + d] : mx[d];
-					mn[d] = b[d] < mn[d] ? b[d] : mn[d];
-				}
-			}
-		}
-	}
-	double* o = sbox + 6 * int64_t(k);
-	for (int d = 0; d < 3; d++) {
-		o[d] = mn[d];
-		o[3 + d] = mx[d];
-	}
-	float span = 0.0f;
-	if (!empty) {
-		double s2 = 0.0;
-		for (int d = 0; d < 3; d++) s2 += (mx[d] - mn[d]) * (mx[d] - mn[d]);
-		span = float(sqrt(s2));
-	}
-	WalkNode w;
-	w.pbegin = nd.pbegin;
-	w.pend = nd.pend;
-	w.c0 = nd.c0;
-	w.c1 = nd.c1;
-	for (int d = 0; d < 3; d++) w.x[d] = m.x[d];
-	w.r = m.r;
-	w.rmax = span;
-	wn[k] = w;
-}
-
 // particle records (x, y, z, mass bits) and the input order
 __global__ __launch_bounds__(256) void k_tw_parts(const int32_t* __restrict__ pos, const float* __restrict__ mass, const int64_t* __restrict__ order,
 		int64_t n, int4* __restrict__ parts, int64_t* __restrict__ order_out) {
@@ -651,29 +598,6 @@ __global__ __launch_bounds__(64) void k_tw_pleaf(const int4* __restrict__ leaf_i
 }
 
 }  // namespace
-
-hipError_t walk_nodes_device(const DeviceTree& D, WalkNode** out, hipStream_t s, std::string& err, std::vector<void*>& later) {
-	*out = nullptr;
-	const int64_t nn = D.nn;
-	WalkNode* wn = nullptr;
-	double* sbox = nullptr;
-	hipError_t e = dev_malloc(&wn, size_t(std::max<int64_t>(nn, 1)) * sizeof(WalkNode));
-	if (e == hipSuccess) e = dev_malloc(&sbox, size_t(std::max<int64_t>(nn, 1)) * 6 * sizeof(double));
-	for (size_t l = D.level_begin.size() - 1; e == hipSuccess && l-- > 0;) {
-		const int b = D.level_begin[l], nl = D.level_begin[l + 1] - b;
-		if (nl <= 0) continue;
-		hipLaunchKernelGGL(k_tw_walk_nodes, dim3(blocks(nl, 256)), dim3(256), 0, s, D.nodes, D.multi, b, nl, sbox, wn);
-		e = hipGetLastError();
-	}
-	if (sbox) later.push_back(sbox);
-	if (e != hipSuccess) {
-		if (wn) later.push_back(wn);
-		err = std::string("walk node table: ") + hipGetErrorString(e);
-		return e;
-	}
-	*out = wn;
-	return hipSuccess;
-}
 
 #define PCHK(call)                                                   \
 	do {                                                             \

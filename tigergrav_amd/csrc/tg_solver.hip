@@ -357,6 +357,16 @@ int Solver::set_particles(const int32_t* x, const float* mass, int64_t count, bo
 		if (stream2) SCHK(hipStreamSynchronize(stream2));
 		if (stream3) SCHK(hipStreamSynchronize(stream3));
 	}
+	// the build's working buffers are freed when its stream has drained, on every way out
+	struct Later {
+		Solver& S;
+		~Later() {
+			if (S.build_later.empty()) return;
+			(void) hipStreamSynchronize(S.stream);
+			for (void* p : S.build_later) dev_free(p);
+			S.build_later.clear();
+		}
+	} later{*this};
 	order_on_device = false;
 	fof_group.clear();
 	n = count;
@@ -374,7 +384,8 @@ int Solver::set_particles(const int32_t* x, const float* mass, int64_t count, bo
 	tree_on_device = false;
 	if (gpu_tree && device >= 0) {
 		double tt[2] = {0.0, 0.0};
-		const hipError_t e = device_build_tree(tree, x, mass, count, P, m, device, stream, err, tt, on_device, keep_tree ? &dtree : nullptr);
+		const hipError_t e = device_build_tree(tree, x, mass, count, P, m, device, stream, err, tt, on_device, keep_tree ? &dtree : nullptr,
+				build_later);
 		if (e != hipSuccess) return e == hipErrorOutOfMemory ? TG_ENOMEM : TG_EHIP;
 		tree_on_device = keep_tree;
 		t1 = t0 + tt[0];
@@ -393,23 +404,13 @@ int Solver::set_particles(const int32_t* x, const float* mass, int64_t count, bo
 	for (auto& w : work)
 		if (!w.list.owned) w.list.release();
 	lists_on_device = false;
-	// the build's working buffers are freed when its stream has drained, on every way out
-	struct Later {
-		Solver& S;
-		~Later() {
-			if (S.build_later.empty()) return;
-			(void) hipStreamSynchronize(S.stream);
-			for (void* p : S.build_later) dev_free(p);
-			S.build_later.clear();
-		}
-	} later{*this};
 	owners_complete = true;
 	if (gpu_walk) {
 		// the lists stay on the device; the work is built from them there (upload_lists_device)
 		WalkNode* wn = nullptr;
 		if (tree_on_device) {
-			const hipError_t e = walk_nodes_device(dtree, &wn, stream, err, build_later);
-			if (e != hipSuccess) return e == hipErrorOutOfMemory ? TG_ENOMEM : TG_EHIP;
+			wn = dtree.walk;  // the walk owns it from here on
+			dtree.walk = nullptr;
 		}
 		const hipError_t e = device_walk(tree, device, stream, err, t_detail, &dlists, wn, n_nodes, &walk_hint, build_later);
 		if (e != hipSuccess) return e == hipErrorOutOfMemory ? TG_ENOMEM : TG_EHIP;

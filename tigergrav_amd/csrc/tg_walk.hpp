@@ -57,11 +57,4 @@ struct WalkHint {
 hipError_t device_walk(Tree& T, int device, hipStream_t s, std::string& err, double* t, DeviceLists* keep, WalkNode* nodes, int64_t nn,
 		WalkHint* hint, std::vector<void*>& later);
 
-struct DeviceTree;
-// the walk's node table of a device-built tree, made on the device (*out: nn nodes, device memory
-// the caller frees): the centres, radii and children, and each node's sink span from a bottom-up
-// union of its non-empty leaves' particle boxes, as Tree::sink_spans forms it.  Enqueued on s; `later`
-// as for device_walk.
-hipError_t walk_nodes_device(const DeviceTree& D, WalkNode** out, hipStream_t s, std::string& err, std::vector<void*>& later);
-
 }  // namespace tg
