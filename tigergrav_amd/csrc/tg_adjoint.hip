@@ -25,6 +25,7 @@
 // atomics (one per source node and item), so their summation order varies between runs; Lambda and
 // the particle gradients are not.
 #include <hip/hip_runtime.h>
+#include <hipcub/hipcub.hpp>  // DeviceRadixSort of the pair keys
 
 #include <algorithm>
 #include <cmath>
@@ -32,6 +33,9 @@
 #include <vector>
 
 #include "tg_adjoint_math.hpp"
+#include "tg_devmem.hpp"
+#include "tg_leaf_waves.hpp"
+#include "tg_scan.hpp"
 #include "tg_gravity.h"
 #include "tg_local.hpp"
 #include "tg_solver.hpp"
@@ -280,53 +284,82 @@ struct AdjItems {
 	int nitems;
 };
 
-// PP direct: one item per group, lane = sink, sources in LDS tiles of 64 with their weights.
+// the lanes of an item's wave: sinks padded to a power of two nsp, the P = 64 / nsp lane groups
+// (phases) splitting the sources, so leaves of 32 or fewer particles keep every lane busy; the
+// NW waves of the group share the list (tg_leaf_waves.hpp)
+template <int NW>
+struct LeafLanes {
+	int lane, wave, ns, nsp, P, si, ph, pi;
+	int2 share;
+	__device__ __forceinline__ LeafLanes(const int4& it) {
+		lane = threadIdx.x & 63;
+		wave = NW == 1 ? 0 : int(threadIdx.x >> 6);
+		ns = it.y & PP_COUNT_MASK;
+		const int lg = ns <= 1 ? 0 : 32 - __clz(ns - 1);
+		nsp = 1 << lg;
+		P = 64 >> lg;
+		si = lane & (nsp - 1);
+		ph = lane >> lg;
+		pi = it.x + min(si, ns - 1);
+		share = wave_share<NW>(it.z, it.w, wave);
+	}
+	// the sums of all phases and waves onto the sink's gradient
+	__device__ __forceinline__ void store(double gm, double* gx, double (*red)[4][64], double* grad) {
+		leaf_sums<NW>(gm, gx, nsp, lane, wave, red);
+		if (wave == 0 && ph == 0 && si < ns) {
+			double* o = grad + 4 * int64_t(pi);
+			o[0] += gx[0];
+			o[1] += gx[1];
+			o[2] += gx[2];
+			o[3] += gm;
+		}
+	}
+};
+
+// PP direct: lane = (sink, phase), sources in LDS tiles of 64 with their weights.
 // The lists are symmetric, so particle k's own list carries its source-side terms as well:
 //   dL/dx_k += sum_j J(d_kj) (m_j w_k - m_k w_j),  J v = -f v - (f'/r)(d.v) d,
 //   dL/dm_k += sum_j f(d_kj) (d_kj . w_j)
-__global__ __launch_bounds__(64) void k_adj_pp(AdjArgs A, AdjItems I) {
+// Bound by FP32 arithmetic (about 45 instructions a pair) where enough waves are in flight: one
+// wave per item left the longest lists of clustered sets to run alone.
+template <int NW, bool WRAP>
+__global__ __launch_bounds__(64 * NW) void k_adj_pp(AdjArgs A, AdjItems I) {
 	const int4 it = I.items[blockIdx.x];
-	const int t = threadIdx.x;
-	const int ns = it.y & PP_COUNT_MASK;
-	// sinks padded to a power of two nsp; the P = 64 / nsp lane groups (phases) split each tile's
-	// sources, so leaves of 32 or fewer particles keep every lane busy
-	const int lg = ns <= 1 ? 0 : 32 - __clz(ns - 1);
-	const int nsp = 1 << lg;
-	const int P = 64 >> lg;
-	const int si = t & (nsp - 1);
-	const int ph = t >> lg;
+	LeafLanes<NW> T(it);
 	const int near_len = int(unsigned(it.y) >> PP_NEAR_SHIFT);
 	const int near_end = near_len == PP_NEAR_ALL ? INT_MAX : it.z + near_len;
-	const int pi = it.x + min(si, ns - 1);
-	const int4 me = A.parts[pi];
-	const float4 wv = A.w[pi];
+	const int4 me = A.parts[T.pi];
+	const float4 wv = A.w[T.pi];
 	const float wi[3] = {wv.x, wv.y, wv.z};
 	const float mi = __int_as_float(me.w);
-	__shared__ int4 tp[64];
-	__shared__ float4 tw[64];
+	__shared__ int4 tps[NW][64];
+	__shared__ float4 tws[NW][64];
+	__shared__ double red[NW > 1 ? NW - 1 : 1][4][64];
+	int4* tp = tps[T.wave];
+	float4* tw = tws[T.wave];
 	double gx[3] = {0.0, 0.0, 0.0}, gm = 0.0;
-	for (int base = it.z; base < it.w; base += 64) {
-		const int n = min(64, it.w - base);
-		__syncthreads();
-		if (t < n) {
-			const int j = I.list[base + t];
-			tp[t] = A.parts[j];
-			tw[t] = A.w[j];
+	for (int base = T.share.x; base < T.share.y; base += 64) {
+		const int n = min(64, T.share.y - base);
+		wave_lds_sync<NW>();
+		if (T.lane < n) {
+			const int j = I.list[base + T.lane];
+			tp[T.lane] = A.parts[j];
+			tw[T.lane] = A.w[j];
 		}
-		__syncthreads();
+		wave_lds_sync<NW>();
 		float fx[3] = {0.f, 0.f, 0.f}, fm = 0.f;
 		// tiles inside the list's near prefix may hold pairs closer than h (spline); later tiles
 		// hold only pairs at least h apart (the forward's split)
 		const bool near = base < near_end;
-		for (int k = ph; k < n; k += P) {
+		auto pair = [&](int k, bool soft) {
 			const int4 s = tp[k];
 			const float4 ws = tw[k];
 			const float mj = __int_as_float(s.w);
-			const float d[3] = {sepf(me.x, s.x, A.wrap), sepf(me.y, s.y, A.wrap), sepf(me.z, s.z, A.wrap)};
+			const float d[3] = {sepf(me.x, s.x, WRAP), sepf(me.y, s.y, WRAP), sepf(me.z, s.z, WRAP)};
 			const float v[3] = {mj * wi[0] - mi * ws.x, mj * wi[1] - mi * ws.y, mj * wi[2] - mi * ws.z};
 			const float r2 = fmaf(d[2], d[2], fmaf(d[1], d[1], d[0] * d[0]));
 			float f, fr;
-			if (near) {
+			if (soft) {
 				spline_f(r2, A.h, f, fr);
 			} else {
 				const float ri = __builtin_amdgcn_rsqf(r2);
@@ -340,52 +373,48 @@ __global__ __launch_bounds__(64) void k_adj_pp(AdjArgs A, AdjItems I) {
 #pragma unroll
 			for (int b = 0; b < 3; b++) fx[b] = fmaf(-f, v[b], fmaf(-frdv, d[b], fx[b]));
 			fm = fmaf(f, dw, fm);
+		};
+		if (near) {
+			for (int k = T.ph; k < n; k += T.P) pair(k, true);
+		} else {
+#pragma unroll 4
+			for (int k = T.ph; k < n; k += T.P) pair(k, false);
 		}
 #pragma unroll
 		for (int b = 0; b < 3; b++) gx[b] += fx[b];
 		gm += fm;
 	}
-	for (int off = nsp; off < 64; off <<= 1) {
-#pragma unroll
-		for (int b = 0; b < 3; b++) gx[b] += __shfl_xor(gx[b], off, 64);
-		gm += __shfl_xor(gm, off, 64);
-	}
-	if (ph == 0 && si < ns) {
-		double* o = A.grad + 4 * int64_t(pi);
-		o[0] += gx[0];
-		o[1] += gx[1];
-		o[2] += gx[2];
-		o[3] += gm;
-	}
+	T.store(gm, gx, red, A.grad);
 }
 
 // PP Ewald: the correction's F = -D1, J = -D2, per pair from the tabulated correction (its
 // real-space images, Fourier terms and n = 0 term together, as the forward's k_pp_ewald reads them):
 //   dL/dx_k += sum_j J(d_kj) (m_j w_k - m_k w_j),  dL/dm_k += sum_j w_j . D1(d_kj)
-__global__ __launch_bounds__(64) void k_adj_pp_ewald(AdjArgs A, AdjItems I) {
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void k_adj_pp_ewald(AdjArgs A, AdjItems I) {
 	const int4 it = I.items[blockIdx.x];
-	const int t = threadIdx.x;
-	const int ns = it.y & PP_COUNT_MASK;
-	const bool sink = t < ns;
-	const int pi = it.x + min(t, ns - 1);
-	const int4 me = A.parts[pi];
-	const float4 wv = A.w[pi];
+	LeafLanes<NW> T(it);
+	const int4 me = A.parts[T.pi];
+	const float4 wv = A.w[T.pi];
 	const float wi[3] = {wv.x, wv.y, wv.z};
 	const float mi = __int_as_float(me.w);
-	__shared__ int4 tp[64];
-	__shared__ float4 tw[64];
+	__shared__ int4 tps[NW][64];
+	__shared__ float4 tws[NW][64];
+	__shared__ double red[NW > 1 ? NW - 1 : 1][4][64];
+	int4* tp = tps[T.wave];
+	float4* tw = tws[T.wave];
 	double gx[3] = {0.0, 0.0, 0.0}, gm = 0.0;
-	for (int base = it.z; base < it.w; base += 64) {
-		const int n = min(64, it.w - base);
-		__syncthreads();
-		if (t < n) {
-			const int j = I.list[base + t];
-			tp[t] = A.parts[j];
-			tw[t] = A.w[j];
+	for (int base = T.share.x; base < T.share.y; base += 64) {
+		const int n = min(64, T.share.y - base);
+		wave_lds_sync<NW>();
+		if (T.lane < n) {
+			const int j = I.list[base + T.lane];
+			tp[T.lane] = A.parts[j];
+			tw[T.lane] = A.w[j];
 		}
-		__syncthreads();
+		wave_lds_sync<NW>();
 		float fx[3] = {0.f, 0.f, 0.f}, fm = 0.f;
-		for (int k = 0; k < n; k++) {
+		for (int k = T.ph; k < n; k += T.P) {
 			const int4 s = tp[k];
 			const float4 ws = tw[k];
 			const float mj = __int_as_float(s.w);
@@ -410,44 +439,41 @@ __global__ __launch_bounds__(64) void k_adj_pp_ewald(AdjArgs A, AdjItems I) {
 		for (int b = 0; b < 3; b++) gx[b] += fx[b];
 		gm += fm;
 	}
-	if (!sink) return;
-	double* o = A.grad + 4 * int64_t(pi);
-	o[0] += gx[0];
-	o[1] += gx[1];
-	o[2] += gx[2];
-	o[3] += gm;
+	T.store(gm, gx, red, A.grad);
 }
 
-// PC, sink side: lane = sink, over the item's multipoles, dL/dx_i += w . dg/dx_i (fifth derivatives)
-template <bool EWALD>
-__global__ __launch_bounds__(64) void k_adj_pc_sink(AdjArgs A, AdjItems I) {
+// PC, sink side: lane = (sink, phase), over the item's multipoles, dL/dx_i += w . dg/dx_i (fifth
+// derivatives)
+template <int NW, bool EWALD>
+__global__ __launch_bounds__(64 * NW) void k_adj_pc_sink(AdjArgs A, AdjItems I) {
 	const int4 it = I.items[blockIdx.x];
-	const int t = threadIdx.x;
-	const int ns = it.y & PP_COUNT_MASK;
-	if (t >= ns) return;
-	const int pi = it.x + t;
-	const int4 me = A.parts[pi];
-	const float4 wv = A.w[pi];
+	LeafLanes<NW> T(it);
+	__shared__ double red[NW > 1 ? NW - 1 : 1][4][64];
+	const int4 me = A.parts[T.pi];
+	const float4 wv = A.w[T.pi];
 	const float wi[3] = {wv.x, wv.y, wv.z};
-	float gx[3] = {0.f, 0.f, 0.f};
+	double dx[3] = {0.0, 0.0, 0.0};
 	const bool wrapx = EWALD || A.wrap;
-	for (int e = it.z; e < it.w; e++) {
-		const MultiSrc& ms = A.multis[I.list[e]];
-		float M[17];
+	for (int base = T.share.x; base < T.share.y; base += 64) {
+		const int end = min(base + 64, T.share.y);
+		float gx[3] = {0.f, 0.f, 0.f};
+		for (int e = base + T.ph; e < end; e += T.P) {
+			const MultiSrc& ms = A.multis[I.list[e]];
+			float M[17];
 #pragma unroll
-		for (int q = 0; q < 17; q++) M[q] = ms.m[q];
-		const float d[3] = {sepf(me.x, ms.x[0], wrapx), sepf(me.y, ms.x[1], wrapx), sepf(me.z, ms.x[2], wrapx)};
-		float D[adj::NS5];
-		if (EWALD)
-			green_ewald_tab<adj::NS5>(D, d, c_adj_ewt);
-		else
-			adj::green_direct_n<adj::NS5>(D, d);
-		m2p_sink_adjoint(gx, M, D, wi);
+			for (int q = 0; q < 17; q++) M[q] = ms.m[q];
+			const float d[3] = {sepf(me.x, ms.x[0], wrapx), sepf(me.y, ms.x[1], wrapx), sepf(me.z, ms.x[2], wrapx)};
+			float D[adj::NS5];
+			if (EWALD)
+				green_ewald_tab<adj::NS5>(D, d, c_adj_ewt);
+			else
+				adj::green_direct_n<adj::NS5>(D, d);
+			m2p_sink_adjoint(gx, M, D, wi);
+		}
+#pragma unroll
+		for (int b = 0; b < 3; b++) dx[b] += double(gx[b]);
 	}
-	double* o = A.grad + 4 * int64_t(pi);
-	o[0] += double(gx[0]);
-	o[1] += double(gx[1]);
-	o[2] += double(gx[2]);
+	T.store(0.0, dx, red, A.grad);
 }
 
 // PC, source side: lane = multipole of the item's list, over the item's sinks (staged in LDS):
@@ -516,7 +542,8 @@ __global__ __launch_bounds__(64) void k_adj_pc_t(AdjPCArgs A) {
 // to one item, so the gradient is added without atomics.
 struct AdjCPArgs {
 	const int4* items;
-	const int* sinks;
+	const uint64_t* keys;  // first particle << sink_bits | sink node, ascending
+	int sink_bits;
 	const int4* nodepos;
 	const int4* parts;
 	const double* Lam;
@@ -524,10 +551,13 @@ struct AdjCPArgs {
 	int wrap;
 };
 
-template <bool EWALD>
-__global__ __launch_bounds__(64) void k_adj_cp_t(AdjCPArgs A) {
+template <int NW, bool EWALD>
+__global__ __launch_bounds__(64 * NW) void k_adj_cp_t(AdjCPArgs A) {
 	const int4 it = A.items[blockIdx.x];
-	const int t = threadIdx.x;
+	if (it.z == it.w) return;  // no node takes this leaf
+	const int t = threadIdx.x & 63;
+	const int wave = NW == 1 ? 0 : int(threadIdx.x >> 6);
+	const int2 share = wave_share<NW>(it.z, it.w, wave);
 	const int ns = it.y;
 	const int lg = ns <= 1 ? 0 : 32 - __clz(ns - 1);
 	const int nsp = 1 << lg;
@@ -537,19 +567,22 @@ __global__ __launch_bounds__(64) void k_adj_cp_t(AdjCPArgs A) {
 	const int pi = it.x + min(si, ns - 1);
 	const int4 me = A.parts[pi];
 	const bool wrapx = EWALD || A.wrap;
-	__shared__ float lam[64][36];
-	__shared__ int4 xs[64];
+	__shared__ float lams[NW][64][36];
+	__shared__ int4 xss[NW][64];
+	__shared__ double red[NW > 1 ? NW - 1 : 1][4][64];
+	float (*lam)[36] = lams[wave];
+	int4* xs = xss[wave];
 	double gm = 0.0, g3[3] = {0.0, 0.0, 0.0};
-	for (int base = it.z; base < it.w; base += 64) {
-		const int n = min(64, it.w - base);
-		__syncthreads();
+	for (int base = share.x; base < share.y; base += 64) {
+		const int n = min(64, share.y - base);
+		wave_lds_sync<NW>();
 		if (t < n) {
-			const int a = A.sinks[base + t];
+			const int a = int(A.keys[base + t] & ((uint64_t(1) << A.sink_bits) - 1));
 			xs[t] = A.nodepos[a];
 #pragma unroll
 			for (int q = 0; q < 35; q++) lam[t][q] = float(A.Lam[35 * int64_t(a) + q]);
 		}
-		__syncthreads();
+		wave_lds_sync<NW>();
 		float fm = 0.0f, f3[3] = {0.f, 0.f, 0.f};
 		for (int k = ph; k < n; k += P) {
 			const int4 X = xs[k];
@@ -573,12 +606,8 @@ __global__ __launch_bounds__(64) void k_adj_cp_t(AdjCPArgs A) {
 #pragma unroll
 		for (int q = 0; q < 3; q++) g3[q] += f3[q];
 	}
-	for (int off = nsp; off < 64; off <<= 1) {
-		gm += __shfl_xor(gm, off, 64);
-#pragma unroll
-		for (int q = 0; q < 3; q++) g3[q] += __shfl_xor(g3[q], off, 64);
-	}
-	if (ph == 0 && si < ns) {
+	leaf_sums<NW>(gm, g3, nsp, t, wave, red);
+	if (wave == 0 && ph == 0 && si < ns) {
 		const double mj = double(__int_as_float(me.w));
 		double* o = A.grad + 4 * int64_t(pi);
 		o[0] -= mj * g3[0];
@@ -592,9 +621,9 @@ __global__ __launch_bounds__(64) void k_adj_cp_t(AdjCPArgs A) {
 // lane forms M2L(., X_a - X_c)^T Lambda_a, then 17 lanes add the wave's entries source by source and
 // issue one atomic per source segment and slot
 struct AdjCCArgs {
-	const int2* waves;
-	const int* src;
-	const int* snk;
+	const uint64_t* keys;  // source << sink_bits | sink node, ascending
+	int64_t n;
+	int sink_bits;
 	const int4* nodepos;
 	const MultiSrc* multis;
 	const double* Lam;
@@ -604,19 +633,20 @@ struct AdjCCArgs {
 
 template <bool EWALD>
 __global__ __launch_bounds__(64) void k_adj_cc_t(AdjCCArgs A) {
-	const int2 wv = A.waves[blockIdx.x];
+	const int64_t begin = 64 * int64_t(blockIdx.x);
 	const int t = threadIdx.x;
-	const int j = wv.x + t;
-	const int cnt = wv.y - wv.x;
+	const int64_t j = begin + t;
+	const int cnt = int(A.n - begin < 64 ? A.n - begin : 64);
 	__shared__ float red[17][65];
 	__shared__ int sc[64];
 	float mu[17];
 #pragma unroll
 	for (int q = 0; q < 17; q++) mu[q] = 0.0f;
 	int c = -1;
-	if (j < wv.y) {
-		c = A.src[j];
-		const int a = A.snk[j];
+	if (j < A.n) {
+		const uint64_t key = A.keys[j];
+		c = int(key >> A.sink_bits);
+		const int a = int(key & ((uint64_t(1) << A.sink_bits) - 1));
 		const int4 X = A.nodepos[a];
 		const MultiSrc& ms = A.multis[c];
 		float Lam[35];
@@ -660,12 +690,13 @@ __global__ __launch_bounds__(64) void k_adj_cc_t(AdjCCArgs A) {
 // sum over leaves B below a of S(X_B - X_a)^T lambda_B.  Shifts compose exactly
 // (S(X_B - X_a) = S(X_B - X_c) S(X_c - X_a) for a child c of a on the way), hence level by level,
 // deepest first:  Lambda_a = sum_children S(X_c - X_a)^T Lambda_c,  with Lambda_B = lambda_B at the
-// leaves.  One lane per (node, child); the two children of a node sit on adjacent lanes and are
-// added with one exchange.  No atomics: every Lambda is written once.
-__global__ __launch_bounds__(64) void k_adj_up(const int2* __restrict__ pairs, int npairs, const int4* __restrict__ nodepos,
+// leaves.  One lane per child of a level (nodes are numbered level by level, the children of a node
+// side by side); the two children of a node sit on adjacent lanes and are added with one exchange (an
+// empty child's Lambda is zero).  No atomics: every Lambda is written once.
+__global__ __launch_bounds__(64) void k_adj_up(const int* __restrict__ parent, int begin, int npairs, const int4* __restrict__ nodepos,
 		double* __restrict__ Lam) {
 	const int j = blockIdx.x * 64 + threadIdx.x;
-	const int2 pc = j < npairs ? pairs[j] : make_int2(-1, -1);
+	const int2 pc = j < npairs ? make_int2(parent[begin + j], begin + j) : make_int2(-1, -1);
 	double out[35];
 #pragma unroll
 	for (int q = 0; q < 35; q++) out[q] = 0.0;
@@ -719,13 +750,12 @@ __device__ __forceinline__ void m2m_adjoint(float* mu, const float* mup, const f
 
 // The forward forms a parent's moments from its children's (M2M), so the multipole adjoint of a
 // node is its own mu plus the M2M transpose of its parent's:  mu~_c = mu_c + M2M(X_c - X_a)^T mu~_a,
-// level by level from the root (the up-sweep's (node, child) pairs in reverse level order); in place.
-__global__ __launch_bounds__(64) void k_adj_down(const int2* __restrict__ pairs, int npairs, const int4* __restrict__ nodepos,
+// level by level from the root; in place.
+__global__ __launch_bounds__(64) void k_adj_down(const int* __restrict__ parent, int begin, int npairs, const int4* __restrict__ nodepos,
 		double* __restrict__ mu) {
 	const int j = blockIdx.x * 64 + threadIdx.x;
 	if (j >= npairs) return;
-	const int2 pc = pairs[j];
-	if (pc.y < 0) return;
+	const int2 pc = make_int2(parent[begin + j], begin + j);
 	const int4 Xa = nodepos[pc.x], Xc = nodepos[pc.y];
 	const float Y[3] = {float(double(int64_t(Xc.x) - int64_t(Xa.x)) * POS_INV), float(double(int64_t(Xc.y) - int64_t(Xa.y)) * POS_INV),
 			float(double(int64_t(Xc.z) - int64_t(Xa.z)) * POS_INV)};
@@ -784,6 +814,137 @@ __global__ void k_adj_zero(double* p, int64_t n) {
 	if (i < n) p[i] = 0.0;
 }
 
+// ---- set-up: the lists by source, on the device ---------------------------------------------------
+// What the source-side passes read follows from the walk's node-order lists by one sort per kind of
+// (source, sink) pairs packed into one word, sink in the low sink_bits.  (On the host, with the lists
+// and the tree copied there, this took 195 ms at 262,144 particles and most of an autograd pass.)
+
+struct AdjKeyArgs {
+	const int64_t* ptr;     // the kind's CSR over the nodes
+	const int32_t* val;
+	const WalkNode* nodes;
+	const int* pleaf;
+	int64_t nn;
+	int sink_bits;
+	int64_t* flag;          // set to 1 where a range is no whole leaf, or holds more than 64 particles where that counts
+};
+
+// kinds of node entries (CC, PC): one wave per sink node
+__global__ __launch_bounds__(256) void k_adj_node_keys(AdjKeyArgs A, uint64_t* __restrict__ keys) {
+	const int64_t a = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
+	if (a >= A.nn) return;
+	for (int64_t q = A.ptr[a] + (threadIdx.x & 63); q < A.ptr[a + 1]; q += 64) keys[q] = uint64_t(uint32_t(A.val[q])) << A.sink_bits | uint64_t(a);
+}
+
+// CP: (first particle of the source leaf, sink node); an empty range sorts past every leaf
+__global__ __launch_bounds__(256) void k_adj_cp_keys(AdjKeyArgs A, uint64_t empty, uint64_t* __restrict__ keys) {
+	const int64_t a = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
+	if (a >= A.nn) return;
+	for (int64_t q = A.ptr[a] / 2 + (threadIdx.x & 63); q < A.ptr[a + 1] / 2; q += 64) {
+		const int b = A.val[2 * q], e = A.val[2 * q + 1];
+		uint64_t key = empty;
+		if (e > b) {
+			const WalkNode& n = A.nodes[A.pleaf[b]];
+			if (n.pbegin != b || n.pend != e || e - b > 64) *A.flag = 1;
+			key = uint64_t(uint32_t(b)) << A.sink_bits | uint64_t(a);
+		}
+		keys[q] = key;
+	}
+}
+
+// PP, for the symmetry check: (sink leaf, source leaf) and (source leaf, sink leaf)
+__global__ __launch_bounds__(256) void k_adj_pp_keys(AdjKeyArgs A, uint64_t* __restrict__ fwd, uint64_t* __restrict__ rev) {
+	const int64_t a = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
+	if (a >= A.nn) return;
+	for (int64_t q = A.ptr[a] / 2 + (threadIdx.x & 63); q < A.ptr[a + 1] / 2; q += 64) {
+		const int b = A.val[2 * q], e = A.val[2 * q + 1];
+		uint64_t src = 0;
+		if (e > b) {
+			src = uint64_t(A.pleaf[b]);
+			const WalkNode& n = A.nodes[src];
+			if (n.pbegin != b || n.pend != e) *A.flag = 1;
+		} else {
+			*A.flag = 1;
+		}
+		fwd[q] = uint64_t(a) << A.sink_bits | src;
+		rev[q] = src << A.sink_bits | uint64_t(a);
+	}
+}
+
+__global__ __launch_bounds__(256) void k_adj_differ(const uint64_t* __restrict__ a, const uint64_t* __restrict__ b, int64_t n, int64_t* flag) {
+	const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+	if (i < n && a[i] != b[i]) *flag = 1;
+}
+
+// the first of n ascending keys that is at least k
+__device__ __forceinline__ int64_t lower_bound(const uint64_t* keys, int64_t n, uint64_t k) {
+	int64_t lo = 0, hi = n;
+	while (lo < hi) {
+		const int64_t mid = (lo + hi) >> 1;
+		if (keys[mid] < k)
+			lo = mid + 1;
+		else
+			hi = mid;
+	}
+	return lo;
+}
+
+// CP items, one per non-empty leaf in leaf order: (first particle, count, its run of keys); the
+// largest leaf
+__global__ __launch_bounds__(256) void k_adj_cp_items(const int4* __restrict__ leaves, int nl, const uint64_t* __restrict__ keys, int64_t n,
+		int sink_bits, int4* __restrict__ items, unsigned long long* __restrict__ maxleaf) {
+	const int i = int(blockIdx.x) * 256 + int(threadIdx.x);
+	if (i >= nl) return;
+	const int4 lf = leaves[i];
+	if (maxleaf) atomicMax(maxleaf, (unsigned long long) (lf.z - lf.y));
+	items[i] = make_int4(lf.y, lf.z - lf.y, int(lower_bound(keys, n, uint64_t(uint32_t(lf.y)) << sink_bits)),
+			int(lower_bound(keys, n, uint64_t(uint32_t(lf.y) + 1) << sink_bits)));
+}
+
+// PC: 1 where an item (a run of at most 16 sink leaves of one source node) starts; the sink leaves
+__global__ __launch_bounds__(256) void k_adj_pc_starts(const uint64_t* __restrict__ keys, int64_t n, int sink_bits,
+		const WalkNode* __restrict__ nodes, int64_t* __restrict__ starts, int2* __restrict__ leaves) {
+	const int64_t q = int64_t(blockIdx.x) * 256 + threadIdx.x;
+	if (q >= n) return;
+	const uint64_t key = keys[q], src = key >> sink_bits;
+	const WalkNode& lf = nodes[key & ((uint64_t(1) << sink_bits) - 1)];
+	leaves[q] = make_int2(lf.pbegin, lf.pend - lf.pbegin);
+	const bool same = q > 0 && keys[q - 1] >> sink_bits == src;
+	starts[q] = !same || (q - lower_bound(keys, n, src << sink_bits)) % 16 == 0;
+}
+
+__global__ __launch_bounds__(256) void k_adj_pc_items(const uint64_t* __restrict__ keys, int64_t n, int sink_bits,
+		const int64_t* __restrict__ starts, const int64_t* __restrict__ place, int4* __restrict__ items) {
+	const int64_t q = int64_t(blockIdx.x) * 256 + threadIdx.x;
+	if (q >= n || !starts[q]) return;
+	int64_t e = q + 1;
+	while (e < n && !starts[e]) e++;
+	items[place[q]] = make_int4(int(keys[q] >> sink_bits), int(q), int(e), 0);
+}
+
+// ---- input and output order -----------------------------------------------------------------------
+__global__ __launch_bounds__(256) void k_adj_weights(const float* __restrict__ w, const int64_t* __restrict__ order, int64_t n,
+		float4* __restrict__ out) {
+	const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+	if (i >= n) return;
+	const int64_t o = order[i];
+	out[i] = make_float4(w[3 * o], w[3 * o + 1], w[3 * o + 2], 0.0f);
+}
+
+__global__ __launch_bounds__(256) void k_adj_output(const double* __restrict__ g, const int64_t* __restrict__ order, int64_t n,
+		double* __restrict__ out) {
+	const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+	if (i >= n) return;
+	const int64_t o = order[i];
+	for (int c = 0; c < 4; c++) out[4 * o + c] = g[4 * i + c];
+}
+
+int bits_of(int64_t v) {  // bits that hold every value up to v
+	int b = 1;
+	while (v >> b) b++;
+	return b;
+}
+
 }  // namespace
 
 #define ACHK(call)                                                   \
@@ -795,8 +956,190 @@ __global__ void k_adj_zero(double* p, int64_t n) {
 		}                                                            \
 	} while (0)
 
+// The lists by source, and what the adjoint asks of the tree (symmetric PP lists, leaves of at most
+// 64 particles), once per tree.  The walk's lists are on the device, or are copied there from a host
+// walk's.
+int Solver::adjoint_lists() {
+	if (adj_lists_ready) return TG_OK;
+	hipStream_t s = stream;
+	// scratch, freed once the stream has drained
+	struct Scratch {
+		hipStream_t s;
+		std::vector<void*> blocks;
+		~Scratch() {
+			(void) hipStreamSynchronize(s);
+			for (void* p : blocks) dev_free(p);
+		}
+		void* get(size_t bytes) {
+			void* p = nullptr;
+			if (dev_malloc(&p, std::max<size_t>(bytes, 16)) != hipSuccess) return nullptr;
+			blocks.push_back(p);
+			return p;
+		}
+	} scratch{s, {}};
+	const int64_t nn = n_nodes;
+	if (!dlists.ptr_all || dlists.nn != nn) {
+		// a host walk's lists
+		const Lists& Ls = tree.lists;
+		const hvec<int64_t>* ptrs[8] = {&Ls.cc_d_ptr, &Ls.cp_d_ptr, &Ls.cc_e_ptr, &Ls.cp_e_ptr, &Ls.pc_d_ptr, &Ls.pp_d_ptr, &Ls.pc_e_ptr, &Ls.pp_e_ptr};
+		const hvec<int32_t>* vals[8] = {&Ls.cc_d, &Ls.cp_d, &Ls.cc_e, &Ls.cp_e, &Ls.pc_d, &Ls.pp_d, &Ls.pc_e, &Ls.pp_e};
+		for (int k = 0; k < 8; k++)
+			if (int64_t(ptrs[k]->size()) != nn + 1) {
+				err = "adjoint: the interaction lists do not belong to this tree";
+				return TG_EINVAL;
+			}
+		dlists.release();
+		dlists.nn = nn;
+		hvec<WalkNode> wn(static_cast<size_t>(nn));
+		walk_nodes(tree, wn.data());
+		ACHK(dev_malloc(&dlists.nodes, size_t(nn) * sizeof(WalkNode)));
+		ACHK(hipMemcpyAsync(dlists.nodes, wn.data(), size_t(nn) * sizeof(WalkNode), hipMemcpyHostToDevice, s));
+		ACHK(dev_malloc(&dlists.ptr_all, size_t(8 * (nn + 1)) * 8));
+		for (int k = 0; k < 8; k++) {
+			dlists.len[k] = int64_t(vals[k]->size());
+			ACHK(hipMemcpyAsync(dlists.ptr_all + int64_t(k) * (nn + 1), ptrs[k]->data(), size_t(nn + 1) * 8, hipMemcpyHostToDevice, s));
+			ACHK(dev_malloc(&dlists.val[k], std::max<size_t>(size_t(dlists.len[k]) * 4, 16)));
+			if (dlists.len[k] > 0)
+				ACHK(hipMemcpyAsync(dlists.val[k], vals[k]->data(), size_t(dlists.len[k]) * 4, hipMemcpyHostToDevice, s));
+		}
+		ACHK(hipStreamSynchronize(s));
+	}
+	const int sink_bits = bits_of(nn), src_bits = bits_of(std::max(nn, n + 1));
+	const int key_bits = sink_bits + src_bits;
+	if (key_bits > 64) {
+		err = "adjoint: more nodes and particles than a 64-bit pair key holds";
+		return TG_EINVAL;
+	}
+	// [0], [1] PP lists (direct, Ewald) not symmetric; [2] a CP range that is no leaf of at most 64; [3] the
+	// largest leaf; [4], [5] PC items
+	int64_t* info = static_cast<int64_t*>(scratch.get(8 * 8));
+	if (!info) ACHK(hipErrorOutOfMemory);
+	hipLaunchKernelGGL(k_adj_zero, dim3(1), dim3(64), 0, s, reinterpret_cast<double*>(info), int64_t(8));
+	ACHK(hipGetLastError());
+	void* sort_tmp = nullptr;
+	size_t sort_bytes = 0;
+	auto sort = [&](const uint64_t* in, uint64_t* out, int64_t m) -> hipError_t {
+		size_t need = 0;
+		hipError_t e = hipcub::DeviceRadixSort::SortKeys(nullptr, need, in, out, m, 0, key_bits, s);
+		if (e != hipSuccess) return e;
+		if (need > sort_bytes) {
+			sort_bytes = need;
+			sort_tmp = scratch.get(need);
+			if (!sort_tmp) return hipErrorOutOfMemory;
+		}
+		return hipcub::DeviceRadixSort::SortKeys(sort_tmp, need, in, out, m, 0, key_bits, s);
+	};
+	const dim3 node_grid(unsigned((nn + 3) / 4));
+	auto grid = [](int64_t m) { return dim3(unsigned((m + 255) / 256)); };
+	AdjKeyArgs A{nullptr, nullptr, dlists.nodes, d_pleaf.as<int>(), nn, sink_bits, nullptr};
+	auto kind = [&](int k, int64_t* flag) {
+		A.ptr = dlists.ptr(k);
+		A.val = dlists.val[k];
+		A.flag = flag;
+	};
+	enum { W_CC_D, W_CP_D, W_CC_E, W_CP_E, W_PC_D, W_PP_D, W_PC_E, W_PP_E };
+	ScanSet pc_scan;
+	int64_t* pc_starts[2] = {nullptr, nullptr};
+	for (int e = 0; e < 2; e++) {
+		// PP: symmetric, leaf by leaf
+		kind(e ? W_PP_E : W_PP_D, info + e);
+		if (const int64_t m = dlists.len[e ? W_PP_E : W_PP_D] / 2) {
+			uint64_t* f = static_cast<uint64_t*>(scratch.get(size_t(m) * 8));
+			uint64_t* r = static_cast<uint64_t*>(scratch.get(size_t(m) * 8));
+			uint64_t* fs = static_cast<uint64_t*>(scratch.get(size_t(m) * 8));
+			uint64_t* rs = static_cast<uint64_t*>(scratch.get(size_t(m) * 8));
+			if (!f || !r || !fs || !rs) ACHK(hipErrorOutOfMemory);
+			hipLaunchKernelGGL(k_adj_pp_keys, node_grid, dim3(256), 0, s, A, f, r);
+			ACHK(hipGetLastError());
+			ACHK(sort(f, fs, m));
+			ACHK(sort(r, rs, m));
+			hipLaunchKernelGGL(k_adj_differ, grid(m), dim3(256), 0, s, fs, rs, m, info + e);
+			ACHK(hipGetLastError());
+		}
+		// CC by source
+		kind(e ? W_CC_E : W_CC_D, nullptr);
+		adj_cct_n[e] = dlists.len[e ? W_CC_E : W_CC_D];
+		ACHK(d_adj_cct_keys[e].alloc(std::max<size_t>(size_t(adj_cct_n[e]) * 8, 16)));
+		if (const int64_t m = adj_cct_n[e]) {
+			uint64_t* k = static_cast<uint64_t*>(scratch.get(size_t(m) * 8));
+			if (!k) ACHK(hipErrorOutOfMemory);
+			hipLaunchKernelGGL(k_adj_node_keys, node_grid, dim3(256), 0, s, A, k);
+			ACHK(hipGetLastError());
+			ACHK(sort(k, d_adj_cct_keys[e].as<uint64_t>(), m));
+		}
+		// CP by source leaf
+		kind(e ? W_CP_E : W_CP_D, info + 2);
+		adj_cpt_n[e] = dlists.len[e ? W_CP_E : W_CP_D] / 2;
+		ACHK(d_adj_cpt_keys[e].alloc(std::max<size_t>(size_t(adj_cpt_n[e]) * 8, 16)));
+		ACHK(d_adj_cpt_items[e].alloc(std::max<size_t>(size_t(n_leaf_items) * sizeof(int4), 16)));
+		if (const int64_t m = adj_cpt_n[e]) {
+			uint64_t* k = static_cast<uint64_t*>(scratch.get(size_t(m) * 8));
+			if (!k) ACHK(hipErrorOutOfMemory);
+			hipLaunchKernelGGL(k_adj_cp_keys, node_grid, dim3(256), 0, s, A, key_bits == 64 ? ~uint64_t(0) : (uint64_t(1) << key_bits) - 1, k);
+			ACHK(hipGetLastError());
+			ACHK(sort(k, d_adj_cpt_keys[e].as<uint64_t>(), m));
+		}
+		if (n_leaf_items > 0) {
+			hipLaunchKernelGGL(k_adj_cp_items, grid(n_leaf_items), dim3(256), 0, s, d_leaf_items.as<int4>(), n_leaf_items,
+					d_adj_cpt_keys[e].as<uint64_t>(), adj_cpt_n[e], sink_bits, d_adj_cpt_items[e].as<int4>(),
+					e == 0 ? reinterpret_cast<unsigned long long*>(info + 3) : nullptr);
+			ACHK(hipGetLastError());
+		}
+		// PC by source node
+		kind(e ? W_PC_E : W_PC_D, nullptr);
+		const int64_t m = dlists.len[e ? W_PC_E : W_PC_D];
+		ACHK(d_adj_pct_leaves[e].alloc(std::max<size_t>(size_t(m) * sizeof(int2), 16)));
+		ACHK(d_adj_pct_items[e].alloc(std::max<size_t>(size_t(m) * sizeof(int4), 16)));
+		uint64_t* k = static_cast<uint64_t*>(scratch.get(size_t(m) * 8));
+		uint64_t* ks = static_cast<uint64_t*>(scratch.get(size_t(m) * 8));
+		pc_starts[e] = static_cast<int64_t*>(scratch.get(size_t(m) * 8));
+		int64_t* place = static_cast<int64_t*>(scratch.get(size_t(m) * 8));
+		if (!k || !ks || !pc_starts[e] || !place) ACHK(hipErrorOutOfMemory);
+		ScanSet sc;
+		sc.add(pc_starts[e], place, m);
+		int64_t* ws = static_cast<int64_t*>(scratch.get(size_t(scan_workspace(sc)) * 8));
+		if (!ws) ACHK(hipErrorOutOfMemory);
+		if (m > 0) {
+			hipLaunchKernelGGL(k_adj_node_keys, node_grid, dim3(256), 0, s, A, k);
+			ACHK(hipGetLastError());
+			ACHK(sort(k, ks, m));
+			hipLaunchKernelGGL(k_adj_pc_starts, grid(m), dim3(256), 0, s, ks, m, sink_bits, dlists.nodes, pc_starts[e], d_adj_pct_leaves[e].as<int2>());
+			ACHK(hipGetLastError());
+			ACHK(scan_columns(sc, ws, info + 4 + e, s));
+			hipLaunchKernelGGL(k_adj_pc_items, grid(m), dim3(256), 0, s, ks, m, sink_bits, pc_starts[e], place, d_adj_pct_items[e].as<int4>());
+			ACHK(hipGetLastError());
+		}
+	}
+	int64_t v[8];
+	ACHK(hipMemcpyAsync(v, info, sizeof(v), hipMemcpyDeviceToHost, s));
+	ACHK(hipStreamSynchronize(s));
+	adj_pp_symmetric = v[0] == 0 && v[1] == 0;
+	adj_cp_whole = v[2] == 0;
+	adj_maxleaf = int(v[3]);
+	adj_pct_nitems[0] = int(v[4]);
+	adj_pct_nitems[1] = int(v[5]);
+	adj_sink_bits = sink_bits;
+	adj_lists_ready = true;
+	return TG_OK;
+}
+
+namespace {
+
+// waves per group of a leaf-kind launch, as the forward's
+template <class F>
+void with_waves(int nitems, int64_t nlist, F launch) {
+	switch (leaf_waves(nitems, nlist, 8)) {
+		case 1: launch(std::integral_constant<int, 1>{}); break;
+		case 2: launch(std::integral_constant<int, 2>{}); break;
+		case 4: launch(std::integral_constant<int, 4>{}); break;
+		default: launch(std::integral_constant<int, 8>{}); break;
+	}
+}
+
+}  // namespace
+
 int Solver::adjoint(const float* w_in, double* grad_out, float* ms) {
-	if (device < 0 || n == 0 || tree.nodes.empty()) {
+	if (device < 0 || n == 0 || n_nodes == 0) {
 		err = "adjoint needs a device solver with particles";
 		return TG_EINVAL;
 	}
@@ -804,149 +1147,47 @@ int Solver::adjoint(const float* w_in, double* grad_out, float* ms) {
 		err = "the adjoint handles leaves of at most 64 particles";
 		return TG_EINVAL;
 	}
-	for (int32_t lf : tree.leaves)
-		if (tree.nodes[size_t(lf)].pend - tree.nodes[size_t(lf)].pbegin > 64) {
-			// only more coincident particles than a leaf holds make one (the tree's depth limit)
-			err = "the adjoint handles leaves of at most 64 particles; a leaf at the tree's depth limit holds more";
-			return TG_EINVAL;
-		}
+	ACHK(hipSetDevice(device));
+	{
+		const int rc = adjoint_lists();
+		if (rc != TG_OK) return rc;
+	}
+	if (adj_maxleaf > 64) {
+		// only more coincident particles than a leaf holds make one (the tree's depth limit)
+		err = "the adjoint handles leaves of at most 64 particles; a leaf at the tree's depth limit holds more";
+		return TG_EINVAL;
+	}
 	if (!adj_pp_symmetric) {
 		err = "the adjoint needs symmetric PP lists";
 		return TG_EINVAL;
 	}
-	ACHK(hipSetDevice(device));
-	if (!adj_lists_ready) {
-		{
-			const int rc = host_lists();  // the by-source transposes read the CC list values
-			if (rc != TG_OK) return rc;
-		}
-		// CC entries by source: (source, sink node) pairs of the direct and Ewald lists, sorted by source
-		auto put_v = [&](DeviceArray& d, const void* h, size_t bytes) -> hipError_t {
-			hipError_t r = d.alloc(std::max<size_t>(bytes, 16));
-			if (r != hipSuccess || bytes == 0) return r;
-			return hipMemcpy(d.p, h, bytes, hipMemcpyHostToDevice);
-		};
-		for (int e = 0; e < 2; e++) {
-			const hvec<int64_t>& ptr = e ? tree.lists.cc_e_ptr : tree.lists.cc_d_ptr;
-			const hvec<int32_t>& v = e ? tree.lists.cc_e : tree.lists.cc_d;
-			std::vector<std::pair<int32_t, int32_t>> pr;
-			for (size_t a = 0; a + 1 < ptr.size(); a++)
-				for (int64_t q = ptr[a]; q < ptr[a + 1]; q++) pr.emplace_back(v[q], int32_t(a));
-			std::sort(pr.begin(), pr.end());
-			std::vector<int> src(pr.size()), snk(pr.size());
-			std::vector<int2> waves;
-			for (size_t q = 0; q < pr.size(); q++) {
-				src[q] = pr[q].first;
-				snk[q] = pr[q].second;
-			}
-			for (size_t q = 0; q < pr.size(); q += 64) waves.push_back(make_int2(int(q), int(std::min(pr.size(), q + 64))));
-			ACHK(put_v(d_adj_cct_src[e], src.data(), src.size() * sizeof(int)));
-			ACHK(put_v(d_adj_cct_snk[e], snk.data(), snk.size() * sizeof(int)));
-			ACHK(put_v(d_adj_cct_waves[e], waves.data(), waves.size() * sizeof(int2)));
-			adj_cct_nwaves[e] = int(waves.size());
-		}
-		// CP entries by source leaf (direct, Ewald): every CP range is a whole leaf's particles
-		std::vector<int32_t> leaf_at(size_t(n) + 1, -1);
-		for (int32_t lf : tree.leaves)
-			if (!tree.nodes[lf].empty()) leaf_at[size_t(tree.nodes[lf].pbegin)] = lf;
-		for (int e = 0; e < 2; e++) {
-			const hvec<int64_t>& ptr = e ? tree.lists.cp_e_ptr : tree.lists.cp_d_ptr;
-			const hvec<int32_t>& v = e ? tree.lists.cp_e : tree.lists.cp_d;
-			std::vector<std::pair<int32_t, int32_t>> pr;  // (source leaf first particle, sink node)
-			for (size_t a = 0; a + 1 < ptr.size(); a++)
-				for (int64_t q = ptr[a]; q < ptr[a + 1]; q += 2) {
-					const int32_t b = v[q], en = v[q + 1];
-					if (en <= b) continue;
-					const int32_t lf = leaf_at[size_t(b)];
-					if (lf < 0 || tree.nodes[lf].pend != en || en - b > 64) {
-						err = "the adjoint needs CP sources that are whole leaves of at most 64 particles";
-						return TG_EINVAL;
-					}
-					pr.emplace_back(b, int32_t(a));
-				}
-			std::sort(pr.begin(), pr.end());
-			std::vector<int> sinks(pr.size());
-			std::vector<int4> items;
-			for (size_t q = 0; q < pr.size(); q++) {
-				sinks[q] = pr[q].second;
-				if (q == 0 || pr[q].first != pr[q - 1].first) {
-					const int32_t b = pr[q].first, lf = leaf_at[size_t(b)];
-					items.push_back(make_int4(b, tree.nodes[lf].pend - b, int(q), int(q)));
-				}
-				items.back().w = int(q + 1);
-			}
-			ACHK(put_v(d_adj_cpt_sinks[e], sinks.data(), sinks.size() * sizeof(int)));
-			ACHK(put_v(d_adj_cpt_items[e], items.data(), items.size() * sizeof(int4)));
-			adj_cpt_nitems[e] = int(items.size());
-		}
-		// PC entries by source node (direct, Ewald): runs of at most 16 sink leaves per item
-		int maxleaf = 1;
-		for (int32_t lf : tree.leaves) maxleaf = std::max(maxleaf, int(tree.nodes[lf].pend - tree.nodes[lf].pbegin));
-		adj_pc_lgL = 0;
-		while ((1 << adj_pc_lgL) < maxleaf) adj_pc_lgL++;
-		if (adj_pc_lgL > 6) {
-			err = "the adjoint handles leaves of at most 64 particles";
-			return TG_EINVAL;
-		}
-		for (int e = 0; e < 2; e++) {
-			const hvec<int64_t>& ptr = e ? tree.lists.pc_e_ptr : tree.lists.pc_d_ptr;
-			const hvec<int32_t>& v = e ? tree.lists.pc_e : tree.lists.pc_d;
-			std::vector<std::pair<int32_t, int32_t>> pr;  // (source node, sink leaf)
-			for (int32_t lf : tree.leaves) {
-				if (tree.nodes[lf].empty() || size_t(lf) + 1 >= ptr.size()) continue;
-				for (int64_t q = ptr[lf]; q < ptr[lf + 1]; q++) pr.emplace_back(v[q], lf);
-			}
-			std::sort(pr.begin(), pr.end());
-			std::vector<int2> sl(pr.size());
-			std::vector<int4> items;
-			for (size_t q = 0; q < pr.size(); q++) {
-				const Node& nd = tree.nodes[pr[q].second];
-				sl[q] = make_int2(nd.pbegin, nd.pend - nd.pbegin);
-				if (q == 0 || pr[q].first != pr[q - 1].first || items.back().z - items.back().y >= 16)
-					items.push_back(make_int4(pr[q].first, int(q), int(q), 0));
-				items.back().z = int(q + 1);
-			}
-			ACHK(put_v(d_adj_pct_leaves[e], sl.data(), sl.size() * sizeof(int2)));
-			ACHK(put_v(d_adj_pct_items[e], items.data(), items.size() * sizeof(int4)));
-			adj_pct_nitems[e] = int(items.size());
-		}
-		// (node, child) pairs of the internal nodes, deepest level first; an empty child gets -1
-		std::vector<std::vector<int2>> by_level(size_t(tree.max_level) + 1);
-		for (size_t i = 0; i < tree.nodes.size(); i++) {
-			const Node& nd = tree.nodes[i];
-			if (nd.leaf()) continue;
-			for (int c = 0; c < 2; c++) {
-				const int ch = nd.child[c];
-				by_level[size_t(nd.level)].push_back(make_int2(int(i), ch >= 0 && !tree.nodes[size_t(ch)].empty() ? ch : -1));
-			}
-		}
-		std::vector<int2> pairs;
-		adj_up_ptr.assign(1, 0);
-		for (int l = tree.max_level; l >= 0; l--) {
-			pairs.insert(pairs.end(), by_level[size_t(l)].begin(), by_level[size_t(l)].end());
-			if (int(pairs.size()) > adj_up_ptr.back()) adj_up_ptr.push_back(int(pairs.size()));
-		}
-		ACHK(d_adj_up.alloc(std::max<size_t>(pairs.size() * sizeof(int2), 16)));
-		if (!pairs.empty()) ACHK(hipMemcpy(d_adj_up.p, pairs.data(), pairs.size() * sizeof(int2), hipMemcpyHostToDevice));
-		adj_lists_ready = true;
+	if (!adj_cp_whole) {
+		err = "the adjoint needs CP sources that are whole leaves of at most 64 particles";
+		return TG_EINVAL;
 	}
+	adj_pc_lgL = 0;
+	while ((1 << adj_pc_lgL) < adj_maxleaf) adj_pc_lgL++;
 	static thread_local int tables_ready = -1;
 	if (tables_ready != device) {
 		ACHK(init_adjoint_tables(device));
 		tables_ready = device;
 	}
-	const int64_t nn = int64_t(tree.nodes.size());
-	std::vector<float4> w(n);
-	for (int64_t i = 0; i < n; i++) {
-		const int64_t o = tree.order[i];
-		w[i] = make_float4(w_in[3 * o], w_in[3 * o + 1], w_in[3 * o + 2], 0.0f);
+	{
+		const int rc = forces_device_order();  // the input index of each tree-order particle
+		if (rc != TG_OK) return rc;
 	}
+	const int64_t nn = n_nodes;
 	ACHK(d_adj_w.alloc(std::max<size_t>(n * sizeof(float4), 16)));
 	ACHK(d_adj_grad.alloc(std::max<size_t>(n * 4 * sizeof(double), 16)));
+	ACHK(d_adj_out.alloc(std::max<size_t>(n * 4 * sizeof(double), 16)));
 	ACHK(d_adj_lam.alloc(std::max<size_t>(nn * 35 * sizeof(double), 16)));
 	ACHK(d_adj_mu.alloc(std::max<size_t>(nn * 17 * sizeof(double), 16)));
 	hipStream_t s = stream;
-	ACHK(hipMemcpyAsync(d_adj_w.p, w.data(), n * sizeof(float4), hipMemcpyHostToDevice, s));
+	const dim3 part_grid(unsigned((n + 255) / 256));
+	// the weights as they come (host or device memory), put into tree order there; d_adj_out holds them so long
+	ACHK(hipMemcpyAsync(d_adj_out.p, w_in, size_t(n) * 12, hipMemcpyDefault, s));
+	hipLaunchKernelGGL(k_adj_weights, part_grid, dim3(256), 0, s, d_adj_out.as<const float>(), d_order.as<const int64_t>(), n, d_adj_w.as<float4>());
+	ACHK(hipGetLastError());
 	if (!adj_ev[0]) {
 		ACHK(hipEventCreate(&adj_ev[0]));
 		ACHK(hipEventCreate(&adj_ev[1]));
@@ -970,40 +1211,49 @@ int Solver::adjoint(const float* w_in, double* grad_out, float* ms) {
 	a.mu = d_adj_mu.as<double>();
 	a.h = float(soft_len);
 	a.wrap = ewald;
-	a.maxdepth = tree.max_level + 1;
+	a.maxdepth = max_level + 1;
 	const size_t lds = size_t(35 * 64 + 35 + 35 * a.maxdepth) * sizeof(double);
 	if (n_leaf_items > 0) {
 		hipLaunchKernelGGL(k_adj_l2p, dim3(n_leaf_items), dim3(64), lds, s, a);
 		ACHK(hipGetLastError());
 	}
-	for (size_t l = 0; l + 1 < adj_up_ptr.size(); l++) {
-		const int b = adj_up_ptr[l], np = adj_up_ptr[l + 1] - b;
-		hipLaunchKernelGGL(k_adj_up, dim3(unsigned((np + 63) / 64)), dim3(64), 0, s, d_adj_up.as<int2>() + b, np, d_nodepos.as<int4>(),
-				d_adj_lam.as<double>());
+	// children of each level, the deepest first
+	const int* parent = d_parent.as<int>();
+	const int levels = int(level_begin.size()) - 1;
+	for (int l = levels - 1; l >= 1; l--) {
+		const int b = level_begin[size_t(l)], np = level_begin[size_t(l) + 1] - b;
+		hipLaunchKernelGGL(k_adj_up, dim3(unsigned((np + 63) / 64)), dim3(64), 0, s, parent, b, np, d_nodepos.as<int4>(), d_adj_lam.as<double>());
 		ACHK(hipGetLastError());
 	}
 	for (int k : {PP_DIRECT, PP_EWALD, PC_DIRECT, PC_EWALD}) {
 		if (work[k].nitems <= 0) continue;
 		AdjItems I{work[k].items.as<int4>(), work[k].list.as<int>(), work[k].nitems};
-		const dim3 g(work[k].nitems), b(64);
-		if (k == PP_DIRECT)
-			hipLaunchKernelGGL(k_adj_pp, g, b, 0, s, a, I);
-		else if (k == PP_EWALD)
-			hipLaunchKernelGGL(k_adj_pp_ewald, g, b, 0, s, a, I);
-		else if (k == PC_DIRECT)
-			hipLaunchKernelGGL(k_adj_pc_sink<false>, g, b, 0, s, a, I);
-		else
-			hipLaunchKernelGGL(k_adj_pc_sink<true>, g, b, 0, s, a, I);
+		const dim3 g(work[k].nitems);
+		with_waves(work[k].nitems, work[k].nlist, [&](auto nw_) {
+			constexpr int NW = decltype(nw_)::value;
+			const dim3 b(64 * NW);
+			if (k == PP_DIRECT && ewald)
+				hipLaunchKernelGGL((k_adj_pp<NW, true>), g, b, 0, s, a, I);
+			else if (k == PP_DIRECT)
+				hipLaunchKernelGGL((k_adj_pp<NW, false>), g, b, 0, s, a, I);
+			else if (k == PP_EWALD)
+				hipLaunchKernelGGL((k_adj_pp_ewald<NW>), g, b, 0, s, a, I);
+			else if (k == PC_DIRECT)
+				hipLaunchKernelGGL((k_adj_pc_sink<NW, false>), g, b, 0, s, a, I);
+			else
+				hipLaunchKernelGGL((k_adj_pc_sink<NW, true>), g, b, 0, s, a, I);
+		});
 		ACHK(hipGetLastError());
 	}
 	for (int e = 0; e < 2; e++) {
-		if (adj_cct_nwaves[e] <= 0) continue;
-		AdjCCArgs ca{d_adj_cct_waves[e].as<int2>(), d_adj_cct_src[e].as<int>(), d_adj_cct_snk[e].as<int>(), d_nodepos.as<int4>(),
-				d_multis.as<MultiSrc>(), d_adj_lam.as<double>(), d_adj_mu.as<double>(), ewald};
+		if (adj_cct_n[e] <= 0) continue;
+		AdjCCArgs ca{d_adj_cct_keys[e].as<uint64_t>(), adj_cct_n[e], adj_sink_bits, d_nodepos.as<int4>(), d_multis.as<MultiSrc>(),
+				d_adj_lam.as<double>(), d_adj_mu.as<double>(), ewald};
+		const dim3 g(unsigned((adj_cct_n[e] + 63) / 64));
 		if (e)
-			hipLaunchKernelGGL(k_adj_cc_t<true>, dim3(adj_cct_nwaves[e]), dim3(64), 0, s, ca);
+			hipLaunchKernelGGL(k_adj_cc_t<true>, g, dim3(64), 0, s, ca);
 		else
-			hipLaunchKernelGGL(k_adj_cc_t<false>, dim3(adj_cct_nwaves[e]), dim3(64), 0, s, ca);
+			hipLaunchKernelGGL(k_adj_cc_t<false>, g, dim3(64), 0, s, ca);
 		ACHK(hipGetLastError());
 	}
 	for (int e = 0; e < 2; e++) {
@@ -1017,19 +1267,22 @@ int Solver::adjoint(const float* w_in, double* grad_out, float* ms) {
 		ACHK(hipGetLastError());
 	}
 	for (int e = 0; e < 2; e++) {
-		if (adj_cpt_nitems[e] <= 0) continue;
-		AdjCPArgs pa{d_adj_cpt_items[e].as<int4>(), d_adj_cpt_sinks[e].as<int>(), d_nodepos.as<int4>(), d_parts.as<int4>(),
+		if (adj_cpt_n[e] <= 0 || n_leaf_items <= 0) continue;
+		AdjCPArgs pa{d_adj_cpt_items[e].as<int4>(), d_adj_cpt_keys[e].as<uint64_t>(), adj_sink_bits, d_nodepos.as<int4>(), d_parts.as<int4>(),
 				d_adj_lam.as<double>(), d_adj_grad.as<double>(), ewald};
-		if (e)
-			hipLaunchKernelGGL(k_adj_cp_t<true>, dim3(adj_cpt_nitems[e]), dim3(64), 0, s, pa);
-		else
-			hipLaunchKernelGGL(k_adj_cp_t<false>, dim3(adj_cpt_nitems[e]), dim3(64), 0, s, pa);
+		// four waves at most: 9 KB of staged expansions each
+		with_waves(n_leaf_items, adj_cpt_n[e], [&](auto nw_) {
+			constexpr int NW = decltype(nw_)::value < 4 ? decltype(nw_)::value : 4;
+			if (e)
+				hipLaunchKernelGGL((k_adj_cp_t<NW, true>), dim3(n_leaf_items), dim3(64 * NW), 0, s, pa);
+			else
+				hipLaunchKernelGGL((k_adj_cp_t<NW, false>), dim3(n_leaf_items), dim3(64 * NW), 0, s, pa);
+		});
 		ACHK(hipGetLastError());
 	}
-	for (size_t l = adj_up_ptr.size(); l-- > 1;) {
-		const int b = adj_up_ptr[l - 1], np = adj_up_ptr[l] - b;
-		hipLaunchKernelGGL(k_adj_down, dim3(unsigned((np + 63) / 64)), dim3(64), 0, s, d_adj_up.as<int2>() + b, np, d_nodepos.as<int4>(),
-				d_adj_mu.as<double>());
+	for (int l = 1; l < levels; l++) {
+		const int b = level_begin[size_t(l)], np = level_begin[size_t(l) + 1] - b;
+		hipLaunchKernelGGL(k_adj_down, dim3(unsigned((np + 63) / 64)), dim3(64), 0, s, parent, b, np, d_nodepos.as<int4>(), d_adj_mu.as<double>());
 		ACHK(hipGetLastError());
 	}
 	if (n_leaf_items > 0) {
@@ -1037,14 +1290,11 @@ int Solver::adjoint(const float* w_in, double* grad_out, float* ms) {
 		ACHK(hipGetLastError());
 	}
 	if (ms) ACHK(hipEventRecord(e1, s));
-	std::vector<double> g(n * 4);
-	ACHK(hipMemcpyAsync(g.data(), d_adj_grad.p, n * 4 * sizeof(double), hipMemcpyDeviceToHost, s));
+	hipLaunchKernelGGL(k_adj_output, part_grid, dim3(256), 0, s, d_adj_grad.as<const double>(), d_order.as<const int64_t>(), n, d_adj_out.as<double>());
+	ACHK(hipGetLastError());
+	ACHK(hipMemcpyAsync(grad_out, d_adj_out.p, size_t(n) * 4 * sizeof(double), hipMemcpyDefault, s));
 	ACHK(hipStreamSynchronize(s));
 	if (ms) ACHK(hipEventElapsedTime(ms, e0, e1));
-	for (int64_t i = 0; i < n; i++) {
-		const int64_t o = tree.order[i];
-		for (int c = 0; c < 4; c++) grad_out[4 * o + c] = g[4 * i + c];
-	}
 	return TG_OK;
 }
 

@@ -299,17 +299,13 @@ Solver::~Solver() {
 		d_adj_grad.release();
 		d_adj_lam.release();
 		d_adj_mu.release();
-		d_adj_up.release();
+		d_adj_out.release();
 		for (int e = 0; e < 2; e++) {
+			d_adj_cct_keys[e].release();
+			d_adj_cpt_keys[e].release();
 			d_adj_cpt_items[e].release();
-			d_adj_cpt_sinks[e].release();
 			d_adj_pct_items[e].release();
 			d_adj_pct_leaves[e].release();
-		}
-		for (int e = 0; e < 2; e++) {
-			d_adj_cct_src[e].release();
-			d_adj_cct_snk[e].release();
-			d_adj_cct_waves[e].release();
 		}
 		d_leaf_items.release();
 		d_slot_node.release();
@@ -470,34 +466,6 @@ int Solver::update_particles(const int32_t* x, const float* mass) {
 }
 
 // particle records and multipoles of the current tree to the device
-// the adjoint gathers each particle's PP source-side terms from its own list, which needs leaf B in
-// leaf A's PP lists exactly when A is in B's (true of the walk's lists, checked here per tree)
-bool Solver::pp_lists_symmetric() const {
-	const Tree& T = tree;
-	std::vector<int32_t> leaf_at(size_t(n) + 1, -1);
-	for (int32_t lf : T.leaves)
-		if (!T.nodes[lf].empty()) leaf_at[T.nodes[lf].pbegin] = lf;
-	for (int kind = 0; kind < 2; kind++) {
-		const hvec<int64_t>& ptr = kind ? T.lists.pp_e_ptr : T.lists.pp_d_ptr;
-		const hvec<int32_t>& v = kind ? T.lists.pp_e : T.lists.pp_d;
-		std::vector<std::pair<int32_t, int32_t>> pairs;
-		for (int32_t lf : T.leaves) {
-			if (size_t(lf) + 1 >= ptr.size()) continue;
-			for (int64_t k = ptr[lf]; k < ptr[lf + 1]; k += 2) {
-				const int32_t src = leaf_at[v[k]];
-				if (src < 0 || T.nodes[src].pend != v[k + 1]) return false;  // not a whole leaf
-				pairs.emplace_back(lf, src);
-			}
-		}
-		std::vector<std::pair<int32_t, int32_t>> rev(pairs.size());
-		for (size_t i = 0; i < pairs.size(); i++) rev[i] = {pairs[i].second, pairs[i].first};
-		std::sort(pairs.begin(), pairs.end());
-		std::sort(rev.begin(), rev.end());
-		if (pairs != rev) return false;
-	}
-	return true;
-}
-
 int Solver::upload_sources() {
 	const Tree& T = tree;
 	const int64_t nn = int64_t(T.nodes.size());
@@ -572,7 +540,6 @@ int Solver::upload() {
 	const double tp0 = now();
 	if (tree_on_device) {
 		// the tree's arrays and the list work, all made on the device
-		adj_checked = false;
 		adj_lists_ready = false;
 		int rc = upload_tree_device();
 		const double tp1 = now();
@@ -629,7 +596,6 @@ int Solver::upload() {
 	SCHK(put(d_multis, multis, s));
 	SCHK(put(d_nodepos, npos, s));
 	SCHK(put(d_leaf_items, leaf_items, s));
-	adj_checked = false;
 	adj_lists_ready = false;
 	SCHK(put(d_path, path, s));
 	path_len = int64_t(path.size());
@@ -1060,13 +1026,6 @@ int tg_solver_tune(tg_solver* h, const char* knob, int value) {
 int tg_solver_adjoint(tg_solver* h, const float* w, double* grad, double* ms) {
 	if (!h || h->s.device < 0 || (h->s.n > 0 && (!w || !grad))) return TG_EINVAL;
 	tg::Solver& S = h->s;
-	if (!S.adj_checked) {
-		int rl = S.host_tree();  // the adjoint's set-up reads the tree and the lists on the host
-		if (rl == TG_OK) rl = S.host_lists();
-		if (rl != TG_OK) return fail(h, rl);
-		S.adj_pp_symmetric = S.pp_lists_symmetric();
-		S.adj_checked = true;
-	}
 	float t = 0.0f;
 	const int rc = S.adjoint(w, grad, ms ? &t : nullptr);
 	if (ms) *ms = t;

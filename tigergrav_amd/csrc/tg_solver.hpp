@@ -66,23 +66,19 @@ struct Solver {
 	std::vector<int> level_begin;          // first node of each level, then the node count
 	// adjoint buffers: loss weights, gradients, expansion and multipole adjoints
 	DeviceArray d_adj_w, d_adj_grad, d_adj_lam, d_adj_mu;
-	bool adj_pp_symmetric = false;  // checked once per tree at the first adjoint call
-	bool adj_checked = false;
+	DeviceArray d_adj_out;  // weights as passed, then gradients in input order
 	hipEvent_t adj_ev[2] = {nullptr, nullptr};
-	// CC entries by source for the adjoint (direct, Ewald): built at the first adjoint call per tree
-	DeviceArray d_adj_cct_src[2], d_adj_cct_snk[2], d_adj_cct_waves[2];
-	int adj_cct_nwaves[2] = {0, 0};
-	// CP entries by source leaf (direct, Ewald): items (first particle, count, sink range) and sink nodes
-	DeviceArray d_adj_cpt_items[2], d_adj_cpt_sinks[2];
-	int adj_cpt_nitems[2] = {0, 0};
-	// PC entries by source node (direct, Ewald): items (node, sink-leaf run) and sink leaves
-	DeviceArray d_adj_pct_items[2], d_adj_pct_leaves[2];
+	// the lists by source (direct, Ewald), made on the device at the first adjoint call per tree: CC
+	// and CP as sorted (source, sink node) keys, CP items (first particle, count, key range) per leaf; PC
+	// items (node, sink-leaf run) and sink leaves
+	DeviceArray d_adj_cct_keys[2], d_adj_cpt_keys[2], d_adj_cpt_items[2], d_adj_pct_items[2], d_adj_pct_leaves[2];
+	int64_t adj_cct_n[2] = {0, 0}, adj_cpt_n[2] = {0, 0};
 	int adj_pct_nitems[2] = {0, 0};
+	int adj_sink_bits = 0;          // of a key
+	bool adj_pp_symmetric = false;  // leaf B is in leaf A's PP lists exactly when A is in B's
+	bool adj_cp_whole = false;      // CP sources are whole leaves of at most 64 particles
+	int adj_maxleaf = 0;
 	int adj_pc_lgL = 6;  // lanes per sink leaf in k_adj_pc_t: 2^adj_pc_lgL >= the largest leaf
-	// (node, child) pairs for the Lambda up-sweep, grouped by level deepest first: batch l is
-	// [adj_up_ptr[l], adj_up_ptr[l + 1])
-	DeviceArray d_adj_up;
-	std::vector<int> adj_up_ptr;
 	bool adj_lists_ready = false;
 	KindWork work[NKINDS];
 	// host-only solvers (device < 0) keep the PP-direct items and flattened source list
@@ -133,7 +129,7 @@ struct Solver {
 	// gradients of sum_i w_i . g_i (w: 3 per particle, input order) with respect to positions and
 	// masses: grad 4 per particle (d/dx, d/dy, d/dz, d/dm), input order; ms: device time, or NULL
 	int adjoint(const float* w, double* grad, float* ms);
-	bool pp_lists_symmetric() const;
+	int adjoint_lists();
 	int enqueue_solve(bool timed);
 	hipGraphExec_t graph_exec = nullptr;
 	int solve_graph();
