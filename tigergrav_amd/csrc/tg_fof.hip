@@ -12,7 +12,12 @@
 //     boxes come within L of its own (minimum image), counted, then written;
 //   * links: one 64-lane group per candidate pair tests every particle pair with the reference's
 //     integer test and unites the linked ones;
-//   * labels: the root of every linked particle, DEFAULT_GROUP for the rest.
+//   * labels: the root of every linked particle, DEFAULT_GROUP for the rest, in tree and in input
+//     order.
+// The nodes come from the device build's tree where that is current, else from the host's; only the
+// labels in input order cross to the host (with set_particles at 2M clustered particles, leaves of 32:
+// 27.8 -> 8.7 ms; before, tree and order were copied, the nodes rebuilt and the labels permuted on
+// the host).
 // The candidate search only has to find a superset of the linked pairs, so its box test is in
 // FP64 with a margin; the link test itself is the reference's exact integer one.
 //
@@ -23,9 +28,10 @@
 // wrap), in either boundary mode, and groups are the plain connected components; every pair away
 // from the edge is treated as the reference treats it.
 #include "tg_fof.hpp"
+#include "tg_devmem.hpp"
+#include "tg_scan.hpp"
 
-#include <hipcub/hipcub.hpp>
-
+#include <algorithm>
 #include <climits>
 #include <cmath>
 #include <vector>
@@ -69,15 +75,33 @@ __device__ __forceinline__ bool boxes_near(const FofNode& a, const FofNode& b, d
 	return s <= L2;
 }
 
+// the search's record of a device-built node
+__global__ __launch_bounds__(256) void k_fof_nodes(const DNode* __restrict__ nodes, const DMulti* __restrict__ multi, int64_t nn,
+		FofNode* __restrict__ out) {
+	const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+	if (i >= nn) return;
+	const DNode d = nodes[i];
+	FofNode o;
+	o.pbegin = d.pbegin;
+	o.pend = d.pend;
+	o.c0 = d.c0;
+	o.c1 = d.c1;
+	for (int k = 0; k < 3; k++) {
+		o.mn[k] = multi[i].rmin[k];
+		o.mx[k] = multi[i].rmax[k];
+	}
+	out[i] = o;
+}
+
 constexpr int STACK = 256;
 
 // pass 0 counts each leaf's candidates (leaves b >= a whose boxes come within L), pass 1 writes
 // them at the leaf's offset
-__global__ void k_fof_candidates(const FofNode* __restrict__ nodes, const int32_t* __restrict__ leaves, int nleaves, double L2, int periodic,
+__global__ void k_fof_candidates(const FofNode* __restrict__ nodes, const int4* __restrict__ leaves, int nleaves, double L2, int periodic,
 		int pass, int64_t* __restrict__ count, const int64_t* __restrict__ offset, int2* __restrict__ pairs, int* __restrict__ overflow) {
 	const int k = blockIdx.x * blockDim.x + threadIdx.x;
 	if (k >= nleaves) return;
-	const int a = leaves[k];
+	const int a = leaves[k].x;
 	const FofNode A = nodes[a];
 	int64_t c = 0;
 	if (A.pend == A.pbegin) {
@@ -124,11 +148,12 @@ __device__ int uf_find(int* parent, int x) {
 	return x;
 }
 
-__device__ void uf_union(int* parent, int a, int b) {
+// unites the sets of a and b; returns their root as of then
+__device__ int uf_union(int* parent, int a, int b) {
 	for (;;) {
 		a = uf_find(parent, a);
 		b = uf_find(parent, b);
-		if (a == b) return;
+		if (a == b) return a;
 		if (a > b) {
 			const int t = a;
 			a = b;
@@ -136,36 +161,92 @@ __device__ void uf_union(int* parent, int a, int b) {
 		}
 		// hook the larger root under the smaller one
 		const int old = atomicCAS(&parent[b], b, a);
-		if (old == b) return;
+		if (old == b) return a;
 		b = old;
 	}
 }
 
-// every particle pair of each candidate leaf pair, the reference's integer test
+// a node's box widened by the linking length, in positions
+struct Reach {
+	int lo[3], hi[3];
+};
+
+__device__ __forceinline__ Reach box_reach(const FofNode& b, double Lb) {
+	Reach r;
+	for (int d = 0; d < 3; d++) {
+		r.lo[d] = int(fmax(floor((b.mn[d] - 0.5 - Lb) * 4294967296.0), -2147483648.0));
+		r.hi[d] = int(fmin(ceil((b.mx[d] - 0.5 + Lb) * 4294967296.0), 2147483647.0));
+	}
+	return r;
+}
+
+__device__ __forceinline__ bool within(const Reach& r, const int4& x) {
+	return x.x >= r.lo[0] && x.x <= r.hi[0] && x.y >= r.lo[1] && x.y <= r.hi[1] && x.z >= r.lo[2] && x.z <= r.hi[2];
+}
+
+// Every particle pair of each candidate leaf pair, the reference's integer test.  A linking length is
+// a fraction of the spacing, so of two neighbouring leaves only the particles next to the common face
+// can link: each leaf's are kept in LDS where they come within reach of the other's box (the
+// candidate search's margin), then lane = (particle of A, phase), the phases splitting B's.  In a
+// cluster most links join particles already in one set, which a parent equal to the last root shows
+// without a walk.  Bound by its chains of loads (pair, node, particles, parents): 2M clustered
+// particles, leaves of 32, 2.46 -> 1.28 ms against every pair of two leaves tested in turn.
 __global__ __launch_bounds__(64) void k_fof_link(const FofNode* __restrict__ nodes, const int2* __restrict__ pairs, int64_t npairs,
-		const int4* __restrict__ parts, uint64_t L2, int* __restrict__ parent, int* __restrict__ linked) {
+		const int4* __restrict__ parts, double Lb, uint64_t L2, int* parent, int* linked) {
+	__shared__ int4 sa[64], sb[64];
 	const int64_t q = blockIdx.x;
 	if (q >= npairs) return;
+	const int lane = int(threadIdx.x);
 	const int2 pr = pairs[q];
-	const FofNode A = nodes[pr.x], B = nodes[pr.y];
+	const FofNode &A = nodes[pr.x], &B = nodes[pr.y];
 	const bool same = pr.x == pr.y;
-	for (int i = A.pbegin + threadIdx.x; i < A.pend; i += 64) {
-		const int4 xi = parts[i];
-		for (int j = same ? i + 1 : B.pbegin; j < B.pend; j++) {
-			const int4 xj = parts[j];
-			// vect<pos_type> difference (int32 wrap), then vect<uint64_t> and its dot product; a
-			// difference that wraps crosses the box edge
-			const int64_t ex = int64_t(xi.x) - int64_t(xj.x), ey = int64_t(xi.y) - int64_t(xj.y), ez = int64_t(xi.z) - int64_t(xj.z);
-			const bool wraps = ex != int64_t(int32_t(ex)) || ey != int64_t(int32_t(ey)) || ez != int64_t(int32_t(ez));
-			const uint64_t dx = uint64_t(int64_t(int32_t(uint32_t(xi.x) - uint32_t(xj.x))));
-			const uint64_t dy = uint64_t(int64_t(int32_t(uint32_t(xi.y) - uint32_t(xj.y))));
-			const uint64_t dz = uint64_t(int64_t(int32_t(uint32_t(xi.z) - uint32_t(xj.z))));
-			const uint64_t d2 = dx * dx + dy * dy + dz * dz;
-			if (d2 < L2 && d2 != 0 && !wraps) {
-				linked[i] = 1;
-				linked[j] = 1;
-				uf_union(parent, i, j);
+	const int ae = A.pend, bb = B.pbegin, be = B.pend;
+	const Reach ra = box_reach(A, Lb), rb = box_reach(B, Lb);
+	const uint64_t before = (uint64_t(1) << lane) - 1;
+	for (int a0 = A.pbegin; a0 < ae; a0 += 64) {
+		int4 x = a0 + lane < ae ? parts[a0 + lane] : make_int4(0, 0, 0, 0);
+		bool in = a0 + lane < ae && (same || within(rb, x));
+		uint64_t m = __ballot(in);
+		const int na = __popcll(m);
+		if (na == 0) continue;
+		x.w = a0 + lane;
+		if (in) sa[__popcll(m & before)] = x;
+		const int lg = na <= 1 ? 0 : 32 - __clz(na - 1);
+		const int P = 64 >> lg, ph = lane >> lg, ia = lane & ((1 << lg) - 1);
+		for (int b0 = same ? a0 : bb; b0 < be; b0 += 64) {
+			x = b0 + lane < be ? parts[b0 + lane] : make_int4(0, 0, 0, 0);
+			in = b0 + lane < be && (same || within(ra, x));
+			m = __ballot(in);
+			const int nb = __popcll(m);
+			x.w = b0 + lane;
+			if (in) sb[__popcll(m & before)] = x;
+			__syncthreads();
+			if (ia < na) {
+				const int4 xi = sa[ia];
+				const int i = xi.w;
+				int root = -1;  // of i's set, when last looked at
+				for (int k = ph; k < nb; k += P) {
+					const int4 xj = sb[k];
+					const int j = xj.w;
+					// vect<pos_type> difference (int32 wrap), then vect<uint64_t> and its dot product; a
+					// difference that wraps crosses the box edge
+					const int64_t ex = int64_t(xi.x) - int64_t(xj.x), ey = int64_t(xi.y) - int64_t(xj.y), ez = int64_t(xi.z) - int64_t(xj.z);
+					const bool wraps = ex != int64_t(int32_t(ex)) || ey != int64_t(int32_t(ey)) || ez != int64_t(int32_t(ez));
+					const uint64_t d2 = uint64_t(int64_t(int32_t(ex)) * int32_t(ex)) + uint64_t(int64_t(int32_t(ey)) * int32_t(ey)) +
+							uint64_t(int64_t(int32_t(ez)) * int32_t(ez));
+					if (d2 < L2 && d2 != 0 && !wraps && (!same || j > i)) {
+						// a parent that was i's root once keeps j in i's set
+						if (root >= 0 && ld(parent + j) == root) {
+							if (!linked[j]) linked[j] = 1;
+							continue;
+						}
+						root = uf_union(parent, i, j);
+						linked[i] = 1;
+						linked[j] = 1;
+					}
+				}
 			}
+			__syncthreads();
 		}
 	}
 }
@@ -178,29 +259,41 @@ __global__ void k_fof_init(int* parent, int* linked, int64_t n) {
 	}
 }
 
-__global__ void k_fof_labels(int* parent, const int* __restrict__ linked, int64_t n, uint64_t* __restrict__ group) {
-	const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-	if (i < n) group[i] = linked[i] ? uint64_t(uf_find(parent, int(i))) : TG_FOF_NONE;
+// the labels in tree and in input order; the groups counted by their roots
+__global__ __launch_bounds__(256) void k_fof_labels(int* parent, const int* __restrict__ linked, const int64_t* __restrict__ order, int64_t n,
+		uint64_t* __restrict__ group, uint64_t* __restrict__ group_in, unsigned long long* __restrict__ ngroups) {
+	const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+	const uint64_t g = i < n && linked[i] ? uint64_t(uf_find(parent, int(i))) : TG_FOF_NONE;
+	const int roots = __syncthreads_count(i < n && g == uint64_t(i));
+	if (threadIdx.x == 0 && roots) atomicAdd(ngroups, (unsigned long long) roots);
+	if (i >= n) return;
+	group[i] = g;
+	group_in[order[i]] = g;
 }
 
-struct Buf {
-	void* p = nullptr;
-	~Buf() {
-		if (p) (void) hipFree(p);
+// device memory of one call, freed once the stream has drained
+struct Scratch {
+	hipStream_t s;
+	std::vector<void*> blocks;
+	~Scratch() {
+		(void) hipStreamSynchronize(s);
+		for (void* p : blocks) dev_free(p);
 	}
-	hipError_t alloc(size_t b) { return hipMalloc(&p, b < 256 ? 256 : b); }
 	template <class T>
-	T* as() const {
-		return static_cast<T*>(p);
+	hipError_t get(T** p, size_t count) {
+		void* q = nullptr;
+		const hipError_t e = dev_malloc(&q, std::max<size_t>(count * sizeof(T), 16));
+		if (e == hipSuccess) blocks.push_back(q);
+		*p = static_cast<T*>(q);
+		return e;
 	}
 };
 
 }  // namespace
 
-hipError_t fof_device(const Tree& T, const int4* d_parts, double link_len, int device, hipStream_t s, uint64_t* group_tree,
-		int64_t* n_candidates, std::string& err) {
-	const int64_t n = int64_t(T.pos.size() / 3);
-	const int64_t nn = int64_t(T.nodes.size());
+hipError_t fof_device(const FofSource& F, double link_len, hipStream_t s, uint64_t* group_tree, uint64_t* group_input, int64_t* n_groups,
+		std::string& err) {
+	const int64_t n = F.n, nn = F.nn;
 	hipError_t e = hipSuccess;
 #define FCHK(call)                                                 \
 	do {                                                           \
@@ -210,52 +303,65 @@ hipError_t fof_device(const Tree& T, const int4* d_parts, double link_len, int d
 			return e;                                              \
 		}                                                          \
 	} while (0)
+	*n_groups = 0;
 	if (n == 0) return hipSuccess;
-	FCHK(hipSetDevice(device));
 	// the reference's integer linking length (src/part_vect.cpp:86-88)
 	const uint64_t L = uint64_t((std::pow(double(n), -1.0 / 3.0) * link_len) * 4294967295.0);
 	const uint64_t L2 = L * L;
 	// candidate boxes within the linking length, with a margin (the exact test is per pair)
 	const double Lb = 1.01 * double(L) / 4294967296.0 + 1e-9;
-	std::vector<FofNode> hn(static_cast<size_t>(nn));
-	for (int64_t i = 0; i < nn; i++) {
-		const Node& d = T.nodes[size_t(i)];
-		FofNode& o = hn[size_t(i)];
-		o.pbegin = d.pbegin;
-		o.pend = d.pend;
-		o.c0 = d.child[0];
-		o.c1 = d.child[1];
-		for (int k = 0; k < 3; k++) {
-			o.mn[k] = d.rmin[k];
-			o.mx[k] = d.rmax[k];
+	const int nleaves = F.n_leaf_items;
+	std::vector<FofNode> hn;
+	Scratch scratch{s, {}};  // drained before hn goes
+	FofNode* nodes;
+	int64_t *count, *offset, *work, *info;  // info: candidate pairs, overflow, groups
+	int *parent, *linked;
+	uint64_t* gin;
+	int2* pairs;
+	ScanSet sc;
+	FCHK(scratch.get(&nodes, size_t(nn)));
+	FCHK(scratch.get(&count, size_t(nleaves)));
+	FCHK(scratch.get(&offset, size_t(nleaves)));
+	FCHK(scratch.get(&info, 3));
+	FCHK(scratch.get(&parent, size_t(n)));
+	FCHK(scratch.get(&linked, size_t(n)));
+	FCHK(scratch.get(&gin, size_t(n)));
+	sc.add(count, offset, nleaves);
+	FCHK(scratch.get(&work, size_t(scan_workspace(sc))));
+	if (F.dtree) {
+		hipLaunchKernelGGL(k_fof_nodes, dim3(unsigned((nn + 255) / 256)), dim3(256), 0, s, F.dtree->nodes, F.dtree->multi, nn, nodes);
+		FCHK(hipGetLastError());
+	} else {
+		hn.resize(static_cast<size_t>(nn));
+		for (int64_t i = 0; i < nn; i++) {
+			const Node& d = F.tree->nodes[size_t(i)];
+			FofNode& o = hn[size_t(i)];
+			o.pbegin = d.pbegin;
+			o.pend = d.pend;
+			o.c0 = d.child[0];
+			o.c1 = d.child[1];
+			for (int k = 0; k < 3; k++) {
+				o.mn[k] = d.rmin[k];
+				o.mx[k] = d.rmax[k];
+			}
 		}
+		FCHK(hipMemcpyAsync(nodes, hn.data(), hn.size() * sizeof(FofNode), hipMemcpyHostToDevice, s));
 	}
-	const int nleaves = int(T.leaves.size());
-	Buf dnodes, dleaves, dcount, doffset, dpairs, dparent, dlinked, dgroup, doverflow, tmp;
-	FCHK(dnodes.alloc(hn.size() * sizeof(FofNode)));
-	FCHK(dleaves.alloc(size_t(nleaves) * 4));
-	FCHK(dcount.alloc(size_t(nleaves + 1) * 8));
-	FCHK(doffset.alloc(size_t(nleaves + 1) * 8));
-	FCHK(doverflow.alloc(4));
-	FCHK(hipMemcpyAsync(dnodes.p, hn.data(), hn.size() * sizeof(FofNode), hipMemcpyHostToDevice, s));
-	FCHK(hipMemcpyAsync(dleaves.p, T.leaves.data(), size_t(nleaves) * 4, hipMemcpyHostToDevice, s));
-	FCHK(hipMemsetAsync(doverflow.p, 0, 4, s));
-	FCHK(hipMemsetAsync(dcount.p, 0, size_t(nleaves + 1) * 8, s));
+	FCHK(hipMemsetAsync(info, 0, 3 * 8, s));
 	const bool periodic = false;  // pairs across the box edge are not friends (above)
-	const unsigned lb = unsigned((nleaves + 127) / 128);
-	hipLaunchKernelGGL(k_fof_candidates, dim3(lb), dim3(128), 0, s, dnodes.as<const FofNode>(), dleaves.as<const int32_t>(), nleaves, Lb * Lb,
-			int(periodic), 0, dcount.as<int64_t>(), nullptr, nullptr, doverflow.as<int>());
+	const unsigned lb = unsigned((nleaves + 127) / 128), pb = unsigned((n + 255) / 256);
+	int* overflow = reinterpret_cast<int*>(info + 1);
+	hipLaunchKernelGGL(k_fof_init, dim3(pb), dim3(256), 0, s, parent, linked, n);
 	FCHK(hipGetLastError());
-	size_t tb = 0;
-	FCHK(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, dcount.as<int64_t>(), doffset.as<int64_t>(), nleaves + 1, s));
-	FCHK(tmp.alloc(tb));
-	FCHK(hipcub::DeviceScan::ExclusiveSum(tmp.p, tb, dcount.as<int64_t>(), doffset.as<int64_t>(), nleaves + 1, s));
-	int64_t npairs = 0;
-	int overflow = 0;
-	FCHK(hipMemcpyAsync(&npairs, doffset.as<int64_t>() + nleaves, 8, hipMemcpyDeviceToHost, s));
-	FCHK(hipMemcpyAsync(&overflow, doverflow.p, 4, hipMemcpyDeviceToHost, s));
+	hipLaunchKernelGGL(k_fof_candidates, dim3(lb), dim3(128), 0, s, nodes, F.leaf_items, nleaves, Lb * Lb, int(periodic), 0, count, nullptr, nullptr,
+			overflow);
+	FCHK(hipGetLastError());
+	FCHK(scan_columns(sc, work, info, s));
+	int64_t v[3];
+	FCHK(hipMemcpyAsync(v, info, sizeof(v), hipMemcpyDeviceToHost, s));
 	FCHK(hipStreamSynchronize(s));
-	if (overflow) {
+	const int64_t npairs = v[0];
+	if (v[1]) {
 		err = "friends-of-friends: tree deeper than the candidate search's stack";
 		return hipErrorInvalidValue;
 	}
@@ -263,23 +369,21 @@ hipError_t fof_device(const Tree& T, const int4* d_parts, double link_len, int d
 		err = "friends-of-friends: more candidate leaf pairs than one launch takes";
 		return hipErrorInvalidValue;
 	}
-	FCHK(dpairs.alloc(size_t(npairs) * sizeof(int2)));
-	hipLaunchKernelGGL(k_fof_candidates, dim3(lb), dim3(128), 0, s, dnodes.as<const FofNode>(), dleaves.as<const int32_t>(), nleaves, Lb * Lb,
-			int(periodic), 1, dcount.as<int64_t>(), doffset.as<const int64_t>(), dpairs.as<int2>(), doverflow.as<int>());
+	FCHK(scratch.get(&pairs, size_t(npairs)));
+	hipLaunchKernelGGL(k_fof_candidates, dim3(lb), dim3(128), 0, s, nodes, F.leaf_items, nleaves, Lb * Lb, int(periodic), 1, count, offset, pairs,
+			overflow);
 	FCHK(hipGetLastError());
-	FCHK(dparent.alloc(size_t(n) * 4));
-	FCHK(dlinked.alloc(size_t(n) * 4));
-	FCHK(dgroup.alloc(size_t(n) * 8));
-	const unsigned pb = unsigned((n + 255) / 256);
-	hipLaunchKernelGGL(k_fof_init, dim3(pb), dim3(256), 0, s, dparent.as<int>(), dlinked.as<int>(), n);
-	if (npairs > 0)
-		hipLaunchKernelGGL(k_fof_link, dim3(unsigned(npairs)), dim3(64), 0, s, dnodes.as<const FofNode>(), dpairs.as<const int2>(), npairs,
-				d_parts, L2, dparent.as<int>(), dlinked.as<int>());
-	hipLaunchKernelGGL(k_fof_labels, dim3(pb), dim3(256), 0, s, dparent.as<int>(), dlinked.as<const int>(), n, dgroup.as<uint64_t>());
+	if (npairs > 0) {
+		hipLaunchKernelGGL(k_fof_link, dim3(unsigned(npairs)), dim3(64), 0, s, nodes, pairs, npairs, F.parts, Lb, L2, parent, linked);
+		FCHK(hipGetLastError());
+	}
+	hipLaunchKernelGGL(k_fof_labels, dim3(pb), dim3(256), 0, s, parent, linked, F.order, n, group_tree, gin,
+			reinterpret_cast<unsigned long long*>(info + 2));
 	FCHK(hipGetLastError());
-	FCHK(hipMemcpyAsync(group_tree, dgroup.p, size_t(n) * 8, hipMemcpyDeviceToHost, s));
+	FCHK(hipMemcpyAsync(v, info, sizeof(v), hipMemcpyDeviceToHost, s));
+	FCHK(hipMemcpyAsync(group_input, gin, size_t(n) * 8, hipMemcpyDeviceToHost, s));
 	FCHK(hipStreamSynchronize(s));
-	if (n_candidates) *n_candidates = npairs;
+	*n_groups = v[2];
 	return hipSuccess;
 #undef FCHK
 }

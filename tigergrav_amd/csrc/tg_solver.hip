@@ -300,6 +300,7 @@ Solver::~Solver() {
 		d_adj_lam.release();
 		d_adj_mu.release();
 		d_adj_out.release();
+		d_fof.release();
 		for (int e = 0; e < 2; e++) {
 			d_adj_cct_keys[e].release();
 			d_adj_cpt_keys[e].release();
@@ -365,6 +366,7 @@ int Solver::set_particles(const int32_t* x, const float* mass, int64_t count, bo
 	} later{*this};
 	order_on_device = false;
 	fof_group.clear();
+	fof_done = false;
 	n = count;
 	TreeParams P;
 	P.ewald = ewald;
@@ -377,13 +379,13 @@ int Solver::set_particles(const int32_t* x, const float* mass, int64_t count, bo
 	// with the walk on the device too, the tree stays there: the walk and the solve's arrays are
 	// made from it on the device, and the host copy only on demand (host_tree)
 	const bool keep_tree = gpu_tree && gpu_walk && device >= 0;
-	tree_on_device = false;
+	tree_on_device = dtree_current = false;
 	if (gpu_tree && device >= 0) {
 		double tt[2] = {0.0, 0.0};
 		const hipError_t e = device_build_tree(tree, x, mass, count, P, m, device, stream, err, tt, on_device, keep_tree ? &dtree : nullptr,
 				build_later);
 		if (e != hipSuccess) return e == hipErrorOutOfMemory ? TG_ENOMEM : TG_EHIP;
-		tree_on_device = keep_tree;
+		tree_on_device = dtree_current = keep_tree;
 		t1 = t0 + tt[0];
 		t2 = now();
 	} else {
@@ -437,6 +439,7 @@ int Solver::update_particles(const int32_t* x, const float* mass) {
 		return TG_EINVAL;
 	}
 	drop_graph();
+	dtree_current = false;  // its boxes are the build's
 	std::vector<int32_t> pt(3 * size_t(n));
 	std::vector<float> mt;
 	for (int64_t i = 0; i < n; i++)
@@ -960,29 +963,55 @@ int tg_solver_get_forces_device(tg_solver* h, tg_force* f) {
 int tg_solver_find_groups(tg_solver* h, double link_len, uint64_t* group, int64_t* n_groups) {
 	if (!h || h->s.device < 0 || (h->s.n > 0 && !group) || !(link_len > 0.0)) return TG_EINVAL;
 	tg::Solver& S = h->s;
-	const int64_t n = S.n;
-	{
-		const int rc = S.host_tree();  // the candidate search walks the host tree
-		if (rc != TG_OK) return fail(h, rc);
-	}
-	S.fof_group.assign(size_t(n), TG_FOF_NONE);
-	int64_t cand = 0;
-	const hipError_t e = tg::fof_device(S.tree, S.d_parts.as<const int4>(), link_len, S.device, S.stream, S.fof_group.data(), &cand, S.err);
-	if (e != hipSuccess) return fail(h, e == hipErrorOutOfMemory ? TG_ENOMEM : TG_EHIP);
+	S.fof_group.clear();
+	S.fof_done = false;
 	int64_t ng = 0;
-	for (int64_t i = 0; i < n; i++) {
-		group[S.tree.order[size_t(i)]] = S.fof_group[size_t(i)];
-		ng += S.fof_group[size_t(i)] == uint64_t(i);
+	if (S.n > 0) {
+		tg::FofSource F;
+		int rc = TG_OK;
+		if (S.dtree.nodes && S.dtree_current)
+			F.dtree = &S.dtree;
+		else
+			rc = S.host_tree();
+		if (rc == TG_OK) rc = S.forces_device_order();  // the input index of each tree-order particle
+		if (rc != TG_OK) return fail(h, rc);
+		F.tree = &S.tree;
+		F.parts = S.d_parts.as<const int4>();
+		F.order = S.d_order.as<const int64_t>();
+		F.leaf_items = S.d_leaf_items.as<const int4>();
+		F.n_leaf_items = S.n_leaf_items;
+		F.n = S.n;
+		F.nn = S.n_nodes;
+		hipError_t e = hipSetDevice(S.device);
+		if (e == hipSuccess) e = S.d_fof.alloc(size_t(S.n) * 8);
+		if (e != hipSuccess)
+			S.err = hipGetErrorString(e);
+		else
+			e = tg::fof_device(F, link_len, S.stream, S.d_fof.as<uint64_t>(), group, &ng, S.err);
+		if (e != hipSuccess) return fail(h, e == hipErrorOutOfMemory ? TG_ENOMEM : TG_EHIP);
 	}
+	S.fof_done = true;
 	if (n_groups) *n_groups = ng;
 	return TG_OK;
 }
 
 int tg_solver_group_catalog(tg_solver* h, const float* v, double a, int32_t min_n, tg_group* out, int64_t capacity, int64_t* n_out) {
 	if (!h || !n_out || !(a > 0.0) || (h->s.n > 0 && !v) || capacity < 0) return TG_EINVAL;
-	if (h->s.fof_group.size() != size_t(h->s.n)) {
+	if (h->s.n > 0 && !h->s.fof_done) {
 		g_solver_err = "tg_solver_group_catalog before tg_solver_find_groups";
 		return TG_EINVAL;
+	}
+	if (h->s.fof_group.size() != size_t(h->s.n)) {
+		// the catalog reads the tree and the groups on the host
+		const int rc = h->s.host_tree();
+		if (rc != TG_OK) return fail(h, rc);
+		h->s.fof_group.resize(size_t(h->s.n));
+		const hipError_t e = hipSetDevice(h->s.device);
+		if (e != hipSuccess || hipMemcpy(h->s.fof_group.data(), h->s.d_fof.p, size_t(h->s.n) * 8, hipMemcpyDeviceToHost) != hipSuccess) {
+			h->s.fof_group.clear();
+			g_solver_err = "tg_solver_group_catalog: device copy failed";
+			return TG_EHIP;
+		}
 	}
 	return tg::group_catalog(h->s.tree, h->s.fof_group, v, a, min_n, out, capacity, n_out);
 }

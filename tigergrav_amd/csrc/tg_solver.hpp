@@ -84,7 +84,9 @@ struct Solver {
 	// host-only solvers (device < 0) keep the PP-direct items and flattened source list
 	hvec<int4> host_pp_items;
 	std::vector<int> host_pp_list;
-	std::vector<uint64_t> fof_group;  // friends-of-friends group per particle, tree order (find_groups)
+	DeviceArray d_fof;                // friends-of-friends group per particle, tree order (find_groups)
+	std::vector<uint64_t> fof_group;  // its host copy, for the catalog
+	bool fof_done = false;
 	int n_leaf_items = 0;
 	int64_t n_slots = 0;
 	int64_t list_bytes = 0;
@@ -93,6 +95,7 @@ struct Solver {
 	// on demand (host_tree)
 	DeviceTree dtree;
 	bool tree_on_device = false;  // tree holds no copy of dtree yet
+	bool dtree_current = false;   // dtree is the solver's tree, particles where it was built
 	int64_t n_nodes = 0;          // nodes of the current tree
 	int64_t n_leaves = 0;         // its leaves, empty ones included
 	int max_level = 0;            // its deepest level
