@@ -401,6 +401,7 @@ __global__ __launch_bounds__(64 * NW) void k_adj_pp_ewald(AdjArgs A, AdjItems I)
 	__shared__ int4 tps[NW][64];
 	__shared__ float4 tws[NW][64];
 	__shared__ double red[NW > 1 ? NW - 1 : 1][4][64];
+	__shared__ EwtStage stages[NW];
 	int4* tp = tps[T.wave];
 	float4* tw = tws[T.wave];
 	double gx[3] = {0.0, 0.0, 0.0}, gm = 0.0;
@@ -414,15 +415,33 @@ __global__ __launch_bounds__(64 * NW) void k_adj_pp_ewald(AdjArgs A, AdjItems I)
 		}
 		wave_lds_sync<NW>();
 		float fx[3] = {0.f, 0.f, 0.f}, fm = 0.f;
-		for (int k = T.ph; k < n; k += T.P) {
-			const int4 s = tp[k];
-			const float4 ws = tw[k];
-			const float mj = __int_as_float(s.w);
+		// the whole wave takes every turn (its table rows are read together), the next turn's rows on
+		// their way while this turn's are evaluated
+		auto at = [&](int k0, bool& on) {
+			const int4 s = tp[min(k0 + T.ph, n - 1)];
 			const float x[3] = {sepf(me.x, s.x, true), sepf(me.y, s.y, true), sepf(me.z, s.z, true)};
 			const float r2 = fmaf(x[2], x[2], fmaf(x[1], x[1], x[0] * x[0]));
-			if (!(r2 > 1e-12f)) continue;  // the reference's constant below r = 1e-6: no derivatives
-			float D[10];
-			green_ewald_tab<10>(D, x, c_adj_ewt);
+			on = k0 + T.ph < n && r2 > 1e-12f;  // the reference's constant below r = 1e-6: no derivatives
+			return ewt_point(x);
+		};
+		bool on;
+		EwtPoint p = at(0, on);
+		EwtRows<10> rows;
+		rows.fetch(p.row, c_adj_ewt, stages[T.wave], T.lane);
+		for (int k0 = 0; k0 < n; k0 += T.P) {
+			float c[EwtRead<10>::F4 * 4], D[10];
+			rows.take(c, stages[T.wave], T.lane);
+			const EwtPoint now = p;
+			const bool add_it = on;
+			const int k = min(k0 + T.ph, n - 1);
+			const float mj = __int_as_float(tp[k].w);
+			const float4 ws = tw[k];
+			if (k0 + T.P < n) {
+				p = at(k0 + T.P, on);
+				rows.fetch(p.row, c_adj_ewt, stages[T.wave], T.lane);
+			}
+			ewt_eval<10>(D, c, now);
+			if (!add_it) continue;
 			const float v[3] = {mj * wi[0] - mi * ws.x, mj * wi[1] - mi * ws.y, mj * wi[2] - mi * ws.z};
 			for_n<3>([&](auto b_) {
 				constexpr int b = decltype(b_)::value;
@@ -449,6 +468,7 @@ __global__ __launch_bounds__(64 * NW) void k_adj_pc_sink(AdjArgs A, AdjItems I) 
 	const int4 it = I.items[blockIdx.x];
 	LeafLanes<NW> T(it);
 	__shared__ double red[NW > 1 ? NW - 1 : 1][4][64];
+	__shared__ EwtStage stages[EWALD ? NW : 1];
 	const int4 me = A.parts[T.pi];
 	const float4 wv = A.w[T.pi];
 	const float wi[3] = {wv.x, wv.y, wv.z};
@@ -457,18 +477,20 @@ __global__ __launch_bounds__(64 * NW) void k_adj_pc_sink(AdjArgs A, AdjItems I) 
 	for (int base = T.share.x; base < T.share.y; base += 64) {
 		const int end = min(base + 64, T.share.y);
 		float gx[3] = {0.f, 0.f, 0.f};
-		for (int e = base + T.ph; e < end; e += T.P) {
-			const MultiSrc& ms = A.multis[I.list[e]];
+		for (int e0 = base; e0 < end; e0 += T.P) {
+			const int e = e0 + T.ph;
+			if (!EWALD && e >= end) break;
+			const MultiSrc& ms = A.multis[I.list[min(e, end - 1)]];
 			float M[17];
 #pragma unroll
 			for (int q = 0; q < 17; q++) M[q] = ms.m[q];
 			const float d[3] = {sepf(me.x, ms.x[0], wrapx), sepf(me.y, ms.x[1], wrapx), sepf(me.z, ms.x[2], wrapx)};
 			float D[adj::NS5];
 			if (EWALD)
-				green_ewald_tab<adj::NS5>(D, d, c_adj_ewt);
+				green_ewald_wave<adj::NS5>(D, d, c_adj_ewt, stages[EWALD ? T.wave : 0], T.lane);
 			else
 				adj::green_direct_n<adj::NS5>(D, d);
-			m2p_sink_adjoint(gx, M, D, wi);
+			if (!EWALD || e < end) m2p_sink_adjoint(gx, M, D, wi);
 		}
 #pragma unroll
 		for (int b = 0; b < 3; b++) dx[b] += double(gx[b]);
@@ -506,21 +528,22 @@ __global__ __launch_bounds__(64) void k_adj_pc_t(AdjPCArgs A) {
 	float mu[17];
 #pragma unroll
 	for (int q = 0; q < 17; q++) mu[q] = 0.0f;
+	__shared__ EwtStage stage[1];
 	for (int k = it.y + qq; k - qq < it.z; k += Q) {
-		if (k >= it.z) continue;
-		const int2 lf = A.leaves[k];
-		if (o >= lf.y) continue;
-		const int pi = lf.x + o;
+		const int2 lf = A.leaves[min(k, it.z - 1)];
+		const bool on = k < it.z && o < lf.y;
+		if (!EWALD && !on) continue;
+		const int pi = lf.x + (on ? o : 0);
 		const int4 me = A.parts[pi];
 		const float4 wv = A.w[pi];
 		const float wi[3] = {wv.x, wv.y, wv.z};
 		const float d[3] = {sepf(me.x, cx0, wrapx), sepf(me.y, cx1, wrapx), sepf(me.z, cx2, wrapx)};
 		float D[35];
 		if (EWALD)
-			green_ewald_tab<35>(D, d, c_adj_ewt);
+			green_ewald_wave<35>(D, d, c_adj_ewt, stage[0], t);
 		else
 			adj::green_direct_n<35>(D, d);
-		m2p_source_adjoint(mu, D, wi);
+		if (on) m2p_source_adjoint(mu, D, wi);
 	}
 	__shared__ float red[17][65];
 #pragma unroll
@@ -570,6 +593,7 @@ __global__ __launch_bounds__(64 * NW) void k_adj_cp_t(AdjCPArgs A) {
 	__shared__ float lams[NW][64][36];
 	__shared__ int4 xss[NW][64];
 	__shared__ double red[NW > 1 ? NW - 1 : 1][4][64];
+	__shared__ EwtStage stages[EWALD ? NW : 1];
 	float (*lam)[36] = lams[wave];
 	int4* xs = xss[wave];
 	double gm = 0.0, g3[3] = {0.0, 0.0, 0.0};
@@ -584,14 +608,17 @@ __global__ __launch_bounds__(64 * NW) void k_adj_cp_t(AdjCPArgs A) {
 		}
 		wave_lds_sync<NW>();
 		float fm = 0.0f, f3[3] = {0.f, 0.f, 0.f};
-		for (int k = ph; k < n; k += P) {
+		for (int k0 = 0; k0 < n; k0 += P) {
+			if (!EWALD && k0 + ph >= n) break;
+			const int k = min(k0 + ph, n - 1);
 			const int4 X = xs[k];
 			const float d[3] = {sepf(X.x, me.x, wrapx), sepf(X.y, me.y, wrapx), sepf(X.z, me.z, wrapx)};
 			float D[adj::NS5];
 			if (EWALD)
-				green_ewald_tab<adj::NS5>(D, d, c_adj_ewt);
+				green_ewald_wave<adj::NS5>(D, d, c_adj_ewt, stages[EWALD ? wave : 0], t);
 			else
 				adj::green_direct_n<adj::NS5>(D, d);
+			if (EWALD && k0 + ph >= n) continue;
 			for_n<35>([&](auto t_) {
 				constexpr int tt = decltype(t_)::value;
 				const float l = lam[k][tt];
@@ -639,12 +666,13 @@ __global__ __launch_bounds__(64) void k_adj_cc_t(AdjCCArgs A) {
 	const int cnt = int(A.n - begin < 64 ? A.n - begin : 64);
 	__shared__ float red[17][65];
 	__shared__ int sc[64];
+	__shared__ EwtStage stage[1];
 	float mu[17];
 #pragma unroll
 	for (int q = 0; q < 17; q++) mu[q] = 0.0f;
 	int c = -1;
-	if (j < A.n) {
-		const uint64_t key = A.keys[j];
+	if (EWALD || j < A.n) {  // the Ewald kind's wave reads its table rows together
+		const uint64_t key = A.keys[j < A.n ? j : A.n - 1];
 		c = int(key >> A.sink_bits);
 		const int a = int(key & ((uint64_t(1) << A.sink_bits) - 1));
 		const int4 X = A.nodepos[a];
@@ -656,10 +684,13 @@ __global__ __launch_bounds__(64) void k_adj_cc_t(AdjCCArgs A) {
 		const float d[3] = {sepf(X.x, ms.x[0], wrapx), sepf(X.y, ms.x[1], wrapx), sepf(X.z, ms.x[2], wrapx)};
 		float D[35];
 		if (EWALD)
-			green_ewald_tab<35>(D, d, c_adj_ewt);
+			green_ewald_wave<35>(D, d, c_adj_ewt, stage[0], t);
 		else
 			adj::green_direct_n<35>(D, d);
-		m2l_adjoint(mu, Lam, D);
+		if (j < A.n)
+			m2l_adjoint(mu, Lam, D);
+		else
+			c = -1;
 	}
 #pragma unroll
 	for (int q = 0; q < 17; q++) red[q][t] = mu[q];

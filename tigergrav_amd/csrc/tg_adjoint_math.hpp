@@ -9,7 +9,7 @@
 // ([0], [1+a], [4+s2], [10+s3], [20+s4]; tigergrav/expansion.hpp:77-137) followed by the 21
 // sorted index quintuples in lexicographic order.  Slot k holds the index multiset with counts
 // (n0, n1, n2) of the values 0, 1, 2; every loop over slots is unrolled with compile-time indices.
-// The periodic correction's derivatives come from the forward's table (green_ewald_tab, tg_math.hpp).
+// The periodic correction's derivatives come from the forward's table (ewt_eval, tg_math.hpp).
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -27,7 +27,7 @@
 #define TG_EWT_P 6545   // grid points with i >= j >= l: TG_EWT_N (TG_EWT_N + 1) (TG_EWT_N + 2) / 6
 #define TG_EWT_ROWS (TG_EWT_P + 1)  // and one row for coincident points: the reference's constants
 #define TG_EWT_C 64      // slots stored per row: those holding the third axis at most once (2 n + 1 of order n)
-#define TG_EWT_STRIDE 68  // floats per row: 272 bytes
+#define TG_EWT_STRIDE 64  // floats per row: two lines of 128 bytes
 
 namespace tg {
 namespace ewt {

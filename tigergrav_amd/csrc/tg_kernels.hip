@@ -10,7 +10,7 @@
 //  * node kinds (CC, CP): lane = source; a wave packs the short lists of several expansion
 //    centres (<= 64 entries), 35 float accumulators per lane, merged per centre in FP64 through
 //    LDS by a segmented scan.
-//  * Ewald kinds use tg::green_ewald (tg_math.hpp) and, for PP, green_ewald1_real below.
+//  * Ewald kinds use tg::ewt_eval (tg_math.hpp).
 #include "tg_kernels.hpp"
 #include "tg_leaf_waves.hpp"
 #include "tg_math.hpp"
@@ -368,6 +368,7 @@ __global__ __launch_bounds__(64 * NW) void k_pc(LeafArgs A) {
 	const int4 me = A.sinks[it.x + min(si, ns - 1)];
 	__shared__ float tiles[NW][64][20];
 	__shared__ double red[NW > 1 ? NW - 1 : 1][4][64];
+	__shared__ EwtStage stages[EWALD ? NW : 1];
 	float (*tile)[20] = tiles[wave];
 	float phi = 0.f, g[3] = {0.f, 0.f, 0.f};
 	double dphi = 0.0, dg[3] = {0.0, 0.0, 0.0};
@@ -386,7 +387,10 @@ __global__ __launch_bounds__(64 * NW) void k_pc(LeafArgs A) {
 			}
 		}
 		wave_lds_sync<NW>();
-		for (int k = ph; k < n; k += P) {
+		// the whole wave takes every turn of the Ewald kind's loop (its rows are read together)
+		for (int k0 = 0; k0 < n; k0 += P) {
+			const int k = min(k0 + ph, n - 1);
+			if (!EWALD && k0 + ph >= n) break;
 			float M[17];
 #pragma unroll
 			for (int q = 0; q < 17; q++) M[q] = tile[k][q];
@@ -395,10 +399,10 @@ __global__ __launch_bounds__(64 * NW) void k_pc(LeafArgs A) {
 					sepu<EWALD || WRAP>(me.z, __float_as_int(tile[k][19])) * POS_INVF};
 			float D[35];
 			if (EWALD)
-				green_ewald(D, x);
+				green_ewald_wave<35>(D, x, c_ewt, stages[EWALD ? wave : 0], lane);
 			else
 				green_direct(D, x);
-			m2p(phi, g, M, D);
+			if (!EWALD || k0 + ph < n) m2p(phi, g, M, D);
 		}
 		dphi += phi;
 		dg[0] += g[0];
@@ -439,16 +443,20 @@ hipError_t launch_pc(const LeafArgs& a, bool ewald, hipStream_t s) {
 
 // ---- PP Ewald correction -------------------------------------------------------------------------
 // The periodic correction between particle pairs (src/gravity.cpp:491-614): per pair the potential
-// and gradient of the tabulated correction (green_ewald_tab<4>: the reference's real-space images,
+// and gradient of the tabulated correction (ewt_eval<4>: the reference's real-space images,
 // Fourier terms, n = 0 term and pi/4 in one table), weighted by the source mass; pairs closer than
 // 1e-6 take the reference's constant 2.8372975 and zero force (its zmask).  Sinks and sources are
 // laid out as in k_pc: 2^lg lanes per sink, the other lane bits split the tile's sources.
+// Bound by the rows' way through the vector cache and LDS (8 KB a turn) beside about 150
+// instructions of arithmetic, at the four waves a SIMD that the stages leave.  32,768 uniform
+// particles, leaves of 64 (4.5e7 pairs): 646 -> 430 us against a row read by each lane and a 19-term
+// sum per component.
 template <int NW>
 __global__ __launch_bounds__(64 * NW) void k_pp_ewald(LeafArgs A) {
 	const int4 it = A.items[blockIdx.x];
 	const int lane = threadIdx.x & 63;
 	const int wave = NW == 1 ? 0 : int(threadIdx.x >> 6);
-	const int2 share = wave_share<NW>(it.z, it.w, wave);
+	const int2 share = wave_share<NW, 8>(it.z, it.w, wave);
 	const int ns = it.y & PP_COUNT_MASK;
 	const int lg = ceil_log2_64(ns);
 	const int nsp = 1 << lg;
@@ -456,8 +464,11 @@ __global__ __launch_bounds__(64 * NW) void k_pp_ewald(LeafArgs A) {
 	const int si = lane & (nsp - 1);
 	const int ph = lane >> lg;
 	const int4 me = A.sinks[it.x + min(si, ns - 1)];
+	// the sums' exchange at the end reuses the stages (16 waves take 152 KB with them)
+	__shared__ EwtStage stages[NW];
 	__shared__ int4 tiles[NW][64];
-	__shared__ double red[NW > 1 ? NW - 1 : 1][4][64];
+	static_assert(sizeof(double) * (NW - 1) * 4 * 64 <= sizeof(stages), "exchange in the stages");
+	double (*red)[4][64] = reinterpret_cast<double (*)[4][64]>(stages);
 	int4* tile = tiles[wave];
 	double dphi = 0.0, dg[3] = {0.0, 0.0, 0.0};
 	for (int base = share.x; base < share.y; base += 64) {
@@ -466,13 +477,25 @@ __global__ __launch_bounds__(64 * NW) void k_pp_ewald(LeafArgs A) {
 		if (lane < n) tile[lane] = A.srcs[A.list ? A.list[base + lane] : base + lane];
 		wave_lds_sync<NW>();
 		float phi = 0.f, g[3] = {0.f, 0.f, 0.f};
-		for (int k = ph; k < n; k += P) {
-			const int4 s = tile[k];
-			const float x[3] = {sepu<true>(me.x, s.x) * POS_INVF, sepu<true>(me.y, s.y) * POS_INVF,
-					sepu<true>(me.z, s.z) * POS_INVF};
-			float D[4];
-			green_ewald_tab<4>(D, x, c_ewt);
-			const float w = __int_as_float(s.w);
+		// the next turn's rows are on their way while this turn's are evaluated
+		auto at = [&](int k0) {
+			const int4 s = tile[min(k0 + ph, n - 1)];
+			const float x[3] = {sepu<true>(me.x, s.x) * POS_INVF, sepu<true>(me.y, s.y) * POS_INVF, sepu<true>(me.z, s.z) * POS_INVF};
+			return ewt_point(x);
+		};
+		EwtPoint p = at(0);
+		EwtRows<4> rows;
+		rows.fetch(p.row, c_ewt, stages[wave], lane);
+		for (int k0 = 0; k0 < n; k0 += P) {
+			float c[EwtRead<4>::F4 * 4], D[4];
+			rows.take(c, stages[wave], lane);
+			const EwtPoint now = p;
+			const float w = k0 + ph < n ? __int_as_float(tile[min(k0 + ph, n - 1)].w) : 0.0f;
+			if (k0 + P < n) {
+				p = at(k0 + P);
+				rows.fetch(p.row, c_ewt, stages[wave], lane);
+			}
+			ewt_eval<4>(D, c, now);
 			phi = fmaf(w, D[0], phi);
 			g[0] = fmaf(-w, D[1], g[0]);
 			g[1] = fmaf(-w, D[2], g[1]);
@@ -483,6 +506,7 @@ __global__ __launch_bounds__(64 * NW) void k_pp_ewald(LeafArgs A) {
 		dg[1] += g[1];
 		dg[2] += g[2];
 	}
+	if (NW > 1) __syncthreads();
 	leaf_sums<NW>(dphi, dg, nsp, lane, wave, red);
 	if (wave == 0 && ph == 0 && si < ns) {
 		double* o = A.out + 4 * (size_t) (it.x + si);
@@ -493,9 +517,16 @@ __global__ __launch_bounds__(64 * NW) void k_pp_ewald(LeafArgs A) {
 	}
 }
 
+// waves of an item: 64 sources or more to each on average
+static int ewald_waves(int nitems, int64_t sources) {
+	int w = 1;
+	while (w < 16 && int64_t(nitems) * (2 * w) <= TARGET_WAVES && sources >= int64_t(nitems) * 64 * (2 * w)) w *= 2;
+	return w;
+}
+
 hipError_t launch_pp_ewald(const LeafArgs& a, hipStream_t s) {
 	if (a.nitems <= 0) return hipSuccess;
-	switch (leaf_waves(a.nitems, a.nlist, 16)) {
+	switch (ewald_waves(a.nitems, a.nlist)) {
 		case 1: hipLaunchKernelGGL(k_pp_ewald<1>, dim3(a.nitems), dim3(64), 0, s, a); break;
 		case 2: hipLaunchKernelGGL(k_pp_ewald<2>, dim3(a.nitems), dim3(128), 0, s, a); break;
 		case 4: hipLaunchKernelGGL(k_pp_ewald<4>, dim3(a.nitems), dim3(256), 0, s, a); break;
@@ -508,11 +539,20 @@ hipError_t launch_pp_ewald(const LeafArgs& a, hipStream_t s) {
 // ---- node kinds ----------------------------------------------------------------------------------
 // Segmented FP64 reduction of the lanes' 35 float accumulators by owner slot, through LDS.  The
 // entries of one slot are consecutive, so lanes 0..34 (one coefficient each) scan the wave once.
-__device__ __forceinline__ void node_segment_store(const float* L, int slot, int cnt, const int* slot_node_unused,
-		double* partial) {
-	__shared__ float red[35][65];
-	__shared__ int sl[64];
+struct NodeSums {
+	float red[35][65];
+	int sl[64];
+};
+union NodeLds {  // the Ewald kinds' rows, then the sums
+	EwtStage rows;
+	NodeSums sums;
+};
+
+__device__ __forceinline__ void node_segment_store(const float* L, int slot, int cnt, NodeSums& S, double* partial) {
+	float (*red)[65] = S.red;
+	int* sl = S.sl;
 	const int lane = threadIdx.x;
+	__syncthreads();
 #pragma unroll
 	for (int c = 0; c < 35; c++) red[c][lane] = L[c];
 	sl[lane] = slot;
@@ -540,11 +580,22 @@ __device__ __forceinline__ void node_segment_store(const float* L, int slot, int
 	}
 }
 
+__device__ __forceinline__ void multi_floats(float* v, const float4* m) {
+#pragma unroll
+	for (int q = 0; q < 5; q++) {
+		v[4 * q] = m[q].x;
+		v[4 * q + 1] = m[q].y;
+		v[4 * q + 2] = m[q].z;
+		v[4 * q + 3] = m[q].w;
+	}
+}
+
 // A wave takes a run of list entries: up to 64 entries of one or more partial slots (one entry per
 // lane), or the entries of one slot beyond 64 (a chunk longer than a wave), which the lanes take
 // 64 apart, each adding its entries' terms in order before the store.
-template <bool EWALD, bool WRAP>
+template <bool WRAP>
 __global__ __launch_bounds__(64) void k_cc(NodeArgs A) {
+	__shared__ NodeSums sums;
 	const int2 wv = A.waves[blockIdx.x];
 	const int lane = threadIdx.x;
 	float L[35];
@@ -555,11 +606,9 @@ __global__ __launch_bounds__(64) void k_cc(NodeArgs A) {
 	if (j < wv.y) {
 		slot = A.owner ? A.owner[j] : int(blockIdx.x);  // the plain drop-in: one slot per wave, one sink
 		const int4 X = A.sinkpos[A.slot_node ? A.slot_node[slot] : 0];
-		// software pipeline (direct kinds): the next entry's multipole and the list index after it
-		// are loaded while the current entry is evaluated, into the other of two buffers (the loop
-		// is unrolled twice, so no copy between them).  The Ewald kinds load in order: their table
-		// row already holds most registers, and the 20 more cost a wave per SIMD (measured: no
-		// gain)
+		// software pipeline: the next entry's multipole and the list index after it are loaded while
+		// the current entry is evaluated, into the other of two buffers (the loop is unrolled twice,
+		// so no copy between them)
 		auto index_at = [&](int jj) { return jj < wv.y ? (A.list ? A.list[jj] : jj) : -1; };
 		auto load_multi = [&](int idx, float4* m) {
 			if (idx >= 0) {
@@ -570,54 +619,74 @@ __global__ __launch_bounds__(64) void k_cc(NodeArgs A) {
 		};
 		auto entry = [&](const float4* m) {
 			float v[20];
-#pragma unroll
-			for (int q = 0; q < 5; q++) {
-				v[4 * q] = m[q].x;
-				v[4 * q + 1] = m[q].y;
-				v[4 * q + 2] = m[q].z;
-				v[4 * q + 3] = m[q].w;
-			}
-			const float x[3] = {sepu<EWALD || WRAP>(X.x, __float_as_int(v[17])) * POS_INVF,
-					sepu<EWALD || WRAP>(X.y, __float_as_int(v[18])) * POS_INVF,
-					sepu<EWALD || WRAP>(X.z, __float_as_int(v[19])) * POS_INVF};
+			multi_floats(v, m);
+			const float x[3] = {sepu<WRAP>(X.x, __float_as_int(v[17])) * POS_INVF, sepu<WRAP>(X.y, __float_as_int(v[18])) * POS_INVF,
+					sepu<WRAP>(X.z, __float_as_int(v[19])) * POS_INVF};
 			float D[35];
-			if (EWALD)
-				green_ewald(D, x);
-			else
-				green_direct(D, x);
-			m2l<!EWALD>(L, v, D);
+			green_direct(D, x);
+			m2l<false>(L, v, D, 0.0f);
 		};
-		float4 ma[5];
-		if (EWALD) {
-			for (; j < wv.y; j += 64) {
-				const float4* src = reinterpret_cast<const float4*>(A.multis + (A.list ? A.list[j] : j));
-#pragma unroll
-				for (int q = 0; q < 5; q++) ma[q] = src[q];
-				entry(ma);
-			}
-		} else {
-			float4 mb[5];
-			load_multi(index_at(j), ma);
-			int next_idx = index_at(j + 64);
-			for (;;) {
-				load_multi(next_idx, mb);
-				next_idx = index_at(j + 128);
-				entry(ma);
-				j += 64;
-				if (j >= wv.y) break;
-				load_multi(next_idx, ma);
-				next_idx = index_at(j + 128);
-				entry(mb);
-				j += 64;
-				if (j >= wv.y) break;
-			}
+		float4 ma[5], mb[5];
+		load_multi(index_at(j), ma);
+		int next_idx = index_at(j + 64);
+		for (;;) {
+			load_multi(next_idx, mb);
+			next_idx = index_at(j + 128);
+			entry(ma);
+			j += 64;
+			if (j >= wv.y) break;
+			load_multi(next_idx, ma);
+			next_idx = index_at(j + 128);
+			entry(mb);
+			j += 64;
+			if (j >= wv.y) break;
 		}
 	}
-	node_segment_store(L, slot, min(wv.y - wv.x, 64), A.slot_node, A.partial);
+	node_segment_store(L, slot, min(wv.y - wv.x, 64), sums, A.partial);
 }
 
-template <bool EWALD, bool WRAP>
+// The Ewald correction of the same: the whole wave takes every turn (its table rows are read
+// together), lanes past the end with the last entry and no weight.  Bound by arithmetic (about 700
+// instructions an entry, 900 before) and by the rows' way through the vector cache and LDS, 16 KB a
+// turn, at three waves a SIMD (two waves with the next turn's rows in flight took 1.16 ms where this
+// takes 1.03: 2M particles at theta 0.3, 3.6e7 entries).
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_cc_ewald(NodeArgs A) {
+	__shared__ NodeLds lds;
+	const int2 wv = A.waves[blockIdx.x];
+	const int lane = threadIdx.x;
+	float L[35];
+#pragma unroll
+	for (int c = 0; c < 35; c++) L[c] = 0.f;
+	int slot = -1;
+	int4 X = make_int4(0, 0, 0, 0);
+	if (wv.x + lane < wv.y) {
+		slot = A.owner ? A.owner[wv.x + lane] : int(blockIdx.x);
+		X = A.sinkpos[A.slot_node ? A.slot_node[slot] : 0];
+	}
+	for (int j0 = wv.x; j0 < wv.y; j0 += 64) {
+		const int j = min(j0 + lane, wv.y - 1);
+		const float4* src = reinterpret_cast<const float4*>(A.multis + (A.list ? A.list[j] : j));
+		float4 m[5];
+#pragma unroll
+		for (int q = 0; q < 5; q++) m[q] = src[q];
+		float v[20];
+		multi_floats(v, m);
+		const float x[3] = {sepu<true>(X.x, __float_as_int(v[17])) * POS_INVF, sepu<true>(X.y, __float_as_int(v[18])) * POS_INVF,
+				sepu<true>(X.z, __float_as_int(v[19])) * POS_INVF};
+		float D[35];
+		const float lap = green_ewald_wave<35>(D, x, c_ewt, lds.rows, lane);
+		if (j0 + 64 > wv.y && j0 + lane >= wv.y) {
+#pragma unroll
+			for (int c = 0; c < 17; c++) v[c] = 0.0f;
+		}
+		m2l<true>(L, v, D, lap);
+	}
+	node_segment_store(L, slot, min(wv.y - wv.x, 64), lds.sums, A.partial);
+}
+
+template <bool WRAP>
 __global__ __launch_bounds__(64) void k_cp(NodeArgs A) {
+	__shared__ NodeSums sums;
 	const int2 wv = A.waves[blockIdx.x];
 	const int lane = threadIdx.x;
 	float L[35];
@@ -630,38 +699,58 @@ __global__ __launch_bounds__(64) void k_cp(NodeArgs A) {
 		const int4 X = A.sinkpos[A.slot_node ? A.slot_node[slot] : 0];
 		for (; j < wv.y; j += 64) {
 			const int4 s = A.srcs[A.list ? A.list[j] : j];
-			const float x[3] = {sepu<EWALD || WRAP>(X.x, s.x) * POS_INVF, sepu<EWALD || WRAP>(X.y, s.y) * POS_INVF,
-					sepu<EWALD || WRAP>(X.z, s.z) * POS_INVF};
+			const float x[3] = {sepu<WRAP>(X.x, s.x) * POS_INVF, sepu<WRAP>(X.y, s.y) * POS_INVF, sepu<WRAP>(X.z, s.z) * POS_INVF};
 			float D[35];
-			if (EWALD)
-				green_ewald(D, x);
-			else
-				green_direct(D, x);
+			green_direct(D, x);
 			p2l(L, __int_as_float(s.w), D);
 		}
 	}
-	node_segment_store(L, slot, min(wv.y - wv.x, 64), A.slot_node, A.partial);
+	node_segment_store(L, slot, min(wv.y - wv.x, 64), sums, A.partial);
+}
+
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_cp_ewald(NodeArgs A) {
+	__shared__ NodeLds lds;
+	const int2 wv = A.waves[blockIdx.x];
+	const int lane = threadIdx.x;
+	float L[35];
+#pragma unroll
+	for (int c = 0; c < 35; c++) L[c] = 0.f;
+	int slot = -1;
+	int4 X = make_int4(0, 0, 0, 0);
+	if (wv.x + lane < wv.y) {
+		slot = A.owner ? A.owner[wv.x + lane] : int(blockIdx.x);
+		X = A.sinkpos[A.slot_node ? A.slot_node[slot] : 0];
+	}
+	for (int j0 = wv.x; j0 < wv.y; j0 += 64) {
+		const int j = min(j0 + lane, wv.y - 1);
+		const int4 s = A.srcs[A.list ? A.list[j] : j];
+		const float x[3] = {sepu<true>(X.x, s.x) * POS_INVF, sepu<true>(X.y, s.y) * POS_INVF, sepu<true>(X.z, s.z) * POS_INVF};
+		float D[35];
+		green_ewald_wave<35>(D, x, c_ewt, lds.rows, lane);
+		p2l(L, j0 + lane < wv.y ? __int_as_float(s.w) : 0.0f, D);
+	}
+	node_segment_store(L, slot, min(wv.y - wv.x, 64), lds.sums, A.partial);
 }
 
 hipError_t launch_cc(const NodeArgs& a, bool ewald, hipStream_t s) {
 	if (a.nwaves <= 0) return hipSuccess;
 	if (ewald)
-		hipLaunchKernelGGL((k_cc<true, true>), dim3(a.nwaves), dim3(64), 0, s, a);
+		hipLaunchKernelGGL(k_cc_ewald, dim3(a.nwaves), dim3(64), 0, s, a);
 	else if (a.wrap)
-		hipLaunchKernelGGL((k_cc<false, true>), dim3(a.nwaves), dim3(64), 0, s, a);
+		hipLaunchKernelGGL(k_cc<true>, dim3(a.nwaves), dim3(64), 0, s, a);
 	else
-		hipLaunchKernelGGL((k_cc<false, false>), dim3(a.nwaves), dim3(64), 0, s, a);
+		hipLaunchKernelGGL(k_cc<false>, dim3(a.nwaves), dim3(64), 0, s, a);
 	return hipGetLastError();
 }
 
 hipError_t launch_cp(const NodeArgs& a, bool ewald, hipStream_t s) {
 	if (a.nwaves <= 0) return hipSuccess;
 	if (ewald)
-		hipLaunchKernelGGL((k_cp<true, true>), dim3(a.nwaves), dim3(64), 0, s, a);
+		hipLaunchKernelGGL(k_cp_ewald, dim3(a.nwaves), dim3(64), 0, s, a);
 	else if (a.wrap)
-		hipLaunchKernelGGL((k_cp<false, true>), dim3(a.nwaves), dim3(64), 0, s, a);
+		hipLaunchKernelGGL(k_cp<true>, dim3(a.nwaves), dim3(64), 0, s, a);
 	else
-		hipLaunchKernelGGL((k_cp<false, false>), dim3(a.nwaves), dim3(64), 0, s, a);
+		hipLaunchKernelGGL(k_cp<false>, dim3(a.nwaves), dim3(64), 0, s, a);
 	return hipGetLastError();
 }
 

@@ -23,29 +23,29 @@ __device__ __forceinline__ void wave_lds_sync() {
 	}
 }
 
-// Leaf kinds: NW waves share an item, each taking a contiguous run of its 64-source tiles; their
-// sums are added in wave order.  [begin, end) of wave w's sources in the list [b, e).
-template <int NW>
+// Leaf kinds: NW waves share an item, each taking a contiguous run of its tiles of TILE sources;
+// their sums are added in wave order.  [begin, end) of wave w's sources in the list [b, e).
+template <int NW, int TILE = 64>
 __device__ __forceinline__ int2 wave_share(int b, int e, int w) {
 	if (NW == 1) return make_int2(b, e);
-	const int tiles = (e - b + 63) >> 6;
+	const int tiles = (e - b + TILE - 1) / TILE;
 	const int per = (tiles + NW - 1) / NW;
-	const int lo = min(int64_t(e), int64_t(b) + int64_t(64) * per * w);
-	const int hi = min(int64_t(e), int64_t(lo) + int64_t(64) * per);
+	const int lo = min(int64_t(e), int64_t(b) + int64_t(TILE) * per * w);
+	const int hi = min(int64_t(e), int64_t(lo) + int64_t(TILE) * per);
 	return make_int2(lo, hi);
 }
 
 // Waves per leaf item.  One wave's chain of tiles is serial, so few items with long lists leave the
 // chip idle, and on clustered sets the longest lists set the kernel's time.  The waves are raised
-// up to TARGET in all (four rounds of the chip: 256 CUs, 4 SIMDs each, eight waves a SIMD, for the
+// up to a target in all (four rounds of the chip: 256 CUs, 4 SIMDs each, eight waves a SIMD, for the
 // uneven lists to even out), as long as each keeps two tiles or more on average.  Sets of more than
-// TARGET / 2 items (2M particles: 65,000 and more) keep one wave each, whose sums need no second
+// half the target's items (2M particles: 65,000 and more) keep one wave each, whose sums need no second
 // pass.
+constexpr int64_t TARGET_WAVES = 32768;
 inline int leaf_waves(int nitems, int64_t sources, int most) {
-	constexpr int64_t TARGET = 32768;
 	const int64_t tiles = (sources / (nitems > 0 ? nitems : 1) + 63) / 64;
 	int w = 1;
-	while (w < most && int64_t(nitems) * (2 * w) <= TARGET && tiles >= 4 * w) w *= 2;
+	while (w < most && int64_t(nitems) * (2 * w) <= TARGET_WAVES && tiles >= 4 * w) w *= 2;
 	return w;
 }
 

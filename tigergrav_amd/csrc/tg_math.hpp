@@ -190,43 +190,42 @@ __device__ __forceinline__ void green_direct(float* D, const float* x) {
 // ---- contractions (src/gravity.cpp:26-169) ----------------------------------------------------
 // M2L: L += contraction of the multipole M with D (reference gravity.cpp:26-90)
 // Every term is added straight into L, in the reference's order of terms (as its loop adds each
-// term into its L).  HARM: D is traceless in any two of its indices (derivatives of 1/r away from
-// the origin), so D_{k,zz} = -D_{k,xx} - D_{k,yy} and a multipole's zz-holding components fold
-// into the others: the quadrupole contracts in 5 terms and the octupole in 7 (each L component
-// whose terms reach D through them: L0, L_a, L_ab), with the 8 folded weights formed once per
-// entry.
-template <bool HARM>
-__device__ __forceinline__ void m2l(float* L, const float* M, const float* D) {
+// term into its L).  D's trace in two of its indices is lap where it is D itself and 0 above
+// (derivatives of 1/r away from the origin: lap = 0; the periodic correction: its constant
+// Laplacian), so D_{k,zz} = -D_{k,xx} - D_{k,yy}, plus lap for D_zz, and a multipole's zz-holding
+// components fold into the others (LAP: with lap's term): the quadrupole contracts in 5 terms and the octupole in 7 (each L
+// component whose terms reach D through them: L0, L_a, L_ab), with the 8 folded weights formed once
+// per entry.
+template <bool LAP>
+__device__ __forceinline__ void m2l(float* L, const float* M, const float* D, float lap) {
 	float q[6], o[10];
 #pragma unroll
 	for (int s = 0; s < 6; s++) q[s] = M[1 + s] * ef2(s);
 #pragma unroll
 	for (int s = 0; s < 10; s++) o[s] = -M[7 + s] * ef3(s);
-	if (HARM) {
-		// quadrupole slots xx 0, xy 1, xz 2, yy 3, yz 4, zz 5; octupole xxx 0, xxy 1, xxz 2, xyy 3,
-		// xyz 4, xzz 5, yyy 6, yyz 7, yzz 8, zzz 9
-		q[0] -= q[5];
-		q[3] -= q[5];
-		o[0] -= o[5];
-		o[3] -= o[5];
-		o[1] -= o[8];
-		o[6] -= o[8];
-		o[2] -= o[9];
-		o[7] -= o[9];
-	}
+	// quadrupole slots xx 0, xy 1, xz 2, yy 3, yz 4, zz 5; octupole xxx 0, xxy 1, xxz 2, xyy 3,
+	// xyz 4, xzz 5, yyy 6, yyz 7, yzz 8, zzz 9
+	q[0] -= q[5];
+	q[3] -= q[5];
+	o[0] -= o[5];
+	o[3] -= o[5];
+	o[1] -= o[8];
+	o[6] -= o[8];
+	o[2] -= o[9];
+	o[7] -= o[9];
 	auto quad = [&](auto slot_of, float acc) {
 #pragma unroll
-		for (int s = 0; s < 6; s++)
-			if (!HARM || s != 5) acc = fmaf(q[s], D[slot_of(s)], acc);
+		for (int s = 0; s < 5; s++) acc = fmaf(q[s], D[slot_of(s)], acc);
 		return acc;
 	};
 	auto oct = [&](auto slot_of, float acc) {
 #pragma unroll
 		for (int s = 0; s < 10; s++)
-			if (!HARM || (s != 5 && s != 8 && s != 9)) acc = fmaf(o[s], D[slot_of(s)], acc);
+			if (s != 5 && s != 8 && s != 9) acc = fmaf(o[s], D[slot_of(s)], acc);
 		return acc;
 	};
 	float l0 = fmaf(M[0], D[0], L[0]);
+	if (LAP) l0 = fmaf(q[5], lap, l0);
 	l0 = quad([](int s) { return 4 + s; }, l0);
 	l0 = oct([](int s) { return 10 + s; }, l0);
 	L[0] = l0;
@@ -282,26 +281,15 @@ __device__ __forceinline__ void m2p(float& phi, float* g, const float* M, const 
 // in tg_kernels.hip; another translation unit keeps its own copy of the pointer).
 extern __constant__ const float* c_ewt;
 
-// slots read for the first nout outputs: every slot up to three orders above the highest output
-// order, rounded up to whole float4 loads
-constexpr int ewt_nload(int nout) {
-	const int o = nout <= 1 ? 0 : nout <= 4 ? 1 : nout <= 10 ? 2 : nout <= 20 ? 3 : 4;
-	const int s = (o + 4) * (o + 5) * (o + 6) / 6;
-	return (s + 3) / 4 * 4;
-}
-
-template <int V>
-constexpr int ewt_cx = V;  // forces a constant slot index to be folded at compile time
-
 template <int... S, class F>
-__device__ __forceinline__ void ewt_for_seq(std::integer_sequence<int, S...>, F&& f) {
+__host__ __device__ __forceinline__ void ewt_for_seq(std::integer_sequence<int, S...>, F&& f) {
 	(f(std::integral_constant<int, S>{}), ...);
 }
 
 // exchanges components k and swap_ab(k, a, b) of D[0..NOUT) where cond holds: the tensor with
 // coordinates a and b exchanged
 template <int NOUT, int A, int B>
-__device__ __forceinline__ void ewt_transpose_if(float* D, bool cond) {
+__host__ __device__ __forceinline__ void ewt_transpose_if(float* D, bool cond) {
 	ewt_for_seq(std::make_integer_sequence<int, NOUT>{}, [&](auto k_) {
 		constexpr int k = decltype(k_)::value;
 		constexpr int p = ewt::swap_ab(k, A, B);
@@ -313,29 +301,25 @@ __device__ __forceinline__ void ewt_transpose_if(float* D, bool cond) {
 	});
 }
 
-// The first NOUT components (all of orders 0..1, 0..2, 0..4 or 0..5: NOUT = 4, 10, 35, 56) of
-// the periodic-correction tensor (tigergrav/green.hpp:189-286) at a wrapped separation x
-// (|x_i| <= 1/2).  |x| is sorted into the wedge u0 >= u1 >= u2 by three compare-exchanges; the
-// components there come from a third-order Taylor expansion about the nearest grid point of
-// `table` (FP64 values of the correction, rounded to float, on a 1/64 grid of the wedge); the
-// exchanges are then undone on the components in reverse order, and the sign of each component is
-// flipped by the coordinates that are negative and occur an odd number of times.  Interpolation
-// error below 5e-6 of each order's largest value (1.7e-6 RMS over orders 0..4, 1.1e-7 at order 1).
-// Order-5 components (the adjoint's) take a second-order expansion, the table ending at order 7:
-// error about 1e-4 of that order's largest value.  At |x| <= 1e-6 the reference's convention
+// where a separation x (|x_i| <= 1/2) lies in the table: the row of the nearest grid point of the
+// wedge u0 >= u1 >= u2 that three compare-exchanges sort |x| into, the offset from it, the exchanges
+// made, the signs, and the Laplacian there.  At |x| <= 1e-6 the reference's convention
 // D = (2.8372975, 0, ..., 0) applies (tigergrav/green.hpp:272): the table's last row, read with a
 // zero offset.
-template <int NOUT>
-__device__ __forceinline__ void green_ewald_tab(float* D, const float* x, const float* table) {
-	constexpr int NLOAD = NOUT == 56 ? TG_EWT_S : ewt_nload(NOUT);
-	static_assert(NOUT == 56 || NOUT == 35 || NOUT == 10 || NOUT == 4, "orders 0..5, 0..4, 0..2 or 0..1");
-	static_assert(NLOAD <= TG_EWT_S, "slots read");
+struct EwtPoint {
+	int row;
+	float d[3], sg[3], lap;
+	bool s1, s2, s3;
+};
+
+__host__ __device__ __forceinline__ EwtPoint ewt_point(const float* x) {
+	EwtPoint p;
 	const float r2 = fmaf(x[2], x[2], fmaf(x[1], x[1], x[0] * x[0]));
-	float u[3], sg[3];
+	float u[3];
 #pragma unroll
 	for (int a = 0; a < 3; a++) {
 		u[a] = fabsf(x[a]);
-		sg[a] = x[a] < 0.0f ? -1.0f : 1.0f;
+		p.sg[a] = x[a] < 0.0f ? -1.0f : 1.0f;
 	}
 	// sort |x| descending: exchange (0,1), (1,2), (0,1) where the later coordinate is larger
 	auto cx = [](float& p, float& q, bool c) {
@@ -343,97 +327,122 @@ __device__ __forceinline__ void green_ewald_tab(float* D, const float* x, const 
 		p = c ? b : a;
 		q = c ? a : b;
 	};
-	const bool s1 = u[1] > u[0];
-	cx(u[0], u[1], s1);
-	const bool s2 = u[2] > u[1];
-	cx(u[1], u[2], s2);
-	const bool s3 = u[1] > u[0];
-	cx(u[0], u[1], s3);
-	// a coincident pair reads the table's last row, (2.8372975, 0, ..., 0), with a zero offset
+	p.s1 = u[1] > u[0];
+	cx(u[0], u[1], p.s1);
+	p.s2 = u[2] > u[1];
+	cx(u[1], u[2], p.s2);
+	p.s3 = u[1] > u[0];
+	cx(u[0], u[1], p.s3);
 	const bool z = !(r2 > 1e-12f);
-	float d[3];
 	int gi[3];
 #pragma unroll
 	for (int a = 0; a < 3; a++) {
-		gi[a] = min(int(fmaf(u[a], float(TG_EWT_INV), 0.5f)), TG_EWT_N - 1);
-		d[a] = z ? 0.0f : u[a] - float(gi[a]) * (1.0f / TG_EWT_INV);
+		const int g = int(fmaf(u[a], float(TG_EWT_INV), 0.5f));
+		gi[a] = g < TG_EWT_N - 1 ? g : TG_EWT_N - 1;
+		p.d[a] = z ? 0.0f : u[a] - float(gi[a]) * (1.0f / TG_EWT_INV);
 	}
-	const int row = z ? TG_EWT_P : ewt::wedge_index(gi[0], gi[1], gi[2]);
-	const float4* tp = reinterpret_cast<const float4*>(table + size_t(row) * TG_EWT_STRIDE);
-	// the row holds the slots with the third axis at most once; the others follow from the trace
-	// relation (a constant Laplacian, -4 pi; 0 for the coincident row), each from two slots before it
-	constexpr int MAXO = ewt::ST.c[NLOAD - 1].n0 + ewt::ST.c[NLOAD - 1].n1 + ewt::ST.c[NLOAD - 1].n2;  // highest order read
-	constexpr int NSTORED = ewt::stored_count(MAXO);
-	float c[(NSTORED + 3) / 4 * 4];
-#pragma unroll
-	for (int q = 0; q < (NSTORED + 3) / 4; q++) {
-		const float4 v = tp[q];
-		c[4 * q] = v.x;
-		c[4 * q + 1] = v.y;
-		c[4 * q + 2] = v.z;
-		c[4 * q + 3] = v.w;
-	}
-	const float lap = z ? 0.0f : -12.566370614359172f;
+	p.row = z ? TG_EWT_P : ewt::wedge_index(gi[0], gi[1], gi[2]);
+	p.lap = z ? 0.0f : -12.566370614359172f;
+	return p;
+}
+
+// what NOUT outputs read: every slot up to three orders above the highest output order, and the row's
+// float4 that hold those stored
+template <int NOUT>
+struct EwtRead {
+	static_assert(NOUT == 56 || NOUT == 35 || NOUT == 10 || NOUT == 4, "orders 0..5, 0..4, 0..2 or 0..1");
+	static constexpr int OUT = NOUT == 4 ? 1 : NOUT == 10 ? 2 : NOUT == 35 ? 4 : 5;
+	static constexpr int ORDER = OUT + 3 < TG_EWT_ORDER ? OUT + 3 : TG_EWT_ORDER;
+	static constexpr int LOAD = (ORDER + 1) * (ORDER + 2) * (ORDER + 3) / 6;
+	static_assert(LOAD <= TG_EWT_S, "slots read");
+	static constexpr int F4 = (ewt::stored_count(ORDER) + 3) / 4;
+};
+
+// Replaces every slot k of t with order < limit and n2 <= 1 by its Taylor sum along axis A about an
+// offset d, of up to third order and as far as the orders read go.  In ascending order: a slot's
+// terms are of higher orders, not yet replaced.
+template <int A, int LIMIT, int ORDER>
+__host__ __device__ __forceinline__ void ewt_shift(float* t, float d) {
+	const float d2 = d * 0.5f, d3 = d * (1.0f / 3.0f);
+	constexpr int N = LIMIT * (LIMIT + 1) * (LIMIT + 2) / 6;
+	ewt_for_seq(std::make_integer_sequence<int, N>{}, [&](auto k_) {
+		constexpr int k = decltype(k_)::value;
+		constexpr int n0 = ewt::ST.c[k].n0, n1 = ewt::ST.c[k].n1, n2 = ewt::ST.c[k].n2, n = n0 + n1 + n2;
+		if constexpr (n2 <= 1 && n < ORDER) {
+			constexpr int k1 = ewt::slot_of(n0 + (A == 0), n1 + (A == 1), n2 + (A == 2));
+			float v = t[k1];
+			if constexpr (n + 2 <= ORDER) {
+				constexpr int k2 = ewt::slot_of(n0 + 2 * (A == 0), n1 + 2 * (A == 1), n2 + 2 * (A == 2));
+				float w = t[k2];
+				if constexpr (n + 3 <= ORDER) {
+					constexpr int k3 = ewt::slot_of(n0 + 3 * (A == 0), n1 + 3 * (A == 1), n2 + 3 * (A == 2));
+					w = fmaf(t[k3], d3, w);
+				}
+				v = fmaf(w, d2, v);
+			}
+			t[k] = fmaf(v, d, t[k]);
+		}
+	});
+}
+
+// The first NOUT components (all of orders 0..1, 0..2, 0..4 or 0..5: NOUT = 4, 10, 35, 56) of
+// the periodic-correction tensor (tigergrav/green.hpp:189-286) at a point of the table, from its
+// row c: in the wedge by third-order Taylor sums about the grid point (FP64 values of the correction,
+// rounded to float, on a 1/64 grid); the exchanges are then undone on the components in reverse
+// order, and the sign of each component is flipped by the coordinates that are negative and occur an
+// odd number of times.  Interpolation error below 5e-6 of each order's largest value (1.7e-6 RMS over
+// orders 0..4, 1.1e-7 at order 1).  Order-5 components (the adjoint's) take a second-order expansion,
+// the table ending at order 7: error about 1e-4 of that order's largest value.
+//
+// The sums are taken one axis at a time, each slot of the orders read moved along z, then y, then x
+// (a few mixed terms beyond third order come with it): about 290 fused multiply-adds for orders 0..4
+// where a 19-term sum per component took 475 and the monomials 30 more.  The correction has a
+// constant Laplacian in the cell (-4 pi: the periodic potential's uniform background), so every
+// component holding the wedge's third axis twice or more is C - D[k - 2z + 2x] - D[k - 2z + 2y],
+// C = -4 pi for D_zz and 0 otherwise: the row leaves those slots out, only the move along z reads
+// them, and the components follow at the end.
+template <int NOUT>
+__host__ __device__ __forceinline__ void ewt_eval(float* D, const float* c, const EwtPoint& p) {
+	using R = EwtRead<NOUT>;
+	constexpr int NLOAD = R::LOAD;
 	float t[NLOAD];
+	auto traced = [&](auto k_, const float* v) {
+		constexpr int k = decltype(k_)::value;
+		constexpr int n0 = ewt::ST.c[k].n0, n1 = ewt::ST.c[k].n1, n2 = ewt::ST.c[k].n2;
+		constexpr int ka = ewt::slot_of(n0 + 2, n1, n2 - 2), kb = ewt::slot_of(n0, n1 + 2, n2 - 2);
+		static_assert(ka >= 0 && ka < k && kb >= 0 && kb < k, "trace terms come first");
+		if constexpr (n0 == 0 && n1 == 0 && n2 == 2)
+			return p.lap - v[ka] - v[kb];
+		else
+			return -v[ka] - v[kb];
+	};
 	ewt_for_seq(std::make_integer_sequence<int, NLOAD>{}, [&](auto k_) {
 		constexpr int k = decltype(k_)::value;
-		constexpr int n0 = ewt::ST.c[k].n0, n1 = ewt::ST.c[k].n1, n2 = ewt::ST.c[k].n2;
-		if constexpr (n2 <= 1) {
+		if constexpr (ewt::ST.c[k].n2 <= 1) {
 			constexpr int si = ewt::stored_index(k);
-			static_assert(si >= 0 && si < (NSTORED + 3) / 4 * 4, "stored slot read");
+			static_assert(si >= 0 && si < R::F4 * 4, "stored slot read");
 			t[k] = c[si];
 		} else {
-			constexpr int ka = ewt::slot_of(n0 + 2, n1, n2 - 2), kb = ewt::slot_of(n0, n1 + 2, n2 - 2);
-			static_assert(ka >= 0 && ka < k && kb >= 0 && kb < k, "trace terms come first");
-			t[k] = ((n0 == 0 && n1 == 0 && n2 == 2) ? lap : 0.0f) - t[ka] - t[kb];
+			t[k] = traced(k_, t);
 		}
 	});
-	// the Taylor monomials d^j / j! of orders 1..3 (slots 1..19)
-	float w[20];
-	w[0] = 1.0f;
-	ewt_for_seq(std::make_integer_sequence<int, 19>{}, [&](auto j_) {
-		constexpr int j = decltype(j_)::value + 1;
-		constexpr int n0 = ewt::ST.c[j].n0, n1 = ewt::ST.c[j].n1, n2 = ewt::ST.c[j].n2;
-		float m = ewt::taylor_coef(j);
-#pragma unroll
-		for (int e = 0; e < n0; e++) m *= d[0];
-#pragma unroll
-		for (int e = 0; e < n1; e++) m *= d[1];
-#pragma unroll
-		for (int e = 0; e < n2; e++) m *= d[2];
-		w[j] = m;
-	});
-	// The correction has a constant Laplacian in the cell (-4 pi: the periodic potential's uniform
-	// background), so every derivative tensor's trace is fixed by lower slots: a component holding
-	// the wedge's third axis twice or more is C - D[k - 2z + 2x] - D[k - 2z + 2y], C = -4 pi for
-	// D_zz and 0 otherwise.  Those components (10 of the 35 to order 4) come from that relation,
-	// in slot order (their two terms come earlier), the others from the Taylor step.
+	ewt_shift<2, R::ORDER, R::ORDER>(t, p.d[2]);
+	ewt_shift<1, R::ORDER, R::ORDER>(t, p.d[1]);
+	ewt_shift<0, R::OUT + 1, R::ORDER>(t, p.d[0]);
 	ewt_for_seq(std::make_integer_sequence<int, NOUT>{}, [&](auto k_) {
 		constexpr int k = decltype(k_)::value;
-		constexpr int n0 = ewt::ST.c[k].n0, n1 = ewt::ST.c[k].n1, n2 = ewt::ST.c[k].n2;
-		if constexpr (n2 >= 2) {
-			constexpr int ka = ewt::slot_of(n0 + 2, n1, n2 - 2), kb = ewt::slot_of(n0, n1 + 2, n2 - 2);
-			static_assert(ka >= 0 && ka < k && kb >= 0 && kb < k, "trace terms come first");
-			const float c = (n0 == 0 && n1 == 0 && n2 == 2) ? lap : 0.0f;
-			D[k] = c - D[ka] - D[kb];
-		} else {
-			// monomials of orders 1..3 (slots 1..19), or 1..2 (slots 1..9) where order 8 would be needed
-			constexpr int jn = n0 + n1 + n2 + 3 <= TG_EWT_ORDER ? 19 : 9;
-			float v = t[k];
-			ewt_for_seq(std::make_integer_sequence<int, jn>{}, [&](auto j_) {
-				constexpr int j = decltype(j_)::value + 1;
-				static_assert(ewt::merge(k, j) >= 0 && ewt::merge(k, j) < NLOAD, "slot read");
-				v = fmaf(t[ewt_cx<ewt::merge(k, j)>], w[j], v);
-			});
-			D[k] = v;
-		}
+		if constexpr (ewt::ST.c[k].n2 <= 1)
+			D[k] = t[k];
+		else
+			D[k] = traced(k_, D);
 	});
 	// back from the wedge to the separation's own axes
-	ewt_transpose_if<NOUT, 0, 1>(D, s3);
-	ewt_transpose_if<NOUT, 1, 2>(D, s2);
-	ewt_transpose_if<NOUT, 0, 1>(D, s1);
+	ewt_transpose_if<NOUT, 0, 1>(D, p.s3);
+	ewt_transpose_if<NOUT, 1, 2>(D, p.s2);
+	ewt_transpose_if<NOUT, 0, 1>(D, p.s1);
 	// the sign of a component is the product of the signs of the coordinates it holds an odd
 	// number of times: one multiply per component from the products of the three signs
+	const float* sg = p.sg;
 	const float sgp[8] = {1.0f, sg[0], sg[1], sg[0] * sg[1], sg[2], sg[0] * sg[2], sg[1] * sg[2], sg[0] * sg[1] * sg[2]};
 	ewt_for_seq(std::make_integer_sequence<int, NOUT>{}, [&](auto k_) {
 		constexpr int k = decltype(k_)::value;
@@ -442,6 +451,82 @@ __device__ __forceinline__ void green_ewald_tab(float* D, const float* x, const 
 	});
 }
 
-__device__ __forceinline__ void green_ewald(float* D, const float* x) { green_ewald_tab<35>(D, x, c_ewt); }
+// A wave reads its lanes' rows together, 128 bytes of each at a time: 8 lanes take a row's line, so a
+// load touches 8 lines where a row per lane touches 64 (the vector cache serves about one a cycle:
+// 16 such loads for orders 0..4 are 1,024 cycles of a compute unit for the 64 entries, more than their
+// arithmetic).  The lines go through LDS, the 16-byte parts of a row rotated so that neither side
+// conflicts.  Every lane of the wave calls this; one wave uses a stage at a time.
+typedef float ewt_f4 __attribute__((ext_vector_type(4)));
+struct EwtStage {
+	ewt_f4 part[64 * 8];
+	int row[64];
+};
+
+template <int NOUT>
+struct EwtRows {
+	// one float4 past a line (orders 0..2 read 9) is read by each lane for itself
+	static constexpr int F4 = EwtRead<NOUT>::F4, REST = F4 % 8 == 1 ? 1 : 0, LINES = (F4 - REST + 7) / 8;
+	ewt_f4 v[LINES][8], rest;
+
+	static __device__ __forceinline__ void settle() {
+		__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+		__builtin_amdgcn_wave_barrier();
+		__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+	}
+	// the loads: lane 8 g + i takes part i of rows g, 8 + g, ..., rotated by half the row's number
+	__device__ __forceinline__ void fetch(int row, const float* table, EwtStage& S, int lane) {
+		const int g = lane >> 3;
+		settle();
+		S.row[(lane & 7) * 8 + g] = row * (TG_EWT_STRIDE * 4);  // rows g, 8 + g, ... of group g side by side
+		settle();
+		unsigned src[8];
+		const unsigned part = 16u * unsigned((lane & 7) ^ (g >> 1));
+		ewt_for_seq(std::make_integer_sequence<int, 8>{}, [&](auto q_) {
+			constexpr int q = decltype(q_)::value;
+			src[q] = unsigned(S.row[g * 8 + q]) + (q & 1 ? part ^ 64u : part);
+		});
+		ewt_for_seq(std::make_integer_sequence<int, LINES * 8>{}, [&](auto i_) {
+			constexpr int h = decltype(i_)::value / 8, q = decltype(i_)::value % 8;
+			v[h][q] = *reinterpret_cast<const ewt_f4*>(reinterpret_cast<const char*>(table) + src[q] + 128 * h);
+		});
+		if (REST) rest = *reinterpret_cast<const ewt_f4*>(table + unsigned(row) * TG_EWT_STRIDE + 32 * LINES);
+	}
+	// the lane's own row
+	__device__ __forceinline__ void take(float* c, EwtStage& S, int lane) const {
+		ewt_for_seq(std::make_integer_sequence<int, LINES>{}, [&](auto h_) {
+			constexpr int h = decltype(h_)::value;
+			settle();
+			ewt_for_seq(std::make_integer_sequence<int, 8>{}, [&](auto q_) { S.part[64 * decltype(q_)::value + lane] = v[h][decltype(q_)::value]; });
+			settle();
+			ewt_for_seq(std::make_integer_sequence<int, (F4 - 8 * h < 8 ? F4 - 8 * h : 8)>{}, [&](auto k_) {
+				constexpr int k = decltype(k_)::value;
+				const ewt_f4 w = S.part[8 * lane + (k ^ ((lane >> 1) & 7))];
+				c[4 * (8 * h + k)] = w.x;
+				c[4 * (8 * h + k) + 1] = w.y;
+				c[4 * (8 * h + k) + 2] = w.z;
+				c[4 * (8 * h + k) + 3] = w.w;
+			});
+		});
+		if constexpr (REST) {
+			c[32 * LINES] = rest.x;
+			c[32 * LINES + 1] = rest.y;
+			c[32 * LINES + 2] = rest.z;
+			c[32 * LINES + 3] = rest.w;
+		}
+	}
+};
+
+// ewt_eval at the separations of a wave's lanes together, x of an idle lane being any; returns the
+// Laplacian
+template <int NOUT>
+__device__ __forceinline__ float green_ewald_wave(float* D, const float* x, const float* table, EwtStage& S, int lane) {
+	const EwtPoint p = ewt_point(x);
+	EwtRows<NOUT> rows;
+	rows.fetch(p.row, table, S, lane);
+	float c[EwtRead<NOUT>::F4 * 4];
+	rows.take(c, S, lane);
+	ewt_eval<NOUT>(D, c, p);
+	return p.lap;
+}
 
 }  // namespace tg
