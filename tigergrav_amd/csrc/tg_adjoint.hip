@@ -287,7 +287,7 @@ struct AdjItems {
 // the lanes of an item's wave: sinks padded to a power of two nsp, the P = 64 / nsp lane groups
 // (phases) splitting the sources, so leaves of 32 or fewer particles keep every lane busy; the
 // NW waves of the group share the list (tg_leaf_waves.hpp)
-template <int NW>
+template <int NW, int TILE = 64>
 struct LeafLanes {
 	int lane, wave, ns, nsp, P, si, ph, pi;
 	int2 share;
@@ -301,7 +301,7 @@ struct LeafLanes {
 		si = lane & (nsp - 1);
 		ph = lane >> lg;
 		pi = it.x + min(si, ns - 1);
-		share = wave_share<NW>(it.z, it.w, wave);
+		share = wave_share<NW, TILE>(it.z, it.w, wave);
 	}
 	// the sums of all phases and waves onto the sink's gradient
 	__device__ __forceinline__ void store(double gm, double* gx, double (*red)[4][64], double* grad) {
@@ -393,7 +393,7 @@ __global__ __launch_bounds__(64 * NW) void k_adj_pp(AdjArgs A, AdjItems I) {
 template <int NW>
 __global__ __launch_bounds__(64 * NW) void k_adj_pp_ewald(AdjArgs A, AdjItems I) {
 	const int4 it = I.items[blockIdx.x];
-	LeafLanes<NW> T(it);
+	LeafLanes<NW, 8> T(it);
 	const int4 me = A.parts[T.pi];
 	const float4 wv = A.w[T.pi];
 	const float wi[3] = {wv.x, wv.y, wv.z};
@@ -401,7 +401,7 @@ __global__ __launch_bounds__(64 * NW) void k_adj_pp_ewald(AdjArgs A, AdjItems I)
 	__shared__ int4 tps[NW][64];
 	__shared__ float4 tws[NW][64];
 	__shared__ double red[NW > 1 ? NW - 1 : 1][4][64];
-	__shared__ EwtStage stages[NW];
+	__shared__ EwtStage<10> stages[NW];
 	int4* tp = tps[T.wave];
 	float4* tw = tws[T.wave];
 	double gx[3] = {0.0, 0.0, 0.0}, gm = 0.0;
@@ -466,9 +466,9 @@ __global__ __launch_bounds__(64 * NW) void k_adj_pp_ewald(AdjArgs A, AdjItems I)
 template <int NW, bool EWALD>
 __global__ __launch_bounds__(64 * NW) void k_adj_pc_sink(AdjArgs A, AdjItems I) {
 	const int4 it = I.items[blockIdx.x];
-	LeafLanes<NW> T(it);
+	LeafLanes<NW, 4> T(it);
 	__shared__ double red[NW > 1 ? NW - 1 : 1][4][64];
-	__shared__ EwtStage stages[EWALD ? NW : 1];
+	__shared__ EwtStage<adj::NS5> stages[EWALD ? NW : 1];
 	const int4 me = A.parts[T.pi];
 	const float4 wv = A.w[T.pi];
 	const float wi[3] = {wv.x, wv.y, wv.z};
@@ -528,7 +528,7 @@ __global__ __launch_bounds__(64) void k_adj_pc_t(AdjPCArgs A) {
 	float mu[17];
 #pragma unroll
 	for (int q = 0; q < 17; q++) mu[q] = 0.0f;
-	__shared__ EwtStage stage[1];
+	__shared__ EwtStage<35> stage[1];
 	for (int k = it.y + qq; k - qq < it.z; k += Q) {
 		const int2 lf = A.leaves[min(k, it.z - 1)];
 		const bool on = k < it.z && o < lf.y;
@@ -580,7 +580,7 @@ __global__ __launch_bounds__(64 * NW) void k_adj_cp_t(AdjCPArgs A) {
 	if (it.z == it.w) return;  // no node takes this leaf
 	const int t = threadIdx.x & 63;
 	const int wave = NW == 1 ? 0 : int(threadIdx.x >> 6);
-	const int2 share = wave_share<NW>(it.z, it.w, wave);
+	const int2 share = wave_share<NW, 4>(it.z, it.w, wave);
 	const int ns = it.y;
 	const int lg = ns <= 1 ? 0 : 32 - __clz(ns - 1);
 	const int nsp = 1 << lg;
@@ -593,7 +593,7 @@ __global__ __launch_bounds__(64 * NW) void k_adj_cp_t(AdjCPArgs A) {
 	__shared__ float lams[NW][64][36];
 	__shared__ int4 xss[NW][64];
 	__shared__ double red[NW > 1 ? NW - 1 : 1][4][64];
-	__shared__ EwtStage stages[EWALD ? NW : 1];
+	__shared__ EwtStage<adj::NS5> stages[EWALD ? NW : 1];
 	float (*lam)[36] = lams[wave];
 	int4* xs = xss[wave];
 	double gm = 0.0, g3[3] = {0.0, 0.0, 0.0};
@@ -666,7 +666,7 @@ __global__ __launch_bounds__(64) void k_adj_cc_t(AdjCCArgs A) {
 	const int cnt = int(A.n - begin < 64 ? A.n - begin : 64);
 	__shared__ float red[17][65];
 	__shared__ int sc[64];
-	__shared__ EwtStage stage[1];
+	__shared__ EwtStage<35> stage[1];
 	float mu[17];
 #pragma unroll
 	for (int q = 0; q < 17; q++) mu[q] = 0.0f;
@@ -1156,10 +1156,10 @@ int Solver::adjoint_lists() {
 
 namespace {
 
-// waves per group of a leaf-kind launch, as the forward's
+// launch for the number of waves per group, 1, 2, 4 or 8
 template <class F>
-void with_waves(int nitems, int64_t nlist, F launch) {
-	switch (leaf_waves(nitems, nlist, 8)) {
+void with_waves(int waves, F launch) {
+	switch (waves) {
 		case 1: launch(std::integral_constant<int, 1>{}); break;
 		case 2: launch(std::integral_constant<int, 2>{}); break;
 		case 4: launch(std::integral_constant<int, 4>{}); break;
@@ -1260,19 +1260,22 @@ int Solver::adjoint(const float* w_in, double* grad_out, float* ms) {
 		if (work[k].nitems <= 0) continue;
 		AdjItems I{work[k].items.as<int4>(), work[k].list.as<int>(), work[k].nitems};
 		const dim3 g(work[k].nitems);
-		with_waves(work[k].nitems, work[k].nlist, [&](auto nw_) {
-			constexpr int NW = decltype(nw_)::value;
+		// as the forward's; the Ewald kinds' rows and tiles take up to 10 KB of LDS a wave
+		const int waves = k == PP_DIRECT ? leaf_waves(work[k].nitems, work[k].nlist, 8) :
+				leaf_waves_fine(work[k].nitems, work[k].nlist, k == PC_DIRECT ? 8 : 4, k == PP_EWALD ? 64 : 8);
+		with_waves(waves, [&](auto nw_) {
+			constexpr int NW = decltype(nw_)::value, NWE = NW < 4 ? NW : 4;
 			const dim3 b(64 * NW);
 			if (k == PP_DIRECT && ewald)
 				hipLaunchKernelGGL((k_adj_pp<NW, true>), g, b, 0, s, a, I);
 			else if (k == PP_DIRECT)
 				hipLaunchKernelGGL((k_adj_pp<NW, false>), g, b, 0, s, a, I);
 			else if (k == PP_EWALD)
-				hipLaunchKernelGGL((k_adj_pp_ewald<NW>), g, b, 0, s, a, I);
+				hipLaunchKernelGGL((k_adj_pp_ewald<NWE>), g, dim3(64 * NWE), 0, s, a, I);
 			else if (k == PC_DIRECT)
 				hipLaunchKernelGGL((k_adj_pc_sink<NW, false>), g, b, 0, s, a, I);
 			else
-				hipLaunchKernelGGL((k_adj_pc_sink<NW, true>), g, b, 0, s, a, I);
+				hipLaunchKernelGGL((k_adj_pc_sink<NWE, true>), g, dim3(64 * NWE), 0, s, a, I);
 		});
 		ACHK(hipGetLastError());
 	}
@@ -1301,11 +1304,11 @@ int Solver::adjoint(const float* w_in, double* grad_out, float* ms) {
 		if (adj_cpt_n[e] <= 0 || n_leaf_items <= 0) continue;
 		AdjCPArgs pa{d_adj_cpt_items[e].as<int4>(), d_adj_cpt_keys[e].as<uint64_t>(), adj_sink_bits, d_nodepos.as<int4>(), d_parts.as<int4>(),
 				d_adj_lam.as<double>(), d_adj_grad.as<double>(), ewald};
-		// four waves at most: 9 KB of staged expansions each
-		with_waves(n_leaf_items, adj_cpt_n[e], [&](auto nw_) {
-			constexpr int NW = decltype(nw_)::value < 4 ? decltype(nw_)::value : 4;
+		// four waves at most, 10 KB of staged expansions each; two where the table's rows take 8 KB more
+		with_waves(leaf_waves_fine(n_leaf_items, adj_cpt_n[e], e ? 2 : 4, 8), [&](auto nw_) {
+			constexpr int NW = decltype(nw_)::value < 4 ? decltype(nw_)::value : 4, NWE = NW < 2 ? NW : 2;
 			if (e)
-				hipLaunchKernelGGL((k_adj_cp_t<NW, true>), dim3(n_leaf_items), dim3(64 * NW), 0, s, pa);
+				hipLaunchKernelGGL((k_adj_cp_t<NWE, true>), dim3(n_leaf_items), dim3(64 * NWE), 0, s, pa);
 			else
 				hipLaunchKernelGGL((k_adj_cp_t<NW, false>), dim3(n_leaf_items), dim3(64 * NW), 0, s, pa);
 		});

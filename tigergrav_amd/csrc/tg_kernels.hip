@@ -358,7 +358,7 @@ __global__ __launch_bounds__(64 * NW) void k_pc(LeafArgs A) {
 	const int4 it = A.items[blockIdx.x];
 	const int lane = threadIdx.x & 63;
 	const int wave = NW == 1 ? 0 : int(threadIdx.x >> 6);
-	const int2 share = wave_share<NW>(it.z, it.w, wave);
+	const int2 share = wave_share<NW, 4>(it.z, it.w, wave);
 	const int ns = it.y & PP_COUNT_MASK;
 	const int lg = ceil_log2_64(ns);
 	const int nsp = 1 << lg;
@@ -368,7 +368,7 @@ __global__ __launch_bounds__(64 * NW) void k_pc(LeafArgs A) {
 	const int4 me = A.sinks[it.x + min(si, ns - 1)];
 	__shared__ float tiles[NW][64][20];
 	__shared__ double red[NW > 1 ? NW - 1 : 1][4][64];
-	__shared__ EwtStage stages[EWALD ? NW : 1];
+	__shared__ EwtStage<35> stages[EWALD ? NW : 1];
 	float (*tile)[20] = tiles[wave];
 	float phi = 0.f, g[3] = {0.f, 0.f, 0.f};
 	double dphi = 0.0, dg[3] = {0.0, 0.0, 0.0};
@@ -387,10 +387,7 @@ __global__ __launch_bounds__(64 * NW) void k_pc(LeafArgs A) {
 			}
 		}
 		wave_lds_sync<NW>();
-		// the whole wave takes every turn of the Ewald kind's loop (its rows are read together)
-		for (int k0 = 0; k0 < n; k0 += P) {
-			const int k = min(k0 + ph, n - 1);
-			if (!EWALD && k0 + ph >= n) break;
+		auto source = [&](int k, bool on) {
 			float M[17];
 #pragma unroll
 			for (int q = 0; q < 17; q++) M[q] = tile[k][q];
@@ -402,7 +399,12 @@ __global__ __launch_bounds__(64 * NW) void k_pc(LeafArgs A) {
 				green_ewald_wave<35>(D, x, c_ewt, stages[EWALD ? wave : 0], lane);
 			else
 				green_direct(D, x);
-			if (!EWALD || k0 + ph < n) m2p(phi, g, M, D);
+			if (on) m2p(phi, g, M, D);
+		};
+		if (EWALD) {  // the whole wave takes every turn (its table rows are read together)
+			for (int k0 = 0; k0 < n; k0 += P) source(min(k0 + ph, n - 1), k0 + ph < n);
+		} else {
+			for (int k = ph; k < n; k += P) source(k, true);
 		}
 		dphi += phi;
 		dg[0] += g[0];
@@ -430,13 +432,21 @@ static void pc_launch(const LeafArgs& a, bool ewald, hipStream_t s) {
 		hipLaunchKernelGGL((k_pc<NW, false, false>), dim3(a.nitems), dim3(64 * NW), 0, s, a);
 }
 
+static void pc_launch8(const LeafArgs& a, hipStream_t s) {
+	if (a.wrap)
+		hipLaunchKernelGGL((k_pc<8, false, true>), dim3(a.nitems), dim3(512), 0, s, a);
+	else
+		hipLaunchKernelGGL((k_pc<8, false, false>), dim3(a.nitems), dim3(512), 0, s, a);
+}
+
 hipError_t launch_pc(const LeafArgs& a, bool ewald, hipStream_t s) {
 	if (a.nitems <= 0) return hipSuccess;
-	switch (leaf_waves(a.nitems, a.nlist, 8)) {
+	// the Ewald kind's rows and tile take 13 KB of LDS a wave
+	switch (leaf_waves_fine(a.nitems, a.nlist, ewald ? 4 : 8, 8)) {
 		case 1: pc_launch<1>(a, ewald, s); break;
 		case 2: pc_launch<2>(a, ewald, s); break;
 		case 4: pc_launch<4>(a, ewald, s); break;
-		default: pc_launch<8>(a, ewald, s); break;
+		default: pc_launch8(a, s); break;
 	}
 	return hipGetLastError();
 }
@@ -449,8 +459,8 @@ hipError_t launch_pc(const LeafArgs& a, bool ewald, hipStream_t s) {
 // laid out as in k_pc: 2^lg lanes per sink, the other lane bits split the tile's sources.
 // Bound by the rows' way through the vector cache and LDS (8 KB a turn) beside about 150
 // instructions of arithmetic, at the four waves a SIMD that the stages leave.  32,768 uniform
-// particles, leaves of 64 (4.5e7 pairs): 646 -> 430 us against a row read by each lane and a 19-term
-// sum per component.
+// particles, leaves of 64 (4.5e7 pairs): 646 -> 460 us against a row read by each lane and a 19-term
+// sum per component (16 waves in 152 KB took 430; a work group keeps to 64 KB).
 template <int NW>
 __global__ __launch_bounds__(64 * NW) void k_pp_ewald(LeafArgs A) {
 	const int4 it = A.items[blockIdx.x];
@@ -464,8 +474,8 @@ __global__ __launch_bounds__(64 * NW) void k_pp_ewald(LeafArgs A) {
 	const int si = lane & (nsp - 1);
 	const int ph = lane >> lg;
 	const int4 me = A.sinks[it.x + min(si, ns - 1)];
-	// the sums' exchange at the end reuses the stages (16 waves take 152 KB with them)
-	__shared__ EwtStage stages[NW];
+	// the sums' exchange at the end reuses the stages (8 waves take 64 KB with the tiles)
+	__shared__ EwtStage<4> stages[NW];
 	__shared__ int4 tiles[NW][64];
 	static_assert(sizeof(double) * (NW - 1) * 4 * 64 <= sizeof(stages), "exchange in the stages");
 	double (*red)[4][64] = reinterpret_cast<double (*)[4][64]>(stages);
@@ -517,21 +527,14 @@ __global__ __launch_bounds__(64 * NW) void k_pp_ewald(LeafArgs A) {
 	}
 }
 
-// waves of an item: 64 sources or more to each on average
-static int ewald_waves(int nitems, int64_t sources) {
-	int w = 1;
-	while (w < 16 && int64_t(nitems) * (2 * w) <= TARGET_WAVES && sources >= int64_t(nitems) * 64 * (2 * w)) w *= 2;
-	return w;
-}
-
 hipError_t launch_pp_ewald(const LeafArgs& a, hipStream_t s) {
 	if (a.nitems <= 0) return hipSuccess;
-	switch (ewald_waves(a.nitems, a.nlist)) {
+	// 64 sources a wave: a turn takes one source per sink's lane group through its rows
+	switch (leaf_waves_fine(a.nitems, a.nlist, 8, 64)) {
 		case 1: hipLaunchKernelGGL(k_pp_ewald<1>, dim3(a.nitems), dim3(64), 0, s, a); break;
 		case 2: hipLaunchKernelGGL(k_pp_ewald<2>, dim3(a.nitems), dim3(128), 0, s, a); break;
 		case 4: hipLaunchKernelGGL(k_pp_ewald<4>, dim3(a.nitems), dim3(256), 0, s, a); break;
-		case 8: hipLaunchKernelGGL(k_pp_ewald<8>, dim3(a.nitems), dim3(512), 0, s, a); break;
-		default: hipLaunchKernelGGL(k_pp_ewald<16>, dim3(a.nitems), dim3(1024), 0, s, a); break;
+		default: hipLaunchKernelGGL(k_pp_ewald<8>, dim3(a.nitems), dim3(512), 0, s, a); break;
 	}
 	return hipGetLastError();
 }
@@ -544,7 +547,7 @@ struct NodeSums {
 	int sl[64];
 };
 union NodeLds {  // the Ewald kinds' rows, then the sums
-	EwtStage rows;
+	EwtStage<35> rows;
 	NodeSums sums;
 };
 

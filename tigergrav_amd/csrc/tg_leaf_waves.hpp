@@ -49,6 +49,16 @@ inline int leaf_waves(int nitems, int64_t sources, int most) {
 	return w;
 }
 
+// The same for kinds whose turn takes one source (or as few as share the wave's lanes) through a long
+// evaluation: shares of per sources or more on average, whatever the tiles.  300 multipoles on 64
+// sinks: 69 us with two waves (the tiles' rule), 22 us with eight; the far multipoles of 262,144
+// clustered particles (39 a leaf): 91 -> 59 us, their adjoint's (65,536) 160 -> 92 us.
+inline int leaf_waves_fine(int nitems, int64_t sources, int most, int per) {
+	int w = 1;
+	while (w < most && int64_t(nitems) * (2 * w) <= TARGET_WAVES && sources >= int64_t(nitems) * per * (2 * w)) w *= 2;
+	return w;
+}
+
 // The waves of a sink add up: the phases of each wave by cross-lane adds, then the waves in order
 // (wave 0's first NSP lanes hold the sums).  Every lane of the group calls this.
 template <int NW>

@@ -455,17 +455,21 @@ __host__ __device__ __forceinline__ void ewt_eval(float* D, const float* c, cons
 // load touches 8 lines where a row per lane touches 64 (the vector cache serves about one a cycle:
 // 16 such loads for orders 0..4 are 1,024 cycles of a compute unit for the 64 entries, more than their
 // arithmetic).  The lines go through LDS, the 16-byte parts of a row rotated so that neither side
-// conflicts.  Every lane of the wave calls this; one wave uses a stage at a time.
+// conflicts (orders 0..1 read 7 parts, an odd stride that needs no rotation).  Every lane of the wave
+// calls this; one wave uses a stage at a time.
 typedef float ewt_f4 __attribute__((ext_vector_type(4)));
+template <int NOUT>
 struct EwtStage {
-	ewt_f4 part[64 * 8];
-	int row[64];
+	static constexpr int PARTS = EwtRead<NOUT>::F4 < 8 ? EwtRead<NOUT>::F4 : 8;
+	static_assert(PARTS == 8 || PARTS == 7, "strides without conflicts");
+	ewt_f4 part[64 * PARTS];  // the wave's row numbers first
 };
 
 template <int NOUT>
 struct EwtRows {
 	// one float4 past a line (orders 0..2 read 9) is read by each lane for itself
 	static constexpr int F4 = EwtRead<NOUT>::F4, REST = F4 % 8 == 1 ? 1 : 0, LINES = (F4 - REST + 7) / 8;
+	static constexpr int PARTS = EwtStage<NOUT>::PARTS;
 	ewt_f4 v[LINES][8], rest;
 
 	static __device__ __forceinline__ void settle() {
@@ -474,16 +478,17 @@ struct EwtRows {
 		__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 	}
 	// the loads: lane 8 g + i takes part i of rows g, 8 + g, ..., rotated by half the row's number
-	__device__ __forceinline__ void fetch(int row, const float* table, EwtStage& S, int lane) {
+	__device__ __forceinline__ void fetch(int row, const float* table, EwtStage<NOUT>& S, int lane) {
 		const int g = lane >> 3;
+		int* rows = reinterpret_cast<int*>(S.part);
 		settle();
-		S.row[(lane & 7) * 8 + g] = row * (TG_EWT_STRIDE * 4);  // rows g, 8 + g, ... of group g side by side
+		rows[(lane & 7) * 8 + g] = row * (TG_EWT_STRIDE * 4);  // rows g, 8 + g, ... of group g side by side
 		settle();
 		unsigned src[8];
-		const unsigned part = 16u * unsigned((lane & 7) ^ (g >> 1));
+		const unsigned part = PARTS == 8 ? 16u * unsigned((lane & 7) ^ (g >> 1)) : 16u * unsigned(min(lane & 7, 6));
 		ewt_for_seq(std::make_integer_sequence<int, 8>{}, [&](auto q_) {
 			constexpr int q = decltype(q_)::value;
-			src[q] = unsigned(S.row[g * 8 + q]) + (q & 1 ? part ^ 64u : part);
+			src[q] = unsigned(rows[g * 8 + q]) + (PARTS == 8 && (q & 1) ? part ^ 64u : part);
 		});
 		ewt_for_seq(std::make_integer_sequence<int, LINES * 8>{}, [&](auto i_) {
 			constexpr int h = decltype(i_)::value / 8, q = decltype(i_)::value % 8;
@@ -492,15 +497,17 @@ struct EwtRows {
 		if (REST) rest = *reinterpret_cast<const ewt_f4*>(table + unsigned(row) * TG_EWT_STRIDE + 32 * LINES);
 	}
 	// the lane's own row
-	__device__ __forceinline__ void take(float* c, EwtStage& S, int lane) const {
+	__device__ __forceinline__ void take(float* c, EwtStage<NOUT>& S, int lane) const {
 		ewt_for_seq(std::make_integer_sequence<int, LINES>{}, [&](auto h_) {
 			constexpr int h = decltype(h_)::value;
 			settle();
-			ewt_for_seq(std::make_integer_sequence<int, 8>{}, [&](auto q_) { S.part[64 * decltype(q_)::value + lane] = v[h][decltype(q_)::value]; });
+			// seven parts: the eighth lane of a row holds the seventh's value
+			const int to = PARTS == 8 ? lane : 7 * (lane >> 3) + min(lane & 7, 6);
+			ewt_for_seq(std::make_integer_sequence<int, 8>{}, [&](auto q_) { S.part[8 * PARTS * decltype(q_)::value + to] = v[h][decltype(q_)::value]; });
 			settle();
 			ewt_for_seq(std::make_integer_sequence<int, (F4 - 8 * h < 8 ? F4 - 8 * h : 8)>{}, [&](auto k_) {
 				constexpr int k = decltype(k_)::value;
-				const ewt_f4 w = S.part[8 * lane + (k ^ ((lane >> 1) & 7))];
+				const ewt_f4 w = S.part[PARTS * lane + (PARTS == 8 ? k ^ ((lane >> 1) & 7) : k)];
 				c[4 * (8 * h + k)] = w.x;
 				c[4 * (8 * h + k) + 1] = w.y;
 				c[4 * (8 * h + k) + 2] = w.z;
@@ -519,7 +526,7 @@ struct EwtRows {
 // ewt_eval at the separations of a wave's lanes together, x of an idle lane being any; returns the
 // Laplacian
 template <int NOUT>
-__device__ __forceinline__ float green_ewald_wave(float* D, const float* x, const float* table, EwtStage& S, int lane) {
+__device__ __forceinline__ float green_ewald_wave(float* D, const float* x, const float* table, EwtStage<NOUT>& S, int lane) {
 	const EwtPoint p = ewt_point(x);
 	EwtRows<NOUT> rows;
 	rows.fetch(p.row, table, S, lane);

@@ -683,7 +683,7 @@ int Solver::upload_lists_device() {
 	const DeviceLists& L = dlists;
 	const int64_t nn = n_nodes;
 	const int64_t nl = n_leaf_items;
-	const int chunk = std::min(NODE_CHUNK_MAX, std::max(1, node_chunk));
+	const int chunk = std::min(NODE_CHUNK_MAX, std::max(1, chunk_of()));
 	if (L.nn != nn || !L.ptr_all) {
 		err = "device list work: the device walk's lists do not belong to this tree";
 		return TG_EINVAL;

@@ -560,7 +560,7 @@ int Solver::upload() {
 	const bool device_lists = lists_on_device && device >= 0;
 	{
 		// with the lists on the device only the tree's arrays are made here
-		const int rc = device_lists ? prepare_tree_work(T, n, W, err) : prepare_work(T, n, ewald, soft_len, node_chunk, W, err);
+		const int rc = device_lists ? prepare_tree_work(T, n, W, err) : prepare_work(T, n, ewald, soft_len, chunk_of(), W, err);
 		if (rc != TG_OK) return rc;
 	}
 	t_detail[4] = now() - tp0;

@@ -45,7 +45,11 @@ struct Solver {
 	double soft_len = 0.0, m = 0.0, theta = 0.7;
 	int parts_per_node = 64;
 	bool uniform_mass = true;
-	int node_chunk = 4096;  // sources per CC/CP partial slot (<= NODE_CHUNK_MAX); applies from the next set_particles
+	int node_chunk = 0;  // sources per CC/CP partial slot (<= NODE_CHUNK_MAX); 0: by the set's size; from the next set_particles
+	// One wave takes a slot's sources, so a slot holds a whole list where the lists are enough waves; sets
+	// of up to 131,072 have a few hundred nodes with particle lists of a thousand (32,768 particles, leaves
+	// of 64: 464 of 1,095, 65 us against 17 us in slots of 256)
+	int chunk_of() const { return node_chunk > 0 ? node_chunk : n <= 131072 ? 256 : 4096; }
 	bool pp_persistent = false;  // PP direct as a persistent queue-driven kernel
 	// graph replays: 0 one stream; 1 the node kinds on a second stream beside the leaf kinds; 2 as 1,
 	// with the Ewald node kinds on a third stream beside the direct ones
