@@ -8,7 +8,7 @@
 //    float, the running sum FP64 (the reference accumulates float terms in FP64 lanes,
 //    src/gravity.cpp:259-261), and phases are merged with cross-lane FP64 shuffles.
 //  * node kinds (CC, CP): lane = source; a wave packs the short lists of several expansion
-//    centres (<= 64 entries), 35 float accumulators per lane, merged per centre in FP64 through
+//    centres (<= 64 entries), 25 float accumulators per lane, merged per centre in FP64 through
 //    LDS by a segmented scan.
 //  * Ewald kinds use tg::ewt_eval (tg_math.hpp).
 #include "tg_kernels.hpp"
@@ -540,46 +540,69 @@ hipError_t launch_pp_ewald(const LeafArgs& a, hipStream_t s) {
 }
 
 // ---- node kinds ----------------------------------------------------------------------------------
-// Segmented FP64 reduction of the lanes' 35 float accumulators by owner slot, through LDS.  The
-// entries of one slot are consecutive, so lanes 0..34 (one coefficient each) scan the wave once.
+// Segmented FP64 reduction of the lanes' 25 float accumulators (26 with the trace) by owner slot,
+// through LDS.  The entries of one slot are consecutive: each half wave adds one coefficient a lane over
+// a segment of its own, or over half of a wave's only segment.
 struct NodeSums {
-	float red[35][65];
+	float red[NODE_SUMS][65];
 	int sl[64];
 };
 union NodeLds {  // the Ewald kinds' rows, then the sums
 	EwtStage<35> rows;
 	NodeSums sums;
 };
+union NodeFoldLds {  // the direct kind's multipoles, then the sums
+	ewt_f4 stage[256];
+	NodeSums sums;
+};
 
-__device__ __forceinline__ void node_segment_store(const float* L, int slot, int cnt, NodeSums& S, double* partial) {
+template <bool TRACE>
+__device__ __forceinline__ void node_segment_store(const float* L, float trace, int slot, int cnt, NodeSums& S, double* partial) {
 	float (*red)[65] = S.red;
 	int* sl = S.sl;
 	const int lane = threadIdx.x;
 	__syncthreads();
-#pragma unroll
-	for (int c = 0; c < 35; c++) red[c][lane] = L[c];
+	static_for<25>([&](auto k_) { red[decltype(k_)::value][lane] = L[KEPT[decltype(k_)::value]]; });
+	if (TRACE) red[25][lane] = trace;
 	sl[lane] = slot;
 	__syncthreads();
-	// the wave's segments (runs of one slot) from a ballot of their first entries; lanes 0..34 then
-	// add one coefficient each over every segment, four FP64 partial sums per segment
+	// the wave's segments (runs of one slot) from a ballot of their first entries, two at a time
 	const bool first = lane < cnt && (lane == 0 || sl[lane] != sl[lane - 1]);
 	unsigned long long starts = __ballot(first);
-	if (lane < 35) {
-		while (starts) {
-			const int b = __ffsll(starts) - 1;
+	const bool single = __popcll(starts) == 1;
+	const int c = lane & 31;
+	const bool high = lane >= 32;
+	while (starts) {
+		int b = __ffsll(starts) - 1;
+		starts &= starts - 1;
+		int e = starts ? __ffsll(starts) - 1 : cnt;
+		int b1 = e, e1 = e;  // the second segment
+		if (single) {
+			b1 = b + ((e - b + 1) >> 1);
+			e = b1;
+		} else if (starts) {
 			starts &= starts - 1;
-			const int e = starts ? __ffsll(starts) - 1 : cnt;
+			e1 = starts ? __ffsll(starts) - 1 : cnt;
+		}
+		if (high) {
+			b = b1;
+			e = e1;
+		}
+		double acc = 0.0;
+		if (c < (TRACE ? 26 : 25)) {
 			double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
 			int j = b;
 			for (; j + 4 <= e; j += 4) {
-				a0 += double(red[lane][j]);
-				a1 += double(red[lane][j + 1]);
-				a2 += double(red[lane][j + 2]);
-				a3 += double(red[lane][j + 3]);
+				a0 += double(red[c][j]);
+				a1 += double(red[c][j + 1]);
+				a2 += double(red[c][j + 2]);
+				a3 += double(red[c][j + 3]);
 			}
-			for (; j < e; j++) a0 += double(red[lane][j]);
-			partial[35 * (size_t) sl[b] + lane] = (a0 + a1) + (a2 + a3);
+			for (; j < e; j++) a0 += double(red[c][j]);
+			acc = (a0 + a1) + (a2 + a3);
 		}
+		if (single) acc += __shfl_xor(acc, 32, 64);
+		if (c < NODE_SUMS && b < e && !(single && high)) partial[NODE_SUMS * (size_t) sl[b] + c] = acc;
 	}
 }
 
@@ -609,43 +632,95 @@ __global__ __launch_bounds__(64) void k_cc(NodeArgs A) {
 	if (j < wv.y) {
 		slot = A.owner ? A.owner[j] : int(blockIdx.x);  // the plain drop-in: one slot per wave, one sink
 		const int4 X = A.sinkpos[A.slot_node ? A.slot_node[slot] : 0];
-		// software pipeline: the next entry's multipole and the list index after it are loaded while
-		// the current entry is evaluated, into the other of two buffers (the loop is unrolled twice,
-		// so no copy between them)
-		auto index_at = [&](int jj) { return jj < wv.y ? (A.list ? A.list[jj] : jj) : -1; };
-		auto load_multi = [&](int idx, float4* m) {
-			if (idx >= 0) {
-				const float4* src = reinterpret_cast<const float4*>(A.multis + idx);
+		for (; j < wv.y; j += 64) {
+			const float4* src = reinterpret_cast<const float4*>(A.multis + (A.list ? A.list[j] : j));
+			float4 f[5];
 #pragma unroll
-				for (int q = 0; q < 5; q++) m[q] = src[q];
-			}
-		};
-		auto entry = [&](const float4* m) {
-			float v[20];
-			multi_floats(v, m);
+			for (int q = 0; q < 5; q++) f[q] = src[q];
+			float v[20], q[5], o[7], qzz, D[35];
+			multi_floats(v, f);
 			const float x[3] = {sepu<WRAP>(X.x, __float_as_int(v[17])) * POS_INVF, sepu<WRAP>(X.y, __float_as_int(v[18])) * POS_INVF,
 					sepu<WRAP>(X.z, __float_as_int(v[19])) * POS_INVF};
-			float D[35];
 			green_direct(D, x);
-			m2l<false>(L, v, D, 0.0f);
-		};
-		float4 ma[5], mb[5];
-		load_multi(index_at(j), ma);
-		int next_idx = index_at(j + 64);
-		for (;;) {
-			load_multi(next_idx, mb);
-			next_idx = index_at(j + 128);
-			entry(ma);
-			j += 64;
-			if (j >= wv.y) break;
-			load_multi(next_idx, ma);
-			next_idx = index_at(j + 128);
-			entry(mb);
-			j += 64;
-			if (j >= wv.y) break;
+			fold_multi(v, q, o, qzz);
+			m2l(L, v[0], q, o, D);
 		}
 	}
-	node_segment_store(L, slot, min(wv.y - wv.x, 64), sums, A.partial);
+	node_segment_store<false>(L, 0.0f, slot, min(wv.y - wv.x, 64), sums, A.partial);
+}
+
+// The same from a solver's folded multipoles, which the wave reads together: four lanes take a record,
+// so a load touches 16 half lines where a record per lane touches 64, and LDS hands each lane its own
+// (parts rotated so that neither side conflicts).  The next turn's records are on their way while this
+// turn's are evaluated; lanes past the end carry the last entry without weight.
+// Bound by FP32 arithmetic, about 175 instructions an entry (222 with 35 components, weights formed
+// per entry).  2M particles at theta 0.3 (3.3e8 entries here, 3.6e7 in the Ewald kind): the whole
+// solve 4.50 -> 4.12 ms; at theta 0.6 1.55 -> 1.50.
+template <bool WRAP>
+__global__ __launch_bounds__(64) void k_cc_folded(NodeArgs A) {
+	__shared__ NodeFoldLds lds;
+	const int2 wv = A.waves[blockIdx.x];
+	const int lane = threadIdx.x;
+	float L[35];
+#pragma unroll
+	for (int c = 0; c < 35; c++) L[c] = 0.f;
+	int slot = -1;
+	int4 X = make_int4(0, 0, 0, 0);
+	if (wv.x + lane < wv.y) {
+		slot = A.owner[wv.x + lane];
+		X = A.sinkpos[A.slot_node[slot]];
+	}
+	if (wv.x < wv.y) {
+		const int part = (lane & 3) ^ (lane >> 4);  // of records 16 q + lane / 4, rotated by record / 4
+		const unsigned at = lane >> 2, last = wv.y - 1;
+		int i0, i1, i2, i3;  // the next turn's records
+		ewt_f4 in0, in1, in2, in3;
+		const ewt_f4* recs = reinterpret_cast<const ewt_f4*>(A.folded) + part;
+#define TG_CC_INDICES(j)                     \
+	i0 = A.list[min(unsigned(j) + at, last)];        \
+	i1 = A.list[min(unsigned(j) + 16 + at, last)];   \
+	i2 = A.list[min(unsigned(j) + 32 + at, last)];   \
+	i3 = A.list[min(unsigned(j) + 48 + at, last)]
+#define TG_CC_RECORDS              \
+	in0 = recs[4 * size_t(i0)];    \
+	in1 = recs[4 * size_t(i1)];    \
+	in2 = recs[4 * size_t(i2)];    \
+	in3 = recs[4 * size_t(i3)]
+		TG_CC_INDICES(wv.x);
+		TG_CC_RECORDS;
+		TG_CC_INDICES(wv.x + 64);
+		for (int j0 = wv.x; j0 < wv.y; j0 += 64) {
+			__syncthreads();
+			lds.stage[lane] = in0;
+			lds.stage[64 + lane] = in1;
+			lds.stage[128 + lane] = in2;
+			lds.stage[192 + lane] = in3;
+			__syncthreads();
+			TG_CC_RECORDS;
+			TG_CC_INDICES(j0 + 128);
+			float v[16];
+			static_for<4>([&](auto q_) {
+				constexpr int q = decltype(q_)::value;
+				const ewt_f4 f = lds.stage[4 * lane + (q ^ ((lane >> 2) & 3))];
+				v[4 * q] = f.x;
+				v[4 * q + 1] = f.y;
+				v[4 * q + 2] = f.z;
+				v[4 * q + 3] = f.w;
+			});
+			const float x[3] = {sepu<WRAP>(X.x, __float_as_int(v[13])) * POS_INVF, sepu<WRAP>(X.y, __float_as_int(v[14])) * POS_INVF,
+					sepu<WRAP>(X.z, __float_as_int(v[15])) * POS_INVF};
+			float D[35];
+			green_direct(D, x);
+			if (j0 + 64 > wv.y && j0 + lane >= wv.y) {
+#pragma unroll
+				for (int c = 0; c < 13; c++) v[c] = 0.0f;
+			}
+			m2l(L, v[0], v + 1, v + 6, D);
+		}
+	}
+#undef TG_CC_INDICES
+#undef TG_CC_RECORDS
+	node_segment_store<false>(L, 0.0f, slot, min(wv.y - wv.x, 64), lds.sums, A.partial);
 }
 
 // The Ewald correction of the same: the whole wave takes every turn (its table rows are read
@@ -661,6 +736,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
 #pragma unroll
 	for (int c = 0; c < 35; c++) L[c] = 0.f;
 	int slot = -1;
+	float trace = 0.0f;
 	int4 X = make_int4(0, 0, 0, 0);
 	if (wv.x + lane < wv.y) {
 		slot = A.owner ? A.owner[wv.x + lane] : int(blockIdx.x);
@@ -682,9 +758,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
 #pragma unroll
 			for (int c = 0; c < 17; c++) v[c] = 0.0f;
 		}
-		m2l<true>(L, v, D, lap);
+		float q[5], o[7], qzz;
+		fold_multi(v, q, o, qzz);
+		m2l(L, v[0], q, o, D);
+		L[0] = fmaf(qzz, lap, L[0]);
+		trace = fmaf(v[0], lap, trace);
 	}
-	node_segment_store(L, slot, min(wv.y - wv.x, 64), lds.sums, A.partial);
+	node_segment_store<true>(L, trace, slot, min(wv.y - wv.x, 64), lds.sums, A.partial);
 }
 
 template <bool WRAP>
@@ -708,7 +788,7 @@ __global__ __launch_bounds__(64) void k_cp(NodeArgs A) {
 			p2l(L, __int_as_float(s.w), D);
 		}
 	}
-	node_segment_store(L, slot, min(wv.y - wv.x, 64), sums, A.partial);
+	node_segment_store<false>(L, 0.0f, slot, min(wv.y - wv.x, 64), sums, A.partial);
 }
 
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_cp_ewald(NodeArgs A) {
@@ -719,6 +799,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
 #pragma unroll
 	for (int c = 0; c < 35; c++) L[c] = 0.f;
 	int slot = -1;
+	float trace = 0.0f;
 	int4 X = make_int4(0, 0, 0, 0);
 	if (wv.x + lane < wv.y) {
 		slot = A.owner ? A.owner[wv.x + lane] : int(blockIdx.x);
@@ -729,20 +810,45 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
 		const int4 s = A.srcs[A.list ? A.list[j] : j];
 		const float x[3] = {sepu<true>(X.x, s.x) * POS_INVF, sepu<true>(X.y, s.y) * POS_INVF, sepu<true>(X.z, s.z) * POS_INVF};
 		float D[35];
-		green_ewald_wave<35>(D, x, c_ewt, lds.rows, lane);
-		p2l(L, j0 + lane < wv.y ? __int_as_float(s.w) : 0.0f, D);
+		const float lap = green_ewald_wave<35>(D, x, c_ewt, lds.rows, lane);
+		const float m = j0 + lane < wv.y ? __int_as_float(s.w) : 0.0f;
+		p2l(L, m, D);
+		trace = fmaf(m, lap, trace);
 	}
-	node_segment_store(L, slot, min(wv.y - wv.x, 64), lds.sums, A.partial);
+	node_segment_store<true>(L, trace, slot, min(wv.y - wv.x, 64), lds.sums, A.partial);
 }
 
 hipError_t launch_cc(const NodeArgs& a, bool ewald, hipStream_t s) {
 	if (a.nwaves <= 0) return hipSuccess;
+	const dim3 g(a.nwaves), b(64);
 	if (ewald)
-		hipLaunchKernelGGL(k_cc_ewald, dim3(a.nwaves), dim3(64), 0, s, a);
+		hipLaunchKernelGGL(k_cc_ewald, g, b, 0, s, a);
+	else if (a.folded && a.wrap)
+		hipLaunchKernelGGL(k_cc_folded<true>, g, b, 0, s, a);
+	else if (a.folded)
+		hipLaunchKernelGGL(k_cc_folded<false>, g, b, 0, s, a);
 	else if (a.wrap)
-		hipLaunchKernelGGL(k_cc<true>, dim3(a.nwaves), dim3(64), 0, s, a);
+		hipLaunchKernelGGL(k_cc<true>, g, b, 0, s, a);
 	else
-		hipLaunchKernelGGL(k_cc<false>, dim3(a.nwaves), dim3(64), 0, s, a);
+		hipLaunchKernelGGL(k_cc<false>, g, b, 0, s, a);
+	return hipGetLastError();
+}
+
+__global__ __launch_bounds__(256) void k_fold_multis(const MultiSrc* __restrict__ multis, int64_t nn, FoldedMulti* __restrict__ out) {
+	const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+	if (i >= nn) return;
+	const MultiSrc s = multis[i];
+	FoldedMulti f;
+	float qzz;
+	f.m = s.m[0];
+	fold_multi(s.m, f.q, f.o, qzz);
+	for (int d = 0; d < 3; d++) f.x[d] = s.x[d];
+	out[i] = f;
+}
+
+hipError_t launch_fold_multis(const MultiSrc* multis, int64_t nn, FoldedMulti* out, hipStream_t s) {
+	if (nn <= 0) return hipSuccess;
+	hipLaunchKernelGGL(k_fold_multis, dim3(unsigned((nn + 255) / 256)), dim3(256), 0, s, multis, nn, out);
 	return hipGetLastError();
 }
 

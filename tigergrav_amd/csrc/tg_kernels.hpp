@@ -51,6 +51,43 @@ struct MultiSrc {
 	int32_t x[3];
 };
 
+// The node kinds' sums.  A direct term's tensor has no trace (derivatives of 1/r away from the origin)
+// and the periodic correction's has the constant Laplacian's, lap for D_zz and 0 above, so of the 35
+// components only the 25 without the third axis twice are summed, with the sum of the traces beside
+// them; the other ten follow from those at the end, in FP64.
+constexpr int NODE_SUMS = 26;
+constexpr int KEPT[25] = {0, 1, 2, 3, 4, 5, 6, 7, 8, 10, 11, 12, 13, 14, 16, 17, 20, 21, 22, 23, 24, 26, 27, 30, 31};
+__host__ __device__ constexpr bool kept(int slot) {
+	for (int k = 0; k < 25; k++)
+		if (KEPT[k] == slot) return true;
+	return false;
+}
+// component q of the expansion whose sums are c
+__host__ __device__ inline double node_component(const double* c, int q) {
+	switch (q) {
+		case 9: return c[25] - c[4] - c[7];        // zz
+		case 15: return -c[9] - c[12];             // xzz
+		case 18: return -c[10] - c[14];            // yzz
+		case 19: return -c[11] - c[15];            // zzz
+		case 25: return -c[16] - c[19];            // xxzz
+		case 28: return -c[17] - c[21];            // xyzz
+		case 29: return -c[18] - c[22];            // xzzz
+		case 32: return -c[19] - c[23];            // yyzz
+		case 33: return -c[20] - c[24];            // yzzz
+		case 34: return (c[16] + c[19]) + (c[19] + c[23]);  // zzzz
+		default: return c[q < 9 ? q : q < 15 ? q - 1 : q < 18 ? q - 2 : q < 25 ? q - 4 : q < 28 ? q - 5 : q - 7];
+	}
+}
+
+// A source multipole as M2L takes it: weights formed (multiplicities and 1/k!, the octupole's sign)
+// and the components with the third axis twice folded into the others by the trace relation, the
+// quadrupole in 5 terms and the octupole in 7.  64 bytes: half a line, where the plain 80 cross lines.
+struct alignas(16) FoldedMulti {
+	float m, q[5], o[7];
+	int32_t x[3];
+};
+static_assert(sizeof(FoldedMulti) == 64, "half a line");
+
 struct LeafArgs {
 	const int4* sinks;       // sink particles (x, y, z, mass bits)
 	const int4* srcs;        // source particles (PP)
@@ -72,11 +109,12 @@ struct NodeArgs {
 	const int4* sinkpos;     // expansion centres (x, y, z, unused)
 	const int4* srcs;        // source particles (CP)
 	const MultiSrc* multis;  // source multipoles (CC)
+	const FoldedMulti* folded;  // the same as M2L takes them (CC direct of a solver), or null
 	const int2* waves;       // [begin, end) runs of list entries, <= 64 each
 	const int* list;         // source index per entry
 	const int* owner;        // partial slot per entry
 	const int* slot_node;    // expansion-centre index per slot
-	double* partial;         // 35 doubles per slot
+	double* partial;         // NODE_SUMS doubles per slot
 	int nwaves;
 	int wrap;
 };
@@ -92,6 +130,8 @@ hipError_t launch_pp_direct(const LeafArgs& a, bool do_phi, hipStream_t s);
 hipError_t launch_pc(const LeafArgs& a, bool ewald, hipStream_t s);
 hipError_t launch_pp_ewald(const LeafArgs& a, hipStream_t s);
 hipError_t launch_cc(const NodeArgs& a, bool ewald, hipStream_t s);
+// a solver's multipoles as launch_cc's folded
+hipError_t launch_fold_multis(const MultiSrc* multis, int64_t nn, FoldedMulti* out, hipStream_t s);
 hipError_t launch_cp(const NodeArgs& a, bool ewald, hipStream_t s);
 
 }  // namespace tg

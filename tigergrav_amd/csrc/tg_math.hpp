@@ -12,6 +12,7 @@
 #include <utility>
 
 #include "tg_ewald_table.hpp"
+#include "tg_kernels.hpp"
 
 namespace tg {
 
@@ -188,31 +189,31 @@ __device__ __forceinline__ void green_direct(float* D, const float* x) {
 }
 
 // ---- contractions (src/gravity.cpp:26-169) ----------------------------------------------------
-// M2L: L += contraction of the multipole M with D (reference gravity.cpp:26-90)
-// Every term is added straight into L, in the reference's order of terms (as its loop adds each
-// term into its L).  D's trace in two of its indices is lap where it is D itself and 0 above
-// (derivatives of 1/r away from the origin: lap = 0; the periodic correction: its constant
-// Laplacian), so D_{k,zz} = -D_{k,xx} - D_{k,yy}, plus lap for D_zz, and a multipole's zz-holding
-// components fold into the others (LAP: with lap's term): the quadrupole contracts in 5 terms and the octupole in 7 (each L
-// component whose terms reach D through them: L0, L_a, L_ab), with the 8 folded weights formed once
-// per entry.
-template <bool LAP>
-__device__ __forceinline__ void m2l(float* L, const float* M, const float* D, float lap) {
-	float q[6], o[10];
-#pragma unroll
-	for (int s = 0; s < 6; s++) q[s] = M[1 + s] * ef2(s);
-#pragma unroll
-	for (int s = 0; s < 10; s++) o[s] = -M[7 + s] * ef3(s);
+// a multipole's folded weights (FoldedMulti); qzz: the zz weight, which meets the Laplacian
+__device__ __forceinline__ void fold_multi(const float* M, float* q, float* o, float& qzz) {
 	// quadrupole slots xx 0, xy 1, xz 2, yy 3, yz 4, zz 5; octupole xxx 0, xxy 1, xxz 2, xyy 3,
 	// xyz 4, xzz 5, yyy 6, yyz 7, yzz 8, zzz 9
-	q[0] -= q[5];
-	q[3] -= q[5];
-	o[0] -= o[5];
-	o[3] -= o[5];
-	o[1] -= o[8];
-	o[6] -= o[8];
-	o[2] -= o[9];
-	o[7] -= o[9];
+	qzz = M[6] * ef2(5);
+	const float ozx = -M[12] * ef3(5), ozy = -M[15] * ef3(8), ozz = -M[16] * ef3(9);
+	q[0] = M[1] * ef2(0) - qzz;
+	q[1] = M[2] * ef2(1);
+	q[2] = M[3] * ef2(2);
+	q[3] = M[4] * ef2(3) - qzz;
+	q[4] = M[5] * ef2(4);
+	o[0] = -M[7] * ef3(0) - ozx;
+	o[1] = -M[8] * ef3(1) - ozy;
+	o[2] = -M[9] * ef3(2) - ozz;
+	o[3] = -M[10] * ef3(3) - ozx;
+	o[4] = -M[11] * ef3(4);
+	o[5] = -M[13] * ef3(6) - ozy;
+	o[6] = -M[14] * ef3(7) - ozz;
+}
+
+// M2L: L += contraction of a folded multipole with D, kept components (reference gravity.cpp:26-90).
+// Every term is added straight into L, in the reference's order of terms (as its loop adds each term
+// into its L).
+__device__ __forceinline__ void m2l(float* L, float m, const float* q, const float* o, const float* D) {
+	constexpr int OS[7] = {0, 1, 2, 3, 4, 6, 7};  // octupole slots
 	auto quad = [&](auto slot_of, float acc) {
 #pragma unroll
 		for (int s = 0; s < 5; s++) acc = fmaf(q[s], D[slot_of(s)], acc);
@@ -220,37 +221,37 @@ __device__ __forceinline__ void m2l(float* L, const float* M, const float* D, fl
 	};
 	auto oct = [&](auto slot_of, float acc) {
 #pragma unroll
-		for (int s = 0; s < 10; s++)
-			if (s != 5 && s != 8 && s != 9) acc = fmaf(o[s], D[slot_of(s)], acc);
+		for (int s = 0; s < 7; s++) acc = fmaf(o[s], D[slot_of(OS[s])], acc);
 		return acc;
 	};
-	float l0 = fmaf(M[0], D[0], L[0]);
-	if (LAP) l0 = fmaf(q[5], lap, l0);
+	float l0 = fmaf(m, D[0], L[0]);
 	l0 = quad([](int s) { return 4 + s; }, l0);
 	l0 = oct([](int s) { return 10 + s; }, l0);
 	L[0] = l0;
 #pragma unroll
 	for (int a = 0; a < 3; a++) {
-		float la = fmaf(M[0], D[1 + a], L[1 + a]);
+		float la = fmaf(m, D[1 + a], L[1 + a]);
 		la = quad([a](int s) { return E3(a, T2[s].i[0], T2[s].i[1]); }, la);
 		la = oct([a](int s) { return E4(a, T3[s].i[0], T3[s].i[1], T3[s].i[2]); }, la);
 		L[1 + a] = la;
 	}
 #pragma unroll
-	for (int t = 0; t < 6; t++) {
+	for (int t = 0; t < 5; t++) {
 		const int a = T2[t].i[0], b = T2[t].i[1];
-		float lab = fmaf(M[0], D[4 + t], L[4 + t]);
+		float lab = fmaf(m, D[4 + t], L[4 + t]);
 		lab = quad([a, b](int s) { return E4(a, b, T2[s].i[0], T2[s].i[1]); }, lab);
 		L[4 + t] = lab;
 	}
 #pragma unroll
-	for (int s = 10; s < 35; s++) L[s] = fmaf(M[0], D[s], L[s]);
+	for (int s = 10; s < 35; s++)
+		if (kept(s)) L[s] = fmaf(m, D[s], L[s]);
 }
 
-// P2L: L += m D (reference gravity.cpp:92-121)
+// P2L: L += m D, kept components (reference gravity.cpp:92-121)
 __device__ __forceinline__ void p2l(float* L, float m, const float* D) {
 #pragma unroll
-	for (int s = 0; s < 35; s++) L[s] = fmaf(m, D[s], L[s]);
+	for (int s = 0; s < 35; s++)
+		if (kept(s)) L[s] = fmaf(m, D[s], L[s]);
 }
 
 // M2P: potential and acceleration at the sink (reference gravity.cpp:123-169).  The potential's

@@ -25,6 +25,7 @@
 #include "tg_gravity.h"
 #include "tg_solver.hpp"
 #include "tg_devmem.hpp"
+#include "tg_math.hpp"
 #include "tg_scan.hpp"
 
 namespace tg {
@@ -560,7 +561,7 @@ __global__ __launch_bounds__(256) void k_tw_parts(const int32_t* __restrict__ po
 // per node: source multipole, centre, level, parent; flags of the non-empty leaves and their
 // root-path lengths, and of every leaf, empty ones included
 __global__ __launch_bounds__(256) void k_tw_nodes(const DNode* __restrict__ nodes, const DMulti* __restrict__ multi, int64_t nn,
-		MultiSrc* __restrict__ multis, int4* __restrict__ npos, int* __restrict__ level, int* __restrict__ parent, int64_t* __restrict__ lflag,
+		MultiSrc* __restrict__ multis, FoldedMulti* __restrict__ folded, int4* __restrict__ npos, int* __restrict__ level, int* __restrict__ parent, int64_t* __restrict__ lflag,
 		int64_t* __restrict__ plen, int64_t* __restrict__ leaves) {
 	const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
 	if (i >= nn) return;
@@ -570,6 +571,12 @@ __global__ __launch_bounds__(256) void k_tw_nodes(const DNode* __restrict__ node
 	for (int q = 0; q < 17; q++) ms.m[q] = m.m[q];
 	for (int d = 0; d < 3; d++) ms.x[d] = m.x[d];
 	multis[i] = ms;
+	FoldedMulti f;
+	float qzz;
+	f.m = ms.m[0];
+	fold_multi(ms.m, f.q, f.o, qzz);
+	for (int d = 0; d < 3; d++) f.x[d] = ms.x[d];
+	folded[i] = f;
 	npos[i] = make_int4(m.x[0], m.x[1], m.x[2], 0);
 	level[i] = nd.level;
 	parent[i] = nd.parent;
@@ -622,6 +629,7 @@ int Solver::upload_tree_device() {
 	}
 	PCHK(d_parts.alloc(std::max<size_t>(size_t(n) * sizeof(int4), 16)));
 	PCHK(d_multis.alloc(std::max<size_t>(size_t(nn) * sizeof(MultiSrc), 16)));
+	PCHK(d_folded.alloc(std::max<size_t>(size_t(nn) * sizeof(FoldedMulti), 16)));
 	PCHK(d_nodepos.alloc(std::max<size_t>(size_t(nn) * sizeof(int4), 16)));
 	PCHK(d_level.alloc(std::max<size_t>(size_t(nn) * 4, 16)));
 	PCHK(d_parent.alloc(std::max<size_t>(size_t(nn) * 4, 16)));
@@ -642,7 +650,7 @@ int Solver::upload_tree_device() {
 	order_on_device = true;
 	int64_t tot[3] = {0, 0, 0};
 	if (nn > 0) {
-		hipLaunchKernelGGL(k_tw_nodes, dim3(blocks(nn, 256)), dim3(256), 0, s, D.nodes, D.multi, nn, d_multis.as<MultiSrc>(), d_nodepos.as<int4>(),
+		hipLaunchKernelGGL(k_tw_nodes, dim3(blocks(nn, 256)), dim3(256), 0, s, D.nodes, D.multi, nn, d_multis.as<MultiSrc>(), d_folded.as<FoldedMulti>(), d_nodepos.as<int4>(),
 				d_level.as<int>(), d_parent.as<int>(), flag, plen, lall);
 		PCHK(hipGetLastError());
 		ScanSet sc;

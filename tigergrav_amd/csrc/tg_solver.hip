@@ -45,17 +45,51 @@ void DeviceArray::release() {
 
 // ---- kernels ---------------------------------------------------------------------------------
 // Each node's own CC/CP contribution: the sum of its partial slots in slot order (the
-// reference adds each list's accumulator into the node's L, src/tree.cpp:400-401,481-491).
-// One thread per (node, coefficient); consecutive threads read consecutive doubles.
+// reference adds each list's accumulator into the node's L, src/tree.cpp:400-401,481-491), its 35
+// components from the 26 sums.  Half a wave per node, each four nodes at a time, 32 nodes a group: two
+// dependent loads a node and 258 MB at 529,000 nodes, so bound by memory with enough of them under way.
+constexpr int NODES_PER_SUM = 32;
 __global__ __launch_bounds__(256) void k_node_sum(const int64_t* __restrict__ slot_ptr,
 		const double* __restrict__ partial, double* __restrict__ dL, int64_t nn) {
-	const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
-	if (i >= nn * 35) return;
-	const int64_t a = i / 35;
-	const int q = int(i - 35 * a);
-	double acc = 0.0;
-	for (int64_t z = slot_ptr[a]; z < slot_ptr[a + 1]; z++) acc += partial[35 * z + q];
-	dL[i] = acc;
+	__shared__ double sums[NODES_PER_SUM][NODE_SUMS];
+	const int64_t a0 = int64_t(blockIdx.x) * NODES_PER_SUM;
+	const int h = int(threadIdx.x) >> 5, c = int(threadIdx.x) & 31;
+	int64_t b[4], e[4];
+	double acc[4];
+#pragma unroll
+	for (int u = 0; u < 4; u++) {
+		const int64_t a = a0 + h + 8 * u;
+		b[u] = a < nn ? slot_ptr[a] : 0;
+		e[u] = a < nn ? slot_ptr[a + 1] : 0;
+	}
+	if (c < NODE_SUMS) {
+		// the first slot of each, most often the only one
+#pragma unroll
+		for (int u = 0; u < 4; u++) acc[u] = b[u] < e[u] ? partial[NODE_SUMS * b[u] + c] : 0.0;
+#pragma unroll
+		for (int u = 0; u < 4; u++) {
+			for (int64_t z = b[u] + 1; z < e[u]; z++) acc[u] += partial[NODE_SUMS * z + c];
+			sums[h + 8 * u][c] = acc[u];
+		}
+	}
+	__syncthreads();
+	// (node_component, without its branches) kept components by the lanes that hold them, the ten that
+	// follow by lanes 0..9: minus two sums, plus the trace for zz; zzzz from xxzz and yyzz
+	constexpr int8_t FIRST[10] = {4, 9, 10, 11, 16, 17, 18, 19, 20, 16}, SECOND[10] = {7, 12, 14, 15, 19, 21, 22, 23, 24, 23};
+	constexpr int8_t TO[10] = {9, 15, 18, 19, 25, 28, 29, 32, 33, 34};
+	const int q = c < 9 ? c : c < 14 ? c + 1 : c < 16 ? c + 2 : c < 21 ? c + 4 : c < 23 ? c + 5 : c + 7;
+	const int f = c < 10 ? FIRST[c] : 0, g = c < 10 ? SECOND[c] : 0, to = c < 10 ? TO[c] : 0;
+#pragma unroll
+	for (int u = 0; u < 4; u++) {
+		const int64_t a = a0 + h + 8 * u;
+		if (a >= nn) continue;
+		const double* m = sums[h + 8 * u];
+		if (c < 25) dL[35 * a + q] = acc[u];
+		if (c < 10) {
+			const double two = -m[f] - m[g];
+			dL[35 * a + to] = c == 0 ? m[25] + two : c == 9 ? (m[16] + m[19]) + (m[19] + m[23]) : two;
+		}
+	}
 }
 
 // The local-expansion pass, LPG leaves per block of 64 (64 / LPG lanes each).  The shift of a
@@ -289,6 +323,7 @@ Solver::~Solver() {
 			if (e) hipEventDestroy(e);
 		d_parts.release();
 		d_multis.release();
+		d_folded.release();
 		d_nodepos.release();
 		d_out.release();
 		d_partial.release();
@@ -485,6 +520,7 @@ int Solver::upload_sources() {
 	}
 	SCHK(put(d_parts, parts, stream));
 	SCHK(put(d_multis, multis, stream));
+	SCHK(launch_fold_multis(d_multis.as<MultiSrc>(), nn, d_folded.as<FoldedMulti>(), stream));
 	SCHK(hipStreamSynchronize(stream));
 	return TG_OK;
 }
@@ -551,7 +587,7 @@ int Solver::upload() {
 		t_detail[4] = now() - tp0;  // preparation: the tree's arrays and the list work
 		t_detail[5] = 0.0;          // no transfers
 		(void) tp1;
-		SCHK(d_partial.alloc(std::max<size_t>(n_slots * 35 * sizeof(double), 16)));
+		SCHK(d_partial.alloc(std::max<size_t>(n_slots * NODE_SUMS * sizeof(double), 16)));
 		SCHK(d_dL.alloc(std::max<size_t>(size_t(n_nodes) * 35 * sizeof(double), 16)));
 		SCHK(d_out.alloc(std::max<size_t>(n * 4 * sizeof(double), 16)));
 		SCHK(hipStreamSynchronize(stream));
@@ -597,6 +633,8 @@ int Solver::upload() {
 	hipStream_t s = stream;
 	SCHK(put(d_parts, parts, s));
 	SCHK(put(d_multis, multis, s));
+	SCHK(d_folded.alloc(std::max<size_t>(multis.size() * sizeof(FoldedMulti), 16)));
+	SCHK(launch_fold_multis(d_multis.as<MultiSrc>(), int64_t(multis.size()), d_folded.as<FoldedMulti>(), s));
 	SCHK(put(d_nodepos, npos, s));
 	SCHK(put(d_leaf_items, leaf_items, s));
 	adj_lists_ready = false;
@@ -629,7 +667,7 @@ int Solver::upload() {
 		if (rc != TG_OK) return rc;
 		t_detail[5] = tp1 - tp0 - t_detail[4];  // transfers: the tree's arrays
 		t_detail[4] += now() - tp1;            // preparation: the tree's arrays (host), the list work (device)
-		SCHK(d_partial.alloc(std::max<size_t>(n_slots * 35 * sizeof(double), 16)));
+		SCHK(d_partial.alloc(std::max<size_t>(n_slots * NODE_SUMS * sizeof(double), 16)));
 		SCHK(d_dL.alloc(std::max<size_t>(T.nodes.size() * 35 * sizeof(double), 16)));
 		SCHK(d_out.alloc(std::max<size_t>(n * 4 * sizeof(double), 16)));
 		SCHK(hipStreamSynchronize(s));
@@ -686,7 +724,7 @@ int Solver::upload() {
 	t_detail[5] = now() - tp0 - t_detail[4];
 	if (rc != TG_OK) return rc;
 	SCHK(es);
-	SCHK(d_partial.alloc(std::max<size_t>(n_slots * 35 * sizeof(double), 16)));
+	SCHK(d_partial.alloc(std::max<size_t>(n_slots * NODE_SUMS * sizeof(double), 16)));
 	SCHK(d_dL.alloc(std::max<size_t>(T.nodes.size() * 35 * sizeof(double), 16)));
 	SCHK(d_out.alloc(std::max<size_t>(n * 4 * sizeof(double), 16)));
 	SCHK(hipStreamSynchronize(s));
@@ -728,6 +766,7 @@ int Solver::enqueue_solve(bool timed) {
 	na.sinkpos = d_nodepos.as<int4>();
 	na.srcs = d_parts.as<int4>();
 	na.multis = d_multis.as<MultiSrc>();
+	na.folded = d_folded.as<FoldedMulti>();
 	na.partial = d_partial.as<double>();
 	na.slot_node = d_slot_node.as<int>();
 	na.wrap = ewald;
@@ -753,7 +792,7 @@ int Solver::enqueue_solve(bool timed) {
 	SCHK(mark(e));
 	const bool local_pass = nn > 0 && n_leaf_items > 0;
 	if (local_pass) {
-		hipLaunchKernelGGL(k_node_sum, dim3(unsigned((nn * 35 + 255) / 256)), dim3(256), 0, sn,
+		hipLaunchKernelGGL(k_node_sum, dim3(unsigned((nn + NODES_PER_SUM - 1) / NODES_PER_SUM)), dim3(256), 0, sn,
 				d_node_slot_ptr.as<int64_t>(), d_partial.as<double>(), d_dL.as<double>(), nn);
 		SCHK(hipGetLastError());
 		if (local_sweep)

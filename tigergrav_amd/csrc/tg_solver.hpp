@@ -64,6 +64,7 @@ struct Solver {
 	Tree tree;
 	int64_t n = 0;
 	// device state
+	DeviceArray d_folded;  // d_multis as CC direct takes them
 	DeviceArray d_parts, d_multis, d_nodepos, d_out, d_partial, d_node_slot_ptr;
 	DeviceArray d_leaf_items, d_slot_node, d_path, d_level, d_dL, d_queue;
 	DeviceArray d_parent, d_pleaf, d_Lnode;  // level-by-level local pass: parents, particle -> leaf, node expansions
