@@ -67,7 +67,8 @@ int tg_solver_solve(tg_solver* s);
  * queue-driven kernel; "node_chunk" 1..4096 (4096: a whole list) sources per CC/CP partial slot (applies from the next
  * tg_solver_set_particles; unset: 256 for up to 131,072 particles, else 4096); "resident" work groups of the persistent form; "local_sweep" 1 runs the
  * local-expansion pass level by level (the reference's order, src/tree.cpp:400-401) instead of
- * per-leaf sums over the root path (0, the default); "gpu_walk" 1 (the default
+ * per-leaf sums over the root path (0, the default; tg_solver_solve_graph enqueues the former
+ * without a graph); "gpu_walk" 1 (the default
  * for device solvers) builds the interaction lists on the device, 0 on the host (the same lists
  * either way: the walk of kick_fmm, src/tree.cpp:378-635; from the next tg_solver_set_particles);
  * with the lists on the device, the work of every kind is built from them there and the host
