@@ -2,8 +2,8 @@
 and multipoles) with lists cut into slots of 1 to 65 entries, so that a wave holds one segment, two,
 an odd number and 64 of them, and segments longer than a wave, against the whole lists.  Slots only
 regroup FP64 sums of float terms: forces agree to a few float roundings (1e-6 RMS, the bound the
-slots' own test takes); and the per-call CC and CP kinds' 35 components against the FP64 kernels: the
-ten components that follow from the trace carry the errors of two or three others."""
+slots' own test takes); and the per-call CC and CP kinds, which sum all 35 components, against the
+FP64 kernels."""
 import numpy as np
 import pytest
 

@@ -193,7 +193,7 @@ int node_call(const tg_params* p, double* L, const int32_t* x, const void* y, in
 	T->hsinks.assign(1, pack(x, 0.0f));
 	HIPCHK(T->sinks.ensure(sizeof(int4)));
 	HIPCHK(T->items.ensure(nitems * sizeof(int2)));
-	HIPCHK(T->out.ensure(nitems * tg::NODE_SUMS * sizeof(double)));
+	HIPCHK(T->out.ensure(nitems * 35 * sizeof(double)));
 	hipStream_t s = T->stream;
 	HIPCHK(hipMemcpyAsync(T->sinks.p, T->hsinks.data(), sizeof(int4), hipMemcpyHostToDevice, s));
 	HIPCHK(hipMemcpyAsync(T->items.p, T->hwaves.data(), nitems * sizeof(int2), hipMemcpyHostToDevice, s));
@@ -224,13 +224,14 @@ int node_call(const tg_params* p, double* L, const int32_t* x, const void* y, in
 		case tg::CP_DIRECT: HIPCHK(tg::launch_cp(a, false, s)); break;
 		case tg::CP_EWALD: HIPCHK(tg::launch_cp(a, true, s)); break;
 	}
-	T->hout.resize(nitems * tg::NODE_SUMS);
-	HIPCHK(hipMemcpyAsync(T->hout.data(), T->out.p, nitems * tg::NODE_SUMS * sizeof(double), hipMemcpyDeviceToHost, s));
+	T->hout.resize(nitems * 35);
+	HIPCHK(hipMemcpyAsync(T->hout.data(), T->out.p, nitems * 35 * sizeof(double), hipMemcpyDeviceToHost, s));
 	HIPCHK(hipStreamSynchronize(s));
-	double sums[tg::NODE_SUMS] = {};
-	for (int64_t i = 0; i < nitems; i++)
-		for (int c = 0; c < tg::NODE_SUMS; c++) sums[c] += T->hout[tg::NODE_SUMS * i + c];
-	for (int c = 0; c < 35; c++) L[c] += tg::node_component(sums, c);
+	for (int c = 0; c < 35; c++) {
+		double acc = 0.0;
+		for (int64_t i = 0; i < nitems; i++) acc += T->hout[35 * i + c];
+		L[c] += acc;
+	}
 	return TG_OK;
 }
 

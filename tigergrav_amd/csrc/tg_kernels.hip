@@ -543,21 +543,26 @@ hipError_t launch_pp_ewald(const LeafArgs& a, hipStream_t s) {
 // Segmented FP64 reduction of the lanes' 25 float accumulators (26 with the trace) by owner slot,
 // through LDS.  The entries of one slot are consecutive: each half wave adds one coefficient a lane over
 // a segment of its own, or over half of a wave's only segment.
+// The plain drop-in's kinds (FULL: no owners, a slot per wave of at most 64 entries) return the
+// expansion itself and sum all 35 components: zz from the others carries their errors, up to twice its
+// own.
+template <bool FULL>
 struct NodeSums {
-	float red[NODE_SUMS][65];
+	float red[FULL ? 35 : NODE_SUMS][65];
 	int sl[64];
 };
+template <bool FULL>
 union NodeLds {  // the Ewald kinds' rows, then the sums
 	EwtStage<35> rows;
-	NodeSums sums;
+	NodeSums<FULL> sums;
 };
 union NodeFoldLds {  // the direct kind's multipoles, then the sums
 	ewt_f4 stage[256];
-	NodeSums sums;
+	NodeSums<false> sums;
 };
 
 template <bool TRACE>
-__device__ __forceinline__ void node_segment_store(const float* L, float trace, int slot, int cnt, NodeSums& S, double* partial) {
+__device__ __forceinline__ void node_segment_store(const float* L, float trace, int slot, int cnt, NodeSums<false>& S, double* partial) {
 	float (*red)[65] = S.red;
 	int* sl = S.sl;
 	const int lane = threadIdx.x;
@@ -606,6 +611,34 @@ __device__ __forceinline__ void node_segment_store(const float* L, float trace, 
 	}
 }
 
+__device__ __forceinline__ void node_full_store(const float* L, int slot, int cnt, NodeSums<true>& S, double* partial) {
+	const int lane = threadIdx.x;
+	__syncthreads();
+#pragma unroll
+	for (int c = 0; c < 35; c++) S.red[c][lane] = L[c];
+	__syncthreads();
+	if (lane < 35) {
+		double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
+		int j = 0;
+		for (; j + 4 <= cnt; j += 4) {
+			a0 += double(S.red[lane][j]);
+			a1 += double(S.red[lane][j + 1]);
+			a2 += double(S.red[lane][j + 2]);
+			a3 += double(S.red[lane][j + 3]);
+		}
+		for (; j < cnt; j++) a0 += double(S.red[lane][j]);
+		partial[35 * (size_t) blockIdx.x + lane] = (a0 + a1) + (a2 + a3);
+	}
+}
+
+template <bool FULL, bool TRACE>
+__device__ __forceinline__ void node_store(const float* L, float trace, int slot, int cnt, NodeSums<FULL>& S, double* partial) {
+	if constexpr (FULL)
+		node_full_store(L, slot, cnt, S, partial);
+	else
+		node_segment_store<TRACE>(L, trace, slot, cnt, S, partial);
+}
+
 __device__ __forceinline__ void multi_floats(float* v, const float4* m) {
 #pragma unroll
 	for (int q = 0; q < 5; q++) {
@@ -621,7 +654,7 @@ __device__ __forceinline__ void multi_floats(float* v, const float4* m) {
 // 64 apart, each adding its entries' terms in order before the store.
 template <bool WRAP>
 __global__ __launch_bounds__(64) void k_cc(NodeArgs A) {
-	__shared__ NodeSums sums;
+	__shared__ NodeSums<true> sums;
 	const int2 wv = A.waves[blockIdx.x];
 	const int lane = threadIdx.x;
 	float L[35];
@@ -643,10 +676,10 @@ __global__ __launch_bounds__(64) void k_cc(NodeArgs A) {
 					sepu<WRAP>(X.z, __float_as_int(v[19])) * POS_INVF};
 			green_direct(D, x);
 			fold_multi(v, q, o, qzz);
-			m2l(L, v[0], q, o, D);
+			m2l<true>(L, v[0], q, o, D);
 		}
 	}
-	node_segment_store<false>(L, 0.0f, slot, min(wv.y - wv.x, 64), sums, A.partial);
+	node_store<true, false>(L, 0.0f, slot, min(wv.y - wv.x, 64), sums, A.partial);
 }
 
 // The same from a solver's folded multipoles, which the wave reads together: four lanes take a record,
@@ -715,7 +748,7 @@ __global__ __launch_bounds__(64) void k_cc_folded(NodeArgs A) {
 #pragma unroll
 				for (int c = 0; c < 13; c++) v[c] = 0.0f;
 			}
-			m2l(L, v[0], v + 1, v + 6, D);
+			m2l<false>(L, v[0], v + 1, v + 6, D);
 		}
 	}
 #undef TG_CC_INDICES
@@ -726,10 +759,11 @@ __global__ __launch_bounds__(64) void k_cc_folded(NodeArgs A) {
 // The Ewald correction of the same: the whole wave takes every turn (its table rows are read
 // together), lanes past the end with the last entry and no weight.  Bound by arithmetic (about 700
 // instructions an entry, 900 before) and by the rows' way through the vector cache and LDS, 16 KB a
-// turn, at three waves a SIMD (two waves with the next turn's rows in flight took 1.16 ms where this
-// takes 1.03: 2M particles at theta 0.3, 3.6e7 entries).
+// turn, at three waves a SIMD: 0.82 ms for 3.6e7 entries (2M particles at theta 0.3), 1.03 with a row per
+// lane and 35 sums; two waves with the next turn's rows in flight took an eighth longer.
+template <bool FULL>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_cc_ewald(NodeArgs A) {
-	__shared__ NodeLds lds;
+	__shared__ NodeLds<FULL> lds;
 	const int2 wv = A.waves[blockIdx.x];
 	const int lane = threadIdx.x;
 	float L[35];
@@ -760,16 +794,16 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
 		}
 		float q[5], o[7], qzz;
 		fold_multi(v, q, o, qzz);
-		m2l(L, v[0], q, o, D);
+		m2l<FULL>(L, v[0], q, o, D);
 		L[0] = fmaf(qzz, lap, L[0]);
 		trace = fmaf(v[0], lap, trace);
 	}
-	node_segment_store<true>(L, trace, slot, min(wv.y - wv.x, 64), lds.sums, A.partial);
+	node_store<FULL, true>(L, trace, slot, min(wv.y - wv.x, 64), lds.sums, A.partial);
 }
 
-template <bool WRAP>
+template <bool FULL, bool WRAP>
 __global__ __launch_bounds__(64) void k_cp(NodeArgs A) {
-	__shared__ NodeSums sums;
+	__shared__ NodeSums<FULL> sums;
 	const int2 wv = A.waves[blockIdx.x];
 	const int lane = threadIdx.x;
 	float L[35];
@@ -785,14 +819,15 @@ __global__ __launch_bounds__(64) void k_cp(NodeArgs A) {
 			const float x[3] = {sepu<WRAP>(X.x, s.x) * POS_INVF, sepu<WRAP>(X.y, s.y) * POS_INVF, sepu<WRAP>(X.z, s.z) * POS_INVF};
 			float D[35];
 			green_direct(D, x);
-			p2l(L, __int_as_float(s.w), D);
+			p2l<FULL>(L, __int_as_float(s.w), D);
 		}
 	}
-	node_segment_store<false>(L, 0.0f, slot, min(wv.y - wv.x, 64), sums, A.partial);
+	node_store<FULL, false>(L, 0.0f, slot, min(wv.y - wv.x, 64), sums, A.partial);
 }
 
+template <bool FULL>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_cp_ewald(NodeArgs A) {
-	__shared__ NodeLds lds;
+	__shared__ NodeLds<FULL> lds;
 	const int2 wv = A.waves[blockIdx.x];
 	const int lane = threadIdx.x;
 	float L[35];
@@ -812,17 +847,19 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
 		float D[35];
 		const float lap = green_ewald_wave<35>(D, x, c_ewt, lds.rows, lane);
 		const float m = j0 + lane < wv.y ? __int_as_float(s.w) : 0.0f;
-		p2l(L, m, D);
+		p2l<FULL>(L, m, D);
 		trace = fmaf(m, lap, trace);
 	}
-	node_segment_store<true>(L, trace, slot, min(wv.y - wv.x, 64), lds.sums, A.partial);
+	node_store<FULL, true>(L, trace, slot, min(wv.y - wv.x, 64), lds.sums, A.partial);
 }
 
 hipError_t launch_cc(const NodeArgs& a, bool ewald, hipStream_t s) {
 	if (a.nwaves <= 0) return hipSuccess;
 	const dim3 g(a.nwaves), b(64);
-	if (ewald)
-		hipLaunchKernelGGL(k_cc_ewald, g, b, 0, s, a);
+	if (ewald && a.owner)
+		hipLaunchKernelGGL(k_cc_ewald<false>, g, b, 0, s, a);
+	else if (ewald)
+		hipLaunchKernelGGL(k_cc_ewald<true>, g, b, 0, s, a);
 	else if (a.folded && a.wrap)
 		hipLaunchKernelGGL(k_cc_folded<true>, g, b, 0, s, a);
 	else if (a.folded)
@@ -852,14 +889,23 @@ hipError_t launch_fold_multis(const MultiSrc* multis, int64_t nn, FoldedMulti* o
 	return hipGetLastError();
 }
 
+template <bool FULL>
+static void cp_launch(const NodeArgs& a, bool ewald, hipStream_t s) {
+	const dim3 g(a.nwaves), b(64);
+	if (ewald)
+		hipLaunchKernelGGL(k_cp_ewald<FULL>, g, b, 0, s, a);
+	else if (a.wrap)
+		hipLaunchKernelGGL((k_cp<FULL, true>), g, b, 0, s, a);
+	else
+		hipLaunchKernelGGL((k_cp<FULL, false>), g, b, 0, s, a);
+}
+
 hipError_t launch_cp(const NodeArgs& a, bool ewald, hipStream_t s) {
 	if (a.nwaves <= 0) return hipSuccess;
-	if (ewald)
-		hipLaunchKernelGGL(k_cp_ewald, dim3(a.nwaves), dim3(64), 0, s, a);
-	else if (a.wrap)
-		hipLaunchKernelGGL(k_cp<true>, dim3(a.nwaves), dim3(64), 0, s, a);
+	if (a.owner)
+		cp_launch<false>(a, ewald, s);
 	else
-		hipLaunchKernelGGL(k_cp<false>, dim3(a.nwaves), dim3(64), 0, s, a);
+		cp_launch<true>(a, ewald, s);
 	return hipGetLastError();
 }
 

@@ -62,23 +62,6 @@ __host__ __device__ constexpr bool kept(int slot) {
 		if (KEPT[k] == slot) return true;
 	return false;
 }
-// component q of the expansion whose sums are c
-__host__ __device__ inline double node_component(const double* c, int q) {
-	switch (q) {
-		case 9: return c[25] - c[4] - c[7];        // zz
-		case 15: return -c[9] - c[12];             // xzz
-		case 18: return -c[10] - c[14];            // yzz
-		case 19: return -c[11] - c[15];            // zzz
-		case 25: return -c[16] - c[19];            // xxzz
-		case 28: return -c[17] - c[21];            // xyzz
-		case 29: return -c[18] - c[22];            // xzzz
-		case 32: return -c[19] - c[23];            // yyzz
-		case 33: return -c[20] - c[24];            // yzzz
-		case 34: return (c[16] + c[19]) + (c[19] + c[23]);  // zzzz
-		default: return c[q < 9 ? q : q < 15 ? q - 1 : q < 18 ? q - 2 : q < 25 ? q - 4 : q < 28 ? q - 5 : q - 7];
-	}
-}
-
 // A source multipole as M2L takes it: weights formed (multiplicities and 1/k!, the octupole's sign)
 // and the components with the third axis twice folded into the others by the trace relation, the
 // quadrupole in 5 terms and the octupole in 7.  64 bytes: half a line, where the plain 80 cross lines.
@@ -114,7 +97,7 @@ struct NodeArgs {
 	const int* list;         // source index per entry
 	const int* owner;        // partial slot per entry
 	const int* slot_node;    // expansion-centre index per slot
-	double* partial;         // NODE_SUMS doubles per slot
+	double* partial;         // NODE_SUMS doubles per slot; 35 without owners
 	int nwaves;
 	int wrap;
 };

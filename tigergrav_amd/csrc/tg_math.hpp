@@ -211,7 +211,8 @@ __device__ __forceinline__ void fold_multi(const float* M, float* q, float* o, f
 
 // M2L: L += contraction of a folded multipole with D, kept components (reference gravity.cpp:26-90).
 // Every term is added straight into L, in the reference's order of terms (as its loop adds each term
-// into its L).
+// into its L).  FULL: all 35 components.
+template <bool FULL>
 __device__ __forceinline__ void m2l(float* L, float m, const float* q, const float* o, const float* D) {
 	constexpr int OS[7] = {0, 1, 2, 3, 4, 6, 7};  // octupole slots
 	auto quad = [&](auto slot_of, float acc) {
@@ -236,7 +237,7 @@ __device__ __forceinline__ void m2l(float* L, float m, const float* q, const flo
 		L[1 + a] = la;
 	}
 #pragma unroll
-	for (int t = 0; t < 5; t++) {
+	for (int t = 0; t < (FULL ? 6 : 5); t++) {
 		const int a = T2[t].i[0], b = T2[t].i[1];
 		float lab = fmaf(m, D[4 + t], L[4 + t]);
 		lab = quad([a, b](int s) { return E4(a, b, T2[s].i[0], T2[s].i[1]); }, lab);
@@ -244,14 +245,15 @@ __device__ __forceinline__ void m2l(float* L, float m, const float* q, const flo
 	}
 #pragma unroll
 	for (int s = 10; s < 35; s++)
-		if (kept(s)) L[s] = fmaf(m, D[s], L[s]);
+		if (FULL || kept(s)) L[s] = fmaf(m, D[s], L[s]);
 }
 
 // P2L: L += m D, kept components (reference gravity.cpp:92-121)
+template <bool FULL>
 __device__ __forceinline__ void p2l(float* L, float m, const float* D) {
 #pragma unroll
 	for (int s = 0; s < 35; s++)
-		if (kept(s)) L[s] = fmaf(m, D[s], L[s]);
+		if (FULL || kept(s)) L[s] = fmaf(m, D[s], L[s]);
 }
 
 // M2P: potential and acceleration at the sink (reference gravity.cpp:123-169).  The potential's

@@ -73,8 +73,8 @@ __global__ __launch_bounds__(256) void k_node_sum(const int64_t* __restrict__ sl
 		}
 	}
 	__syncthreads();
-	// (node_component, without its branches) kept components by the lanes that hold them, the ten that
-	// follow by lanes 0..9: minus two sums, plus the trace for zz; zzzz from xxzz and yyzz
+	// kept components by the lanes that hold them, the ten that follow by lanes 0..9 (component TO from
+	// the sums FIRST and SECOND): minus both, plus the trace for zz; zzzz from xxzz and yyzz
 	constexpr int8_t FIRST[10] = {4, 9, 10, 11, 16, 17, 18, 19, 20, 16}, SECOND[10] = {7, 12, 14, 15, 19, 21, 22, 23, 24, 23};
 	constexpr int8_t TO[10] = {9, 15, 18, 19, 25, 28, 29, 32, 33, 34};
 	const int q = c < 9 ? c : c < 14 ? c + 1 : c < 16 ? c + 2 : c < 21 ? c + 4 : c < 23 ? c + 5 : c + 7;
