@@ -49,3 +49,31 @@ def test_fof_from_either_tree(n, leaf, link, kind, gpu_tree):
     assert ng == len(ids)
     assert [(c.id, c.N) for c in cat] == list(zip(ids.tolist(), counts.tolist()))
     assert np.array_equal(_groups(s, link)[0], g)  # with the tree on the host by now
+
+
+@pytest.mark.parametrize("gpu_tree", [1, 0])
+@pytest.mark.parametrize("n,leaf,link,move", [(2, 1, 0.3, 0.0), (3000, 16, 0.3, 0.5), (2000, 64, 0.2, 20.0), (1500, 1, 0.5, 2.0)])
+def test_fof_after_update(n, leaf, link, move, gpu_tree):
+    """Groups of particles moved under the kept tree (move: RMS displacement in mean spacings), out of
+    their leaves' boxes and across the box edge: ids and counts equal the oracle's on the moved positions."""
+    from tigergrav_amd.solver import Solver
+
+    print(f"fof after update: N={n} leaf={leaf} move={move} gpu_tree={gpu_tree}", flush=True)
+    if n == 2:  # two leaves with boxes far apart, then two particles side by side
+        x = np.array([[-2 ** 30, 0, 0], [2 ** 30, 0, 0]], np.int32)
+        y = np.array([[2 ** 28, 0, 0], [2 ** 30, 0, 0]], np.int32)
+    else:
+        x = _set(n, "cluster")
+        d = np.random.default_rng(n).standard_normal((n, 3)) * (move * n ** (-1.0 / 3.0) * 2.0 ** 32)
+        y = (x.astype(np.int64) + d.astype(np.int64)).astype(np.int32)  # wraps
+    s = Solver(ewald=True, soft_len=ics.soft_len(n), m=1.0 / n, theta=0.7, parts_per_node=leaf, device=0)
+    s.tune("gpu_tree", gpu_tree)
+    s.set_particles(x)
+    s.update_particles(y)
+    g, ng = _groups(s, link)
+    order = s.export("order")
+    want = ob.fof(y[order], ob.fof_link2(n, link))
+    assert np.array_equal(g[order], want)
+    ids, counts = np.unique(want[want != NONE], return_counts=True)
+    assert ng == len(ids) and ng > 0
+    assert [(c.id, c.N) for c in _catalog(s, np.zeros((n, 3), np.float32), 1.0, 2)] == list(zip(ids.tolist(), counts.tolist()))

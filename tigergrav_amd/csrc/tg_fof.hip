@@ -14,7 +14,8 @@
 //     integer test and unites the linked ones;
 //   * labels: the root of every linked particle, DEFAULT_GROUP for the rest, in tree and in input
 //     order.
-// The nodes come from the device build's tree where that is current, else from the host's; only the
+// The nodes come from the device build's tree where that is current, else from the host's, whose boxes are
+// then made anew from the particles (tg_solver_update_particles moves them under the tree); only the
 // labels in input order cross to the host (with set_particles at 2M clustered particles, leaves of 32:
 // 27.8 -> 8.7 ms; before, tree and order were copied, the nodes rebuilt and the labels permuted on
 // the host).
@@ -332,6 +333,8 @@ hipError_t fof_device(const FofSource& F, double link_len, hipStream_t s, uint64
 		hipLaunchKernelGGL(k_fof_nodes, dim3(unsigned((nn + 255) / 256)), dim3(256), 0, s, F.dtree->nodes, F.dtree->multi, nn, nodes);
 		FCHK(hipGetLastError());
 	} else {
+		// the boxes of the particles where they are: those of a tree kept under moved particles are stale
+		const std::vector<double> box = F.tree->particle_boxes();
 		hn.resize(static_cast<size_t>(nn));
 		for (int64_t i = 0; i < nn; i++) {
 			const Node& d = F.tree->nodes[size_t(i)];
@@ -341,8 +344,8 @@ hipError_t fof_device(const FofSource& F, double link_len, hipStream_t s, uint64
 			o.c0 = d.child[0];
 			o.c1 = d.child[1];
 			for (int k = 0; k < 3; k++) {
-				o.mn[k] = d.rmin[k];
-				o.mx[k] = d.rmax[k];
+				o.mn[k] = box[6 * size_t(i) + size_t(k)];
+				o.mx[k] = box[6 * size_t(i) + 3 + size_t(k)];
 			}
 		}
 		FCHK(hipMemcpyAsync(nodes, hn.data(), hn.size() * sizeof(FofNode), hipMemcpyHostToDevice, s));

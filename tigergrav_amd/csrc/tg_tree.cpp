@@ -402,10 +402,9 @@ static void walk_rec(Tree& T, const WalkCtx& W, int ni, std::vector<int32_t> dli
 // per node, the span of its particles' bounding box (src/tree.cpp:406, part_vect_range): leaves
 // from their particles, interior nodes as the union of their non-empty children's boxes (min and
 // max are exact, so this equals a scan of the node's particles)
-std::vector<float> Tree::sink_spans() const {
+std::vector<double> Tree::particle_boxes() const {
 	const size_t nn = nodes.size();
-	std::vector<double> mn(3 * nn, 1.0), mx(3 * nn, 0.0);
-	std::vector<float> span(nn, 0.0f);
+	std::vector<double> box(6 * nn);
 	// nodes are numbered level by level: levels from the deepest up, each level's nodes in parallel
 	std::vector<size_t> level_begin;
 	for (size_t i = 0; i < nn; i++)
@@ -416,27 +415,40 @@ std::vector<float> Tree::sink_spans() const {
 		for (int64_t ki = int64_t(level_begin[l]); ki < int64_t(level_begin[l + 1]); ki++) {
 			const size_t k = size_t(ki);
 			const Node& nd = nodes[k];
+			double *mn = &box[6 * k], *mx = mn + 3;
+			for (int d = 0; d < 3; d++) {
+				mn[d] = 1.0;
+				mx[d] = 0.0;
+			}
 			if (nd.empty()) continue;
 			if (nd.leaf()) {
 				for (int64_t i = nd.pbegin; i < nd.pend; i++)
 					for (int d = 0; d < 3; d++) {
 						const double x = pos_to_double(pos[3 * i + d]);
-						mx[3 * k + d] = std::max(mx[3 * k + d], x);
-						mn[3 * k + d] = std::min(mn[3 * k + d], x);
+						mx[d] = std::max(mx[d], x);
+						mn[d] = std::min(mn[d], x);
 					}
 			} else {
 				for (int c = 0; c < 2; c++) {
 					const size_t ch = size_t(nd.child[c]);
 					if (nodes[ch].empty()) continue;
 					for (int d = 0; d < 3; d++) {
-						mx[3 * k + d] = std::max(mx[3 * k + d], mx[3 * ch + d]);
-						mn[3 * k + d] = std::min(mn[3 * k + d], mn[3 * ch + d]);
+						mx[d] = std::max(mx[d], box[6 * ch + 3 + d]);
+						mn[d] = std::min(mn[d], box[6 * ch + d]);
 					}
 				}
 			}
-			span[k] = float(range_max_span(&mn[3 * k], &mx[3 * k]));
 		}
 	}
+	return box;
+}
+
+std::vector<float> Tree::sink_spans() const {
+	const std::vector<double> box = particle_boxes();
+	std::vector<float> span(nodes.size(), 0.0f);
+#pragma omp parallel for schedule(static)
+	for (int64_t k = 0; k < int64_t(nodes.size()); k++)
+		if (!nodes[size_t(k)].empty()) span[size_t(k)] = float(range_max_span(&box[6 * size_t(k)], &box[6 * size_t(k) + 3]));
 	return span;
 }
 

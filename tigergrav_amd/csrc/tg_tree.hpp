@@ -114,6 +114,10 @@ public:
 	void update_moments(const int32_t* pos_tree, const float* mass_tree);
 	// dual-tree walk from the root with the reference's MAC; fills `lists` and `census`
 	void walk();
+	// per node the bounding box of its particles where they are now (lowest, highest coordinates): a leaf's
+	// own, the union of its non-empty children's above.  rmin and rmax are the build's, also after
+	// update_moments
+	std::vector<double> particle_boxes() const;
 	// per node, the span of its particles' bounding box (the walk's sink rmax)
 	std::vector<float> sink_spans() const;
 	// the interaction census of `lists`
