@@ -106,7 +106,8 @@ int tg_solver_info(tg_solver* s, tg_solve_info* info);
  * "slot_node", "slot_ptr" (each slot's node; each node's first slot), and the tree arrays the
  * solve reads: "solve_parts" (int4 x, y, z, mass bits), "solve_multis", "solve_nodepos",
  * "solve_level", "solve_parent", "solve_leaf_items" (node, first particle, end, path offset),
- * "solve_path", "solve_pleaf" (each particle's leaf), "solve_order").  Returns the size in bytes;
+ * "solve_path", "solve_pleaf" (each particle's leaf), "solve_order"); and the last solve's
+ * "solve_expansions" (per node 35 doubles: the sum of its own CC and CP lists).  Returns the size in bytes;
  * dst may be NULL to query it. */
 int64_t tg_solver_export(tg_solver* s, const char* name, void* dst, int64_t capacity);
 const char* tg_solver_last_error(void);

@@ -1,9 +1,9 @@
-"""The node kinds' 26 sums and folded multipoles: a solver's node expansions (direct and Ewald, particles
-and multipoles) with lists cut into slots of 1 to 65 entries, so that a wave holds one segment, two,
-an odd number and 64 of them, and segments longer than a wave, against the whole lists.  Slots only
+"""The node kinds' segment sums and folded multipoles: a solver's node expansions (direct and Ewald,
+particles and multipoles) with lists cut into slots of 1 to 65 entries, so that a wave holds one segment,
+two, an odd number and 64 of them, and segments longer than a wave, against the whole lists.  Slots only
 regroup FP64 sums of float terms: forces agree to a few float roundings (1e-6 RMS, the bound the
-slots' own test takes); and the per-call CC and CP kinds, which sum all 35 components, against the
-FP64 kernels."""
+slots' own test takes); the per-call CC and CP kinds against the FP64 kernels; and the solver's node
+expansions against the per-call kinds."""
 import numpy as np
 import pytest
 
@@ -48,3 +48,41 @@ def test_components(kind, nj):
     ref = ob.call_kernel("tgo64_", kind, P, x, y)[0]
     for lo, hi in ((0, 1), (1, 4), (4, 10), (10, 20), (20, 35)):
         assert np.abs(L[lo:hi] - ref[lo:hi]).max() < 1e-5 * np.abs(ref[lo:hi]).max()
+
+
+@pytest.mark.parametrize("n,theta,leaf,ewald", [(1500, 0.5, 16, True), (1500, 0.6, 16, False), (400, 0.4, 4, True)])
+def test_expansions(n, theta, leaf, ewald):
+    """Every component of orders 2..4 of a node's expansion is the per-call kinds' sum of the same float
+    terms (one per entry, slots of 64): they differ by the order of FP64 additions, 1e-12 for the few
+    thousand terms of a node, where a component taken from others differs by float roundings, 1e-7."""
+    from tigergrav_amd import gravity as tg
+    from tigergrav_amd import ics
+    from tigergrav_amd._lib import MULTI_DTYPE
+    from tigergrav_amd.solver import Solver
+
+    x = ics.plummer_spheres(n, n) if not ewald else ics.uniform(n, n)
+    print(f"expansions n={n} theta={theta} ewald={ewald}", flush=True)
+    m, h = 1.0 / n, ics.soft_len(n)
+    s = Solver(ewald=ewald, soft_len=h, m=m, theta=theta, parts_per_node=leaf, device=0)
+    s.tune("node_chunk", 64)
+    s.set_particles(x)
+    s.solve()
+    s.synchronize()
+    got = s.export("solve_expansions")
+    T = s.tree_arrays()
+    multi = np.zeros(len(T["node_x"]), MULTI_DTYPE)
+    multi["m"], multi["x"] = T["node_m"], T["node_x"]
+    opts = tg.Options(ewald=ewald, soft_len=h, m=m, device=0)
+    entries = 0
+    for a in range(len(multi)):
+        L = np.zeros(35)
+        for name, kind in (("cc_d", "CC_direct"), ("cp_d", "CP_direct"), ("cc_e", "CC_ewald"), ("cp_e", "CP_ewald")):
+            v = T[name][T[name + "_ptr"][a]:T[name + "_ptr"][a + 1]]
+            if name[1] == "p" and len(v):
+                v = np.concatenate([np.arange(b, e) for b, e in v.reshape(-1, 2)])
+            if len(v):
+                tg.KERNELS[kind](L, T["node_x"][a], multi[v] if name[1] == "c" else T["pos"][v], opts=opts)
+            entries += len(v)
+        for lo, hi in ((4, 10), (10, 20), (20, 35)):
+            assert np.abs(got[a, lo:hi] - L[lo:hi]).max() <= 1e-11 * np.abs(L[lo:hi]).max(), (a, lo)
+    assert entries > n  # the lists are not empty

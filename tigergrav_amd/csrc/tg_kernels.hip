@@ -8,7 +8,7 @@
 //    float, the running sum FP64 (the reference accumulates float terms in FP64 lanes,
 //    src/gravity.cpp:259-261), and phases are merged with cross-lane FP64 shuffles.
 //  * node kinds (CC, CP): lane = source; a wave packs the short lists of several expansion
-//    centres (<= 64 entries), 25 float accumulators per lane, merged per centre in FP64 through
+//    centres (<= 64 entries), 35 float accumulators per lane, merged per centre in FP64 through
 //    LDS by a segmented scan.
 //  * Ewald kinds use tg::ewt_eval (tg_math.hpp).
 #include "tg_kernels.hpp"
@@ -540,103 +540,52 @@ hipError_t launch_pp_ewald(const LeafArgs& a, hipStream_t s) {
 }
 
 // ---- node kinds ----------------------------------------------------------------------------------
-// Segmented FP64 reduction of the lanes' 25 float accumulators (26 with the trace) by owner slot,
-// through LDS.  The entries of one slot are consecutive: each half wave adds one coefficient a lane over
-// a segment of its own, or over half of a wave's only segment.
-// The plain drop-in's kinds (FULL: no owners, a slot per wave of at most 64 entries) return the
-// expansion itself and sum all 35 components: zz from the others carries their errors, up to twice its
-// own.
-template <bool FULL>
+// Segmented FP64 reduction of the lanes' 35 float accumulators by owner slot, through LDS.  The entries
+// of one slot are consecutive: lanes 0..34 add one coefficient each over every segment.
+// All 35 components are summed, though the tensor's trace is known (zero for derivatives of 1/r, a
+// constant for the periodic correction): one taken from two others carries their errors, up to 1.8
+// times its own against FP64.  Ten sums fewer took 0.1 ms off the 4.2 ms solve of 2M particles at
+// theta 0.3.
 struct NodeSums {
-	float red[FULL ? 35 : NODE_SUMS][65];
+	float red[35][65];
 	int sl[64];
 };
-template <bool FULL>
 union NodeLds {  // the Ewald kinds' rows, then the sums
 	EwtStage<35> rows;
-	NodeSums<FULL> sums;
+	NodeSums sums;
 };
 union NodeFoldLds {  // the direct kind's multipoles, then the sums
 	ewt_f4 stage[256];
-	NodeSums<false> sums;
+	NodeSums sums;
 };
 
-template <bool TRACE>
-__device__ __forceinline__ void node_segment_store(const float* L, float trace, int slot, int cnt, NodeSums<false>& S, double* partial) {
-	float (*red)[65] = S.red;
-	int* sl = S.sl;
-	const int lane = threadIdx.x;
-	__syncthreads();
-	static_for<25>([&](auto k_) { red[decltype(k_)::value][lane] = L[KEPT[decltype(k_)::value]]; });
-	if (TRACE) red[25][lane] = trace;
-	sl[lane] = slot;
-	__syncthreads();
-	// the wave's segments (runs of one slot) from a ballot of their first entries, two at a time
-	const bool first = lane < cnt && (lane == 0 || sl[lane] != sl[lane - 1]);
-	unsigned long long starts = __ballot(first);
-	const bool single = __popcll(starts) == 1;
-	const int c = lane & 31;
-	const bool high = lane >= 32;
-	while (starts) {
-		int b = __ffsll(starts) - 1;
-		starts &= starts - 1;
-		int e = starts ? __ffsll(starts) - 1 : cnt;
-		int b1 = e, e1 = e;  // the second segment
-		if (single) {
-			b1 = b + ((e - b + 1) >> 1);
-			e = b1;
-		} else if (starts) {
-			starts &= starts - 1;
-			e1 = starts ? __ffsll(starts) - 1 : cnt;
-		}
-		if (high) {
-			b = b1;
-			e = e1;
-		}
-		double acc = 0.0;
-		if (c < (TRACE ? 26 : 25)) {
-			double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-			int j = b;
-			for (; j + 4 <= e; j += 4) {
-				a0 += double(red[c][j]);
-				a1 += double(red[c][j + 1]);
-				a2 += double(red[c][j + 2]);
-				a3 += double(red[c][j + 3]);
-			}
-			for (; j < e; j++) a0 += double(red[c][j]);
-			acc = (a0 + a1) + (a2 + a3);
-		}
-		if (single) acc += __shfl_xor(acc, 32, 64);
-		if (c < NODE_SUMS && b < e && !(single && high)) partial[NODE_SUMS * (size_t) sl[b] + c] = acc;
-	}
-}
-
-__device__ __forceinline__ void node_full_store(const float* L, int slot, int cnt, NodeSums<true>& S, double* partial) {
+__device__ __forceinline__ void node_store(const float* L, int slot, int cnt, NodeSums& S, double* partial) {
 	const int lane = threadIdx.x;
 	__syncthreads();
 #pragma unroll
 	for (int c = 0; c < 35; c++) S.red[c][lane] = L[c];
+	S.sl[lane] = slot;
 	__syncthreads();
-	if (lane < 35) {
+	// the wave's segments (runs of one slot) from a ballot of their first entries, four FP64 partial sums
+	// per segment
+	const bool first = lane < cnt && (lane == 0 || S.sl[lane] != S.sl[lane - 1]);
+	unsigned long long starts = __ballot(first);
+	if (lane >= 35) return;
+	while (starts) {
+		const int b = __ffsll(starts) - 1;
+		starts &= starts - 1;
+		const int e = starts ? __ffsll(starts) - 1 : cnt;
 		double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-		int j = 0;
-		for (; j + 4 <= cnt; j += 4) {
+		int j = b;
+		for (; j + 4 <= e; j += 4) {
 			a0 += double(S.red[lane][j]);
 			a1 += double(S.red[lane][j + 1]);
 			a2 += double(S.red[lane][j + 2]);
 			a3 += double(S.red[lane][j + 3]);
 		}
-		for (; j < cnt; j++) a0 += double(S.red[lane][j]);
-		partial[35 * (size_t) blockIdx.x + lane] = (a0 + a1) + (a2 + a3);
+		for (; j < e; j++) a0 += double(S.red[lane][j]);
+		partial[35 * (size_t) S.sl[b] + lane] = (a0 + a1) + (a2 + a3);
 	}
-}
-
-template <bool FULL, bool TRACE>
-__device__ __forceinline__ void node_store(const float* L, float trace, int slot, int cnt, NodeSums<FULL>& S, double* partial) {
-	if constexpr (FULL)
-		node_full_store(L, slot, cnt, S, partial);
-	else
-		node_segment_store<TRACE>(L, trace, slot, cnt, S, partial);
 }
 
 __device__ __forceinline__ void multi_floats(float* v, const float4* m) {
@@ -654,7 +603,7 @@ __device__ __forceinline__ void multi_floats(float* v, const float4* m) {
 // 64 apart, each adding its entries' terms in order before the store.
 template <bool WRAP>
 __global__ __launch_bounds__(64) void k_cc(NodeArgs A) {
-	__shared__ NodeSums<true> sums;
+	__shared__ NodeSums sums;
 	const int2 wv = A.waves[blockIdx.x];
 	const int lane = threadIdx.x;
 	float L[35];
@@ -676,19 +625,19 @@ __global__ __launch_bounds__(64) void k_cc(NodeArgs A) {
 					sepu<WRAP>(X.z, __float_as_int(v[19])) * POS_INVF};
 			green_direct(D, x);
 			fold_multi(v, q, o, qzz);
-			m2l<true>(L, v[0], q, o, D);
+			m2l(L, v[0], q, o, D);
 		}
 	}
-	node_store<true, false>(L, 0.0f, slot, min(wv.y - wv.x, 64), sums, A.partial);
+	node_store(L, slot, min(wv.y - wv.x, 64), sums, A.partial);
 }
 
 // The same from a solver's folded multipoles, which the wave reads together: four lanes take a record,
 // so a load touches 16 half lines where a record per lane touches 64, and LDS hands each lane its own
 // (parts rotated so that neither side conflicts).  The next turn's records are on their way while this
 // turn's are evaluated; lanes past the end carry the last entry without weight.
-// Bound by FP32 arithmetic, about 175 instructions an entry (222 with 35 components, weights formed
-// per entry).  2M particles at theta 0.3 (3.3e8 entries here, 3.6e7 in the Ewald kind): the whole
-// solve 4.50 -> 4.12 ms; at theta 0.6 1.55 -> 1.50.
+// Bound by FP32 arithmetic: 1.37e9 wave instructions for 3.3e8 entries (2M particles at theta 0.3), 2.10 ->
+// 2.05 ms against records per lane with the weights formed per entry; at theta 0.6 (1.05e7 entries)
+// 0.210 -> 0.179 ms.
 template <bool WRAP>
 __global__ __launch_bounds__(64) void k_cc_folded(NodeArgs A) {
 	__shared__ NodeFoldLds lds;
@@ -748,29 +697,29 @@ __global__ __launch_bounds__(64) void k_cc_folded(NodeArgs A) {
 #pragma unroll
 				for (int c = 0; c < 13; c++) v[c] = 0.0f;
 			}
-			m2l<false>(L, v[0], v + 1, v + 6, D);
+			m2l(L, v[0], v + 1, v + 6, D);
 		}
 	}
 #undef TG_CC_INDICES
 #undef TG_CC_RECORDS
-	node_segment_store<false>(L, 0.0f, slot, min(wv.y - wv.x, 64), lds.sums, A.partial);
+	node_store(L, slot, min(wv.y - wv.x, 64), lds.sums, A.partial);
 }
 
 // The Ewald correction of the same: the whole wave takes every turn (its table rows are read
-// together), lanes past the end with the last entry and no weight.  Bound by arithmetic (about 700
-// instructions an entry, 900 before) and by the rows' way through the vector cache and LDS, 16 KB a
-// turn, at three waves a SIMD: 0.82 ms for 3.6e7 entries (2M particles at theta 0.3), 1.03 with a row per
-// lane and 35 sums; two waves with the next turn's rows in flight took an eighth longer.
-template <bool FULL>
+// together), lanes past the end with the last entry and no weight.  Its multipoles fold with the
+// Laplacian (error against FP64 no larger than unfolded).  Bound by arithmetic (4.0e8 wave
+// instructions for 3.6e7 entries, 5.2e8 with a row per lane and a 19-term sum per component) and by the
+// rows' way through the vector cache and LDS, 16 KB a turn, at three waves a SIMD: 0.86 ms (2M
+// particles at theta 0.3), 0.93 before; two waves with the next turn's rows in flight took an eighth
+// longer.
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_cc_ewald(NodeArgs A) {
-	__shared__ NodeLds<FULL> lds;
+	__shared__ NodeLds lds;
 	const int2 wv = A.waves[blockIdx.x];
 	const int lane = threadIdx.x;
 	float L[35];
 #pragma unroll
 	for (int c = 0; c < 35; c++) L[c] = 0.f;
 	int slot = -1;
-	float trace = 0.0f;
 	int4 X = make_int4(0, 0, 0, 0);
 	if (wv.x + lane < wv.y) {
 		slot = A.owner ? A.owner[wv.x + lane] : int(blockIdx.x);
@@ -786,24 +735,23 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
 		multi_floats(v, m);
 		const float x[3] = {sepu<true>(X.x, __float_as_int(v[17])) * POS_INVF, sepu<true>(X.y, __float_as_int(v[18])) * POS_INVF,
 				sepu<true>(X.z, __float_as_int(v[19])) * POS_INVF};
-		float D[35];
-		const float lap = green_ewald_wave<35>(D, x, c_ewt, lds.rows, lane);
 		if (j0 + 64 > wv.y && j0 + lane >= wv.y) {
 #pragma unroll
 			for (int c = 0; c < 17; c++) v[c] = 0.0f;
 		}
-		float q[5], o[7], qzz;
+		// folded before the tensor is evaluated: 14 weights to hold meanwhile instead of 17
+		float q[5], o[7], qzz, D[35];
 		fold_multi(v, q, o, qzz);
-		m2l<FULL>(L, v[0], q, o, D);
+		const float lap = green_ewald_wave<35>(D, x, c_ewt, lds.rows, lane);
 		L[0] = fmaf(qzz, lap, L[0]);
-		trace = fmaf(v[0], lap, trace);
+		m2l(L, v[0], q, o, D);
 	}
-	node_store<FULL, true>(L, trace, slot, min(wv.y - wv.x, 64), lds.sums, A.partial);
+	node_store(L, slot, min(wv.y - wv.x, 64), lds.sums, A.partial);
 }
 
-template <bool FULL, bool WRAP>
+template <bool WRAP>
 __global__ __launch_bounds__(64) void k_cp(NodeArgs A) {
-	__shared__ NodeSums<FULL> sums;
+	__shared__ NodeSums sums;
 	const int2 wv = A.waves[blockIdx.x];
 	const int lane = threadIdx.x;
 	float L[35];
@@ -819,22 +767,20 @@ __global__ __launch_bounds__(64) void k_cp(NodeArgs A) {
 			const float x[3] = {sepu<WRAP>(X.x, s.x) * POS_INVF, sepu<WRAP>(X.y, s.y) * POS_INVF, sepu<WRAP>(X.z, s.z) * POS_INVF};
 			float D[35];
 			green_direct(D, x);
-			p2l<FULL>(L, __int_as_float(s.w), D);
+			p2l(L, __int_as_float(s.w), D);
 		}
 	}
-	node_store<FULL, false>(L, 0.0f, slot, min(wv.y - wv.x, 64), sums, A.partial);
+	node_store(L, slot, min(wv.y - wv.x, 64), sums, A.partial);
 }
 
-template <bool FULL>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_cp_ewald(NodeArgs A) {
-	__shared__ NodeLds<FULL> lds;
+	__shared__ NodeLds lds;
 	const int2 wv = A.waves[blockIdx.x];
 	const int lane = threadIdx.x;
 	float L[35];
 #pragma unroll
 	for (int c = 0; c < 35; c++) L[c] = 0.f;
 	int slot = -1;
-	float trace = 0.0f;
 	int4 X = make_int4(0, 0, 0, 0);
 	if (wv.x + lane < wv.y) {
 		slot = A.owner ? A.owner[wv.x + lane] : int(blockIdx.x);
@@ -847,19 +793,16 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
 		float D[35];
 		const float lap = green_ewald_wave<35>(D, x, c_ewt, lds.rows, lane);
 		const float m = j0 + lane < wv.y ? __int_as_float(s.w) : 0.0f;
-		p2l<FULL>(L, m, D);
-		trace = fmaf(m, lap, trace);
+		p2l(L, m, D);
 	}
-	node_store<FULL, true>(L, trace, slot, min(wv.y - wv.x, 64), lds.sums, A.partial);
+	node_store(L, slot, min(wv.y - wv.x, 64), lds.sums, A.partial);
 }
 
 hipError_t launch_cc(const NodeArgs& a, bool ewald, hipStream_t s) {
 	if (a.nwaves <= 0) return hipSuccess;
 	const dim3 g(a.nwaves), b(64);
-	if (ewald && a.owner)
-		hipLaunchKernelGGL(k_cc_ewald<false>, g, b, 0, s, a);
-	else if (ewald)
-		hipLaunchKernelGGL(k_cc_ewald<true>, g, b, 0, s, a);
+	if (ewald)
+		hipLaunchKernelGGL(k_cc_ewald, g, b, 0, s, a);
 	else if (a.folded && a.wrap)
 		hipLaunchKernelGGL(k_cc_folded<true>, g, b, 0, s, a);
 	else if (a.folded)
@@ -889,23 +832,15 @@ hipError_t launch_fold_multis(const MultiSrc* multis, int64_t nn, FoldedMulti* o
 	return hipGetLastError();
 }
 
-template <bool FULL>
-static void cp_launch(const NodeArgs& a, bool ewald, hipStream_t s) {
-	const dim3 g(a.nwaves), b(64);
-	if (ewald)
-		hipLaunchKernelGGL(k_cp_ewald<FULL>, g, b, 0, s, a);
-	else if (a.wrap)
-		hipLaunchKernelGGL((k_cp<FULL, true>), g, b, 0, s, a);
-	else
-		hipLaunchKernelGGL((k_cp<FULL, false>), g, b, 0, s, a);
-}
-
 hipError_t launch_cp(const NodeArgs& a, bool ewald, hipStream_t s) {
 	if (a.nwaves <= 0) return hipSuccess;
-	if (a.owner)
-		cp_launch<false>(a, ewald, s);
+	const dim3 g(a.nwaves), b(64);
+	if (ewald)
+		hipLaunchKernelGGL(k_cp_ewald, g, b, 0, s, a);
+	else if (a.wrap)
+		hipLaunchKernelGGL(k_cp<true>, g, b, 0, s, a);
 	else
-		cp_launch<true>(a, ewald, s);
+		hipLaunchKernelGGL(k_cp<false>, g, b, 0, s, a);
 	return hipGetLastError();
 }
 

@@ -51,17 +51,6 @@ struct MultiSrc {
 	int32_t x[3];
 };
 
-// The node kinds' sums.  A direct term's tensor has no trace (derivatives of 1/r away from the origin)
-// and the periodic correction's has the constant Laplacian's, lap for D_zz and 0 above, so of the 35
-// components only the 25 without the third axis twice are summed, with the sum of the traces beside
-// them; the other ten follow from those at the end, in FP64.
-constexpr int NODE_SUMS = 26;
-constexpr int KEPT[25] = {0, 1, 2, 3, 4, 5, 6, 7, 8, 10, 11, 12, 13, 14, 16, 17, 20, 21, 22, 23, 24, 26, 27, 30, 31};
-__host__ __device__ constexpr bool kept(int slot) {
-	for (int k = 0; k < 25; k++)
-		if (KEPT[k] == slot) return true;
-	return false;
-}
 // A source multipole as M2L takes it: weights formed (multiplicities and 1/k!, the octupole's sign)
 // and the components with the third axis twice folded into the others by the trace relation, the
 // quadrupole in 5 terms and the octupole in 7.  64 bytes: half a line, where the plain 80 cross lines.
@@ -97,7 +86,7 @@ struct NodeArgs {
 	const int* list;         // source index per entry
 	const int* owner;        // partial slot per entry
 	const int* slot_node;    // expansion-centre index per slot
-	double* partial;         // NODE_SUMS doubles per slot; 35 without owners
+	double* partial;         // 35 doubles per slot
 	int nwaves;
 	int wrap;
 };

@@ -209,10 +209,8 @@ __device__ __forceinline__ void fold_multi(const float* M, float* q, float* o, f
 	o[6] = -M[14] * ef3(7) - ozz;
 }
 
-// M2L: L += contraction of a folded multipole with D, kept components (reference gravity.cpp:26-90).
-// Every term is added straight into L, in the reference's order of terms (as its loop adds each term
-// into its L).  FULL: all 35 components.
-template <bool FULL>
+// M2L: L += contraction of a folded multipole with D (reference gravity.cpp:26-90).  Every term is added
+// straight into L, in the reference's order of terms (as its loop adds each term into its L).
 __device__ __forceinline__ void m2l(float* L, float m, const float* q, const float* o, const float* D) {
 	constexpr int OS[7] = {0, 1, 2, 3, 4, 6, 7};  // octupole slots
 	auto quad = [&](auto slot_of, float acc) {
@@ -237,23 +235,20 @@ __device__ __forceinline__ void m2l(float* L, float m, const float* q, const flo
 		L[1 + a] = la;
 	}
 #pragma unroll
-	for (int t = 0; t < (FULL ? 6 : 5); t++) {
+	for (int t = 0; t < 6; t++) {
 		const int a = T2[t].i[0], b = T2[t].i[1];
 		float lab = fmaf(m, D[4 + t], L[4 + t]);
 		lab = quad([a, b](int s) { return E4(a, b, T2[s].i[0], T2[s].i[1]); }, lab);
 		L[4 + t] = lab;
 	}
 #pragma unroll
-	for (int s = 10; s < 35; s++)
-		if (FULL || kept(s)) L[s] = fmaf(m, D[s], L[s]);
+	for (int s = 10; s < 35; s++) L[s] = fmaf(m, D[s], L[s]);
 }
 
-// P2L: L += m D, kept components (reference gravity.cpp:92-121)
-template <bool FULL>
+// P2L: L += m D (reference gravity.cpp:92-121)
 __device__ __forceinline__ void p2l(float* L, float m, const float* D) {
 #pragma unroll
-	for (int s = 0; s < 35; s++)
-		if (FULL || kept(s)) L[s] = fmaf(m, D[s], L[s]);
+	for (int s = 0; s < 35; s++) L[s] = fmaf(m, D[s], L[s]);
 }
 
 // M2P: potential and acceleration at the sink (reference gravity.cpp:123-169).  The potential's

@@ -45,51 +45,17 @@ void DeviceArray::release() {
 
 // ---- kernels ---------------------------------------------------------------------------------
 // Each node's own CC/CP contribution: the sum of its partial slots in slot order (the
-// reference adds each list's accumulator into the node's L, src/tree.cpp:400-401,481-491), its 35
-// components from the 26 sums.  Half a wave per node, each four nodes at a time, 32 nodes a group: two
-// dependent loads a node and 258 MB at 529,000 nodes, so bound by memory with enough of them under way.
-constexpr int NODES_PER_SUM = 32;
+// reference adds each list's accumulator into the node's L, src/tree.cpp:400-401,481-491).
+// One thread per (node, coefficient); consecutive threads read consecutive doubles.
 __global__ __launch_bounds__(256) void k_node_sum(const int64_t* __restrict__ slot_ptr,
 		const double* __restrict__ partial, double* __restrict__ dL, int64_t nn) {
-	__shared__ double sums[NODES_PER_SUM][NODE_SUMS];
-	const int64_t a0 = int64_t(blockIdx.x) * NODES_PER_SUM;
-	const int h = int(threadIdx.x) >> 5, c = int(threadIdx.x) & 31;
-	int64_t b[4], e[4];
-	double acc[4];
-#pragma unroll
-	for (int u = 0; u < 4; u++) {
-		const int64_t a = a0 + h + 8 * u;
-		b[u] = a < nn ? slot_ptr[a] : 0;
-		e[u] = a < nn ? slot_ptr[a + 1] : 0;
-	}
-	if (c < NODE_SUMS) {
-		// the first slot of each, most often the only one
-#pragma unroll
-		for (int u = 0; u < 4; u++) acc[u] = b[u] < e[u] ? partial[NODE_SUMS * b[u] + c] : 0.0;
-#pragma unroll
-		for (int u = 0; u < 4; u++) {
-			for (int64_t z = b[u] + 1; z < e[u]; z++) acc[u] += partial[NODE_SUMS * z + c];
-			sums[h + 8 * u][c] = acc[u];
-		}
-	}
-	__syncthreads();
-	// kept components by the lanes that hold them, the ten that follow by lanes 0..9 (component TO from
-	// the sums FIRST and SECOND): minus both, plus the trace for zz; zzzz from xxzz and yyzz
-	constexpr int8_t FIRST[10] = {4, 9, 10, 11, 16, 17, 18, 19, 20, 16}, SECOND[10] = {7, 12, 14, 15, 19, 21, 22, 23, 24, 23};
-	constexpr int8_t TO[10] = {9, 15, 18, 19, 25, 28, 29, 32, 33, 34};
-	const int q = c < 9 ? c : c < 14 ? c + 1 : c < 16 ? c + 2 : c < 21 ? c + 4 : c < 23 ? c + 5 : c + 7;
-	const int f = c < 10 ? FIRST[c] : 0, g = c < 10 ? SECOND[c] : 0, to = c < 10 ? TO[c] : 0;
-#pragma unroll
-	for (int u = 0; u < 4; u++) {
-		const int64_t a = a0 + h + 8 * u;
-		if (a >= nn) continue;
-		const double* m = sums[h + 8 * u];
-		if (c < 25) dL[35 * a + q] = acc[u];
-		if (c < 10) {
-			const double two = -m[f] - m[g];
-			dL[35 * a + to] = c == 0 ? m[25] + two : c == 9 ? (m[16] + m[19]) + (m[19] + m[23]) : two;
-		}
-	}
+	const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+	if (i >= nn * 35) return;
+	const int64_t a = i / 35;
+	const int q = int(i - 35 * a);
+	double acc = 0.0;
+	for (int64_t z = slot_ptr[a]; z < slot_ptr[a + 1]; z++) acc += partial[35 * z + q];
+	dL[i] = acc;
 }
 
 // The local-expansion pass, LPG leaves per block of 64 (64 / LPG lanes each).  The shift of a
@@ -591,7 +557,7 @@ int Solver::upload() {
 		t_detail[4] = now() - tp0;  // preparation: the tree's arrays and the list work
 		t_detail[5] = 0.0;          // no transfers
 		(void) tp1;
-		SCHK(d_partial.alloc(std::max<size_t>(n_slots * NODE_SUMS * sizeof(double), 16)));
+		SCHK(d_partial.alloc(std::max<size_t>(n_slots * 35 * sizeof(double), 16)));
 		SCHK(d_dL.alloc(std::max<size_t>(size_t(n_nodes) * 35 * sizeof(double), 16)));
 		SCHK(d_out.alloc(std::max<size_t>(n * 4 * sizeof(double), 16)));
 		SCHK(hipStreamSynchronize(stream));
@@ -671,7 +637,7 @@ int Solver::upload() {
 		if (rc != TG_OK) return rc;
 		t_detail[5] = tp1 - tp0 - t_detail[4];  // transfers: the tree's arrays
 		t_detail[4] += now() - tp1;            // preparation: the tree's arrays (host), the list work (device)
-		SCHK(d_partial.alloc(std::max<size_t>(n_slots * NODE_SUMS * sizeof(double), 16)));
+		SCHK(d_partial.alloc(std::max<size_t>(n_slots * 35 * sizeof(double), 16)));
 		SCHK(d_dL.alloc(std::max<size_t>(T.nodes.size() * 35 * sizeof(double), 16)));
 		SCHK(d_out.alloc(std::max<size_t>(n * 4 * sizeof(double), 16)));
 		SCHK(hipStreamSynchronize(s));
@@ -728,7 +694,7 @@ int Solver::upload() {
 	t_detail[5] = now() - tp0 - t_detail[4];
 	if (rc != TG_OK) return rc;
 	SCHK(es);
-	SCHK(d_partial.alloc(std::max<size_t>(n_slots * NODE_SUMS * sizeof(double), 16)));
+	SCHK(d_partial.alloc(std::max<size_t>(n_slots * 35 * sizeof(double), 16)));
 	SCHK(d_dL.alloc(std::max<size_t>(T.nodes.size() * 35 * sizeof(double), 16)));
 	SCHK(d_out.alloc(std::max<size_t>(n * 4 * sizeof(double), 16)));
 	SCHK(hipStreamSynchronize(s));
@@ -796,7 +762,7 @@ int Solver::enqueue_solve(bool timed) {
 	SCHK(mark(e));
 	const bool local_pass = nn > 0 && n_leaf_items > 0;
 	if (local_pass) {
-		hipLaunchKernelGGL(k_node_sum, dim3(unsigned((nn + NODES_PER_SUM - 1) / NODES_PER_SUM)), dim3(256), 0, sn,
+		hipLaunchKernelGGL(k_node_sum, dim3(unsigned((nn * 35 + 255) / 256)), dim3(256), 0, sn,
 				d_node_slot_ptr.as<int64_t>(), d_partial.as<double>(), d_dL.as<double>(), nn);
 		SCHK(hipGetLastError());
 		if (local_sweep)
@@ -1241,6 +1207,7 @@ int64_t tg_solver_export(tg_solver* h, const char* name, void* dst, int64_t capa
 		else if (nm == "solve_level") { a = &S.d_level; bytes = nnd * 4; }
 		else if (nm == "solve_parent") { a = &S.d_parent; bytes = nnd * 4; }
 		else if (nm == "solve_leaf_items") { a = &S.d_leaf_items; bytes = size_t(S.n_leaf_items) * 16; }
+		else if (nm == "solve_expansions") { a = &S.d_dL; bytes = nnd * 35 * sizeof(double); }
 		else if (nm == "solve_path") { a = &S.d_path; bytes = size_t(S.path_len) * 4; }
 		else if (nm == "solve_pleaf") { a = &S.d_pleaf; bytes = n * 4; }
 		else if (nm == "solve_order") {
