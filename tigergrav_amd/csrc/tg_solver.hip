@@ -247,6 +247,9 @@ int Solver::init(int dev) {
 
 void Solver::drop_graph() {
 	if (graph_exec) {
+		// replays may be under way
+		(void) hipSetDevice(device);
+		(void) hipStreamSynchronize(stream);
 		(void) hipGraphExecDestroy(graph_exec);
 		graph_exec = nullptr;
 	}
