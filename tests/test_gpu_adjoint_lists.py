@@ -47,3 +47,34 @@ def test_adjoint_lists(make, n, ewald, theta, leaf):
     assert np.max(np.abs(g.cpu().numpy() - a)) <= 1e-9 * np.max(np.abs(a))
     dev.close()
     host.close()
+
+
+@pytest.mark.parametrize("device_lists", [0, 1])
+def test_out_of_memory_while_the_lists_are_made(device_lists):
+    """The first adjoint call of a tree that runs out of device memory, at every allocation it makes in
+    turn, reports it; the next call starts again and gives the gradients (1e-9, as above)."""
+    from tigergrav_amd._lib import TG_ENOMEM, ptr
+
+    x = ics.uniform(700, 3)
+    w = np.random.default_rng(3).standard_normal((700, 3)).astype(np.float32)
+    print(f"adjoint out of memory, device_lists={device_lists}", flush=True)
+    ref = _solver(x, None, True, 0.5, 8, device_lists)
+    want = ref.adjoint(w)
+    ref.close()
+    failed = 0
+    for k in range(200):
+        s = _solver(x, None, True, 0.5, 8, device_lists)
+        s.synchronize()
+        g = np.zeros((700, 4))
+        lib().tg_devmem_fail_after(k)
+        rc = lib().tg_solver_adjoint(s._h, ptr(w), ptr(g), None)
+        lib().tg_devmem_fail_after(-1)
+        assert rc in (0, TG_ENOMEM)
+        failed += rc == TG_ENOMEM
+        g = s.adjoint(w)
+        s.close()
+        for cols in (slice(0, 3), slice(3, 4)):
+            assert np.max(np.abs(g[:, cols] - want[:, cols])) <= 1e-9 * np.max(np.abs(want[:, cols]))
+        if rc == 0:
+            break
+    assert rc == 0 and failed > 20

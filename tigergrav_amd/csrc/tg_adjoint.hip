@@ -1019,21 +1019,27 @@ int Solver::adjoint_lists() {
 				err = "adjoint: the interaction lists do not belong to this tree";
 				return TG_EINVAL;
 			}
-		dlists.release();
-		dlists.nn = nn;
+		// built aside and taken whole: after an error the next call starts again
+		struct Fresh : DeviceLists {
+			~Fresh() { release(); }
+		} fresh;
+		fresh.nn = nn;
 		hvec<WalkNode> wn(static_cast<size_t>(nn));
 		walk_nodes(tree, wn.data());
-		ACHK(dev_malloc(&dlists.nodes, size_t(nn) * sizeof(WalkNode)));
-		ACHK(hipMemcpyAsync(dlists.nodes, wn.data(), size_t(nn) * sizeof(WalkNode), hipMemcpyHostToDevice, s));
-		ACHK(dev_malloc(&dlists.ptr_all, size_t(8 * (nn + 1)) * 8));
+		ACHK(dev_malloc(&fresh.nodes, size_t(nn) * sizeof(WalkNode)));
+		ACHK(dev_malloc(&fresh.ptr_all, size_t(8 * (nn + 1)) * 8));
 		for (int k = 0; k < 8; k++) {
-			dlists.len[k] = int64_t(vals[k]->size());
-			ACHK(hipMemcpyAsync(dlists.ptr_all + int64_t(k) * (nn + 1), ptrs[k]->data(), size_t(nn + 1) * 8, hipMemcpyHostToDevice, s));
-			ACHK(dev_malloc(&dlists.val[k], std::max<size_t>(size_t(dlists.len[k]) * 4, 16)));
-			if (dlists.len[k] > 0)
-				ACHK(hipMemcpyAsync(dlists.val[k], vals[k]->data(), size_t(dlists.len[k]) * 4, hipMemcpyHostToDevice, s));
+			fresh.len[k] = int64_t(vals[k]->size());
+			ACHK(dev_malloc(&fresh.val[k], std::max<size_t>(size_t(fresh.len[k]) * 4, 16)));
+		}
+		ACHK(hipMemcpyAsync(fresh.nodes, wn.data(), size_t(nn) * sizeof(WalkNode), hipMemcpyHostToDevice, s));
+		for (int k = 0; k < 8; k++) {
+			ACHK(hipMemcpyAsync(fresh.ptr_all + int64_t(k) * (nn + 1), ptrs[k]->data(), size_t(nn + 1) * 8, hipMemcpyHostToDevice, s));
+			if (fresh.len[k] > 0) ACHK(hipMemcpyAsync(fresh.val[k], vals[k]->data(), size_t(fresh.len[k]) * 4, hipMemcpyHostToDevice, s));
 		}
 		ACHK(hipStreamSynchronize(s));
+		dlists.release();
+		std::swap(dlists, static_cast<DeviceLists&>(fresh));
 	}
 	const int sink_bits = bits_of(nn), src_bits = bits_of(std::max(nn, n + 1));
 	const int key_bits = sink_bits + src_bits;

@@ -28,10 +28,15 @@ size_t size_class(size_t b) {
 	return (b + step - 1) / step * step;
 }
 
+thread_local int g_fail_in = -1;  // allocations of this thread until one fails on purpose; -1: none
+
 }  // namespace
+
+void dev_fail_after(int count) { g_fail_in = count; }
 
 hipError_t dev_malloc(void** p, size_t bytes) {
 	*p = nullptr;
+	if (g_fail_in >= 0 && g_fail_in-- == 0) return hipErrorOutOfMemory;
 	int device = 0;
 	hipError_t e = hipGetDevice(&device);
 	if (e != hipSuccess) return e;
@@ -107,3 +112,6 @@ size_t dev_trim(int device) {
 }
 
 }  // namespace tg
+
+// the error paths' tests (no header declares it)
+extern "C" void tg_devmem_fail_after(int count) { tg::dev_fail_after(count); }

@@ -19,6 +19,9 @@ template <class T>
 hipError_t dev_malloc(T** p, size_t bytes) {
 	return dev_malloc(reinterpret_cast<void**>(p), bytes);
 }
+// lets this thread's allocation after the next count ones fail with hipErrorOutOfMemory, once (-1: none
+// does): the error paths' tests
+void dev_fail_after(int count);
 // back to the cache (null: nothing)
 void dev_free(void* p);
 // frees every cached block of `device` (blocks in use stay); returns the bytes freed
