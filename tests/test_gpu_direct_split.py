@@ -23,3 +23,18 @@ def test_direct_split(n, ns, h, ewald):
     phi, g = ob.direct64(ewald, h, x[sinks], x, np.full(n, 1.0 / n))
     assert np.linalg.norm(f[:, 1:] - g) < 1e-10 * np.linalg.norm(g)
     assert np.all(np.abs(f[:, 0] - phi) <= (1e-7 / n if ewald else 0.0) + 1e-10 * np.abs(phi))
+
+
+@pytest.mark.parametrize("ewald", [True, False], ids=["periodic", "open"])
+def test_more_sinks_than_a_launch_has_blocks(ewald):
+    """2^24 + 5 sinks: a block of 256 threads each would pass a launch's 2^32 threads.  The sinks repeat
+    the few particles, and so do the forces (1e-12: the pair sums' order depends on the sink count)."""
+    from tigergrav_amd.accuracy import direct_forces
+
+    n, ns = 7, 2 ** 24 + 5
+    x = ics.uniform(n, seed=n)
+    print(f"direct split ns={ns} ewald={ewald}", flush=True)
+    few = direct_forces(x, np.arange(n), ewald, 1e-3, 1.0 / n)
+    f = direct_forces(x, np.arange(ns) % n, ewald, 1e-3, 1.0 / n)
+    for i in range(n):
+        assert np.abs(f[i::n] - few[i]).max() <= 1e-12 * np.abs(few[i]).max()

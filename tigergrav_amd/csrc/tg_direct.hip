@@ -303,62 +303,65 @@ __global__ __launch_bounds__(64) void k_pairs(const int* __restrict__ x, const f
 	}
 }
 
-// Per sink (one block): pair partials, then the Fourier part over the octant vectors, thread by
+// Per sink (a block each at a time): pair partials, then the Fourier part over the octant vectors, thread by
 // thread, and the constant.  With K = exp(-pi^2 h^2 / alpha^2) / h^2 and every sign of (a, b, c) distinct
 // (half for each zero component), phi = -(8 / pi) sum K C_x C_y C_z, where C = cos_i cos_j + sin_i sin_j per axis;
 // the gradient along an axis takes k (cos_i sin_j - sin_i cos_j) there.
-__global__ __launch_bounds__(256) void k_finish(const int* __restrict__ x, const int64_t* __restrict__ sinks, int chunks,
+constexpr int64_t kFinishBlocks = 1 << 20;  // a launch takes fewer than 2^32 threads
+__global__ __launch_bounds__(256) void k_finish(const int* __restrict__ x, const int64_t* __restrict__ sinks, int64_t ns, int chunks,
 		const double* __restrict__ part, int ewald, const int4* __restrict__ tasks, const double* __restrict__ cs, int nt,
 		double mtot, double* __restrict__ out) {
 	__shared__ double2 tab[3][kTab];
 	__shared__ double red[4][256];
-	const int64_t si = blockIdx.x;
 	const int t = threadIdx.x;
-	double v[4] = {0.0, 0.0, 0.0, 0.0};
-	for (int c = t; c < chunks; c += 256)
-		for (int q = 0; q < 4; q++) v[q] += part[4 * (si * chunks + c) + q];
-	if (ewald) {
-		if (t < 3 * kTab) {
-			const int axis = t / kTab, k = t % kTab;
-			double2 w = make_double2(0.0, 0.0);
-			if (k <= kHF) sincospi(2.0 * k * (double(x[3 * sinks[si] + axis]) * kPosInv + 0.5), &w.y, &w.x);
-			tab[axis][k] = w;
+	for (int64_t si = blockIdx.x; si < ns; si += gridDim.x) {
+		__syncthreads();  // the last sink's tables and sums are read
+		double v[4] = {0.0, 0.0, 0.0, 0.0};
+		for (int c = t; c < chunks; c += 256)
+			for (int q = 0; q < 4; q++) v[q] += part[4 * (si * chunks + c) + q];
+		if (ewald) {
+			if (t < 3 * kTab) {
+				const int axis = t / kTab, k = t % kTab;
+				double2 w = make_double2(0.0, 0.0);
+				if (k <= kHF) sincospi(2.0 * k * (double(x[3 * sinks[si] + axis]) * kPosInv + 0.5), &w.y, &w.x);
+				tab[axis][k] = w;
+			}
+			__syncthreads();
+			const double pi = 3.141592653589793;
+			for (int j = t; j < nt * kZG; j += 256) {
+				const int4 task = tasks[j / kZG];
+				const int a = task.x, b = task.y, c = kZG * task.z + j % kZG;
+				const int h2 = a * a + b * b + c * c;
+				if (h2 == 0 || h2 > kHF2) continue;
+				const double K = exp(-pi * pi / (kAlphaF * kAlphaF) * h2) / h2 * (a ? 2.0 : 1.0) * (b ? 2.0 : 1.0) * (c ? 2.0 : 1.0);
+				const double2 X = tab[0][a], Y = tab[1][b], Z = tab[2][c];
+				const double* T = cs + int64_t(j) * 8;  // (cos, sin) of x, y, z from the highest bit down
+				// contract z, then y, then x: P with C, Q with the derivative's sine
+				double Pz[4], Qz[4], PP[2], QP[2], PQ[2];
+				for (int q = 0; q < 4; q++) {
+					Pz[q] = Z.x * T[2 * q] + Z.y * T[2 * q + 1];
+					Qz[q] = Z.x * T[2 * q + 1] - Z.y * T[2 * q];
+				}
+				for (int q = 0; q < 2; q++) {
+					PP[q] = Y.x * Pz[2 * q] + Y.y * Pz[2 * q + 1];
+					QP[q] = Y.x * Pz[2 * q + 1] - Y.y * Pz[2 * q];
+					PQ[q] = Y.x * Qz[2 * q] + Y.y * Qz[2 * q + 1];
+				}
+				v[0] -= K / pi * (X.x * PP[0] + X.y * PP[1]);
+				v[1] += 2.0 * K * a * (X.x * PP[1] - X.y * PP[0]);
+				v[2] += 2.0 * K * b * (X.x * QP[0] + X.y * QP[1]);
+				v[3] += 2.0 * K * c * (X.x * PQ[0] + X.y * PQ[1]);
+			}
+		}
+		for (int q = 0; q < 4; q++) red[q][t] = v[q];
+		for (int o = 128; o > 0; o >>= 1) {
+			__syncthreads();
+			if (t < o)
+				for (int q = 0; q < 4; q++) red[q][t] += red[q][t + o];
 		}
 		__syncthreads();
-		const double pi = 3.141592653589793;
-		for (int j = t; j < nt * kZG; j += 256) {
-			const int4 task = tasks[j / kZG];
-			const int a = task.x, b = task.y, c = kZG * task.z + j % kZG;
-			const int h2 = a * a + b * b + c * c;
-			if (h2 == 0 || h2 > kHF2) continue;
-			const double K = exp(-pi * pi / (kAlphaF * kAlphaF) * h2) / h2 * (a ? 2.0 : 1.0) * (b ? 2.0 : 1.0) * (c ? 2.0 : 1.0);
-			const double2 X = tab[0][a], Y = tab[1][b], Z = tab[2][c];
-			const double* T = cs + int64_t(j) * 8;  // (cos, sin) of x, y, z from the highest bit down
-			// contract z, then y, then x: P with C, Q with the derivative's sine
-			double Pz[4], Qz[4], PP[2], QP[2], PQ[2];
-			for (int q = 0; q < 4; q++) {
-				Pz[q] = Z.x * T[2 * q] + Z.y * T[2 * q + 1];
-				Qz[q] = Z.x * T[2 * q + 1] - Z.y * T[2 * q];
-			}
-			for (int q = 0; q < 2; q++) {
-				PP[q] = Y.x * Pz[2 * q] + Y.y * Pz[2 * q + 1];
-				QP[q] = Y.x * Pz[2 * q + 1] - Y.y * Pz[2 * q];
-				PQ[q] = Y.x * Qz[2 * q] + Y.y * Qz[2 * q + 1];
-			}
-			v[0] -= K / pi * (X.x * PP[0] + X.y * PP[1]);
-			v[1] += 2.0 * K * a * (X.x * PP[1] - X.y * PP[0]);
-			v[2] += 2.0 * K * b * (X.x * QP[0] + X.y * QP[1]);
-			v[3] += 2.0 * K * c * (X.x * PQ[0] + X.y * PQ[1]);
-		}
+		if (t < 4) out[4 * si + t] = red[t][0] + (t == 0 && ewald ? mtot * 3.141592653589793 / (kAlphaF * kAlphaF) : 0.0);
 	}
-	for (int q = 0; q < 4; q++) red[q][t] = v[q];
-	for (int o = 128; o > 0; o >>= 1) {
-		__syncthreads();
-		if (t < o)
-			for (int q = 0; q < 4; q++) red[q][t] += red[q][t + o];
-	}
-	__syncthreads();
-	if (t < 4) out[4 * si + t] = red[t][0] + (t == 0 && ewald ? mtot * 3.141592653589793 / (kAlphaF * kAlphaF) : 0.0);
 }
 
 // gradient: structure factors C, S (mass weighted) and Cw, Sw (weight weighted), 8 per h
@@ -545,7 +548,6 @@ extern "C" int tg_direct_forces(const tg_params* prm, const int32_t* x, const fl
 	while (lanes < 64 && lanes < ns) lanes *= 2;
 	const int64_t sblocks = (ns + lanes - 1) / lanes;
 	const int src_chunks = int(std::max<int64_t>(1, std::min<int64_t>((16384 + sblocks - 1) / sblocks, n / 512)));
-	if (sblocks > INT32_MAX || ns > INT32_MAX) return TG_EINVAL;
 	Buf dx, dm, ds, dh, dsf, dcs, dpart, dout;
 	hipStream_t st = nullptr;
 	int rc = TG_OK;
@@ -592,8 +594,8 @@ extern "C" int tg_direct_forces(const tg_params* prm, const int32_t* x, const fl
 					static_cast<double*>(dpart.p));
 		DCHK(hipGetLastError());
 		DCHK(hipMalloc(&dout.p, size_t(ns) * 32));
-		hipLaunchKernelGGL(k_finish, dim3(unsigned(ns)), dim3(256), 0, st, static_cast<const int*>(dx.p),
-				static_cast<const int64_t*>(ds.p), src_chunks, static_cast<const double*>(dpart.p), ewald, static_cast<const int4*>(dh.p),
+		hipLaunchKernelGGL(k_finish, dim3(unsigned(std::min(ns, kFinishBlocks))), dim3(256), 0, st, static_cast<const int*>(dx.p),
+				static_cast<const int64_t*>(ds.p), ns, src_chunks, static_cast<const double*>(dpart.p), ewald, static_cast<const int4*>(dh.p),
 				static_cast<const double*>(dcs.p), nt, mtot, static_cast<double*>(dout.p));
 		DCHK(hipGetLastError());
 		DCHK(hipMemcpyAsync(out, dout.p, size_t(ns) * 32, hipMemcpyDeviceToHost, st));
