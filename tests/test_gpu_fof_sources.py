@@ -77,3 +77,25 @@ def test_fof_after_update(n, leaf, link, move, gpu_tree):
     ids, counts = np.unique(want[want != NONE], return_counts=True)
     assert ng == len(ids) and ng > 0
     assert [(c.id, c.N) for c in _catalog(s, np.zeros((n, 3), np.float32), 1.0, 2)] == list(zip(ids.tolist(), counts.tolist()))
+
+
+def test_fof_more_pairs_than_a_launch_takes():
+    """A clump of 11,700 single-particle leaves within the linking length of each other, 6.8e7 candidate
+    pairs and so more than 2^32 threads of 64 a pair, and a tighter one whose pairs, deepest in the tree,
+    come last."""
+    from tigergrav_amd.solver import Solver
+
+    rng = np.random.default_rng(1)
+    wide, tight = 11700, 60
+    x = np.concatenate([rng.integers(-2 ** 24, 2 ** 24, (wide, 3)), 2 ** 30 + rng.integers(-2 ** 8, 2 ** 8, (tight, 3))]).astype(np.int32)
+    n = wide + tight
+    link = 2.0 ** 26 / 2.0 ** 32 * n ** (1.0 / 3.0)
+    print(f"fof many pairs: N={n}", flush=True)
+    s = Solver(ewald=False, soft_len=ics.soft_len(n), m=1.0 / n, theta=0.7, parts_per_node=1, device=0)
+    s.set_particles(x)
+    g, ng = _groups(s, link)
+    assert ng == 2
+    order = s.export("order")
+    want = np.full(n, np.min(np.flatnonzero(order < wide)), np.uint64)
+    want[order >= wide] = np.min(np.flatnonzero(order >= wide))
+    assert np.array_equal(g[order], want)

@@ -192,6 +192,7 @@ __device__ __forceinline__ bool within(const Reach& r, const int4& x) {
 // cluster most links join particles already in one set, which a parent equal to the last root shows
 // without a walk.  Bound by its chains of loads (pair, node, particles, parents): 2M clustered
 // particles, leaves of 32, 2.46 -> 1.28 ms against every pair of two leaves tested in turn.
+constexpr int64_t LINK_PAIRS = 1 << 25;  // of a launch, which takes fewer than 2^32 threads
 __global__ __launch_bounds__(64) void k_fof_link(const FofNode* __restrict__ nodes, const int2* __restrict__ pairs, int64_t npairs,
 		const int4* __restrict__ parts, double Lb, uint64_t L2, int* parent, int* linked) {
 	__shared__ int4 sa[64], sb[64];
@@ -369,15 +370,16 @@ hipError_t fof_device(const FofSource& F, double link_len, hipStream_t s, uint64
 		return hipErrorInvalidValue;
 	}
 	if (npairs > int64_t(INT32_MAX)) {
-		err = "friends-of-friends: more candidate leaf pairs than one launch takes";
+		err = "friends-of-friends: more than 2^31 candidate leaf pairs";
 		return hipErrorInvalidValue;
 	}
 	FCHK(scratch.get(&pairs, size_t(npairs)));
 	hipLaunchKernelGGL(k_fof_candidates, dim3(lb), dim3(128), 0, s, nodes, F.leaf_items, nleaves, Lb * Lb, int(periodic), 1, count, offset, pairs,
 			overflow);
 	FCHK(hipGetLastError());
-	if (npairs > 0) {
-		hipLaunchKernelGGL(k_fof_link, dim3(unsigned(npairs)), dim3(64), 0, s, nodes, pairs, npairs, F.parts, Lb, L2, parent, linked);
+	for (int64_t q0 = 0; q0 < npairs; q0 += LINK_PAIRS) {
+		const int64_t m = std::min(npairs - q0, LINK_PAIRS);
+		hipLaunchKernelGGL(k_fof_link, dim3(unsigned(m)), dim3(64), 0, s, nodes, pairs + q0, m, F.parts, Lb, L2, parent, linked);
 		FCHK(hipGetLastError());
 	}
 	hipLaunchKernelGGL(k_fof_labels, dim3(pb), dim3(256), 0, s, parent, linked, F.order, n, group_tree, gin,
