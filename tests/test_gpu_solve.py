@@ -248,6 +248,32 @@ def test_graph_replay_matches_eager():
             np.testing.assert_array_equal(s.forces(), eager2)
 
 
+def test_solvers_give_their_memory_back():
+    """Solvers made, solved and closed one after the other leave as much device memory free as before (4
+    bytes a particle, and what the runtime keeps of its own); every buffer that a solve, the forces, an
+    adjoint and a group search make is among them."""
+    import torch
+
+    from tigergrav_amd import ics
+    from tigergrav_amd.solver import Solver
+
+    n, free = 400000, []
+    x, w = ics.uniform(n, 8), np.ones((n, 3), np.float32)
+    print(f"solver memory: N={n}", flush=True)
+    for k in range(8):
+        s = Solver(ewald=False, soft_len=ics.soft_len(n), m=1.0 / n, theta=0.8, parts_per_node=64, device=0)
+        s.set_particles(x)
+        s.solve()
+        s.forces()
+        s.adjoint(w)
+        s.find_groups(0.2)
+        s.close()
+        torch.cuda.synchronize()
+        free.append(torch.cuda.mem_get_info(0)[0])
+    print("  free MiB:", [f >> 20 for f in free], flush=True)
+    assert free[2] - free[7] < 5 * 4 * n
+
+
 def test_overlap_knob_is_bit_identical():
     """Graph replays with the node kinds on a second stream ("overlap" 1, the default), with the
     Ewald node kinds on a third ("overlap" 2) and on one stream give the eager solve's forces bit

@@ -299,6 +299,8 @@ Solver::~Solver() {
 		d_folded.release();
 		d_nodepos.release();
 		d_out.release();
+		d_order.release();
+		d_fin.release();
 		d_partial.release();
 		d_node_slot_ptr.release();
 		d_dL.release();
