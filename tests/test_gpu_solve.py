@@ -265,6 +265,8 @@ def test_solvers_give_their_memory_back():
         s.set_particles(x)
         s.solve()
         s.forces()
+        s.solve_graph()
+        s.synchronize()
         s.adjoint(w)
         s.find_groups(0.2)
         s.close()

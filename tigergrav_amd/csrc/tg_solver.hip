@@ -193,9 +193,16 @@ __global__ __launch_bounds__(256) void k_pp_near_all(int4* __restrict__ items, i
 	if (i < n) items[i].y = pp_item_y(items[i].y & PP_COUNT_MASK, PP_NEAR_ALL);
 }
 
-__global__ __launch_bounds__(256) void k_zero_f64(double* __restrict__ p, int64_t n) {
+// The array's pointer goes inside a struct: as an argument of its own, the first kernel of a captured
+// solve kept the array allocated after the graph and the array were gone (32 bytes a particle for every
+// solver that replayed).
+struct ZeroArgs {
+	double* p;
+	int64_t n;
+};
+__global__ __launch_bounds__(256) void k_zero_f64(ZeroArgs A) {
 	const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
-	if (i < n) p[i] = 0.0;
+	if (i < A.n) A.p[i] = 0.0;
 }
 
 static size_t local_lds_bytes(int maxdepth) { return size_t(LOCAL_LPG) * size_t(35 * maxdepth + 35) * sizeof(double); }
@@ -780,7 +787,7 @@ int Solver::enqueue_solve(bool timed) {
 	}
 	if (n > 0) {
 		// a kernel, not a memset, so the launch sequence stays graph-safe
-		hipLaunchKernelGGL(k_zero_f64, dim3(unsigned((4 * n + 255) / 256)), dim3(256), 0, s, d_out.as<double>(), int64_t(4 * n));
+		hipLaunchKernelGGL(k_zero_f64, dim3(unsigned((4 * n + 255) / 256)), dim3(256), 0, s, ZeroArgs{d_out.as<double>(), int64_t(4 * n)});
 		SCHK(hipGetLastError());
 	}
 	SCHK(mark(e + 1));
