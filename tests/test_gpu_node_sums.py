@@ -86,3 +86,26 @@ def test_expansions(n, theta, leaf, ewald):
         for lo, hi in ((4, 10), (10, 20), (20, 35)):
             assert np.abs(got[a, lo:hi] - L[lo:hi]).max() <= 1e-11 * np.abs(L[lo:hi]).max(), (a, lo)
     assert entries > n  # the lists are not empty
+
+
+@pytest.mark.parametrize("make,n,leaf,theta,slot", [("uniform", 3000, 64, 0.5, 256), ("plummer_spheres", 40000, 32, 0.6, 512),
+                                                    ("uniform", 100000, 8, 0.8, 4096), ("plummer_spheres", 150000, 64, 0.7, 512)])
+def test_slot_sizes(make, n, leaf, theta, slot):
+    """Without the knob the slots' size follows the number of nodes (and so of lists), not of particles: each
+    node's slots are its lists cut into runs of that many entries."""
+    from tigergrav_amd import ics
+    from tigergrav_amd.solver import Solver
+
+    s = Solver(ewald=True, soft_len=ics.soft_len(n), m=1.0 / n, theta=theta, parts_per_node=leaf, device=0)
+    s.set_particles(getattr(ics, make)(n, 3))
+    nn = s.info()["n_nodes"]
+    print(f"slot sizes {make} n={n} nodes={nn}", flush=True)
+    assert slot == (256 if nn <= 2048 else 512 if nn <= 32768 else 4096)
+    want = np.zeros(nn, np.int64)
+    for name in ("cc_d", "cp_d", "cc_e", "cp_e"):
+        v, p = s.export(name), s.export(name + "_ptr")
+        each = np.ones(len(v), np.int64) if name[1] == "c" else np.repeat(v[1::2] - v[::2], 2)
+        each = np.concatenate([[0], np.cumsum(each)])
+        entries = (each[p[1:]] - each[p[:-1]]) // (1 if name[1] == "c" else 2)
+        want += (entries + slot - 1) // slot
+    assert np.array_equal(np.diff(s.export("slot_ptr").view(np.int64)), want)

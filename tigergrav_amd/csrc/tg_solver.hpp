@@ -45,11 +45,14 @@ struct Solver {
 	double soft_len = 0.0, m = 0.0, theta = 0.7;
 	int parts_per_node = 64;
 	bool uniform_mass = true;
-	int node_chunk = 0;  // sources per CC/CP partial slot (<= NODE_CHUNK_MAX); 0: by the set's size; from the next set_particles
-	// One wave takes a slot's sources, so a slot holds a whole list where the lists are enough waves; sets
-	// of up to 131,072 have a few hundred nodes with particle lists of a thousand (32,768 particles, leaves
-	// of 64: 464 of 1,095, 65 us against 17 us in slots of 256)
-	int chunk_of() const { return node_chunk > 0 ? node_chunk : n <= 131072 ? 256 : 4096; }
+	int node_chunk = 0;  // sources per CC/CP partial slot (<= NODE_CHUNK_MAX); 0: by the tree's size; from the next set_particles
+	// One wave takes a slot's sources, so a slot holds a whole list where the lists are enough waves; trees
+	// of few nodes have few lists, of up to thousands of particles.  Node kinds and their sums, eager,
+	// in slots of 256 / 512 / 4096: 1,491 nodes (32,768 uniform particles, leaves of 64) 68 / 75 / 119 us;
+	// 3,289 (65,536 Plummer) 107 / 101 / 203; 12,181 (262,144 Plummer) 186 / 175 / 263; 24,253 (131,072
+	// Plummer, leaves of 16) 267 / 243 / 290; 24,053 (524,288 uniform) 156 / 147 / 145; 43,343 (1,000,000
+	// uniform) 208 / 191 / 185, and replayed 36,119 (100,000 uniform, leaves of 8) 290 / 296 / 276
+	int chunk_of() const { return node_chunk > 0 ? node_chunk : n_nodes <= 2048 ? 256 : n_nodes <= 32768 ? 512 : 4096; }
 	bool pp_persistent = false;  // PP direct as a persistent queue-driven kernel
 	// graph replays: 0 one stream; 1 the node kinds on a second stream beside the leaf kinds; 2 as 1,
 	// with the Ewald node kinds on a third stream beside the direct ones
