@@ -65,7 +65,7 @@ int tg_solver_adjoint(tg_solver* s, const float* w, double* grad, double* ms);
 int tg_solver_solve(tg_solver* s);
 /* tuning knobs (no reference counterpart): "pp_persistent" 0/1 runs PP direct as a persistent
  * queue-driven kernel; "node_chunk" 1..4096 (4096: a whole list) sources per CC/CP partial slot (applies from the next
- * tg_solver_set_particles; unset: 256 for up to 2,048 nodes, 512 for up to 32,768, else 4096); "resident" work groups of the persistent form; "local_sweep" 1 runs the
+ * tg_solver_set_particles; unset: 256 for up to 2,048 nodes, 512 for up to 32,768, else 4096); "resident" waves of the persistent form (at least one work group); "local_sweep" 1 runs the
  * local-expansion pass level by level (the reference's order, src/tree.cpp:400-401) instead of
  * per-leaf sums over the root path (0, the default; tg_solver_solve_graph enqueues the former
  * without a graph); "gpu_walk" 1 (the default

@@ -297,8 +297,8 @@ __global__ __launch_bounds__(64 * NW) void k_pp_direct(LeafArgs A) {
 	pp_item<NW, WRAP, PHI, UNIFORM>(A, A.items[blockIdx.x], S);
 }
 
-// persistent form: as many work groups as the machine keeps resident, each taking the next
-// item from a queue counter (A.queue, zero at launch) until the items run out
+// persistent form: work groups of as many waves in all as the machine keeps resident, each taking the
+// next item from a queue counter (A.queue, zero at launch) until the items run out
 template <int NW, bool WRAP, bool PHI, bool UNIFORM>
 __global__ __launch_bounds__(64 * NW) void k_pp_direct_queue(LeafArgs A) {
 	__shared__ PPShared S[NW];
@@ -322,7 +322,8 @@ static void pp_launch(const LeafArgs& a, hipStream_t s) {
 	if (a.queue) {
 		// the counter is cleared by a kernel (not a memset) so the launch sequence stays graph-safe
 		hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, s, a.queue);
-		const int groups = a.nitems < a.resident ? a.nitems : a.resident;
+		const int most = a.resident > NW ? a.resident / NW : 1;
+		const int groups = a.nitems < most ? a.nitems : most;
 		hipLaunchKernelGGL((k_pp_direct_queue<NW, WRAP, PHI, UNIFORM>), dim3(groups), dim3(64 * NW), 0, s, a);
 	} else {
 		hipLaunchKernelGGL((k_pp_direct<NW, WRAP, PHI, UNIFORM>), dim3(a.nitems), dim3(64 * NW), 0, s, a);

@@ -74,7 +74,7 @@ struct LeafArgs {
 	float m;                 // the common mass when uniform
 	float h2u, hinvu, hinv3u;  // softening in position units (2^32 per box length)
 	int* queue;              // PP direct: work counter of the persistent form (NULL: one group per item)
-	int resident;            // PP direct persistent form: work groups to launch
+	int resident;            // PP direct persistent form: waves to launch, in groups of those that share an item
 };
 
 struct NodeArgs {

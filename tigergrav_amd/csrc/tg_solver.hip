@@ -246,7 +246,7 @@ int Solver::init(int dev) {
 	SCHK(d_queue.alloc(256));
 	int cus = 0;
 	SCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-	resident_groups = cus * 4 * 6;  // six 64-lane work groups per SIMD
+	resident_waves = cus * 4 * 6;  // six per SIMD
 	ev.resize(size_t(2) * TIMER_EVSPANS * TIMER_RING);
 	for (auto& e : ev) SCHK(hipEventCreate(&e));
 	return TG_OK;
@@ -806,7 +806,7 @@ int Solver::enqueue_solve(bool timed) {
 	const int leaf_kinds[4] = {PC_DIRECT, PP_DIRECT, PC_EWALD, PP_EWALD};
 	for (int k : leaf_kinds) {
 		la.queue = (k == PP_DIRECT && pp_persistent) ? d_queue.as<int>() : nullptr;
-		la.resident = resident_groups;
+		la.resident = resident_waves;
 		la.items = work[k].items.as<int4>();
 		la.list = work[k].list.as<int>();
 		la.nitems = work[k].nitems;
@@ -1053,7 +1053,7 @@ int tg_solver_tune(tg_solver* h, const char* knob, int value) {
 		S.node_chunk = value;
 	} else if (k == "resident") {
 		if (value < 1) return TG_EINVAL;
-		S.resident_groups = value;
+		S.resident_waves = value;
 	} else if (k == "overlap") {
 		if (value < 0 || value > 2) return TG_EINVAL;
 		S.overlap = value;

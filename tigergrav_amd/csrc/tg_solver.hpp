@@ -63,7 +63,7 @@ struct Solver {
 	bool gpu_walk = false;       // build the interaction lists on the device (device_walk); on for device solvers
 	WalkHint walk_hint;          // the buffer sizes the last device walk reached: the next one starts there
 	bool gpu_tree = false;       // build the tree and multipoles on the device (device_build_tree); on for device solvers
-	int resident_groups = 1024;  // work groups of the persistent form (set from the CU count)
+	int resident_waves = 1024;  // waves of the persistent form (set from the CU count)
 	Tree tree;
 	int64_t n = 0;
 	// device state

@@ -132,7 +132,7 @@ class Solver:
 
     def tune(self, knob, value):
         """Set a tuning knob: "pp_persistent" (0/1), "node_chunk" (1..4096, from the next
-        set_particles), "resident" (work groups of the persistent PP kernel)."""
+        set_particles), "resident" (waves of the persistent PP kernel)."""
         _check(lib().tg_solver_tune(self._h, knob.encode(), int(value)), "tg_solver_tune")
 
     def solve_graph(self):
