@@ -11,7 +11,8 @@ kernel form, the form of the local pass and the stream overlap are autotuned on 
 own graph-replay time, among the leaf sizes whose error on the same FP64 sample meets the bound
 (the leaf size moves the error too: smaller leaves turn near pairs into multipole interactions);
 --leaf N with --node-chunk/--pp-persistent/--local-sweep/--overlap fixes them instead.  The timed
-steps replay the solve from a captured HIP graph.  A second leg, `theta07`, times the same particles at
+steps replay the solve from a captured HIP graph (the level-by-level local pass is enqueued without
+one).  A second leg, `theta07`, times the same particles at
 theta = 0.7 (the workload's specified angle; about 10x faster, with RMS error ~0.15, which does not
 meet 1e-3).
 
@@ -468,7 +469,8 @@ def main():
                    "local_sweep": best.get("local_sweep"), "overlap": best.get("overlap"), "accumulation": "f64",
                    "parallelism": "single GPU"},
         "s_per_force_solve": ms / 1e3,
-        "step": "eager solves" if args.no_graph else "HIP-graph replays",
+        "step": "eager solves" if args.no_graph else
+                "solves enqueued without a graph (level-by-level local pass)" if best.get("local_sweep") else "HIP-graph replays",
         "ms_per_step_eager": ms_eager,
         "s_per_force_solve_end_to_end": None,  # filled below from the rebuilds
         "build_s": None,

@@ -59,6 +59,9 @@ int tg_solver_update_particles(tg_solver* s, const int32_t* x, const float* mass
  * (dL/dx, dL/dy, dL/dz, dL/dm) in input order, positions in box units -- the derivatives of the
  * solve with its tree, lists and expansion centres held fixed (see tg_solver_update_particles).
  * Interactions are recomputed from the stored lists.  Needs leaves of at most 64 particles.
+ * w and grad may be host memory or memory of the solver's device; the solver's stream waits for no
+ * other, so what other streams do with the latter must have ended.  The call returns when grad is
+ * written.
  * *ms, if not NULL, receives the device time of the adjoint kernels. */
 int tg_solver_adjoint(tg_solver* s, const float* w, double* grad, double* ms);
 /* enqueue one force solve on the solver's stream (replaces tree::kick_fmm's kernel calls) */
@@ -72,7 +75,7 @@ int tg_solver_solve(tg_solver* s);
  * for device solvers) builds the interaction lists on the device, 0 on the host (the same lists
  * either way: the walk of kick_fmm, src/tree.cpp:378-635; from the next tg_solver_set_particles);
  * with the lists on the device, the work of every kind is built from them there and the host
- * receives a copy only when something asks for it (tg_solver_export, the adjoint);
+ * receives a copy only when something asks for it (tg_solver_export);
  * "gpu_tree" 1 (the default for device solvers) builds the tree and multipoles on the device, 0 on
  * the host (the same tree bit for bit; from the next tg_solver_set_particles);
  * "overlap" 1 (the default) lets graph replays run the node kinds on a second stream beside the
@@ -81,7 +84,7 @@ int tg_solver_solve(tg_solver* s);
 int tg_solver_tune(tg_solver* s, const char* knob, int value);
 /* the same solve replayed from a HIP graph captured on its first call after set_particles (one
  * submission instead of 11 or more launches; records no per-kind timings; with "overlap" the node and
- * leaf kinds run concurrently) */
+ * leaf kinds run concurrently; "local_sweep" 1 is enqueued without a graph) */
 int tg_solver_solve_graph(tg_solver* s);
 int tg_solver_synchronize(tg_solver* s);
 /* forces of the last solve, in input particle order (the reference's `force` per particle) */

@@ -498,8 +498,6 @@ __global__ __launch_bounds__(64 * NW) void k_adj_pc_sink(AdjArgs A, AdjItems I) 
 	T.store(0.0, dx, red, A.grad);
 }
 
-// PC, source side: lane = multipole of the item's list, over the item's sinks (staged in LDS):
-// mu_c += dg/dM_c^T w (fourth derivatives), one FP64 atomic per slot and entry
 // PC source side by source node: mu_c += sum over the sinks i of every leaf whose PC list holds c of
 // dg_i/dM_c^T w_i.  One work group per item (node c, a run of at most 16 sink leaves); the lanes
 // cover 64 / L leaves at a time, L = 2^lgL lanes per leaf (L >= the largest leaf), one sink each;

@@ -136,7 +136,8 @@ class Solver:
         _check(lib().tg_solver_tune(self._h, knob.encode(), int(value)), "tg_solver_tune")
 
     def solve_graph(self):
-        """The same solve replayed from a captured HIP graph (no per-kind timings)."""
+        """The same solve replayed from a captured HIP graph (no per-kind timings); with "local_sweep" it
+        is enqueued without one."""
         _check(lib().tg_solver_solve_graph(self._h), "tg_solver_solve_graph")
 
     def synchronize(self):
