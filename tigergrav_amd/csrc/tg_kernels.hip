@@ -545,7 +545,7 @@ hipError_t launch_pp_ewald(const LeafArgs& a, hipStream_t s) {
 // of one slot are consecutive: lanes 0..34 add one coefficient each over every segment.
 // All 35 components are summed, though the tensor's trace is known (zero for derivatives of 1/r, a
 // constant for the periodic correction): one taken from two others carries their errors, up to 1.8
-// times its own against FP64.  Ten sums fewer took 0.1 ms off the 4.2 ms solve of 2M particles at
+// times its own against FP64.  Ten sums fewer took 0.2 ms off the 4.35 ms solve of 2M particles at
 // theta 0.3.
 struct NodeSums {
 	float red[35][65];
@@ -710,7 +710,7 @@ __global__ __launch_bounds__(64) void k_cc_folded(NodeArgs A) {
 // together), lanes past the end with the last entry and no weight.  Its multipoles fold with the
 // Laplacian (error against FP64 no larger than unfolded).  Bound by arithmetic (4.0e8 wave
 // instructions for 3.6e7 entries, 5.2e8 with a row per lane and a 19-term sum per component) and by the
-// rows' way through the vector cache and LDS, 16 KB a turn, at three waves a SIMD: 0.86 ms (2M
+// rows' way through the vector cache and LDS, 16 KB a turn, at three waves a SIMD: 0.78 ms (2M
 // particles at theta 0.3), 0.93 before; two waves with the next turn's rows in flight took an eighth
 // longer.
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_cc_ewald(NodeArgs A) {
@@ -740,12 +740,28 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
 #pragma unroll
 			for (int c = 0; c < 17; c++) v[c] = 0.0f;
 		}
-		// folded before the tensor is evaluated: 14 weights to hold meanwhile instead of 17
 		float q[5], o[7], qzz, D[35];
 		fold_multi(v, q, o, qzz);
-		const float lap = green_ewald_wave<35>(D, x, c_ewt, lds.rows, lane);
-		L[0] = fmaf(qzz, lap, L[0]);
-		m2l(L, v[0], q, o, D);
+		const EwtPoint p = ewt_point(x);
+		EwtRows<35> rows;
+		rows.fetch(p.row, c_ewt, lds.rows, lane);
+		float c[EwtRead<35>::F4 * 4];
+		rows.take(c, lds.rows, lane);
+		// the folded weights wait in LDS while the tensor is evaluated: in registers they are seven too many
+		// for three waves a SIMD, which the compiler keeps in scratch memory (0.86 ms)
+		ewt_f4* wait = lds.rows.part;
+		EwtRows<35>::settle();
+		wait[lane] = ewt_f4{v[0], q[0], q[1], q[2]};
+		wait[64 + lane] = ewt_f4{q[3], q[4], o[0], o[1]};
+		wait[128 + lane] = ewt_f4{o[2], o[3], o[4], o[5]};
+		wait[192 + lane] = ewt_f4{o[6], qzz, 0.0f, 0.0f};
+		EwtRows<35>::settle();
+		ewt_eval<35>(D, c, p);
+		EwtRows<35>::settle();
+		const ewt_f4 w0 = wait[lane], w1 = wait[64 + lane], w2 = wait[128 + lane], w3 = wait[192 + lane];
+		const float qw[5] = {w0.y, w0.z, w0.w, w1.x, w1.y}, ow[7] = {w1.z, w1.w, w2.x, w2.y, w2.z, w2.w, w3.x};
+		L[0] = fmaf(w3.y, p.lap, L[0]);
+		m2l(L, w0.x, qw, ow, D);
 	}
 	node_store(L, slot, min(wv.y - wv.x, 64), lds.sums, A.partial);
 }
