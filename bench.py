@@ -1,20 +1,22 @@
 """Benchmark: periodic force solve of 2,097,152 particles on one MI355X.
 
-    python bench.py [--steps K] [--warmup W] [--workload zeldovich128] [--theta 0.3] [--leaf 0] [--no-graph]
+    python bench.py [--steps K] [--warmup W] [--workload zeldovich128] [--theta 0.3] [--leaf 8] [--no-graph]
 
 Workload (default): 128^3 particles displaced by a Zel'dovich field of a seeded Gaussian random
 field with P(k) ~ k^-2 (cut at the grid Nyquist), rms displacement 0.3 cell, periodic (Ewald),
 softening 0.02 N^(-1/3), equal masses 1/N.  The timed solve runs at theta = 0.3: the largest
 opening angle whose force error meets RMS |da|/|a| <= 1e-3 against the FP64 direct sum on this
-workload (the `accuracy` field shows it).  The leaf size (8/16/32/64/128), the CC/CP chunk, the PP
-kernel form, the form of the local pass and the stream overlap are autotuned on this workload's
-own graph-replay time, among the leaf sizes whose error on the same FP64 sample meets the bound
-(the leaf size moves the error too: smaller leaves turn near pairs into multipole interactions);
---leaf N with --node-chunk/--pp-persistent/--local-sweep/--overlap fixes them instead.  The timed
-steps replay the solve from a captured HIP graph (the level-by-level local pass is enqueued without
-one).  A second leg, `theta07`, times the same particles at
-theta = 0.7 (the workload's specified angle; about 10x faster, with RMS error ~0.15, which does not
-meet 1e-3).
+workload (the `accuracy` field shows it).  It runs leaves of 8 and the solver's defaults for the rest
+(within a few percent of what the autotuner finds on this workload); --leaf N with
+--node-chunk/--pp-persistent/--local-sweep/--overlap fixes others.  --leaf 0 searches: the leaf size
+(8/16/32/64/128), the CC/CP chunk, the PP kernel form, the form of the local pass and the stream
+overlap, on this workload's own graph-replay time, among the leaf sizes whose error on the same FP64
+sample meets the bound (the leaf size moves the error too: smaller leaves turn near pairs into
+multipole interactions).  The search is not the default: a default run with it once stopped without
+a message, for a cause that is not known.  The timed steps replay the solve from a captured HIP graph
+(the level-by-level local pass is enqueued without one).  A second leg, `theta07`, times the same
+particles at theta = 0.7 with leaves of 32 (the workload's specified angle; about 3x faster, with RMS
+error ~0.15, which does not meet 1e-3).  Each part's start is a line on stderr.
 
 One step = one force solve on the device over the resident tree and interaction lists: the CC/CP
 node kernels, the local-expansion pass (reduce + L2L + L2P) and the PC/PP leaf kernels.  The tree,
@@ -24,8 +26,7 @@ state of a time step; `s_per_force_solve_end_to_end` is that rebuild plus one so
 particles to forces).  Per-kind kernel times (and the
 roofline) come from HIP events on the solver's stream around each kind's kernels, over K eager
 solves run right after the graph-replayed ones (a captured graph carries no timers).
-`profile_cmd` is the command that reruns the timed configuration with its knobs fixed, under
-which the committed profiler summaries of the dominant kernel were taken.
+`profile_cmd` is a short command that reruns the timed configuration with its knobs fixed.
 
 Prints one JSON line.  `value` is interactions per second (the reference's interaction census,
 src/tree.cpp:483-494,618-628, divided by the device time of one solve).
@@ -223,6 +224,11 @@ def build_solver(x, ewald, h, m, theta, leaf, leaves, knobs, host_walk=False, ac
     return s, best, table, time.time() - t0
 
 
+def stage(what):
+    """A part of the run begins: a line on stderr (stdout holds the JSON line only)."""
+    print(f"bench.py: {what}", file=sys.stderr, flush=True)
+
+
 def build_times(info, total):
     """A build's wall time (s) with its parts: tree, multipoles, interaction lists, upload and the
     finer split of the last two (walk set-up, steps, assembly, census; work preparation, transfers)."""
@@ -256,8 +262,8 @@ def time_solves(s, steps, warmup, graph):
 
 
 def profile_command(workload, theta, best, steps=3):
-    """The bench command that reruns exactly this configuration with every knob fixed (what the
-    committed rocprofv3 summaries of the dominant kernel were taken from)."""
+    """The bench command that reruns exactly this configuration with every knob fixed, short enough
+    for a profiler."""
     cmd = f"python3 bench.py --workload {workload} --theta {theta} --leaf {best['leaf']}"
     for k, flag in (("node_chunk", "--node-chunk"), ("pp_persistent", "--pp-persistent"), ("local_sweep", "--local-sweep"),
                     ("overlap", "--overlap")):
@@ -379,7 +385,7 @@ def main():
     ap.add_argument("--workload", default="zeldovich128")
     ap.add_argument("--theta", type=float, default=0.3,
                     help="opening angle of the timed solve (0.3: the largest that meets RMS 1e-3 on the 2M workload)")
-    ap.add_argument("--leaf", type=int, default=0,
+    ap.add_argument("--leaf", type=int, default=8,
                     help="particles per leaf; 0 autotunes leaf (8, 16, 32, 64, 128), CC/CP chunk, PP kernel form and "
                          "local pass")
     ap.add_argument("--wide-autotune", action="store_true", help="autotune over leaves of 4, 12, 24 and 48 as well")
@@ -430,6 +436,7 @@ def main():
     from tigergrav_amd import ics
     from tigergrav_amd.accuracy import direct_forces
 
+    stage(f"particles of {args.workload}")
     x, ewald, desc = make_workload(args.workload)
     N = x.shape[0]
     h, m = ics.soft_len(N), 1.0 / N
@@ -442,6 +449,7 @@ def main():
     # sample of sinks; the autotuner keeps the leaf sizes that meet the bound on it
     ns = min(N, args.accuracy_sample)
     sinks = np.sort(np.random.default_rng(7).choice(N, ns, replace=False)) if ns < N else np.arange(N)
+    stage(f"FP64 direct sum, {ns} sinks")
     t0 = time.perf_counter()
     fref = direct_forces(x, sinks, ewald, h, m)
     t_ref = time.perf_counter() - t0
@@ -451,12 +459,14 @@ def main():
             rms = accuracy_of(solver.forces(), sinks, fref, ns)["rms"]
             return rms <= args.max_rms, {"rms": rms, "bound": args.max_rms}
     free0 = device_free_bytes()
+    stage(f"solver, theta {args.theta:g}, leaf {args.leaf or 'searched'}")
     s, best, tuning, t_host = build_solver(x, ewald, h, m, args.theta, args.leaf, leaves, knobs, args.host_walk, accept)
     info = s.info()
     count = info["count"]
     total = sum(count.values())
     graph = not args.no_graph
     # timed region: K solves back to back on the resident data (graph replays by default)
+    stage("timed solves")
     ms, ms_eager, kms = time_solves(s, args.steps, args.warmup, graph)
     value = total / (ms / 1e3)
 
@@ -480,6 +490,7 @@ def main():
         "profile_cmd": profile_command(args.workload, args.theta, best),
     }
     # force accuracy of the timed solve against the reference above
+    stage("forces and rebuilds")
     f = s.forces()
     # end to end: host particles to forces.  The first build on a fresh solver allocates its device
     # buffers; a time step rebuilds on the same solver, so the steady state is the median of three
@@ -502,15 +513,19 @@ def main():
     # after the forward, and after the adjoint's buffers are added
     fp = {"forward_bytes": free0 - device_free_bytes()}
     if args.adjoint:
+        stage("adjoint")
         out["adjoint"] = adjoint_leg(s, x, ewald, h, m, ms, args.steps) if best["leaf"] <= 64 else {
             "skipped": "the adjoint handles leaves of at most 64 particles"}
         fp["forward_plus_adjoint_bytes"] = free0 - device_free_bytes()
     fp["method"] = "hipMemGetInfo difference from before the solver was created (the accuracy checks free their buffers)"
     out["hbm_footprint"] = fp
     if not args.no_step:
+        stage("kick and drift")
         out["step"] = step_leg(s, x, h, m, ewald)
+        stage("friends-of-friends")
         out["fof"] = fof_leg()
     if not args.no_cpu:
+        stage("CPU baseline")
         out["cpu_baseline"], f_cpu = cpu_baseline(s, ewald, h, m, args.theta, best["leaf"])
         if f_cpu is not None:
             # the same solve done on the host by the CPU baseline: its error on the same sample
@@ -518,9 +533,10 @@ def main():
     s.close()
     if not args.no_theta07 and args.workload == "zeldovich128" and abs(args.theta - 0.7) > 1e-9:
         # the workload's specified opening angle, 0.7: faster, but its error is the reference
-        # algorithm's own truncation on near-lattice forces, far above 1e-3 (autotuned on the
-        # workload's leaf set 32/64/128, timed the same way, same accuracy sample)
-        s7, best7, _, t7 = build_solver(x, ewald, h, m, 0.7, 0, (32, 64, 128), knobs)
+        # algorithm's own truncation on near-lattice forces, far above 1e-3 (leaves of 32, or with
+        # --leaf 0 autotuned on 32/64/128; timed the same way, same accuracy sample)
+        stage("theta 0.7")
+        s7, best7, _, t7 = build_solver(x, ewald, h, m, 0.7, 32 if args.leaf else 0, (32, 64, 128), knobs)
         ms7, _, kms7 = time_solves(s7, args.steps, args.warmup, graph)
         c7 = s7.info()["count"]
         out["theta07"] = {"theta": 0.7, "best": best7, "ms_per_solve": ms7,

@@ -2,10 +2,11 @@
 longer than 64 entries are one wave each, its lanes adding several entries), the PP-direct kernel
 form (one work group per item, or persistent queue-driven), the form of the local-expansion pass
 (per-leaf path sums, or level by level) and whether graph replays run the node kinds on a second
-stream.  The criterion is the time per solve of tg_solver_solve_graph on the caller's own particle set
-(replays; level by level, solves enqueued without a graph: what the benchmark measures: with the node kinds beside the leaf kinds, so the sum of per-kind
-kernel times would misjudge it), among the leaf sizes an optional acceptance test passes (the
-leaf size and the opening angle set the force error; the other knobs do not)."""
+stream.  The criterion is the time per solve of tg_solver_solve_graph on the caller's own particle set:
+replays, or for the level-by-level form solves enqueued without a graph.  (The node kinds run beside
+the leaf kinds there, so the sum of per-kind kernel times would misjudge it.)  Only leaf sizes that an
+optional acceptance test passes are timed (the leaf size and the opening angle set the force error; the
+other knobs do not)."""
 import itertools
 import time
 
